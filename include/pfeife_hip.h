@@ -84,7 +84,7 @@ int pf_graph_destroy(void* graph_exec);
  *   C[m*ldc+n] = v  (stored as c_dtype)
  * bias/aux/residual require batch1*batch2 == 1.
  *
- * in_dtype PF_F16/PF_BF16 run on v_mfma_f32_32x32x16 with fp32 accumulation;
+ * in_dtype PF_F16/PF_BF16 run on v_mfma_f32_16x16x32 / 32x32x16 with fp32 accumulation;
  * in_dtype PF_F32 runs a full-precision fp32 FMA kernel (the fp32 parity path).
  * 16-bit products whose operands are both reduction-contiguous (a_trans = b_trans = 0,
  * K a multiple of 64) or both reduction-strided (a_trans = b_trans = 1) take the
@@ -131,8 +131,8 @@ typedef struct pf_gemm_desc {
                       harnesses): 1..4 direct-to-LDS kernel with 256x256 / 256x128 / 128x128 /
                       192x256 tiles shared by four wavefronts, 5 / 6 its 128x128 / 256x128 tiles
                       with eight wavefronts as two grids that split each tile step's reduction
-                      depth, 7 / 8 / 9 its 256x256 / 128x128 / 256x128 tiles with eight
-                      wavefronts side by side, 11..14 register-staged kernel with 128x128 (8 wavefronts),
+                      depth, 7 / 8 / 9 / 10 its 256x256 / 128x128 / 256x128 / 192x256 tiles
+                      with eight wavefronts side by side, 11..14 register-staged kernel with 128x128 (8 wavefronts),
                       128x128, 128x64, 64x64 tiles; PF_ERR_INVALID if it cannot run the problem */
   float* colsum_ws; /* optional, with dact on the direct-to-LDS kernel (pf_gemm_variant ends in ", 5>"): the
                        launch also leaves the column sums of the 16-bit values it stores in C as partial

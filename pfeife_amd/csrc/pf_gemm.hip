@@ -20,15 +20,15 @@
   int pf_gemm_x_##DT##_##XT(const pf_gemm_desc& d, hipStream_t st);    \
   int pf_gemm_xgroup_##DT##_##XT(const pf_gemm_desc* d, int n, hipStream_t st);
 #define PF_X_DECL_DT(DT) \
-  PF_X_DECL(DT, 1) PF_X_DECL(DT, 2) PF_X_DECL(DT, 3) PF_X_DECL(DT, 4) PF_X_DECL(DT, 5) PF_X_DECL(DT, 6) PF_X_DECL(DT, 7) PF_X_DECL(DT, 8) PF_X_DECL(DT, 9)
+  PF_X_DECL(DT, 1) PF_X_DECL(DT, 2) PF_X_DECL(DT, 3) PF_X_DECL(DT, 4) PF_X_DECL(DT, 5) PF_X_DECL(DT, 6) PF_X_DECL(DT, 7) PF_X_DECL(DT, 8) PF_X_DECL(DT, 9) PF_X_DECL(DT, 10)
 PF_X_DECL_DT(1)
 PF_X_DECL_DT(2)
 #undef PF_X_DECL_DT
 #undef PF_X_DECL
-static_assert(PF_F16 == 1 && PF_BF16 == 2 && PF_XT_COUNT == 10, "the table below is written out for these ids");
+static_assert(PF_F16 == 1 && PF_BF16 == 2 && PF_XT_COUNT == 11, "the table below is written out for these ids");
 typedef int (*pf_x_fn)(const pf_gemm_desc&, hipStream_t);
 typedef int (*pf_xgroup_fn)(const pf_gemm_desc*, int, hipStream_t);
-#define PF_X_ROW(P, DT) {nullptr, P##DT##_1, P##DT##_2, P##DT##_3, P##DT##_4, P##DT##_5, P##DT##_6, P##DT##_7, P##DT##_8, P##DT##_9}
+#define PF_X_ROW(P, DT) {nullptr, P##DT##_1, P##DT##_2, P##DT##_3, P##DT##_4, P##DT##_5, P##DT##_6, P##DT##_7, P##DT##_8, P##DT##_9, P##DT##_10}
 static const pf_x_fn pf_x_table[3][PF_XT_COUNT] = {{}, PF_X_ROW(pf_gemm_x_, 1), PF_X_ROW(pf_gemm_x_, 2)};
 static const pf_xgroup_fn pf_xgroup_table[3][PF_XT_COUNT] = {{}, PF_X_ROW(pf_gemm_xgroup_, 1), PF_X_ROW(pf_gemm_xgroup_, 2)};
 #undef PF_X_ROW
@@ -616,12 +616,12 @@ int launch16(const pf_gemm_desc& d, hipStream_t st) {
 }
 
 // Variant ids (pf_gemm_desc.variant; 0 = automatic):
-//   1..9   direct-to-LDS kernel, tiles PF_XT_256x256 / 256x128 / 128x128 / 192x256 / 128x128k2 / 256x128k2 /
-//          256x256w8 / 128x128w8 / 256x128w8
+//   1..10  direct-to-LDS kernel, tiles PF_XT_256x256 / 256x128 / 128x128 / 192x256 / 128x128k2 / 256x128k2 /
+//          256x256w8 / 128x128w8 / 256x128w8 / 192x256w8
 //   11..14 register-staged kernel: 128x128 by 8 wavefronts, 128x128, 128x64, 64x64 by 4
-enum { V_AUTO = 0, V_X256 = 1, V_X256x128 = 2, V_X128 = 3, V_X192x256 = 4, V_X128K2 = 5, V_X256x128K2 = 6, V_X256W8 = 7, V_X128W8 = 8, V_X256x128W8 = 9,
+enum { V_AUTO = 0, V_X256 = 1, V_X256x128 = 2, V_X128 = 3, V_X192x256 = 4, V_X128K2 = 5, V_X256x128K2 = 6, V_X256W8 = 7, V_X128W8 = 8, V_X256x128W8 = 9, V_X192x256W8 = 10,
        V_R128W8 = 11, V_R128 = 12, V_R128x64 = 13, V_R64 = 14 };
-inline bool is_x_variant(int v) { return v >= V_X256 && v <= V_X256x128W8; }
+inline bool is_x_variant(int v) { return v >= V_X256 && v <= V_X192x256W8; }
 
 // Register-staged tiles: 128x128 with two workgroups resident per CU is the largest that keeps
 // accumulators, two sets of staging registers and fragments in the register file; smaller tiles
@@ -643,7 +643,7 @@ int choose_staged(const pf_gemm_desc& d) {
 // hardware range check only in the second case (whole k-rows fall outside the operand).
 bool x_supports(const pf_gemm_desc& d, int xt) {
   const int bk = x_tile_bk(xt);
-  if (xt == PF_XT_192x256 && d.a_trans) return false;   // no reduction-strided 192-row tile
+  if ((xt == PF_XT_192x256 || xt == PF_XT_192x256w8) && d.a_trans) return false;   // no reduction-strided 192-row tile
   if (d.a_trans != d.b_trans) return false;
   if (!d.a_trans && d.K % bk != 0) return false;
   return d.K >= bk;
@@ -669,7 +669,7 @@ int choose_variant(const pf_gemm_desc& d) {
   if (d.M < 128 || d.N < 128 || d.M * d.N < 128 * 128 * 16) return choose_staged(d);
   struct Cand { int v, xt, bm, bn; double t64, t64_busy, fixed; };
   static const Cand cands[4] = {{V_X256W8, PF_XT_256x256w8, 256, 256, 1.20, 1.20, 8.0},
-                                {V_X192x256, PF_XT_192x256, 192, 256, 1.05, 1.05, 8.0},
+                                {V_X192x256W8, PF_XT_192x256w8, 192, 256, 1.05, 1.05, 8.0},
                                 {V_X256x128W8, PF_XT_256x128w8, 256, 128, 0.70, 0.70, 8.0},
                                 {V_X128W8, PF_XT_128x128w8, 128, 128, 0.45, 0.55, 8.0}};
   int best = -1;
@@ -719,14 +719,14 @@ int dispatch16(const pf_gemm_desc& d, hipStream_t st) {
   if (d.nonfinite_flag != nullptr) {   // only the fp32 classes of the direct-to-LDS kernel check what they write
     const int ec = epi_class(d, epi_vec_ok(d));
     if (!is_x_variant(v) || !x_supports(d, v) || (ec != EC_STORE32 && ec != EC_ACC32) ||
-        (d.a_trans != d.b_trans)) {
+        (d.a_trans != d.b_trans) || (d.a_trans && d.bias != nullptr)) {
       pf_set_error("pf_gemm: nonfinite_flag needs a 16-bit product with fp32 C (stored or accumulated) on the direct-to-LDS kernel");
       return PF_ERR_UNSUPPORTED;
     }
   }
   switch (v) {
-    case V_X256: case V_X256x128: case V_X128: case V_X192x256: case V_X128K2: case V_X256x128K2: case V_X256W8: case V_X128W8: case V_X256x128W8: {
-      const int xt = v;   // variant ids 1..9 are the PF_XT_* tile ids
+    case V_X256: case V_X256x128: case V_X128: case V_X192x256: case V_X128K2: case V_X256x128K2: case V_X256W8: case V_X128W8: case V_X256x128W8: case V_X192x256W8: {
+      const int xt = v;   // variant ids 1..10 are the PF_XT_* tile ids
       if (!x_supports(d, xt)) {
         pf_set_error("pf_gemm: variant %d needs both operands stored alike and (unless transposed) K a multiple of the stage depth", v);
         return PF_ERR_INVALID;
@@ -853,7 +853,7 @@ bool groupable(const pf_gemm_desc& d, int& variant) {
   const int64_t a_bytes = (d.K + 256) * d.lda * 2, b_bytes = (d.K + 256) * d.ldb * 2;
   if (a_bytes >= (1ll << 31) || b_bytes >= (1ll << 31)) return false;
   variant = resolve_variant(d);
-  if (!is_x_variant(variant) || variant == V_X192x256) return false;
+  if (!is_x_variant(variant)) return false;
   if (!x_supports(d, variant)) return false;
   // (a product that stores rides in the accumulate launch: its old C reads as zeros)
   const int ec = epi_class(d, epi_vec_ok(d));
@@ -907,18 +907,19 @@ extern "C" int pf_gemm_variant(const pf_gemm_desc* desc, char* out, int cap) {
   const char* bt = d.b_trans ? "true" : "false";
   const int v = resolve_variant(d);
   switch (v) {
-    case V_X256: case V_X256x128: case V_X128: case V_X192x256: case V_X128K2: case V_X256x128K2: case V_X256W8: case V_X128W8: case V_X256x128W8: {
+    case V_X256: case V_X256x128: case V_X128: case V_X192x256: case V_X128K2: case V_X256x128K2: case V_X256W8: case V_X128W8: case V_X256x128W8: case V_X192x256W8: {
       // BM, BN, BK, wavefront rows, columns, reduction split, stages: as rocprofv3 prints the instantiation
       static const char* shapes[PF_XT_COUNT] = {"", "256, 256, 32, 2, 2, 1, 5", "256, 128, 64, 2, 2, 1, 3", "128, 128, 64, 2, 2, 1, 3",
                                                 "192, 256, 32, 2, 2, 1, 5", "128, 128, 64, 2, 2, 2, 3", "256, 128, 64, 2, 2, 2, 3",
-                                                "256, 256, 32, 2, 4, 1, 5", "128, 128, 64, 2, 4, 1, 3", "256, 128, 64, 4, 2, 1, 3"};
+                                                "256, 256, 32, 2, 4, 1, 5", "128, 128, 64, 2, 4, 1, 3", "256, 128, 64, 4, 2, 1, 3",
+                                                "192, 256, 32, 2, 4, 1, 5"};
       if (!x_supports(d, v)) {   // a pinned tile that cannot run this product: say so here, not at launch time
         pf_set_error("pf_gemm_variant: variant %d needs both operands stored alike, K >= %d and (unless both are "
                      "reduction-strided) K a multiple of %d", v, x_tile_bk(v), x_tile_bk(v));
         return PF_ERR_INVALID;
       }
       int ec = epi_class(d, epi_vec_ok(d));
-      if (d.a_trans && ec != EC_ACC32 && ec != EC_STORE32) ec = EC_GENERIC;
+      if (d.a_trans && ((ec != EC_ACC32 && ec != EC_STORE32) || d.bias != nullptr)) ec = EC_GENERIC;
       snprintf(out, (size_t)cap, "gemm16x_kernel<%d, %s, %s, %s, %d>", d.in_dtype, shapes[v], at, bt, ec);
       return PF_OK;
     }

@@ -140,8 +140,8 @@ __device__ __forceinline__ void static_for(F&& f) {
 
 template <int DT> struct Mfma;
 template <> struct Mfma<PF_F16> {
-  static __device__ __forceinline__ float16_t run8(short __attribute__((ext_vector_type(8))) a, short __attribute__((ext_vector_type(8))) b, float16_t c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), c, 0, 0, 0);
+  static __device__ __forceinline__ float4_t run16(short __attribute__((ext_vector_type(8))) a, short __attribute__((ext_vector_type(8))) b, float4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), c, 0, 0, 0);
   }
   static __device__ __forceinline__ float16_t run(uint4 a, uint4 b, float16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), c, 0,
@@ -149,8 +149,8 @@ template <> struct Mfma<PF_F16> {
   }
 };
 template <> struct Mfma<PF_BF16> {
-  static __device__ __forceinline__ float16_t run8(short __attribute__((ext_vector_type(8))) a, short __attribute__((ext_vector_type(8))) b, float16_t c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+  static __device__ __forceinline__ float4_t run16(short __attribute__((ext_vector_type(8))) a, short __attribute__((ext_vector_type(8))) b, float4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
   }
   static __device__ __forceinline__ float16_t run(uint4 a, uint4 b, float16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c,
@@ -181,11 +181,11 @@ __device__ __forceinline__ uint4 buf_load16(__amdgpu_buffer_rsrc_t r, uint32_t b
 //   256x256 (32 deep, 5 stages): one 128x128 block per wavefront, the least operand traffic per FLOP
 //   256x128 (64 deep, 3 stages), 128x128 (64 deep, 3 stages): more workgroups for smaller outputs
 //   192x256 (32 deep, 5 stages): for outputs that 256-row blocks cover badly
-//   ids 1-4: four wavefronts (2 x 2); ids 7-9: the same tiles shared by EIGHT wavefronts (2 x 4,
+//   ids 1-4: four wavefronts (2 x 2); ids 7-10: the same tiles shared by EIGHT wavefronts (2 x 4 or 4 x 2,
 //   two per SIMD); ids 5, 6: 128x128 and 256x128 with eight wavefronts as TWO 2 x 2 grids that
 //   split every tile's reduction depth between them ("k2")
 enum { PF_XT_256x256 = 1, PF_XT_256x128 = 2, PF_XT_128x128 = 3, PF_XT_192x256 = 4, PF_XT_128x128k2 = 5,
-       PF_XT_256x128k2 = 6, PF_XT_256x256w8 = 7, PF_XT_128x128w8 = 8, PF_XT_256x128w8 = 9, PF_XT_COUNT = 10 };
+       PF_XT_256x128k2 = 6, PF_XT_256x256w8 = 7, PF_XT_128x128w8 = 8, PF_XT_256x128w8 = 9, PF_XT_192x256w8 = 10, PF_XT_COUNT = 11 };
 // BM, BN, reduction depth per stage, stages, wavefront grid (rows x columns x reduction split) of each tile id
 template <int XT> struct XTile;
 template <> struct XTile<PF_XT_256x256> { static constexpr int BM = 256, BN = 256, BK = 32, ST = 5, WGM = 2, WGN = 2, KS = 1; };
@@ -197,7 +197,8 @@ template <> struct XTile<PF_XT_256x128k2> { static constexpr int BM = 256, BN = 
 template <> struct XTile<PF_XT_256x256w8> { static constexpr int BM = 256, BN = 256, BK = 32, ST = 5, WGM = 2, WGN = 4, KS = 1; };
 template <> struct XTile<PF_XT_128x128w8> { static constexpr int BM = 128, BN = 128, BK = 64, ST = 3, WGM = 2, WGN = 4, KS = 1; };
 template <> struct XTile<PF_XT_256x128w8> { static constexpr int BM = 256, BN = 128, BK = 64, ST = 3, WGM = 4, WGN = 2, KS = 1; };
-inline int x_tile_bk(int xt) { return (xt == PF_XT_256x256 || xt == PF_XT_192x256 || xt == PF_XT_256x256w8) ? 32 : 64; }
+template <> struct XTile<PF_XT_192x256w8> { static constexpr int BM = 192, BN = 256, BK = 32, ST = 5, WGM = 2, WGN = 4, KS = 1; };
+inline int x_tile_bk(int xt) { return (xt == PF_XT_256x256 || xt == PF_XT_192x256 || xt == PF_XT_256x256w8 || xt == PF_XT_192x256w8) ? 32 : 64; }
 
 // Epilogue classes with straight-line code (which operands exist, and their dtypes, fixed at
 // compile time).  Everything else takes EC_GENERIC: one rolled loop with runtime switches.

@@ -20,13 +20,20 @@ namespace {
 //                                           c ^ 4*(k%4)) and read with ds_read_b64_tr_b16,
 //                                           the transposing LDS read, which hands a lane
 //                                           four consecutive k of one row.
-// Each wavefront owns a (BM/WGM) x (BN/WGN) block of accumulators (up to 128x128 =
-// 16 MFMA tiles, one fragment read per two MFMAs).  The K loop has ONE barrier per tile,
-// placed before the tile's last 16-deep MFMA group: by then the group's fragments are in
-// registers, so the buffer can be refilled at once, and the first fragments of the next
-// tile are read under that last group's MFMAs (no LDS latency exposed at the barrier).
+// Each wavefront owns a (BM/WGM) x (BN/WGN) block of accumulators, computed with v_mfma_f32_16x16x32.  That
+// shape instead of 32x32x16 because of power: at the same peak rate the matrix pipes of the whole chip sustain
+// 1.99 against 1.72 PFLOP/s (fp16, random data; bf16 2.15 / 1.89), and a large product is bound by the board's
+// power.  The price is twice as many instructions of half the length, so the K loop deals out its LDS reads and
+// loads one at a time between them.  The K loop has ONE barrier per tile, before the tile's last MFMA group: by
+// then the group's fragments are in registers, so the buffer can be refilled at once, and the first fragments
+// of the next tile are read under that last group's MFMAs (no LDS latency exposed at the barrier).
+// Measured against the 32x32x16 form with an epilogue through LDS (us): 8192^3 fp16 946 -> 852;
+// [3152 x 1024] . [1024 x 1024] 11.9 -> 10.7, [3152 x 4096] . [4096 x 1024] 34.0 -> 30.1,
+// [3152 x 1024] . [1024 x 4096] 33.7 -> 30.9; one workgroup's fixed cost at K = 64: 256x256 7.6 -> 6.3,
+// 128x128 4.2 -> 3.4; weight gradient 4096x4096 over 4096 rows 128.5 -> 113.6.
 // ---------------------------------------------------------------------------
 #define PF_LDS(T) __attribute__((address_space(3))) T*
+typedef int v2i_t __attribute__((ext_vector_type(2)));
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
@@ -52,11 +59,18 @@ __device__ __forceinline__ void frag_hold(Frag<true>& f) { asm volatile("" : "+v
 template <int N> __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-template <int R, int BK, int NW, bool TRANS> struct DTile {
+// PW > 1 (right-hand operand of a row-major product): inside every 16*PW rows the tile holds row PW*i + t
+// as row i of MFMA tile t, so that the accumulators a lane keeps of PW tiles are PW CONSECUTIVE columns
+// of the result.
+template <int R, int BK, int NW, bool TRANS, int PW> struct DTile {
   static constexpr int BYTES = R * BK * 2;
   static constexpr int NI = BYTES / 1024;  // wavefront-wide load instructions per tile
-  static constexpr int IPW = NI / NW;      // ... per wavefront
-  static_assert(NI % NW == 0 && IPW >= 1, "tile does not divide over the wavefronts");
+  static constexpr int IPW = (NI + NW - 1) / NW;   // ... per wavefront
+  // (12 instructions over 8 wavefronts, the 192-row tile: the last two wavefronts repeat the last one, the
+  // same bytes to the same place, so that every wavefront has the same number of loads in flight)
+  static __device__ __forceinline__ int instr(int wave, int q) {
+    return NI % NW == 0 || wave * IPW + q < NI ? wave * IPW + q : NI - 1;
+  }
   static constexpr int CPR = BK / 8;       // [row][k]: 16-byte chunks per row
   static constexpr int RPI = 64 / CPR;     //           rows per instruction
   static constexpr int ROWB = TRANS ? R * 2 : BK * 2;  // bytes per LDS row
@@ -64,10 +78,9 @@ template <int R, int BK, int NW, bool TRANS> struct DTile {
   static constexpr int KPI = 64 / CPK;     //           k-rows per instruction
   static_assert(!TRANS || (R == 128 || R == 256), "transposed tiles are 128 or 256 rows wide");
   static_assert(BK == 64 || BK == 32, "BK is 32 or 64");
-  static constexpr int NFRAG = TRANS ? 0 : BK / 16;
 
-  static __device__ __forceinline__ int swz_row(int row) { return BK == 64 ? ((row >> 1) & 7) : ((row >> 2) & 3); }
-  static __device__ __forceinline__ int swz_k(int k) { return (k & 3) << 2; }
+  static __device__ __forceinline__ int swz_row(int row) { return BK == 64 ? ((row >> 1) & 7) : ((row >> 1) & 3); }
+  static __device__ __forceinline__ int swz_k(int k) { return ((k & 3) << 2) ^ (((k >> 3) & 1) << 1); }
 
   static __device__ __forceinline__ uint32_t extent(int64_t R_total, int64_t K, int64_t ld) {
     return TRANS ? (uint32_t)(((K - 1) * ld + (R_total + 7) / 8 * 8) * 2)
@@ -77,11 +90,12 @@ template <int R, int BK, int NW, bool TRANS> struct DTile {
   static __device__ __forceinline__ void init(uint32_t (&off)[IPW], int64_t ld, int64_t r0, int wave, int lane) {
 #pragma unroll
     for (int q = 0; q < IPW; ++q) {
-      const int ii = wave * IPW + q;
+      const int ii = instr(wave, q);
       if (!TRANS) {
         const int row = ii * RPI + lane / CPR;
         const int c = (lane % CPR) ^ swz_row(row);
-        off[q] = (uint32_t)(((r0 + row) * ld + c * 8) * 2);
+        const int src = PW > 1 ? row / (16 * PW) * (16 * PW) + (row & 15) * PW + (row >> 4) % PW : row;
+        off[q] = (uint32_t)(((r0 + src) * ld + c * 8) * 2);
       } else {
         const int k = ii * KPI + lane / CPK;
         const int mc = (lane % CPK) ^ swz_k(k);
@@ -97,84 +111,101 @@ template <int R, int BK, int NW, bool TRANS> struct DTile {
                                                uint32_t lds, int wave) {
 #pragma unroll
     for (int q = (Q0 < 0 ? 0 : Q0); q < (Q1 > IPW ? IPW : Q1); ++q)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (PF_LDS(void))(uintptr_t)(lds + (uint32_t)(wave * IPW + q) * 1024u), 16,
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (PF_LDS(void))(uintptr_t)(lds + (uint32_t)instr(wave, q) * 1024u), 16,
                                                (int)(off[q] + adv), 0, 0, 0);
   }
   // Fragment addressing.  w0: first row of the wavefront's block inside the tile.
-  //   [row][k]: foff[kk] = byte offset of (row w0 + lane%32, chunk 2*kk + lane/32); + i*32*ROWB per MFMA tile
-  //   [k][row]: foff[i]  = byte offset for MFMA tile i at kk = 0, first half; + (16*kk + 4*h)*ROWB
-  static constexpr int NOFF_T = 4;
-  // kk0: first 16-deep MFMA group of a tile that this wavefront multiplies (wavefronts that split
+  //   [row][k]: foff[kk] = byte offset of (row w0 + lane%16, chunk 4*kk + lane/16); + i*16*ROWB per MFMA tile
+  //   [k][row]: foff[0]  = byte offset for MFMA tile 0 at kk = 0, first half; + (32*kk + 4*h)*ROWB; tile i
+  //             differs in address bits that only the swizzle touches, by exclusive or: ^ tile_xor(i)
+  // kk0: first 32-deep MFMA group of a tile that this wavefront multiplies (wavefronts that split
   // a tile's reduction depth between them start at different groups)
+  // (a wavefront's block starts at a multiple of its own width, a power of two times 16 rows)
+  static constexpr uint32_t tile_xor(int i) { return (uint32_t)(i * 32); }
   template <int NF>
   static __device__ __forceinline__ void frag_init(uint32_t (&foff)[NF], int w0, int lane, int kk0) {
     if constexpr (!TRANS) {
-      const int row = w0 + (lane & 31), half = lane >> 5;
+      const int row = w0 + (lane & 15), quarter = lane >> 4;
 #pragma unroll
-      for (int kk = 0; kk < NF; ++kk) foff[kk] = (uint32_t)(row * ROWB + ((((kk0 + kk) * 2 + half) ^ swz_row(row)) * 16));
+      for (int kk = 0; kk < NF; ++kk) foff[kk] = (uint32_t)(row * ROWB + ((((kk0 + kk) * 4 + quarter) ^ swz_row(row)) * 16));
     } else {
       const int g = lane >> 4, j = lane & 15;
-      const int k = (g >> 1) * 8 + (j >> 2);
+      const int k = g * 8 + (j >> 2);
+      const int m = w0 + 4 * (j & 3);
 #pragma unroll
-      for (int i = 0; i < NF; ++i) {
-        const int m = w0 + i * 32 + (g & 1) * 16 + 4 * (j & 3);
-        foff[i] = (uint32_t)((k + kk0 * 16) * ROWB + (((m >> 3) ^ swz_k(k)) * 16) + (m & 7) * 2);
-      }
+      for (int i = 0; i < NF; ++i) foff[i] = (uint32_t)((k + kk0 * 32) * ROWB + (((m >> 3) ^ swz_k(k)) * 16) + (m & 7) * 2) ^ tile_xor(i);
     }
   }
-  template <int NF, int I, int KKI>
-  static __device__ __forceinline__ Frag<TRANS> frag(uint32_t lds, const uint32_t (&foff)[NF]) {
-    Frag<TRANS> f;
+  static constexpr int NRD = TRANS ? 2 : 1;   // LDS reads per fragment
+  // read H of MFMA tile I's fragment of group KKI
+  template <int NF, int I, int KKI, int H>
+  static __device__ __forceinline__ void read(Frag<TRANS>& f, uint32_t lds, const uint32_t (&foff)[NF]) {
     if constexpr (!TRANS) {
-      f.v = *(PF_LDS(const short8_t))(uintptr_t)(lds + foff[KKI] + (uint32_t)(I * 32 * ROWB));
+      f.v = *(PF_LDS(const short8_t))(uintptr_t)(lds + foff[KKI] + (uint32_t)(I * 16 * ROWB));
     } else {
       // Inline assembly on purpose: the compiler makes an LDS read it cannot tell apart from the
       // destination of an earlier direct-to-LDS load wait for ALL outstanding loads, and it cannot
       // for this instruction, which would serialise the whole tile pipeline.  The price: it does
-      // not know that these results arrive asynchronously either; the K loop waits for them by
-      // hand (TR_READS instructions per fragment count in lgkmcnt).
-      const uint32_t a = lds + foff[I];
-      asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(f.lo) : "v"(a), "n"(KKI * 16 * ROWB) : "memory");
-      asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(f.hi) : "v"(a), "n"(KKI * 16 * ROWB + 4 * ROWB) : "memory");
+      // not know that these results arrive asynchronously either; the K loop waits for them by hand.
+      const uint32_t a = lds + (NF > 1 ? foff[NF > 1 ? I : 0] : (foff[0] ^ tile_xor(I)));
+      if constexpr (H == 0) asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(f.lo) : "v"(a), "n"(KKI * 32 * ROWB) : "memory");
+      else asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(f.hi) : "v"(a), "n"(KKI * 32 * ROWB + 4 * ROWB) : "memory");
     }
-    return f;
   }
-  static constexpr int TR_READS = 2;
+  template <int NF, int I>
+  static __device__ __forceinline__ void read_first(Frag<TRANS>& f, uint32_t lds, const uint32_t (&foff)[NF]) {
+    static_for<NRD>([&](auto hc) { read<NF, I, 0, decltype(hc)::value>(f, lds, foff); });
+  }
 };
 
-// 32-row accumulator blocks each wavefront stages through LDS at a time in the epilogue
-// (nw wavefronts, wn columns per wavefront block, tm blocks in all): as many as 160 KB hold.
-constexpr int epi_row_blocks(int nw, int wn, int tm) {
-  const int fit = (160 * 1024) / (nw * 32 * (wn + 8) * 4);
-  int rb = fit >= tm ? tm : fit;
-  while (rb > 1 && tm % rb != 0) --rb;
-  return rb < 1 ? 1 : rb;
+// reads among the events e = 0 .. ne-1 (nl of them loads, spread evenly) dealt to the slots 0 .. m of ns
+constexpr int count_reads(int ne, int ns, int nl, int m) {
+  int n = 0;
+  for (int e = 0; e < ne; ++e)
+    if (e * ns / ne <= m && (e + 1) * nl / ne == e * nl / ne) ++n;
+  return n;
 }
 
-typedef float float8_t __attribute__((ext_vector_type(8)));
-
-template <int DT> __device__ __forceinline__ float8_t unpack16(v4i_t r) {
-  float8_t o;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const uint32_t w = (uint32_t)r[k];
-    if (DT == PF_BF16) {
-      o[2 * k] = __uint_as_float(w << 16);
-      o[2 * k + 1] = __uint_as_float(w & 0xffff0000u);
+template <int DT> __device__ __forceinline__ float unpack1(uint32_t w, int hi) {
+  if (DT == PF_BF16) return __uint_as_float(hi ? (w & 0xffff0000u) : (w << 16));
+  return pf_f16_bits_to_f32((uint16_t)(hi ? (w >> 16) : (w & 0xffffu)));
+}
+template <int DT> __device__ __forceinline__ uint32_t pack2(float a, float b) {
+  return DT == PF_BF16 ? pf_pack2_bf16(a, b) : pf_pack2_f16(a, b);
+}
+// N 32-bit words that travel in one buffer access (8 words: two)
+template <int N> struct Words {
+  int w[N];
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
+    if constexpr (N == 1) {
+      w[0] = __builtin_amdgcn_raw_buffer_load_b32(rs, (int)off, 0, 0);
+    } else if constexpr (N == 2) {
+      const v2i_t t = __builtin_amdgcn_raw_buffer_load_b64(rs, (int)off, 0, 0);
+      w[0] = t.x; w[1] = t.y;
     } else {
-      o[2 * k] = pf_f16_bits_to_f32((uint16_t)(w & 0xffffu));
-      o[2 * k + 1] = pf_f16_bits_to_f32((uint16_t)(w >> 16));
+#pragma unroll
+      for (int q = 0; q < N; q += 4) {
+        const v4i_t t = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(off + q * 4), 0, 0);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w[q + k] = t[k];
+      }
     }
   }
-  return o;
-}
-template <int DT> __device__ __forceinline__ v4i_t pack16(const float8_t& v) {
-  v4i_t o;
+  __device__ __forceinline__ void store(__amdgpu_buffer_rsrc_t rs, uint32_t off) const {
+    if constexpr (N == 1) {
+      __builtin_amdgcn_raw_buffer_store_b32(w[0], rs, (int)off, 0, 0);
+    } else if constexpr (N == 2) {
+      const v2i_t t = {w[0], w[1]};
+      __builtin_amdgcn_raw_buffer_store_b64(t, rs, (int)off, 0, 0);
+    } else {
 #pragma unroll
-  for (int k = 0; k < 4; ++k)
-    o[k] = (int)(DT == PF_BF16 ? pf_pack2_bf16(v[2 * k], v[2 * k + 1]) : pf_pack2_f16(v[2 * k], v[2 * k + 1]));
-  return o;
-}
+      for (int q = 0; q < N; q += 4) {
+        const v4i_t t = {w[q], w[q + 1], w[q + 2], w[q + 3]};
+        __builtin_amdgcn_raw_buffer_store_b128(t, rs, (int)(off + q * 4), 0, 0);
+      }
+    }
+  }
+};
 
 // `pid`: index of this workgroup among the workgroups of its problem (the launch may hold several
 // problems, see gemm16x_group_kernel)
@@ -189,17 +220,20 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
   constexpr int NWMN = WGM * WGN;
   constexpr int NW = NWMN * KS;
   constexpr int WM = BM / WGM, WN = BN / WGN;
-  constexpr int TM = WM / 32, TN = WN / 32;
-  constexpr int KK = BK / 16 / KS;     // MFMA groups per tile and wavefront
+  constexpr int TM = WM / 16, TN = WN / 16;
+  constexpr int KK = BK / 32 / KS;     // 32-deep MFMA groups per tile and wavefront
   static_assert(KS == 1 || KS == 2, "the reduction depth of a tile is split over one or two wavefront grids");
-  static_assert((BK / 16) % KS == 0, "MFMA groups do not divide over the wavefront grids");
-  using TA = DTile<BM, BK, NW, AT>;
-  using TB = DTile<BN, BK, NW, BT>;
+  static_assert((BK / 32) % KS == 0 && KK >= 1, "MFMA groups do not divide over the wavefront grids");
+  constexpr bool C32 = EC == EC_STORE32 || EC == EC_RES32 || EC == EC_ACC32;
+  using TA = DTile<BM, BK, NW, AT, 1>;
+  using TB = DTile<BN, BK, NW, BT, BT ? 1 : TN>;
   constexpr int STAGE = TA::BYTES + TB::BYTES;
   constexpr int LPW = TA::IPW + TB::IPW;  // load instructions per wavefront per tile
-  static_assert((ST - 2) * LPW <= 63, "too many loads in flight for the 6-bit counter");
-  static_assert(KK % 2 == 0, "fragment double buffer assumes an even number of MFMA groups per tile");
-  constexpr int NFA = AT ? TM : KK, NFB = BT ? TN : KK;
+  static_assert((ST - 1) * LPW <= 63, "too many loads in flight for the 6-bit counter");
+  // (transposing reads: an address per MFMA tile where the block leaves the registers for it; the small blocks
+  // are bound by instruction issue)
+  constexpr int NFA = AT ? (TM * TN <= 16 ? TM : 1) : KK, NFB = BT ? (TM * TN <= 16 ? TN : 1) : KK;
+  static_assert((!AT || (WM & (WM - 1)) == 0) && (!BT || (WN & (WN - 1)) == 0), "tile_xor");
   extern __shared__ __align__(16) uint16_t smem[];
 
   const int t = gemm_tile_id(pid, g.tiles_m * g.tiles_n, g.per_xcd);
@@ -213,21 +247,19 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
   const uint16_t* B = (const uint16_t*)p.B + z1 * p.b_stride1 + z2 * p.b_stride2;
   const int64_t c_base = z1 * p.c_stride1 + z2 * p.c_stride2;
   const Epi epi = make_epi(p);
-  const int vec_epi = g.vec_epi;
-
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wave_k = wave / NWMN, wave_mn = wave % NWMN;
   const int wm0 = (wave_mn / WGN) * WM, wn0 = (wave_mn % WGN) * WN;
   const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
 
-  float16_t acc[TM][TN];
+  float4_t acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
 
   const __amdgpu_buffer_rsrc_t rs_a = make_rsrc(A, TA::extent(M, K, lda));
   const __amdgpu_buffer_rsrc_t rs_b = make_rsrc(B, TB::extent(N, K, ldb));
@@ -241,121 +273,182 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
 
   const int nk = (int)((K + BK - 1) / BK);
 
-  // fast epilogues: this lane's 8 bias values, fetched now so that the K loop hides the latency
-  constexpr int LPR = WN / 8;        // epilogue: lanes per row of the wavefront's block
-  constexpr int RPP = 64 / LPR;      //           rows per pass
-  const int rd_row = lane / LPR, rd_col = (lane % LPR) * 8;
-  const int64_t c8 = n0 + wn0 + rd_col;
-  float8_t bias8 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  if constexpr (EC != EC_GENERIC) {
-    if (epi.bias != nullptr && c8 < N) {
-      float t[8];
-      ld_vec<8>(epi.bias, c8, epi.bias_dtype, t);
+  // This lane's part of C: rows row0 + 16 i + r (r = 0..3); columns c0 .. c0 + TN - 1, one per MFMA tile, of a
+  // row-major product (see DTile's PW), c0 + 16 j of a reduction-strided one (the transposing LDS reads fix
+  // the order of its columns).  16 neighbouring lanes cover 16 * TN (or 16) consecutive columns of a row:
+  // neighbouring lanes have to, the address coalescer joins the accesses of lanes 4 k .. 4 k + 3 only.
+  const int64_t row0 = m0 + wm0 + (lane >> 4) * 4;
+  const int64_t c0 = n0 + wn0 + (lane & 15) * (BT ? 1 : TN);
+  float bias[TN];
+  // One branch on the dtype around all of the bias loads; a missing bias, and columns past N, read as zeros
+  // through the buffer's extent.
+  auto load_bias = [&]() {
+    const bool b32 = epi.bias_dtype == PF_F32;
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(epi.bias, epi.bias != nullptr ? (uint32_t)(N * (b32 ? 4 : 2)) : 0u);
+    if (b32) {
 #pragma unroll
-      for (int k = 0; k < 8; ++k) bias8[k] = t[k];
+      for (int j = 0; j < TN; ++j) bias[j] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, (int)((c0 + j) * 4), 0, 0));
+    } else {
+      uint32_t raw[TN / 2];
+#pragma unroll
+      for (int j = 0; j < TN / 2; ++j) raw[j] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, (int)((c0 + 2 * j) * 2), 0, 0);
+      const bool bf = epi.bias_dtype == PF_BF16;
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const uint32_t h = (raw[j / 2] >> (16 * (j % 2))) & 0xffffu;
+        bias[j] = bf ? __uint_as_float(h << 16) : pf_f16_bits_to_f32((uint16_t)h);
+      }
     }
-  }
-
-  // Tiles past the end of K are requested too: their addresses lie beyond the buffer
-  // extent, so the hardware range check drops them, and every iteration of the K loop
-  // is the same straight-line code with the same number of loads in flight.
-  // The loads of one tile are issued in KK-1 slices, one per MFMA group: a burst of them
-  // would fill the memory pipeline's queue and stall the wavefront (and with it the SIMD's
-  // MFMA pipe, there is one wavefront per SIMD) for as long as the tile takes to stream in.
-  static_assert(ST >= 3, "the refill of a stage is spread over the following tile's MFMA groups");
-  constexpr int NSL = KK - 1;                         // slices
-  constexpr int SLW = (LPW + NSL - 1) / NSL;          // loads per slice
-  auto issue_all = [&](int kt, uint32_t sb) {
-    TA::template issue<0, TA::IPW>(rs_a, offa, (uint32_t)kt * step_a, sb, wave);
-    TB::template issue<0, TB::IPW>(rs_b, offb, (uint32_t)kt * step_b, sb + TA::BYTES, wave);
   };
-  // One 16-deep MFMA group ("phase") = NMFMA matrix instructions on the fragments in register
-  // set kk&1, the LDS reads that fill the other set for the next phase, and (all phases but a
-  // tile's last) one slice of the loads that refill the stage freed by the previous tile.  The
-  // three kinds are dealt round-robin into G sub-groups fenced by scheduling barriers, so the
-  // single wavefront of a SIMD always has matrix work queued while its LDS reads and its
-  // load instructions (which wait for room in the memory pipeline) trickle out.
-  constexpr int NFRAG = TM + TN;
-  constexpr int NMFMA = TM * TN;
-  constexpr int G = NFRAG < NMFMA ? NFRAG : NMFMA;
-  Frag<AT> fa[2][TM];
-  Frag<BT> fb[2][TN];
-  // kkn: MFMA group whose fragments are read (from stage sbr) into register set `slot`;
-  // kk: MFMA group multiplied now; SL: slice of tile loads issued now (-1: none)
-  auto phase = [&](uint32_t sbr, auto kknc, auto kkc, auto slc, int ktl, uint32_t sbl) {
-    constexpr int kkn = decltype(kknc)::value, kk = decltype(kkc)::value, SL = decltype(slc)::value;
-    constexpr int slot = kkn & 1, cur = kk & 1;
-    static_for<G>([&](auto gc) {
-      constexpr int gi = decltype(gc)::value;
-      {
-        static_for<NFRAG>([&](auto fc) {
-          constexpr int f = decltype(fc)::value;
-          if constexpr (f * G / NFRAG == gi) {
-            if constexpr (f < TM) fa[slot][f] = TA::template frag<NFA, f, kkn>(sbr, foa);
-            else fb[slot][f - TM] = TB::template frag<NFB, f - TM, kkn>(sbr + TA::BYTES, fob);
-          }
-        });
-      }
-      if constexpr (AT && BT && gi == 0) {
-        // fragments of this phase's MFMAs were read (by inline assembly) during the previous
-        // phase: LDS returns in order, so they are all there once no more reads are outstanding
-        // than this group has just issued
-        constexpr int mine = ((NFRAG + G - 1) / G) * 2;
-        asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(mine) : "memory");
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      if constexpr (SL >= 0) {
-        {
-          static_for<SLW>([&](auto qc) {
-            constexpr int q = SL * SLW + decltype(qc)::value;   // index into A's then B's list of loads
-            if constexpr (decltype(qc)::value * G / SLW == gi && q < LPW) {
-              if constexpr (q < TA::IPW) TA::template issue<q, q + 1>(rs_a, offa, (uint32_t)ktl * step_a, sbl, wave);
-              else TB::template issue<q - TA::IPW, q - TA::IPW + 1>(rs_b, offb, (uint32_t)ktl * step_b, sbl + TA::BYTES, wave);
+  // Fetched before the K loop, which hides the latency; after it in the GELU' class, which hardly ever has a
+  // bias and has no registers to spare for one.  Weight-gradient products with a bias take the generic class.
+  constexpr bool HAS_BIAS = EC != EC_GENERIC && !AT;
+  constexpr bool BIAS_EARLY = HAS_BIAS && EC != EC_DACT16;
+  if constexpr (BIAS_EARLY) load_bias();
+
+  // Tiles past the end of K are requested too, at an offset beyond the buffer extent: the hardware
+  // range check drops them (no memory traffic), and every iteration of the K loop is the same
+  // straight-line code with the same number of loads in flight.
+  // The loads of one tile are dealt over the sub-groups of one MFMA group: a burst of them would fill the
+  // memory pipeline's queue and stall the wavefront for as long as the tile takes to stream in.
+  static_assert(ST >= 3, "a stage is refilled while the next tile is multiplied");
+  auto adv_of = [&](int kt, uint32_t step) { return kt < nk ? (uint32_t)kt * step : 0x80000000u; };
+  auto issue_all = [&](int kt, uint32_t sb) {
+    TA::template issue<0, TA::IPW>(rs_a, offa, adv_of(kt, step_a), sb, wave);
+    TB::template issue<0, TB::IPW>(rs_b, offb, adv_of(kt, step_b), sb + TA::BYTES, wave);
+  };
+  // One 32-deep MFMA group ("phase") = NM matrix instructions on the fragments in register set `cur`, the
+  // LDS reads that fill the other set for the next phase, and its share of the loads that refill the
+  // stage that is free.  An MFMA occupies the matrix pipe for 16 cycles and the wavefront issues in order:
+  // the reads and loads are dealt out ONE at a time between the MFMAs (each followed by a scheduling
+  // barrier), evenly over the first 7/8 of the phase; two or three of them side by side leave the pipe idle.
+  // (The phase that starts with a barrier waits for all of its predecessor's reads.)
+  // Blocks of more than 128 accumulator registers (the four-wavefront 256x256 and 192x256 tiles), and those that exchange
+  // half their sums with another wavefront, have no room for two sets of fragments: they read a phase's fragments at its start (SINGLE).
+  constexpr int NM = TM * TN;
+  constexpr bool SINGLE = NM > 32 || (KS == 2 && NM == 32);
+  constexpr int NREADS = TM * TA::NRD + TN * TB::NRD;
+  Frag<AT> fa[SINGLE ? 1 : 2][TM];
+  Frag<BT> fb[SINGLE ? 1 : 2][TN];
+  // kkn: MFMA group (of the tile in stage sbr) whose fragments are read into the other register set;
+  // loads PART * LPW / PARTS .. (PART + 1) * LPW / PARTS - 1 of tile ktl go into stage sbl
+  auto phase = [&](uint32_t sbr, auto kknc, auto curc, auto partc, auto partsc, int ktl, uint32_t sbl) {
+    constexpr int kkn = decltype(kknc)::value, cur = SINGLE ? 0 : decltype(curc)::value, slot = cur ^ 1;
+    constexpr int PART = decltype(partc)::value, PARTS = decltype(partsc)::value;
+    constexpr int Q0 = PART * LPW / PARTS, NL = (PART + 1) * LPW / PARTS - Q0;
+    constexpr int NRE = SINGLE ? 0 : NREADS;
+    constexpr int NE = NRE + NL;                     // reads and loads, interleaved evenly
+    if constexpr (SINGLE) {
+      static_for<TN>([&](auto jc) {
+        static_for<TB::NRD>([&](auto hc) { TB::template read<NFB, decltype(jc)::value, kkn, decltype(hc)::value>(fb[0][decltype(jc)::value], sbr + TA::BYTES, fob); });
+      });
+      static_for<TM>([&](auto ic) {
+        static_for<TA::NRD>([&](auto hc) { TA::template read<NFA, decltype(ic)::value, kkn, decltype(hc)::value>(fa[0][decltype(ic)::value], sbr, foa); });
+      });
+    }
+    constexpr int NS = NM > 8 ? NM * 7 / 8 : NM;
+    const uint32_t adv_a = adv_of(ktl, step_a), adv_b = adv_of(ktl, step_b);
+    if constexpr (AT && BT && SINGLE) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int i = 0; i < TM; ++i) frag_hold(fa[0][i]);   // (nothing that uses them may move above the wait)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) frag_hold(fb[0][j]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    static_for<NM>([&](auto mc) {
+      constexpr int m = decltype(mc)::value;
+      static_for<NE>([&](auto ec) {
+        constexpr int e = decltype(ec)::value;
+        if constexpr (e * NS / NE == m) {
+          // event e is a load where the running count of loads steps up, else a read
+          constexpr int l0 = e * NL / NE, l1 = (e + 1) * NL / NE;
+          if constexpr (l1 > l0) {
+            constexpr int q = Q0 + l0;                   // index into A's then B's list of loads
+            if constexpr (q < TA::IPW) TA::template issue<q, q + 1>(rs_a, offa, adv_a, sbl, wave);
+            else TB::template issue<q - TA::IPW, q - TA::IPW + 1>(rs_b, offb, adv_b, sbl + TA::BYTES, wave);
+          } else {
+            constexpr int r = e - l0;                    // B's fragments first, then A's
+            if constexpr (r < TN * TB::NRD) TB::template read<NFB, r / TB::NRD, kkn, r % TB::NRD>(fb[slot][r / TB::NRD], sbr + TA::BYTES, fob);
+            else {
+              constexpr int ra = r - TN * TB::NRD;
+              TA::template read<NFA, ra / TA::NRD, kkn, ra % TA::NRD>(fa[slot][ra / TA::NRD], sbr, foa);
             }
-          });
-        }
-      }
-      // 256x128 shared by eight wavefronts: the wavefront that has MFMAs to issue goes first among
-      // the two of its SIMD (measured -2 % on 4096-row products; no gain on the other tiles)
-      constexpr bool PRIO = NW == 8 && KS == 1 && BM == 256 && BN == 128;
-      if constexpr (PRIO) __builtin_amdgcn_s_setprio(1);
-      static_for<NMFMA>([&](auto mc) {
-        constexpr int m = decltype(mc)::value;
-        if constexpr (m * G / NMFMA == gi) {
-          constexpr int i = m / TN, j = m % TN;
-          acc[i][j] = Mfma<DT>::run8(fa[cur][i].get(), fb[cur][j].get(), acc[i][j]);
+          }
         }
       });
-      if constexpr (PRIO) __builtin_amdgcn_s_setprio(0);
+      if constexpr (AT && BT && !SINGLE && m % TN == 0) {
+        // This row of MFMAs takes fragments read by inline assembly during the previous phase, B's and A's up
+        // to row m / TN.  LDS answers in order: they are there once no more reads are outstanding than came after.
+        constexpr int need = TN * TB::NRD + (m / TN + 1) * TA::NRD;
+        constexpr int issued = count_reads(NE, NS, NL, m);
+        constexpr int later = NREADS - need + issued;
+        asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(later < 15 ? later : 15) : "memory");
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      constexpr int i = m / TN, j = (i & 1) ? TN - 1 - m % TN : m % TN;   // (serpentine: one operand changes at a time)
+      acc[i][j] = Mfma<DT>::run16(fa[cur][i].get(), fb[cur][j].get(), acc[i][j]);
       __builtin_amdgcn_sched_barrier(0);
     });
   };
-
-  // prologue: fill all stages but the last, wait for tile 0
+  // A tile's fragments are in registers at the barrier that opens its last phase: from there on its stage is
+  // refilled with the tile ST further on, the first part in that phase, the others in the next tile's
+  // phases but its last (one part per phase keeps the stream of loads even).  With one phase per tile the
+  // register sets alternate by tile.  (SINGLE reads a phase's fragments inside it: its stage is free one
+  // barrier later.)
+  // prologue: fill the stages, wait for tile 0
 #pragma unroll
   for (int s = 0; s < ST - 1; ++s) issue_all(s, lds0 + (uint32_t)s * STAGE);
-  wait_vm<(ST - 2) * LPW>();
+  constexpr int P0 = SINGLE ? 0 : LPW / KK;    // loads of tile ST - 1 that go out here
+  {
+    const uint32_t sbl = lds0 + (uint32_t)(ST - 1) * STAGE, adv_a = adv_of(ST - 1, step_a), adv_b = adv_of(ST - 1, step_b);
+    TA::template issue<0, P0>(rs_a, offa, adv_a, sbl, wave);
+    TB::template issue<0, P0 - TA::IPW>(rs_b, offb, adv_b, sbl + TA::BYTES, wave);
+  }
+  wait_vm<(ST - 2) * LPW + P0>();
   lds_barrier();
-  static_for<TM>([&](auto ic) { fa[0][decltype(ic)::value] = TA::template frag<NFA, decltype(ic)::value, 0>(lds0, foa); });
-  static_for<TN>([&](auto jc) { fb[0][decltype(jc)::value] = TB::template frag<NFB, decltype(jc)::value, 0>(lds0 + TA::BYTES, fob); });
+  if constexpr (!SINGLE) {
+    static_for<TM>([&](auto ic) { TA::template read_first<NFA, decltype(ic)::value>(fa[0][decltype(ic)::value], lds0, foa); });
+    static_for<TN>([&](auto jc) { TB::template read_first<NFB, decltype(jc)::value>(fb[0][decltype(jc)::value], lds0 + TA::BYTES, fob); });
+  }
   __builtin_amdgcn_sched_barrier(0);
 
   uint32_t sb = lds0;                                   // stage of tile kt
-  uint32_t sb_prev = lds0 + (uint32_t)(ST - 1) * STAGE; // stage of tile kt-1: free, refilled with tile kt+ST-1
-  for (int kt = 0; kt < nk; ++kt) {
+  uint32_t sb_prev = lds0 + (uint32_t)(ST - 1) * STAGE; // stage of tile kt-1
+  // one tile; `par`: register set its first phase multiplies
+  auto tile = [&](int kt, auto parc) {
+    constexpr int par = decltype(parc)::value;
     const uint32_t sb_next = (sb + STAGE == lds0 + (uint32_t)ST * STAGE) ? lds0 : sb + STAGE;
     static_for<KK>([&](auto kkc) {
       constexpr int kk = decltype(kkc)::value;
-      if constexpr (kk + 1 < KK) {
-        phase(sb, std::integral_constant<int, kk + 1>{}, kkc, std::integral_constant<int, kk>{}, kt + ST - 1, sb_prev);
+      constexpr std::integral_constant<int, (par + kk) & 1> cur{};
+      constexpr std::integral_constant<int, KK> parts{};
+      if constexpr (SINGLE) {
+        if (kk == 0 && kt > 0) {
+          wait_vm<(ST - 2) * LPW>();
+          lds_barrier();                            // tile kt landed everywhere, stage of tile kt-1 no longer read
+        }
+        phase(sb, kkc, cur, kkc, parts, kt + ST - 1, sb_prev);
+      } else if constexpr (kk + 1 < KK) {
+        phase(sb, std::integral_constant<int, kk + 1>{}, cur, std::integral_constant<int, kk + 1>{}, parts, kt + ST - 1, sb_prev);
       } else {
         wait_vm<(ST - 2) * LPW>();
         lds_barrier();                              // tile kt+1 landed everywhere, stage sb no longer read
-        phase(sb_next, std::integral_constant<int, 0>{}, kkc, std::integral_constant<int, -1>{}, 0, 0u);
+        phase(sb_next, std::integral_constant<int, 0>{}, cur, std::integral_constant<int, 0>{}, parts, kt + ST, sb);
       }
     });
     sb_prev = sb;
     sb = sb_next;
+  };
+  if constexpr (KK % 2 == 0 || SINGLE) {
+    for (int kt = 0; kt < nk; ++kt) tile(kt, std::integral_constant<int, 0>{});
+  } else {
+    int kt = 0;
+    for (; kt + 1 < nk; kt += 2) {
+      tile(kt, std::integral_constant<int, 0>{});
+      tile(kt + 1, std::integral_constant<int, 1>{});
+    }
+    if (kt < nk) tile(kt, std::integral_constant<int, 0>{});
   }
   // The last tile's last phase has read fragments of a tile that does not exist, and nothing
   // consumes them: the reads issued by inline assembly may still be in flight here, and the
@@ -365,7 +458,7 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
   // lane of row 0 and 15 rows in 16 of the wavefront's block were never written).
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
-  for (int sl = 0; sl < 2; ++sl) {
+  for (int sl = 0; sl < (SINGLE ? 1 : 2); ++sl) {
 #pragma unroll
     for (int i = 0; i < TM; ++i) frag_hold(fa[sl][i]);
 #pragma unroll
@@ -377,218 +470,195 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
   // stores to drain, once per row pass.
   __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
 
-  // Epilogue.  D layout of v_mfma_f32_32x32x*: lane l holds column (l % 32) and rows
-  // 8*(r/4) + 4*(l/32) + (r%4), r = 0..15.  Each wavefront re-lays its block through a private
-  // LDS patch (no workgroup barrier, no wait for earlier stores to drain), as many 32-row blocks
-  // at a time as LDS holds; afterwards WN/8 adjacent lanes cover one whole row of the block, 8
-  // columns each, so every store instruction writes complete rows of 2*WN (16-bit C) or 4*WN
-  // (fp32 C) bytes.  The arithmetic exists ONCE, in a rolled loop over the staged rows: a kernel
-  // of a few tens of microseconds cannot afford to stream 100 KB of unrolled epilogue code
-  // through the instruction cache, which starts cold at every launch.
+  // Epilogue.  D layout of v_mfma_f32_16x16x*: lane l holds column l % 16 and rows 4*(l/16) + r, r = 0..3, and
+  // with the order of the columns chosen for it (above) every access goes straight from the accumulators'
+  // layout to whole runs of a row: no trip through LDS, no barrier.
   lds_barrier();  // every wavefront is done with the operand tiles
   if constexpr (KS == 2) {
     // the second grid hands its partial sums over (16 bytes per lane, lanes side by side: no bank
     // conflicts) and leaves; a barrier only counts the wavefronts that are still running
-    float4* xch = (float4*)smem + wave_mn * (TM * TN * 4 * 64) + lane;
+    float4_t* xch = (float4_t*)smem + wave_mn * (TM * TN * 64) + lane;
     if (wave_k == 1) {
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-            xch[((i * TN + j) * 4 + q) * 64] = make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+        for (int j = 0; j < TN; ++j) xch[(i * TN + j) * 64] = acc[i][j];
     }
     lds_barrier();
     if (wave_k == 1) return;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float4 t = xch[((i * TN + j) * 4 + q) * 64];
-          acc[i][j][4 * q] += t.x; acc[i][j][4 * q + 1] += t.y; acc[i][j][4 * q + 2] += t.z; acc[i][j][4 * q + 3] += t.w;
-        }
+      for (int j = 0; j < TN; ++j) acc[i][j] += xch[(i * TN + j) * 64];
     lds_barrier();  // all partial sums are read before the epilogue patches overwrite them
   }
-  constexpr int SLD = WN + 8;        // floats per staged row: lanes 32..63 (4 rows down) land 32 banks away
-  constexpr int RB = epi_row_blocks(NWMN, WN, TM);   // 32-row blocks staged together
-  float* stage = (float*)smem + wave * (RB * 32 * SLD);
-  const int wr_off = ((lane >> 5) * 4) * SLD + (lane & 31);
-
-  if constexpr (EC != EC_GENERIC) {
-    // Compact branch-free epilogue: 16 rows of the wavefront's block at a time, ONE copy of the
-    // arithmetic in a rolled loop (unrolled, an epilogue runs to 200 KB of code that streams once
-    // through an instruction cache which starts cold at every launch).
-    // All global accesses are raw buffer operations whose range check drops rows past M (and
-    // lanes past N, which get an out-of-range offset): no branch, so no join at which the
-    // compiler would wait for every outstanding vector memory operation (loads AND the stores of
-    // the previous pass share one in-order counter).  The one operand a class reads (residual,
-    // old C or aux_in) comes in by direct-to-LDS loads, double buffered: the loads of the next 16
-    // rows are issued before the stores of the current ones, and since the counter retires in
-    // order, "those loads have landed" is "at most <the operations issued after them>
-    // outstanding", a compile-time number because nothing here is predicated.
-    constexpr bool C32 = EC == EC_STORE32 || EC == EC_RES32 || EC == EC_ACC32;
+  if constexpr (HAS_BIAS && !BIAS_EARLY) load_bias();
+  static_assert(BT || TN == 2 || TN == 4 || TN == 8, "whole vectors per lane and row");
+  if constexpr (EC == EC_GENERIC) {
+    // one rolled loop over 16-row blocks (unrolled, the run-time switches of this class fill the instruction cache)
+#pragma nounroll
+    for (int h = 0; h < TM; ++h) {
+      float4_t x[TN];
+      static_for<TM>([&](auto hc) {
+        constexpr int c = decltype(hc)::value;
+        if (h == c) {
+#pragma unroll
+          for (int j = 0; j < TN; ++j) x[j] = acc[c][j];
+        }
+      });
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t row = row0 + h * 16 + r;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const int64_t col = c0 + (BT ? 16 : 1) * j;
+          if (row < M && col < N) epilogue_scalar(epi, c_base, row, col, x[j][r]);
+        }
+      }
+    }
+    return;
+  } else {
+    // Straight-line classes.  All global accesses are raw buffer operations whose range check drops rows
+    // past M (lanes past N get an out-of-range offset): no branch, so no join at which the compiler would
+    // wait for every outstanding memory operation.  The one operand a class reads (residual, old C or
+    // aux_in) is requested DEPTH row blocks ahead, into the registers the operand fragments have left.
     constexpr bool LOADS = EC == EC_RES32 || EC == EC_ACC32 || EC == EC_DACT16 || EC == EC_ACC16 || EC == EC_RES16;
-    constexpr bool LOAD32 = EC == EC_RES32 || EC == EC_ACC32;
-    constexpr int HB = 16;                 // rows per step
-    constexpr int NHB = TM * 2;            // steps
-    constexpr int NP = HB / RPP;           // passes per step (a pass: every lane 8 columns of one row)
-    constexpr int LPP = LOADS ? (LOAD32 ? 2 : 1) : 0;               // load instructions per pass
-    constexpr int SPP = (C32 ? 2 : 1) + (EC == EC_ACT16 ? 1 : 0);   // store instructions per pass
-    constexpr int ESC = C32 ? 4 : 2;
-    constexpr int WAVE_LDS = HB * SLD * 4 + 2 * NP * 2 * 1024;      // stage + two operand buffers
-    static_assert(NWMN * WAVE_LDS <= 160 * 1024, "epilogue patches exceed LDS");
-    static_assert(NP * (SPP + LPP) <= 63, "too many operations in flight for the 6-bit counter");
-    float* stg = (float*)((char*)smem + wave * WAVE_LDS);
-    const uint32_t raw0 = lds0 + (uint32_t)(wave * WAVE_LDS + HB * SLD * 4);
+    constexpr int ESC = C32 ? 4 : 2;       // (the operand read has the element size of C in every class)
+    constexpr int NG = BT ? TN : 1;        // runs of columns per lane and row
+    constexpr int GW = BT ? 1 : TN;        // columns per run
+    constexpr int NV = GW * ESC / 4;       // 32-bit words per run
+    static_assert(!BT || C32, "reduction-strided products have fp32 results");
+    constexpr int DEPTH = !LOADS ? 1 : (TM * NG * NV <= 16 ? TM : (16 / (NG * NV) > 0 ? 16 / (NG * NV) : 1));
     const uint32_t OOB = 0x80000000u;
-    const int64_t row0 = m0 + wm0 + rd_row;
-    const bool col_ok = c8 < N;
     const __amdgpu_buffer_rsrc_t rs_c = make_rsrc((const char*)epi.C + c_base * ESC, (uint32_t)(((M - 1) * epi.ldc + N) * ESC));
-    const uint32_t off_c = col_ok ? (uint32_t)((row0 * epi.ldc + c8) * ESC) : OOB;
-    const uint32_t step_c = (uint32_t)(epi.ldc * ESC);
     const void* lp = (EC == EC_RES32 || EC == EC_RES16) ? epi.residual
-                                                            : (EC == EC_DACT16 ? epi.aux_in : (const void*)((const char*)epi.C + c_base * ESC));
+                                                        : (EC == EC_DACT16 ? epi.aux_in : (const void*)((const char*)epi.C + c_base * ESC));
     const int64_t ld_l = (EC == EC_RES32 || EC == EC_RES16) ? epi.ld_res : (EC == EC_DACT16 ? epi.ld_aux_in : epi.ldc);
-    constexpr int ESL = LOAD32 ? 4 : 2;
     // (a product that stores, beta = 0, inside a launch of the accumulate class, i.e. one member of a
     // grouped weight-gradient launch, reads its old C through a descriptor of extent 0: all zeros)
     const bool loads_on = LOADS && !(EC == EC_ACC32 && epi.beta == 0);
-    const __amdgpu_buffer_rsrc_t rs_l = make_rsrc(LOADS ? lp : epi.C, loads_on ? (uint32_t)(((M - 1) * ld_l + N) * ESL) : 0u);
-    const uint32_t off_l = col_ok ? (uint32_t)((row0 * ld_l + c8) * ESL) : OOB;
-    const uint32_t step_l = (uint32_t)(ld_l * ESL);
+    const __amdgpu_buffer_rsrc_t rs_l = make_rsrc(LOADS ? lp : epi.C, loads_on ? (uint32_t)(((M - 1) * ld_l + N) * ESC) : 0u);
     const __amdgpu_buffer_rsrc_t rs_x = make_rsrc(EC == EC_ACT16 ? epi.aux_out : epi.C,
                                                   EC == EC_ACT16 ? (uint32_t)(((M - 1) * epi.ld_aux_out + N) * 2) : 0u);
-    const uint32_t off_x = col_ok ? (uint32_t)((row0 * epi.ld_aux_out + c8) * 2) : OOB;
-    const uint32_t step_x = (uint32_t)(epi.ld_aux_out * 2);
+    uint32_t off_c[NG], off_l[NG], off_x[NG];
+#pragma unroll
+    for (int j = 0; j < NG; ++j) {
+      const bool ok = c0 + j * 16 < N;
+      off_c[j] = ok ? (uint32_t)((row0 * epi.ldc + c0 + j * 16) * ESC) : OOB;
+      off_l[j] = ok ? (uint32_t)((row0 * ld_l + c0 + j * 16) * ESC) : OOB;
+      off_x[j] = ok ? (uint32_t)((row0 * epi.ld_aux_out + c0 + j * 16) * 2) : OOB;
+    }
+    const uint32_t step_c = (uint32_t)(epi.ldc * ESC), step_l = (uint32_t)(ld_l * ESC), step_x = (uint32_t)(epi.ld_aux_out * 2);
     const float alpha = epi.alpha;
     const bool round_mid = epi.round_mid != 0;
+    float csum[TN];      // EC_DACT16: column sums of the stored values
+    float worst = 0.f;   // fp32 classes: sum of v * 0 over the values written: 0 if all are finite, NaN otherwise
+#pragma unroll
+    for (int j = 0; j < TN; ++j) csum[j] = 0.f;
 
-    auto fetch = [&](int hb) {   // rows past the block (hb == NHB) are requested too; nobody reads them
-      if constexpr (LOADS) {
-        const uint32_t dst = raw0 + (uint32_t)((hb & 1) * NP * LPP) * 1024u;
+    // one 16-row block: x = its accumulators, old = the operand read
+    auto block = [&](uint32_t h, const float4_t (&x)[TN], const Words<NV> (&old)[4][NG]) {
 #pragma unroll
-        for (int pp = 0; pp < NP; ++pp) {
-          const uint32_t o = off_l + (uint32_t)(hb * HB + pp * RPP) * step_l;
+      for (int r = 0; r < 4; ++r) {
+        const bool row_ok = row0 + (int64_t)(h * 16 + r) < M;
+        float bad = 0.f;
 #pragma unroll
-          for (int h = 0; h < LPP; ++h)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_l, (PF_LDS(void))(uintptr_t)(dst + (uint32_t)(pp * LPP + h) * 1024u), 16,
-                                                     (int)(o + 16 * h), 0, 0, 0);
+        for (int g = 0; g < NG; ++g) {
+          float v[GW];
+#pragma unroll
+          for (int k = 0; k < GW; ++k) {
+            v[k] = x[BT ? g : k][r] * alpha;
+            if constexpr (HAS_BIAS) v[k] += bias[k];
+          }
+          // (the plain 16-bit store rounds once, when it packs: rounding to the same format before
+          // that changes nothing)
+          if constexpr (EC != EC_STORE16 && !BT) {
+            if (round_mid) {
+#pragma unroll
+              for (int k = 0; k < GW; ++k) v[k] = Codec<DT>::round(v[k]);
+            }
+          }
+          const uint32_t oc = off_c[g] + (h * 16 + (uint32_t)r) * step_c;
+          Words<NV> o;
+          if constexpr (C32) {
+            if constexpr (LOADS) {
+#pragma unroll
+              for (int k = 0; k < GW; ++k) v[k] += __int_as_float(old[r][g].w[k]);
+            }
+            if constexpr (EC == EC_STORE32 || EC == EC_ACC32) {
+#pragma unroll
+              for (int k = 0; k < GW; ++k) bad = fmaf(v[k], 0.f, bad);
+            }
+#pragma unroll
+            for (int k = 0; k < GW; ++k) o.w[k] = __float_as_int(v[k]);
+          } else {
+            if constexpr (EC == EC_ACT16) {   // GELU only (other activations take the generic class)
+#pragma unroll
+              for (int k = 0; k < NV; ++k) o.w[k] = (int)pack2<DT>(v[2 * k], v[2 * k + 1]);
+              o.store(rs_x, off_x[g] + (h * 16 + (uint32_t)r) * step_x);
+#pragma unroll
+              for (int k = 0; k < GW; ++k) v[k] = pf_gelu_erf(v[k]);
+            }
+            if constexpr (LOADS) {
+#pragma unroll
+              for (int k = 0; k < GW; ++k) {
+                const float t = unpack1<DT>((uint32_t)old[r][g].w[k / 2], k % 2);
+                if constexpr (EC == EC_DACT16) v[k] *= pf_gelu_erf_grad(t);
+                else v[k] += t;
+              }
+            }
+#pragma unroll
+            for (int k = 0; k < NV; ++k) o.w[k] = (int)pack2<DT>(v[2 * k], v[2 * k + 1]);
+            if constexpr (EC == EC_DACT16) {   // sums run over the ROUNDED values, rows past M excluded
+              const float keep = row_ok ? 1.f : 0.f;
+#pragma unroll
+              for (int k = 0; k < GW; ++k) csum[k] += unpack1<DT>((uint32_t)o.w[k / 2], k % 2) * keep;
+            }
+          }
+          o.store(rs_c, oc);
         }
+        if constexpr (EC == EC_STORE32 || EC == EC_ACC32) worst += row_ok ? bad : 0.f;
       }
     };
-    float8_t csum = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};   // EC_DACT16: column sums of the stored values
-    float worst = 0.f;   // fp32 classes: sum of v - v over the values written: 0 if all are finite, NaN otherwise
-    fetch(0);
-#pragma nounroll
-    for (int hb = 0; hb < NHB; ++hb) {
-      static_for<NHB>([&](auto cc) {
-        constexpr int c = decltype(cc)::value;
-        if (hb == c) {
-          static_for<TN>([&](auto jc) {
-            constexpr int j = decltype(jc)::value;
-#pragma unroll
-            for (int r8 = 0; r8 < 8; ++r8)
-              stg[wr_off + (8 * (r8 >> 2) + (r8 & 3)) * SLD + j * 32] = acc[c / 2][j][(c % 2) * 8 + r8];
-          });
-        }
-      });
+    auto fetch = [&](uint32_t h, Words<NV> (&old)[4][NG]) {
       if constexpr (LOADS) {
-        fetch(hb + 1);
-        if (hb == 0) wait_vm<NP * LPP>(); else wait_vm<NP * (SPP + LPP)>();
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int g = 0; g < NG; ++g) old[r][g].load(rs_l, off_l[g] + (h * 16 + (uint32_t)r) * step_l);
       }
-      const uint32_t rawb = raw0 + (uint32_t)((hb & 1) * NP * LPP) * 1024u + (uint32_t)lane * 16u;
-      const uint32_t stg_addr = lds0 + (uint32_t)(wave * WAVE_LDS + (rd_row * SLD + rd_col) * 4);
-      // LDS reads by inline assembly: the compiler cannot tell these addresses from the
-      // destinations of the direct-to-LDS loads in flight and would wait for all of them (and,
-      // the counter being shared, for every store issued so far) before each ordinary read.
-      // The reads of all passes of a step are issued together and waited for once: a rolled
-      // pass loop exposed one LDS round trip per pass.
-      v4i_t sxs[NP], sys[NP], ras[NP], rbs[NP];
+    };
+    if constexpr (EC == EC_ACT16 || EC == EC_DACT16) {
+      // the arithmetic exists once, in a rolled loop: unrolled, its code would stream through an instruction
+      // cache that is cold at every launch
+      Words<NV> old[4][NG], next[4][NG];
+      fetch(0u, old);
+#pragma nounroll
+      for (int h = 0; h < TM; ++h) {
+        fetch((uint32_t)(h + 1), next);   // (of the block past the last one nobody reads anything)
+        float4_t x[TN];
+        static_for<TM>([&](auto cc) {
+          constexpr int c = decltype(cc)::value;
+          if (h == c) {
 #pragma unroll
-      for (int pp = 0; pp < NP; ++pp) {
-        const uint32_t sa = stg_addr + (uint32_t)((pp * RPP) * SLD * 4);
-        asm volatile("ds_read_b128 %0, %1" : "=v"(sxs[pp]) : "v"(sa) : "memory");
-        asm volatile("ds_read_b128 %0, %1 offset:16" : "=v"(sys[pp]) : "v"(sa) : "memory");
-        if constexpr (LOADS) {
-          const uint32_t rp = rawb + (uint32_t)(pp * LPP) * 1024u;
-          asm volatile("ds_read_b128 %0, %1" : "=v"(ras[pp]) : "v"(rp) : "memory");
-          if constexpr (LOAD32) asm volatile("ds_read_b128 %0, %1 offset:1024" : "=v"(rbs[pp]) : "v"(rp) : "memory");
-        }
+            for (int j = 0; j < TN; ++j) x[j] = acc[c][j];
+          }
+        });
+        block((uint32_t)h, x, old);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int g = 0; g < NG; ++g) old[r][g] = next[r][g];
       }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      // (the values are only complete from here on: nothing that uses them may move above the wait)
-#pragma unroll
-      for (int pp = 0; pp < NP; ++pp) {
-        asm volatile("" : "+v"(sxs[pp]), "+v"(sys[pp]));
-        if constexpr (LOADS) asm volatile("" : "+v"(ras[pp]));
-        if constexpr (LOAD32) asm volatile("" : "+v"(rbs[pp]));
-      }
-#pragma unroll
-      for (int pp = 0; pp < NP; ++pp) {
-        const v4i_t sx = sxs[pp], sy = sys[pp], ra = ras[pp], rb = rbs[pp];
-        float8_t v;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          v[k] = __int_as_float(sx[k]);
-          v[4 + k] = __int_as_float(sy[k]);
-        }
-        v = v * alpha + bias8;
-        // (the plain 16-bit store rounds once, when it packs: rounding to the same format before
-        // that changes nothing and cost 16 of the pass's 30 vector instructions)
-        if constexpr (EC != EC_STORE16) {
-          if (round_mid) {
-#pragma unroll
-            for (int k = 0; k < 8; ++k) v[k] = Codec<DT>::round(v[k]);
-          }
-        }
-        const uint32_t rowk = (uint32_t)(hb * HB + pp * RPP);
-        if constexpr (EC == EC_ACT16) {   // GELU only (other activations take the generic class)
-          __builtin_amdgcn_raw_buffer_store_b128(pack16<DT>(v), rs_x, (int)(off_x + rowk * step_x), 0, 0);
-#pragma unroll
-          for (int k = 0; k < 8; ++k) v[k] = pf_gelu_erf(v[k]);
-        }
-        if constexpr (EC == EC_DACT16 || EC == EC_ACC16 || EC == EC_RES16) {
-          const float8_t t = unpack16<DT>(ra);
-          if constexpr (EC == EC_DACT16) {
-#pragma unroll
-            for (int k = 0; k < 8; ++k) v[k] *= pf_gelu_erf_grad(t[k]);
-          } else {
-            v += t;
-          }
-        }
-        if constexpr (LOAD32) {
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            v[k] += __int_as_float(ra[k]);
-            v[4 + k] += __int_as_float(rb[k]);
-          }
-        }
-        const uint32_t oc = off_c + rowk * step_c;
-        if constexpr (C32) {
-          if constexpr (EC == EC_STORE32 || EC == EC_ACC32) {
-#pragma unroll
-            for (int k = 0; k < 8; ++k) worst += (row0 + (int64_t)rowk < M) ? (v[k] - v[k]) : 0.f;
-          }
-          v4i_t lo, hi;
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            lo[k] = __float_as_int(v[k]);
-            hi[k] = __float_as_int(v[4 + k]);
-          }
-          __builtin_amdgcn_raw_buffer_store_b128(lo, rs_c, (int)oc, 0, 0);
-          __builtin_amdgcn_raw_buffer_store_b128(hi, rs_c, (int)(oc + 16), 0, 0);
-        } else {
-          const v4i_t packed = pack16<DT>(v);
-          if constexpr (EC == EC_DACT16) {   // sums run over the ROUNDED values, rows past M excluded
-            const float keep = (row0 + (int64_t)rowk < M) ? 1.f : 0.f;
-            csum += unpack16<DT>(packed) * keep;
-          }
-          __builtin_amdgcn_raw_buffer_store_b128(packed, rs_c, (int)oc, 0, 0);
-        }
-      }
+    } else {
+      Words<NV> old[DEPTH][4][NG];
+      static_for<DEPTH>([&](auto hc) { fetch((uint32_t)decltype(hc)::value, old[decltype(hc)::value]); });
+      static_for<TM>([&](auto hc) {
+        constexpr int h = decltype(hc)::value;
+        block((uint32_t)h, acc[h], old[h % DEPTH]);
+        if constexpr (LOADS && h + DEPTH < TM) fetch((uint32_t)(h + DEPTH), old[h % DEPTH]);
+        __builtin_amdgcn_sched_barrier(0);   // (left alone, the scheduler starts every block at once and spills)
+      });
     }
     if constexpr (EC == EC_STORE32 || EC == EC_ACC32) {
       // every writer writes the same value: no atomic needed
@@ -596,73 +666,31 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
     }
     if constexpr (EC == EC_DACT16) {
       if (epi.colsum_ws != nullptr) {   // uniform over the grid
-        // lanes l, l + LPR, l + 2 LPR, ... hold the same 8 columns (different rows)
+        // lanes with the same lane % 16 hold the same columns (different rows)
 #pragma unroll
-        for (int off = LPR; off < 64; off <<= 1)
+        for (int off = 16; off < 64; off <<= 1)
 #pragma unroll
-          for (int k = 0; k < 8; ++k) csum[k] += __shfl_xor(csum[k], off, 64);
-        // wavefronts of one block column add up in wavefront-row order through LDS (every wavefront
-        // is done with its own epilogue patch at the barrier; the patch of partial sums lies below
-        // the first wavefront's operand buffers, which the last, unused prefetch may still be filling)
+          for (int k = 0; k < TN; ++k) csum[k] += __shfl_xor(csum[k], off, 64);
+        // wavefronts of one block column add up in wavefront-row order through LDS
         float* red = (float*)smem;
-        static_assert(NWMN * WN * 4 <= HB * SLD * 4, "partial column sums overlap the operand buffers");
         lds_barrier();
-        if (lane < LPR) {
+        if (lane < 16) {
 #pragma unroll
-          for (int k = 0; k < 8; ++k) red[wave * WN + lane * 8 + k] = csum[k];
+          for (int k = 0; k < TN; ++k) red[wave * WN + lane * TN + k] = csum[k];
         }
         lds_barrier();
-        if (wave / WGN == 0 && lane < LPR && c8 < N) {
-          float t[8];
+        if (wave / WGN == 0) {
+          for (int c = lane * 4; c < WN; c += 256) {
+            if (n0 + wn0 + c >= N) continue;
+            float4_t t = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int k = 0; k < 8; ++k) t[k] = 0.f;
-#pragma unroll
-          for (int w = 0; w < WGM; ++w)
-#pragma unroll
-            for (int k = 0; k < 8; ++k) t[k] += red[(w * WGN + wave % WGN) * WN + lane * 8 + k];
-          float* dst = epi.colsum_ws + (int64_t)tm * N + c8;
-          *(float4*)dst = make_float4(t[0], t[1], t[2], t[3]);
-          *(float4*)(dst + 4) = make_float4(t[4], t[5], t[6], t[7]);
+            for (int w = 0; w < WGM; ++w) t += *(const float4_t*)(red + (w * WGN + wave % WGN) * WN + c);
+            *(float4_t*)(epi.colsum_ws + (int64_t)tm * N + n0 + wn0 + c) = t;
+          }
         }
       }
     }
-    return;
   }
-
-#pragma nounroll
-  for (int h = 0; h < TM / RB; ++h) {
-    static_for<TM / RB>([&](auto hc) {
-      constexpr int c = decltype(hc)::value;
-      if (h == c) {
-        static_for<RB>([&](auto ibc) {
-          constexpr int ib = decltype(ibc)::value;
-          static_for<TN>([&](auto jc) {
-            constexpr int j = decltype(jc)::value;
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-              stage[ib * 32 * SLD + wr_off + (8 * (r >> 2) + (r & 3)) * SLD + j * 32] = acc[c * RB + ib][j][r];
-          });
-        });
-      }
-    });
-#pragma nounroll
-    for (int it = 0; it < RB * 32 / RPP; ++it) {
-      const int rr = it * RPP + rd_row;
-      const int64_t row = m0 + wm0 + h * (RB * 32) + rr;
-      if (row >= M || c8 >= N) continue;
-      const float4* src = (const float4*)(stage + rr * SLD + rd_col);
-      const float4 x = src[0], y = src[1];
-      float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
-      if (vec_epi && c8 + 8 <= N) {
-        epilogue_vec8(epi, c_base, row, c8, v);
-      } else {
-#pragma nounroll
-        for (int k = 0; k < 8; ++k)
-          if (c8 + k < N) epilogue_scalar(epi, c_base, row, c8 + k, v[k]);
-      }
-    }
-  }
-  __builtin_amdgcn_s_waitcnt(0x0F70);
 }
 
 #define PF_X_BOUNDS __launch_bounds__(64 * WGM * WGN * KS, (ST * (BM + BN) * BK * 2 <= 80 * 1024 && 64 * WGM * WGN * KS <= 256) ? 2 : 1)
@@ -697,10 +725,7 @@ int launch16x_t(const pf_gemm_desc& d, const GemmGrid& g, hipStream_t st) {
   constexpr int NT = 64 * WGM * WGN * KS;
   constexpr size_t lds_xch = KS == 2 ? (size_t)BM * BN * 4 : 0;   // one grid's partial sums on their way to the other
   constexpr size_t lds_main = ((size_t)ST * (BM + BN) * BK * 2 > lds_xch) ? (size_t)ST * (BM + BN) * BK * 2 : lds_xch;
-  constexpr size_t lds_gen = (size_t)(WGM * WGN) * epi_row_blocks(WGM * WGN, BN / WGN, BM / WGM / 32) * 32 * (BN / WGN + 8) * sizeof(float);
-  constexpr size_t lds_fast = (size_t)(WGM * WGN) * (16 * (BN / WGN + 8) * 4 + 2 * (16 / (64 / (BN / WGN / 8))) * 2 * 1024);
-  constexpr size_t lds_epi = EC == EC_GENERIC ? lds_gen : lds_fast;
-  constexpr size_t lds = lds_main > lds_epi ? lds_main : lds_epi;
+  constexpr size_t lds = lds_main;
   static_assert(lds <= 160 * 1024, "tile pipeline exceeds the 160 KB of LDS");
   auto kern = gemm16x_kernel<DT, BM, BN, BK, WGM, WGN, KS, ST, AT, BT, EC>;
   if (lds > 64 * 1024) {  // opt in to the large LDS carve-out once per instantiation and device
@@ -756,8 +781,8 @@ int launch16x(const pf_gemm_desc& d, hipStream_t st) {
   // transposed (reduction-strided) tiles exist for 128 and 256 rows only
   if constexpr ((BM == 128 || BM == 256) && (BN == 128 || BN == 256)) {
     if (d.a_trans && d.b_trans) {   // weight-gradient products
-      if (ec == EC_ACC32) return PF_X(true, true, EC_ACC32);
-      if (ec == EC_STORE32) return PF_X(true, true, EC_STORE32);
+      if (ec == EC_ACC32 && d.bias == nullptr) return PF_X(true, true, EC_ACC32);
+      if (ec == EC_STORE32 && d.bias == nullptr) return PF_X(true, true, EC_STORE32);
       return PF_X(true, true, EC_GENERIC);
     }
   }
@@ -774,8 +799,7 @@ int launch16x_group(const pf_gemm_desc* d, int n, hipStream_t st) {
     constexpr int NT = 64 * WGM * WGN * KS;
     constexpr size_t lds_xch = KS == 2 ? (size_t)BM * BN * 4 : 0;
     constexpr size_t lds_main = ((size_t)ST * (BM + BN) * BK * 2 > lds_xch) ? (size_t)ST * (BM + BN) * BK * 2 : lds_xch;
-    constexpr size_t lds_fast = (size_t)(WGM * WGN) * (16 * (BN / WGN + 8) * 4 + 2 * (16 / (64 / (BN / WGN / 8))) * 2 * 1024);
-    constexpr size_t lds = lds_main > lds_fast ? lds_main : lds_fast;
+    constexpr size_t lds = lds_main;
     GemmGroup ga;
     int blocks = 0;
     for (int i = 0; i < n; ++i) {

@@ -28,7 +28,7 @@ __global__ __launch_bounds__(256, 1) void mfma_rate_kernel(const uint16_t* __res
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = Mfma<DT>::run8(fa[i], fb[j], acc[i][j]);
+      for (int j = 0; j < 4; ++j) acc[i][j] = Mfma<DT>::run(__builtin_bit_cast(uint4, fa[i]), __builtin_bit_cast(uint4, fb[j]), acc[i][j]);
   }
   float s = 0.f;
 #pragma unroll
