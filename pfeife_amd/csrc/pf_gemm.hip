@@ -20,15 +20,15 @@
   int pf_gemm_x_##DT##_##XT(const pf_gemm_desc& d, hipStream_t st);    \
   int pf_gemm_xgroup_##DT##_##XT(const pf_gemm_desc* d, int n, hipStream_t st);
 #define PF_X_DECL_DT(DT) \
-  PF_X_DECL(DT, 1) PF_X_DECL(DT, 2) PF_X_DECL(DT, 3) PF_X_DECL(DT, 4) PF_X_DECL(DT, 5) PF_X_DECL(DT, 6) PF_X_DECL(DT, 7) PF_X_DECL(DT, 8) PF_X_DECL(DT, 9) PF_X_DECL(DT, 10)
+  PF_X_DECL(DT, 1) PF_X_DECL(DT, 2) PF_X_DECL(DT, 3) PF_X_DECL(DT, 4) PF_X_DECL(DT, 5) PF_X_DECL(DT, 6) PF_X_DECL(DT, 7) PF_X_DECL(DT, 8) PF_X_DECL(DT, 9) PF_X_DECL(DT, 10) PF_X_DECL(DT, 11)
 PF_X_DECL_DT(1)
 PF_X_DECL_DT(2)
 #undef PF_X_DECL_DT
 #undef PF_X_DECL
-static_assert(PF_F16 == 1 && PF_BF16 == 2 && PF_XT_COUNT == 11, "the table below is written out for these ids");
+static_assert(PF_F16 == 1 && PF_BF16 == 2 && PF_XT_COUNT == 12, "the table below is written out for these ids");
 typedef int (*pf_x_fn)(const pf_gemm_desc&, hipStream_t);
 typedef int (*pf_xgroup_fn)(const pf_gemm_desc*, int, hipStream_t);
-#define PF_X_ROW(P, DT) {nullptr, P##DT##_1, P##DT##_2, P##DT##_3, P##DT##_4, P##DT##_5, P##DT##_6, P##DT##_7, P##DT##_8, P##DT##_9, P##DT##_10}
+#define PF_X_ROW(P, DT) {nullptr, P##DT##_1, P##DT##_2, P##DT##_3, P##DT##_4, P##DT##_5, P##DT##_6, P##DT##_7, P##DT##_8, P##DT##_9, P##DT##_10, P##DT##_11}
 static const pf_x_fn pf_x_table[3][PF_XT_COUNT] = {{}, PF_X_ROW(pf_gemm_x_, 1), PF_X_ROW(pf_gemm_x_, 2)};
 static const pf_xgroup_fn pf_xgroup_table[3][PF_XT_COUNT] = {{}, PF_X_ROW(pf_gemm_xgroup_, 1), PF_X_ROW(pf_gemm_xgroup_, 2)};
 #undef PF_X_ROW
@@ -618,10 +618,16 @@ int launch16(const pf_gemm_desc& d, hipStream_t st) {
 // Variant ids (pf_gemm_desc.variant; 0 = automatic):
 //   1..10  direct-to-LDS kernel, tiles PF_XT_256x256 / 256x128 / 128x128 / 192x256 / 128x128k2 / 256x128k2 /
 //          256x256w8 / 128x128w8 / 256x128w8 / 192x256w8
+//   15     direct-to-LDS kernel, tile PF_XT_64x64; 16, 17: 128x128w8 and 256x128w8 for row-major products whose
+//          K is a multiple of 8 only (15 takes these too)
 //   11..14 register-staged kernel: 128x128 by 8 wavefronts, 128x128, 128x64, 64x64 by 4
 enum { V_AUTO = 0, V_X256 = 1, V_X256x128 = 2, V_X128 = 3, V_X192x256 = 4, V_X128K2 = 5, V_X256x128K2 = 6, V_X256W8 = 7, V_X128W8 = 8, V_X256x128W8 = 9, V_X192x256W8 = 10,
-       V_R128W8 = 11, V_R128 = 12, V_R128x64 = 13, V_R64 = 14 };
-inline bool is_x_variant(int v) { return v >= V_X256 && v <= V_X192x256W8; }
+       V_X64 = 15, V_X128W8R = 16, V_X256x128W8R = 17, V_R128W8 = 11, V_R128 = 12, V_R128x64 = 13, V_R64 = 14 };
+inline bool is_x_variant(int v) { return (v >= V_X256 && v <= V_X192x256W8) || (v >= V_X64 && v <= V_X256x128W8R); }
+// tile id (PF_XT_*) of a direct-to-LDS variant
+inline int x_tile_of(int v) {
+  return v == V_X64 ? (int)PF_XT_64x64 : v == V_X128W8R ? (int)PF_XT_128x128w8 : v == V_X256x128W8R ? (int)PF_XT_256x128w8 : v;
+}
 
 // Register-staged tiles: 128x128 with two workgroups resident per CU is the largest that keeps
 // accumulators, two sets of staging registers and fragments in the register file; smaller tiles
@@ -638,47 +644,59 @@ int choose_staged(const pf_gemm_desc& d) {
   return V_R64;
 }
 
-// Can the direct-to-LDS kernel run this problem with tile `xt`?  It takes both operands
+// Can the direct-to-LDS kernel run this problem as variant `v`?  It takes both operands
 // reduction-contiguous or both reduction-strided; a ragged reduction tail is zero-filled by the
-// hardware range check only in the second case (whole k-rows fall outside the operand).
-bool x_supports(const pf_gemm_desc& d, int xt) {
-  const int bk = x_tile_bk(xt);
+// hardware range check in the second case (whole k-rows fall outside the operand), and by a mask on the last
+// tile's loads in the first (some tiles, K a multiple of 8).
+bool x_supports(const pf_gemm_desc& d, int v) {
+  const int xt = x_tile_of(v), bk = x_tile_bk(xt);
   if ((xt == PF_XT_192x256 || xt == PF_XT_192x256w8) && d.a_trans) return false;   // no reduction-strided 192-row tile
   if (d.a_trans != d.b_trans) return false;
-  if (!d.a_trans && d.K % bk != 0) return false;
+  if (!d.a_trans && d.K % bk != 0 && !(v >= V_X64 && d.K % 8 == 0)) return false;
   return d.K >= bk;
 }
 
-// Automatic choice: a small cost model fitted to measurements on MI355X (microseconds).  One
-// workgroup per CU; a tile step of 64 along K costs t64 (MFMA issue for the big tile, operand
-// delivery from L2 for the small ones, which also slow down once every CU streams at the same
-// time); a launch costs ~8 us of fixed latency (dispatch, first tile, epilogue).  The candidates
-// are the eight-wavefront tiles (two wavefronts per SIMD: one's LDS reads, waits and barrier
-// arrivals run under the other's MFMAs; 4-13 % faster than the same tiles shared by four
-// wavefronts on every shape of the five workloads) and the 192x256 tile for outputs that 256-wide
-// row blocks cover badly.  On a sweep of 21 forward / input-gradient shapes of the workloads the
-// choice is the fastest variant or within 3 % of it, but for long reductions: from about 4300
-// deep on, the 256x128 tile whose eight wavefronts split every tile step's depth between two
-// 2 x 2 grids (variant 6) is 4-8 % faster when launches of one shape run back to back (each
-// wavefront reads half the fragment bytes from LDS per MFMA; the exchange of partial sums costs
-// about 3 us).  It is NOT a candidate: inside the pipeline step, with other streams' kernels
-// around it, the Llama and UNet-stage steps that would use it ran 0.7 % slower with it in two
-// A/B runs each, so it stays a variant that can be pinned.
+// Automatic choice: a cost model fitted to measurements on MI355X (microseconds; sweeps of 32 row-major and 21
+// reduction-strided shapes, 16 to 8192 rows).  A workgroup's fixed cost (dispatch, first tile, epilogue) plus, per
+// round of 256 workgroups, K / 64 tile steps; a step gets slower the more CUs stream operands at the same time, so
+// a step costs t0 in an empty device and t0 + t1 in a full one.  The 64x64 tile runs two workgroups to a CU
+// and its cost grows with their number.  On the sweeps the choice is the fastest variant or within 8 % of it.
+// (The tiles whose eight wavefronts split every tile step's depth, variants 5 and 6, are no candidates: inside a
+// pipeline step, next to other streams' kernels, they lost what they gain alone.)
 int choose_variant(const pf_gemm_desc& d) {
   const int64_t nb = d.batch1 * d.batch2;
-  if (d.M < 128 || d.N < 128 || d.M * d.N < 128 * 128 * 16) return choose_staged(d);
-  struct Cand { int v, xt, bm, bn; double t64, t64_busy, fixed; };
-  static const Cand cands[4] = {{V_X256W8, PF_XT_256x256w8, 256, 256, 1.20, 1.20, 8.0},
-                                {V_X192x256W8, PF_XT_192x256w8, 192, 256, 1.05, 1.05, 8.0},
-                                {V_X256x128W8, PF_XT_256x128w8, 256, 128, 0.70, 0.70, 8.0},
-                                {V_X128W8, PF_XT_128x128w8, 128, 128, 0.45, 0.55, 8.0}};
+  struct Cand { int v, bm, bn; double fixed, t0, t1, again; };
+  static const Cand nn[7] = {{V_X256W8, 256, 256, 6.3, 1.05, 0.50, 3.5},
+                             {V_X192x256W8, 192, 256, 5.5, 0.90, 0.40, 3.0},
+                             {V_X256x128W8, 256, 128, 4.5, 0.50, 0.35, 2.0},
+                             {V_X128W8, 128, 128, 3.4, 0.26, 0.27, 1.0},
+                             {V_X256x128W8R, 256, 128, 4.7, 0.52, 0.36, 2.0},   // (ragged K: only where the two above cannot)
+                             {V_X128W8R, 128, 128, 3.5, 0.27, 0.28, 1.0},
+                             {V_X64, 64, 64, 3.0, 0.16, 0.0, 0.6}};
+  static const Cand tt[4] = {{V_X256W8, 256, 256, 6.9, 1.10, 0.55, 3.5},
+                             {V_X256x128W8, 256, 128, 4.8, 0.58, 0.20, 2.0},
+                             {V_X128W8, 128, 128, 3.7, 0.37, 0.17, 1.0},
+                             {V_X64, 64, 64, 3.0, 0.20, 0.0, 0.6}};
+  const bool strided = d.a_trans && d.b_trans;
+  // A weight gradient rarely runs alone: the lowering puts several into one launch once it knows how many
+  // there are, and then the larger tile moves half the bytes.  Alone, 64x64 pays while it fills less than the device.
+  const int64_t t64 = ((d.M + 63) / 64) * ((d.N + 63) / 64) * nb;
   int best = -1;
   double best_t = 0;
-  for (const Cand& c : cands) {
-    if (!x_supports(d, c.xt)) continue;
+  for (int i = 0; i < (strided ? 4 : 7); ++i) {
+    const Cand& c = strided ? tt[i] : nn[i];
+    if (!x_supports(d, c.v)) continue;
+    if (strided && c.v == V_X64 && t64 > 160) continue;
     const int64_t tiles = ((d.M + c.bm - 1) / c.bm) * ((d.N + c.bn - 1) / c.bn) * nb;
-    const int64_t rounds = (tiles + 255) / 256;
-    const double t = c.fixed + (double)rounds * ((double)d.K / 64.0) * (tiles > 256 ? c.t64_busy : c.t64);
+    const int64_t full = tiles / 256, rest = tiles % 256;
+    double step;
+    if (c.v == V_X64) {
+      step = 0.05 + 0.19 * (double)tiles / 256.0;
+      if (step < c.t0) step = c.t0;
+    } else {
+      step = (double)full * (c.t0 + c.t1) + (rest ? c.t0 + c.t1 * (double)rest / 256.0 : 0.0);
+    }
+    const double t = c.fixed + (double)d.K / 64.0 * step + c.again * (double)(full - (rest ? 0 : 1));
     if (best < 0 || t < best_t) { best = c.v; best_t = t; }
   }
   return best < 0 ? choose_staged(d) : best;
@@ -694,12 +712,12 @@ int remap_variant(const pf_gemm_desc& d, int v) {
     const char* e = getenv("PF_GEMM_TILE_MAP");
     while (e && *e) {
       int a = 0, b = 0, used = 0;
-      if (sscanf(e, "%d:%d%n", &a, &b, &used) == 2 && a > 0 && a < PF_XT_COUNT && b > 0 && b < PF_XT_COUNT) map[a] = b;
+      if (sscanf(e, "%d:%d%n", &a, &b, &used) == 2 && a > 0 && a <= V_X192x256W8 && b > 0 && b <= V_X192x256W8) map[a] = b;
       e += used > 0 ? used : 1;
       while (*e == ',' || *e == ' ') ++e;
     }
   });
-  if (!is_x_variant(v)) return v;
+  if (!is_x_variant(v) || v >= V_X64) return v;
   const int w = map[v];
   return (w != v && x_supports(d, w)) ? w : v;
 }
@@ -725,9 +743,9 @@ int dispatch16(const pf_gemm_desc& d, hipStream_t st) {
     }
   }
   switch (v) {
-    case V_X256: case V_X256x128: case V_X128: case V_X192x256: case V_X128K2: case V_X256x128K2: case V_X256W8: case V_X128W8: case V_X256x128W8: case V_X192x256W8: {
-      const int xt = v;   // variant ids 1..10 are the PF_XT_* tile ids
-      if (!x_supports(d, xt)) {
+    case V_X256: case V_X256x128: case V_X128: case V_X192x256: case V_X128K2: case V_X256x128K2: case V_X256W8: case V_X128W8: case V_X256x128W8: case V_X192x256W8: case V_X64: case V_X128W8R: case V_X256x128W8R: {
+      const int xt = x_tile_of(v);
+      if (!x_supports(d, v)) {
         pf_set_error("pf_gemm: variant %d needs both operands stored alike and (unless transposed) K a multiple of the stage depth", v);
         return PF_ERR_INVALID;
       }
@@ -880,7 +898,7 @@ extern "C" int pf_gemm_grouped(const pf_gemm_desc* descs, int n, void* stream) {
         d[k] = descs[i + k];
         d[k].batch1 = d[k].batch2 = 1;
       }
-      const int rc = pf_xgroup_table[descs[i].in_dtype][v0](d, run, (hipStream_t)stream);
+      const int rc = pf_xgroup_table[descs[i].in_dtype][x_tile_of(v0)](d, run, (hipStream_t)stream);
       if (rc != PF_OK) return rc;
       i += run;
     } else {
@@ -907,20 +925,21 @@ extern "C" int pf_gemm_variant(const pf_gemm_desc* desc, char* out, int cap) {
   const char* bt = d.b_trans ? "true" : "false";
   const int v = resolve_variant(d);
   switch (v) {
-    case V_X256: case V_X256x128: case V_X128: case V_X192x256: case V_X128K2: case V_X256x128K2: case V_X256W8: case V_X128W8: case V_X256x128W8: case V_X192x256W8: {
+    case V_X256: case V_X256x128: case V_X128: case V_X192x256: case V_X128K2: case V_X256x128K2: case V_X256W8: case V_X128W8: case V_X256x128W8: case V_X192x256W8: case V_X64: case V_X128W8R: case V_X256x128W8R: {
       // BM, BN, BK, wavefront rows, columns, reduction split, stages: as rocprofv3 prints the instantiation
       static const char* shapes[PF_XT_COUNT] = {"", "256, 256, 32, 2, 2, 1, 5", "256, 128, 64, 2, 2, 1, 3", "128, 128, 64, 2, 2, 1, 3",
                                                 "192, 256, 32, 2, 2, 1, 5", "128, 128, 64, 2, 2, 2, 3", "256, 128, 64, 2, 2, 2, 3",
                                                 "256, 256, 32, 2, 4, 1, 5", "128, 128, 64, 2, 4, 1, 3", "256, 128, 64, 4, 2, 1, 3",
-                                                "192, 256, 32, 2, 4, 1, 5"};
+                                                "192, 256, 32, 2, 4, 1, 5", "64, 64, 64, 2, 2, 1, 5"};
       if (!x_supports(d, v)) {   // a pinned tile that cannot run this product: say so here, not at launch time
         pf_set_error("pf_gemm_variant: variant %d needs both operands stored alike, K >= %d and (unless both are "
-                     "reduction-strided) K a multiple of %d", v, x_tile_bk(v), x_tile_bk(v));
+                     "reduction-strided) K a multiple of %d", v, x_tile_bk(x_tile_of(v)), x_tile_bk(x_tile_of(v)));
         return PF_ERR_INVALID;
       }
       int ec = epi_class(d, epi_vec_ok(d));
       if (d.a_trans && ((ec != EC_ACC32 && ec != EC_STORE32) || d.bias != nullptr)) ec = EC_GENERIC;
-      snprintf(out, (size_t)cap, "gemm16x_kernel<%d, %s, %s, %s, %d>", d.in_dtype, shapes[v], at, bt, ec);
+      const bool ragged = !d.a_trans && d.K % x_tile_bk(x_tile_of(v)) != 0;
+      snprintf(out, (size_t)cap, "gemm16x_%skernel<%d, %s, %s, %s, %d>", ragged ? "ragged_" : "", d.in_dtype, shapes[x_tile_of(v)], at, bt, ec);
       return PF_OK;
     }
     case V_R128W8: snprintf(out, (size_t)cap, "gemm16_kernel<%d, 128, 128, 64, 4, 2, %s, %s>", d.in_dtype, at, bt); return PF_OK;

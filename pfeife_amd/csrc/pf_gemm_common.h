@@ -182,10 +182,10 @@ __device__ __forceinline__ uint4 buf_load16(__amdgpu_buffer_rsrc_t r, uint32_t b
 //   256x128 (64 deep, 3 stages), 128x128 (64 deep, 3 stages): more workgroups for smaller outputs
 //   192x256 (32 deep, 5 stages): for outputs that 256-row blocks cover badly
 //   ids 1-4: four wavefronts (2 x 2); ids 7-10: the same tiles shared by EIGHT wavefronts (2 x 4 or 4 x 2,
-//   two per SIMD); ids 5, 6: 128x128 and 256x128 with eight wavefronts as TWO 2 x 2 grids that
+//   two per SIMD); id 11: 64x64 by four wavefronts, two workgroups to a CU, for small outputs; ids 5, 6: 128x128 and 256x128 with eight wavefronts as TWO 2 x 2 grids that
 //   split every tile's reduction depth between them ("k2")
 enum { PF_XT_256x256 = 1, PF_XT_256x128 = 2, PF_XT_128x128 = 3, PF_XT_192x256 = 4, PF_XT_128x128k2 = 5,
-       PF_XT_256x128k2 = 6, PF_XT_256x256w8 = 7, PF_XT_128x128w8 = 8, PF_XT_256x128w8 = 9, PF_XT_192x256w8 = 10, PF_XT_COUNT = 11 };
+       PF_XT_256x128k2 = 6, PF_XT_256x256w8 = 7, PF_XT_128x128w8 = 8, PF_XT_256x128w8 = 9, PF_XT_192x256w8 = 10, PF_XT_64x64 = 11, PF_XT_COUNT = 12 };
 // BM, BN, reduction depth per stage, stages, wavefront grid (rows x columns x reduction split) of each tile id
 template <int XT> struct XTile;
 template <> struct XTile<PF_XT_256x256> { static constexpr int BM = 256, BN = 256, BK = 32, ST = 5, WGM = 2, WGN = 2, KS = 1; };
@@ -198,6 +198,10 @@ template <> struct XTile<PF_XT_256x256w8> { static constexpr int BM = 256, BN = 
 template <> struct XTile<PF_XT_128x128w8> { static constexpr int BM = 128, BN = 128, BK = 64, ST = 3, WGM = 2, WGN = 4, KS = 1; };
 template <> struct XTile<PF_XT_256x128w8> { static constexpr int BM = 256, BN = 128, BK = 64, ST = 3, WGM = 4, WGN = 2, KS = 1; };
 template <> struct XTile<PF_XT_192x256w8> { static constexpr int BM = 192, BN = 256, BK = 32, ST = 5, WGM = 2, WGN = 4, KS = 1; };
+template <> struct XTile<PF_XT_64x64> { static constexpr int BM = 64, BN = 64, BK = 64, ST = 5, WGM = 2, WGN = 2, KS = 1; };
+// tiles with a kernel for row-major products whose reduction length is no multiple of the stage depth: the
+// eight-wavefront 128x128 and 256x128 tiles and 64x64
+constexpr bool x_tile_ragged(int bm, int bn, int nw) { return (nw == 8 && bn == 128) || (bm == 64 && bn == 64); }
 inline int x_tile_bk(int xt) { return (xt == PF_XT_256x256 || xt == PF_XT_192x256 || xt == PF_XT_256x256w8 || xt == PF_XT_192x256w8) ? 32 : 64; }
 
 // Epilogue classes with straight-line code (which operands exist, and their dtypes, fixed at

@@ -76,18 +76,24 @@ template <int R, int BK, int NW, bool TRANS, int PW> struct DTile {
   static constexpr int ROWB = TRANS ? R * 2 : BK * 2;  // bytes per LDS row
   static constexpr int CPK = R / 8;        // [k][row]: chunks per k-row
   static constexpr int KPI = 64 / CPK;     //           k-rows per instruction
-  static_assert(!TRANS || (R == 128 || R == 256), "transposed tiles are 128 or 256 rows wide");
+  static_assert(!TRANS || R == 64 || R == 128 || R == 256, "transposed tiles are 64, 128 or 256 rows wide");
   static_assert(BK == 64 || BK == 32, "BK is 32 or 64");
 
   static __device__ __forceinline__ int swz_row(int row) { return BK == 64 ? ((row >> 1) & 7) : ((row >> 1) & 3); }
-  static __device__ __forceinline__ int swz_k(int k) { return ((k & 3) << 2) ^ (((k >> 3) & 1) << 1); }
+  // (the four k-rows and two neighbouring k-groups that transposing reads touch together land on different banks;
+  // 64-row tiles have two k-rows per 256 bytes of banks)
+  static __device__ __forceinline__ int swz_k(int k) {
+    return R == 64 ? (((k >> 1) & 1) << 2) ^ (((k >> 3) & 1) << 1) : ((k & 3) << 2) ^ (((k >> 3) & 1) << 1);
+  }
 
   static __device__ __forceinline__ uint32_t extent(int64_t R_total, int64_t K, int64_t ld) {
     return TRANS ? (uint32_t)(((K - 1) * ld + (R_total + 7) / 8 * 8) * 2)
                  : (uint32_t)(((R_total - 1) * ld + (K + 7) / 8 * 8) * 2);
   }
   // byte offset (inside K-tile 0) of the chunk this lane fetches in its q-th instruction
-  static __device__ __forceinline__ void init(uint32_t (&off)[IPW], int64_t ld, int64_t r0, int wave, int lane) {
+  // tail[q]: all ones if that chunk lies past the `left` reduction elements of the last K-tile (RAG kernels)
+  static __device__ __forceinline__ void init(uint32_t (&off)[IPW], uint32_t (&tail)[IPW], int64_t ld, int64_t r0, int left, int wave,
+                                              int lane) {
 #pragma unroll
     for (int q = 0; q < IPW; ++q) {
       const int ii = instr(wave, q);
@@ -96,23 +102,26 @@ template <int R, int BK, int NW, bool TRANS, int PW> struct DTile {
         const int c = (lane % CPR) ^ swz_row(row);
         const int src = PW > 1 ? row / (16 * PW) * (16 * PW) + (row & 15) * PW + (row >> 4) % PW : row;
         off[q] = (uint32_t)(((r0 + src) * ld + c * 8) * 2);
+        tail[q] = c * 8 >= left ? 0xffffffffu : 0u;
       } else {
         const int k = ii * KPI + lane / CPK;
         const int mc = (lane % CPK) ^ swz_k(k);
         off[q] = (uint32_t)((k * ld + r0 + mc * 8) * 2);
+        tail[q] = 0u;   // (whole k-rows past K fall outside the buffer)
       }
     }
   }
   static __device__ __forceinline__ uint32_t tile_step(int64_t ld) { return TRANS ? (uint32_t)(BK * ld * 2) : (uint32_t)(BK * 2); }
   // lds: byte address of this operand's tile inside LDS (wave-uniform); issues the wavefront's
   // instructions Q0 <= q < Q1 (clipped to [0, IPW))
-  template <int Q0, int Q1>
-  static __device__ __forceinline__ void issue(__amdgpu_buffer_rsrc_t rs, const uint32_t (&off)[IPW], uint32_t adv,
-                                               uint32_t lds, int wave) {
+  // (RAG: sel = ~0 for the last K-tile sends the chunks past K out of the buffer's range, which reads zeros)
+  template <int Q0, int Q1, bool RAG>
+  static __device__ __forceinline__ void issue(__amdgpu_buffer_rsrc_t rs, const uint32_t (&off)[IPW], const uint32_t (&tail)[IPW],
+                                               uint32_t adv, uint32_t sel, uint32_t lds, int wave) {
 #pragma unroll
     for (int q = (Q0 < 0 ? 0 : Q0); q < (Q1 > IPW ? IPW : Q1); ++q)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (PF_LDS(void))(uintptr_t)(lds + (uint32_t)instr(wave, q) * 1024u), 16,
-                                               (int)(off[q] + adv), 0, 0, 0);
+                                               (int)(RAG ? (off[q] + adv) | (tail[q] & sel & 0x80000000u) : off[q] + adv), 0, 0, 0);
   }
   // Fragment addressing.  w0: first row of the wavefront's block inside the tile.
   //   [row][k]: foff[kk] = byte offset of (row w0 + lane%16, chunk 4*kk + lane/16); + i*16*ROWB per MFMA tile
@@ -209,7 +218,7 @@ template <int N> struct Words {
 
 // `pid`: index of this workgroup among the workgroups of its problem (the launch may hold several
 // problems, see gemm16x_group_kernel)
-template <int DT, int BM, int BN, int BK, int WGM, int WGN, int KS, int ST, bool AT, bool BT, int EC>
+template <int DT, int BM, int BN, int BK, int WGM, int WGN, int KS, int ST, bool AT, bool BT, int EC, bool RAG = false>
 __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGrid& g, const int pid) {
   // KS = 2: the wavefronts form two WGM x WGN grids; grid h multiplies the h-th half of every
   // tile's 16-deep MFMA groups, and the two partial accumulator blocks are added through LDS
@@ -263,15 +272,14 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
 
   const __amdgpu_buffer_rsrc_t rs_a = make_rsrc(A, TA::extent(M, K, lda));
   const __amdgpu_buffer_rsrc_t rs_b = make_rsrc(B, TB::extent(N, K, ldb));
-  uint32_t offa[TA::IPW], offb[TB::IPW];
-  TA::init(offa, lda, m0, wave, lane);
-  TB::init(offb, ldb, n0, wave, lane);
+  uint32_t offa[TA::IPW], offb[TB::IPW], taila[TA::IPW], tailb[TB::IPW];
+  const int nk = (int)((K + BK - 1) / BK);
+  TA::init(offa, taila, lda, m0, (int)(K - (int64_t)(nk - 1) * BK), wave, lane);
+  TB::init(offb, tailb, ldb, n0, (int)(K - (int64_t)(nk - 1) * BK), wave, lane);
   const uint32_t step_a = TA::tile_step(lda), step_b = TB::tile_step(ldb);
   uint32_t foa[NFA], fob[NFB];
   TA::template frag_init<NFA>(foa, wm0, lane, wave_k * KK);
   TB::template frag_init<NFB>(fob, wn0, lane, wave_k * KK);
-
-  const int nk = (int)((K + BK - 1) / BK);
 
   // This lane's part of C: rows row0 + 16 i + r (r = 0..3); columns c0 .. c0 + TN - 1, one per MFMA tile, of a
   // row-major product (see DTile's PW), c0 + 16 j of a reduction-strided one (the transposing LDS reads fix
@@ -313,9 +321,10 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
   // memory pipeline's queue and stall the wavefront for as long as the tile takes to stream in.
   static_assert(ST >= 3, "a stage is refilled while the next tile is multiplied");
   auto adv_of = [&](int kt, uint32_t step) { return kt < nk ? (uint32_t)kt * step : 0x80000000u; };
+  auto sel_of = [&](int kt) { return RAG && kt == nk - 1 ? 0xffffffffu : 0u; };
   auto issue_all = [&](int kt, uint32_t sb) {
-    TA::template issue<0, TA::IPW>(rs_a, offa, adv_of(kt, step_a), sb, wave);
-    TB::template issue<0, TB::IPW>(rs_b, offb, adv_of(kt, step_b), sb + TA::BYTES, wave);
+    TA::template issue<0, TA::IPW, RAG>(rs_a, offa, taila, adv_of(kt, step_a), sel_of(kt), sb, wave);
+    TB::template issue<0, TB::IPW, RAG>(rs_b, offb, tailb, adv_of(kt, step_b), sel_of(kt), sb + TA::BYTES, wave);
   };
   // One 32-deep MFMA group ("phase") = NM matrix instructions on the fragments in register set `cur`, the
   // LDS reads that fill the other set for the next phase, and its share of the loads that refill the
@@ -347,7 +356,7 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
       });
     }
     constexpr int NS = NM > 8 ? NM * 7 / 8 : NM;
-    const uint32_t adv_a = adv_of(ktl, step_a), adv_b = adv_of(ktl, step_b);
+    const uint32_t adv_a = adv_of(ktl, step_a), adv_b = adv_of(ktl, step_b), sel = sel_of(ktl);
     if constexpr (AT && BT && SINGLE) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
@@ -365,8 +374,8 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
           constexpr int l0 = e * NL / NE, l1 = (e + 1) * NL / NE;
           if constexpr (l1 > l0) {
             constexpr int q = Q0 + l0;                   // index into A's then B's list of loads
-            if constexpr (q < TA::IPW) TA::template issue<q, q + 1>(rs_a, offa, adv_a, sbl, wave);
-            else TB::template issue<q - TA::IPW, q - TA::IPW + 1>(rs_b, offb, adv_b, sbl + TA::BYTES, wave);
+            if constexpr (q < TA::IPW) TA::template issue<q, q + 1, RAG>(rs_a, offa, taila, adv_a, sel, sbl, wave);
+            else TB::template issue<q - TA::IPW, q - TA::IPW + 1, RAG>(rs_b, offb, tailb, adv_b, sel, sbl + TA::BYTES, wave);
           } else {
             constexpr int r = e - l0;                    // B's fragments first, then A's
             if constexpr (r < TN * TB::NRD) TB::template read<NFB, r / TB::NRD, kkn, r % TB::NRD>(fb[slot][r / TB::NRD], sbr + TA::BYTES, fob);
@@ -402,14 +411,15 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
   constexpr int P0 = SINGLE ? 0 : LPW / KK;    // loads of tile ST - 1 that go out here
   {
     const uint32_t sbl = lds0 + (uint32_t)(ST - 1) * STAGE, adv_a = adv_of(ST - 1, step_a), adv_b = adv_of(ST - 1, step_b);
-    TA::template issue<0, P0>(rs_a, offa, adv_a, sbl, wave);
-    TB::template issue<0, P0 - TA::IPW>(rs_b, offb, adv_b, sbl + TA::BYTES, wave);
+    TA::template issue<0, P0, RAG>(rs_a, offa, taila, adv_a, sel_of(ST - 1), sbl, wave);
+    TB::template issue<0, P0 - TA::IPW, RAG>(rs_b, offb, tailb, adv_b, sel_of(ST - 1), sbl + TA::BYTES, wave);
   }
   wait_vm<(ST - 2) * LPW + P0>();
   lds_barrier();
   if constexpr (!SINGLE) {
-    static_for<TM>([&](auto ic) { TA::template read_first<NFA, decltype(ic)::value>(fa[0][decltype(ic)::value], lds0, foa); });
+    // (B's first: the phases count on that order when they wait for part of the reads)
     static_for<TN>([&](auto jc) { TB::template read_first<NFB, decltype(jc)::value>(fb[0][decltype(jc)::value], lds0 + TA::BYTES, fob); });
+    static_for<TM>([&](auto ic) { TA::template read_first<NFA, decltype(ic)::value>(fa[0][decltype(ic)::value], lds0, foa); });
   }
   __builtin_amdgcn_sched_barrier(0);
 
@@ -699,6 +709,13 @@ __global__ PF_X_BOUNDS void gemm16x_kernel(const pf_gemm_desc p, const GemmGrid 
   gemm16x_body<DT, BM, BN, BK, WGM, WGN, KS, ST, AT, BT, EC>(p, g, (int)blockIdx.x);
 }
 
+// Row-major products whose reduction length is a multiple of 8 but not of the stage depth (head dimensions 80 and
+// 88 give such widths): a kernel of its own, the mask costs an instruction and a register per load.
+template <int DT, int BM, int BN, int BK, int WGM, int WGN, int KS, int ST, bool AT, bool BT, int EC>
+__global__ PF_X_BOUNDS void gemm16x_ragged_kernel(const pf_gemm_desc p, const GemmGrid g) {
+  gemm16x_body<DT, BM, BN, BK, WGM, WGN, KS, ST, AT, BT, EC, true>(p, g, (int)blockIdx.x);
+}
+
 // Several independent problems of the same kind in one launch: problem i owns the workgroups
 // [start[i], start[i+1]).  Weight-gradient products are independent of everything that follows
 // them in a backward job; small ones (64 tiles for a 1024x1024 weight) are launched together so
@@ -720,14 +737,16 @@ __global__ PF_X_BOUNDS void gemm16x_group_kernel(const GemmGroup ga) {
   gemm16x_body<DT, BM, BN, BK, WGM, WGN, KS, ST, AT, BT, EC>(ga.p[i], ga.g[i], (int)blockIdx.x - ga.start[i]);
 }
 
-template <int DT, int BM, int BN, int BK, int WGM, int WGN, int KS, int ST, bool AT, bool BT, int EC>
+template <int DT, int BM, int BN, int BK, int WGM, int WGN, int KS, int ST, bool AT, bool BT, int EC, bool RAG>
 int launch16x_t(const pf_gemm_desc& d, const GemmGrid& g, hipStream_t st) {
   constexpr int NT = 64 * WGM * WGN * KS;
   constexpr size_t lds_xch = KS == 2 ? (size_t)BM * BN * 4 : 0;   // one grid's partial sums on their way to the other
   constexpr size_t lds_main = ((size_t)ST * (BM + BN) * BK * 2 > lds_xch) ? (size_t)ST * (BM + BN) * BK * 2 : lds_xch;
   constexpr size_t lds = lds_main;
   static_assert(lds <= 160 * 1024, "tile pipeline exceeds the 160 KB of LDS");
-  auto kern = gemm16x_kernel<DT, BM, BN, BK, WGM, WGN, KS, ST, AT, BT, EC>;
+  void (*kern)(const pf_gemm_desc, const GemmGrid);
+  if constexpr (RAG) kern = gemm16x_ragged_kernel<DT, BM, BN, BK, WGM, WGN, KS, ST, AT, BT, EC>;
+  else kern = gemm16x_kernel<DT, BM, BN, BK, WGM, WGN, KS, ST, AT, BT, EC>;
   if (lds > 64 * 1024) {  // opt in to the large LDS carve-out once per instantiation and device
     static std::mutex mu;
     static bool raised[64] = {};
@@ -759,12 +778,31 @@ int launch16x(const pf_gemm_desc& d, hipStream_t st) {
   g.vec_epi = epi_vec_ok(d);
   // A ragged reduction tail is zero-filled by the hardware range check only when whole k-rows
   // fall outside the operand, i.e. when both operands are stored [k][row].
-  if (d.K % BK != 0 && !(d.a_trans && d.b_trans)) {
+  const bool ragged = d.K % BK != 0 && !(d.a_trans && d.b_trans);
+  constexpr bool HAS_RAGGED = x_tile_ragged(BM, BN, WGM * WGN);
+  if (ragged && !(HAS_RAGGED && d.K % 8 == 0)) {
     pf_set_error("pf_gemm: this variant needs K %% %d == 0 unless both operands are transposed", BK);
     return PF_ERR_INVALID;
   }
   const int ec = epi_class(d, g.vec_epi);
-#define PF_X(AT, BT, EC) launch16x_t<DT, BM, BN, BK, WGM, WGN, KS, ST, AT, BT, EC>(d, g, st)
+#define PF_X(AT, BT, EC) launch16x_t<DT, BM, BN, BK, WGM, WGN, KS, ST, AT, BT, EC, false>(d, g, st)
+#define PF_XR(EC) launch16x_t<DT, BM, BN, BK, WGM, WGN, KS, ST, false, false, EC, HAS_RAGGED>(d, g, st)
+  if constexpr (HAS_RAGGED) {
+    if (ragged) {
+      if (d.a_trans || d.b_trans) return PF_ERR_INVALID;
+      switch (ec) {
+        case EC_STORE16: return PF_XR(EC_STORE16);
+        case EC_STORE32: return PF_XR(EC_STORE32);
+        case EC_ACT16: return PF_XR(EC_ACT16);
+        case EC_RES32: return PF_XR(EC_RES32);
+        case EC_ACC32: return PF_XR(EC_ACC32);
+        case EC_DACT16: return PF_XR(EC_DACT16);
+        case EC_ACC16: return PF_XR(EC_ACC16);
+        case EC_RES16: return PF_XR(EC_RES16);
+        default: return PF_XR(EC_GENERIC);
+      }
+    }
+  }
   if (!d.a_trans && !d.b_trans) {   // forward and input-gradient products
     switch (ec) {
       case EC_STORE16: return PF_X(false, false, EC_STORE16);
@@ -779,7 +817,7 @@ int launch16x(const pf_gemm_desc& d, hipStream_t st) {
     }
   }
   // transposed (reduction-strided) tiles exist for 128 and 256 rows only
-  if constexpr ((BM == 128 || BM == 256) && (BN == 128 || BN == 256)) {
+  if constexpr (BM != 192) {
     if (d.a_trans && d.b_trans) {   // weight-gradient products
       if (ec == EC_ACC32 && d.bias == nullptr) return PF_X(true, true, EC_ACC32);
       if (ec == EC_STORE32 && d.bias == nullptr) return PF_X(true, true, EC_STORE32);
@@ -787,6 +825,7 @@ int launch16x(const pf_gemm_desc& d, hipStream_t st) {
     }
   }
 #undef PF_X
+#undef PF_XR
   pf_set_error("pf_gemm: tile %dx%d has no variant for a_trans=%d b_trans=%d", BM, BN, d.a_trans, d.b_trans);
   return PF_ERR_INVALID;
 }
@@ -795,7 +834,7 @@ int launch16x(const pf_gemm_desc& d, hipStream_t st) {
 // launch; the caller has checked that they all take tile BMxBN and the EC_ACC32 epilogue.
 template <int DT, int BM, int BN, int BK, int WGM, int WGN, int KS, int ST>
 int launch16x_group(const pf_gemm_desc* d, int n, hipStream_t st) {
-  if constexpr ((BM == 128 || BM == 256) && (BN == 128 || BN == 256)) {
+  if constexpr (BM != 192) {
     constexpr int NT = 64 * WGM * WGN * KS;
     constexpr size_t lds_xch = KS == 2 ? (size_t)BM * BN * 4 : 0;
     constexpr size_t lds_main = ((size_t)ST * (BM + BN) * BK * 2 > lds_xch) ? (size_t)ST * (BM + BN) * BK * 2 : lds_xch;

@@ -34,6 +34,7 @@ ACT_NONE, ACT_GELU, ACT_GELU_TANH, ACT_SILU, ACT_RELU = 0, 1, 2, 3, 4
 # tile the automatic choice itself uses (eight wavefronts), so that products that chose it on their own and
 # products moved onto it share launches
 BIG_TILE_VARIANT = int(os.environ.get("PFEIFE_BIG_TILE", "7"))
+MID_TILE_VARIANT, SMALL_TILE_VARIANT = 8, 15    # 128x128 and 64x64
 
 
 class Unsupported(RuntimeError):
@@ -425,8 +426,18 @@ class BwdCtx:
 
     @staticmethod
     def _tiles(launch):
-        bm, bn = (int(x) for x in launch.variant.split("<")[1].split(",")[1:3])
-        return ((launch.desc.M + bm - 1) // bm) * ((launch.desc.N + bn - 1) // bn)
+        return ((launch.desc.M + 127) // 128) * ((launch.desc.N + 127) // 128)
+
+    def _retile_held(self, launches):
+        """The held products on the tile that suits how many there are.  On 64x64 tiles a step of 64 rows costs
+        0.2 us while the device has room and grows with the number of tiles, on 128x128 tiles 0.37-0.54 us
+        (measured): the small tile is ahead up to about 112 tiles of 128x128 in all."""
+        retile = getattr(self.k, "gemm_retiled", None)
+        if retile is None:
+            return launches
+        want = SMALL_TILE_VARIANT if sum(self._tiles(l) for l in launches) <= 112 else MID_TILE_VARIANT
+        new = [retile(l, want) for l in launches]
+        return launches if any(l is None or not self.k.gemm_groupable(l) for l in new) else new
 
     def emit_dw(self, launch, grad):
         """A weight-gradient product: only the optimizer reads its result, and its inputs (a
@@ -448,7 +459,7 @@ class BwdCtx:
             self._offer_big(launch, [(launch, grad)])
             return
         held = sum(t for _, _, t in self._dw)
-        if self._dw and (self._dw[0][0].group_key != launch.group_key or held + tiles > self.FULL_GRID
+        if self._dw and (self._dw[0][0].desc.in_dtype != launch.desc.in_dtype or held + tiles > self.FULL_GRID
                          or len(self._dw) == self.k.GEMM_GROUP_MAX):
             self.flush_dw()
             held = 0
@@ -522,14 +533,18 @@ class BwdCtx:
             self._close_set(self._dw_big[0])
 
     def flush_dw(self):
-        if len(self._dw) == 1:
-            self.emit(self._dw[0][0])
-            self._offer_big(self._dw[0][0], [(self._dw[0][0], self._dw[0][1])])
-        elif self._dw:
-            group = self.k.gemm_group([l for l, _, _ in self._dw])
-            self.emit(group)
-            self._offer_big(group, [(l, g) for l, g, _ in self._dw])
+        if not self._dw:
+            return
+        launches, grads = self._retile_held([l for l, _, _ in self._dw]), [g for _, g, _ in self._dw]
         self._dw = []
+        if len(launches) > 1 and len({l.group_key for l in launches}) > 1:   # (a tile that cannot run one of them)
+            for launch, grad in zip(launches, grads):
+                self.emit(launch)
+                self._offer_big(launch, [(launch, grad)])
+            return
+        issued = launches[0] if len(launches) == 1 else self.k.gemm_group(launches)
+        self.emit(issued)
+        self._offer_big(issued, list(zip(launches, grads)))
 
     def register_lp(self, full, copy, colsum=None):
         """`copy` holds the values of the fp32 gradient `full` in the compute dtype; `colsum`:

@@ -321,7 +321,7 @@ class HipKernels:
         launch runs on another kernel."""
         v = getattr(launch, "variant", "")
         d = getattr(launch, "desc", None)
-        if d is None or not (v.startswith("gemm16x_kernel<") and v.endswith(", false, false, 5>")):
+        if d is None or not (v.startswith(("gemm16x_kernel<", "gemm16x_ragged_kernel<")) and v.endswith(", false, false, 5>")):
             return None
         if d.batch1 * d.batch2 != 1 or d.colsum_ws:
             return None

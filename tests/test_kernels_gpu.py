@@ -228,6 +228,71 @@ def test_gemm_gelu_grad_epilogue_leaves_column_sums(hip, dtype, variant, bm):
         other(torch.cuda.current_stream().cuda_stream)
 
 
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("variant,tile,K", [(10, "192, 256, 32, 2, 4, 1, 5", 320), (15, "64, 64, 64, 2, 2, 1, 5", 320),
+                                            (15, "64, 64, 64, 2, 2, 1, 5", 88), (15, "64, 64, 64, 2, 2, 1, 5", 1320),
+                                            (16, "128, 128, 64, 2, 4, 1, 3", 72), (16, "128, 128, 64, 2, 4, 1, 3", 1144),
+                                            (17, "256, 128, 64, 4, 2, 1, 3", 328)])
+@pytest.mark.parametrize("M,N", [(1, 8), (63, 72), (65, 200), (1000, 1160)])
+def test_gemm_small_and_ragged_direct_to_lds_tiles(hip, oracle, dtype, variant, tile, K, M, N):
+    """The eight-wavefront 192x256 tile, the 64x64 tile, and the kernels for a row-major reduction that is no
+    multiple of the stage depth: every epilogue class, outputs from a single row to ragged ones, operands whose
+    rows are wider than the reduction (what lies behind a row's end must not get into its products)."""
+    dt = {F16: 1, BF16: 2}[dtype]
+    rt, at = TOL[dtype]
+    x, w = rnd((M, K + 8), dtype, 1), rnd((N, K + 16), dtype, 2, 0.1)
+    x[:, K:], w[:, K:] = float("nan"), float("nan")
+    bias = rnd((N,), dtype, 3)
+    name = "gemm16x_%skernel<%d, %s, false, false, %%d>" % ("ragged_" if K % int(tile.split(", ")[2]) else "", dt, tile)
+
+    def run(ec, tensors, outs, rtol, atol, **kw):
+        print("gemm variant", variant, "class", ec, M, N, K, flush=True)
+        dev = {k: v.cuda() for k, v in tensors.items()}
+        cpu = {k: v.clone() for k, v in tensors.items()}
+        launch = hip.gemm(**dev, variant=variant, **kw)
+        assert launch.variant == name % ec, launch.variant
+        launch(torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        oracle.gemm(**cpu, **kw)()
+        for o in outs:
+            close((dev[o].cpu(), cpu[o]), rtol, atol)
+
+    base = dict(M=M, N=N, K=K, lda=K + 8, ldb=K + 16, ldc=N)
+    z16 = lambda: torch.zeros(M, N, dtype=dtype)
+    run(0, dict(a=x, b=w, c=z16(), bias=bias), ["c"], rt, at * 2, round_mid=1, **base)
+    run(1, dict(a=x, b=w, c=torch.zeros(M, N), bias=rnd((N,), F32, 3)), ["c"], 1e-3, 1e-2, **base)
+    run(2, dict(a=x, b=w, c=z16(), bias=bias, aux_out=z16()), ["c", "aux_out"], rt, at * 2, round_mid=1, act=1, ld_aux_out=N, **base)
+    run(3, dict(a=x, b=w, c=torch.zeros(M, N), bias=bias, residual=rnd((M, N), F32, 4)), ["c"], rt, at * 2, round_mid=1, ld_res=N, **base)
+    run(4, dict(a=x, b=w, c=rnd((M, N), F32, 5)), ["c"], 1e-3, 1e-2, beta=1, **base)
+    run(5, dict(a=x, b=w, c=z16(), aux_in=rnd((M, N), dtype, 6)), ["c"], rt, at * 4, dact=1, ld_aux_in=N, **base)
+    run(6, dict(a=x, b=w, c=rnd((M, N), dtype, 7)), ["c"], rt, at * 4, beta=1, **base)
+    run(7, dict(a=x, b=w, c=z16(), bias=bias, residual=rnd((M, N + 8), dtype, 8)), ["c"], rt, at * 4, round_mid=1, ld_res=N + 8, **base)
+    run(-1, dict(a=x, b=w, c=z16(), bias=bias, aux_out=z16()), ["c"], rt, at * 4, round_mid=1, act=3, ld_aux_out=N, **base)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("rows,M,N", [(64, 8, 8), (100, 72, 136), (333, 520, 72)])
+def test_gemm_weight_gradients_on_64x64_tiles(hip, oracle, dtype, rows, M, N):
+    """The reduction-strided form of the 64x64 tile, stored and accumulated, alone and grouped."""
+    dy, x = rnd((rows, M), dtype, 1), rnd((rows, N), dtype, 2, 0.1)
+    s = torch.cuda.current_stream().cuda_stream
+    kw = dict(M=M, N=N, K=rows, lda=M, ldb=N, ldc=N, a_trans=1, b_trans=1)
+    launches, outs = [], []
+    for beta in (0, 1):
+        c0 = rnd((M, N), F32, 3 + beta)
+        dev, both_c = c0.clone().cuda(), c0.clone().cuda()
+        hip.gemm(dy.cuda(), x.cuda(), dev, beta=beta, variant=15, **kw)(s)
+        launches.append(hip.gemm(dy.cuda(), x.cuda(), both_c, beta=beta, variant=15, **kw))
+        cpu = c0.clone()
+        oracle.gemm(dy, x, cpu, beta=beta, **kw)()
+        outs.append((dev, both_c, cpu))
+    hip.gemm_group(launches)(s)
+    torch.cuda.synchronize()
+    for dev, both_c, cpu in outs:
+        close((dev.cpu(), cpu), 1e-3, 2e-2)
+        assert torch.equal(dev, both_c)
+
+
 def test_gemm_full_size_vit_l(hip, oracle):
     # qkv projection of ViT-L/16 at micro-batch 16: [3152 x 1024] . [1024 x 3072]
     M, N, K = 3152, 3072, 1024
