@@ -393,15 +393,16 @@ __global__ __launch_bounds__(256) void gemm32_kernel(const pf_gemm_desc p, const
 }
 
 // ---------------------------------------------------------------------------
-// fp32 MFMA kernel (v_mfma_f32_32x32x2_f32): BM x BN tile, TK deep, four wavefronts as 2 x 2, each
+// fp32 MFMA kernel (v_mfma_f32_32x32x2_f32) for operands that are not 16-byte aligned (everything else runs on
+// gemm32d_kernel): BM x BN tile, TK deep, four wavefronts as 2 x 2, each
 // owning (BM/2) x (BN/2) outputs.  Operand tiles sit in LDS reduction-major ([k][row], the order in
 // which a lane reads its one element per matrix instruction: row = lane % 32, k = lane / 32); the
 // next tile is fetched into registers while the current one is multiplied (two LDS buffers where
-// they fit, else one and a second barrier).  The small tile is 64 deep: its problems leave one
-// workgroup per CU, so a tile's matrix work has to cover the latency of the next tile's loads.
+// they fit, else one and a second barrier).  The tile is 64 deep so that its matrix work covers the
+// latency of the next tile's loads.
 // Any layout and any size: rows / reduction indices out of range read as zero.
 // ---------------------------------------------------------------------------
-template <int BM, int BN, int TK, bool AT, bool BT, bool VEC>
+template <int BM, int BN, int TK, bool AT, bool BT>
 __global__ __launch_bounds__(256) void gemm32x_kernel(const pf_gemm_desc p, const GemmGrid g) {
   constexpr int PAD = 4;
   constexpr int NBUF = (2 * TK * (BM + BN + 2 * PAD) * 4 <= 60 * 1024) ? 2 : 1;
@@ -431,8 +432,7 @@ __global__ __launch_bounds__(256) void gemm32x_kernel(const pf_gemm_desc p, cons
   // (reduction index for a row-major operand, row index for a reduction-strided one).  No branches:
   // indices are clamped into the operand and out-of-range elements are zeroed afterwards, so all of
   // a tile's loads are in flight together (a branch around a load makes the compiler wait for it at
-  // the join).  VEC: one 16-byte load (the launcher has checked alignment and that the extent along
-  // the contiguous dimension is a multiple of 4, so a group of 4 is inside or outside as a whole).
+  // the join).
   auto fetch = [&](const float* X, int64_t ld, auto trans_c, int64_t r0, int64_t R, int64_t k0, int rows, int q,
                    float (&v)[4]) {
     constexpr bool TR = decltype(trans_c)::value;
@@ -440,21 +440,13 @@ __global__ __launch_bounds__(256) void gemm32x_kernel(const pf_gemm_desc p, cons
     int r, k;
     if (TR) { r = (e % (rows / 4)) * 4; k = e / (rows / 4); } else { k = (e % (TK / 4)) * 4; r = e / (TK / 4); }
     const int64_t gr = r0 + r, gk = k0 + k;
-    if (VEC) {
-      const bool ok = gr < R && gk < K;
-      const int64_t cr = TR ? (gr < R ? gr : R - 4) : (gr < R ? gr : R - 1);
-      const int64_t ck = TR ? (gk < K ? gk : K - 1) : (gk < K ? gk : K - 4);
-      const float4 x = *(const float4*)(X + (TR ? ck * ld + cr : cr * ld + ck));
-      v[0] = ok ? x.x : 0.f; v[1] = ok ? x.y : 0.f; v[2] = ok ? x.z : 0.f; v[3] = ok ? x.w : 0.f;
-    } else {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int64_t er = TR ? gr + j : gr, ek = TR ? gk : gk + j;
-        const bool ok = er < R && ek < K;
-        const int64_t cr = er < R ? er : R - 1, ck = ek < K ? ek : K - 1;
-        const float x = X[TR ? ck * ld + cr : cr * ld + ck];
-        v[j] = ok ? x : 0.f;
-      }
+    for (int j = 0; j < 4; ++j) {
+      const int64_t er = TR ? gr + j : gr, ek = TR ? gk : gk + j;
+      const bool ok = er < R && ek < K;
+      const int64_t cr = er < R ? er : R - 1, ck = ek < K ? ek : K - 1;
+      const float x = X[TR ? ck * ld + cr : cr * ld + ck];
+      v[j] = ok ? x : 0.f;
     }
   };
   auto stash = [&](float* S, int ldS, auto trans_c, int rows, int q, const float (&v)[4]) {   // S: [TK][ldS]
@@ -563,16 +555,6 @@ __global__ __launch_bounds__(256) void gemm32x_kernel(const pf_gemm_desc p, cons
       }
     }
   }
-}
-
-// fp32 problems: the matrix-instruction kernel with 128x128 tiles when those fill the GPU, with 64x64
-// tiles otherwise (also for a handful of rows: its staged epilogue beats the FMA kernel's element-wise
-// one); the plain FMA kernel for an empty reduction.
-inline int f32_variant(const pf_gemm_desc& d) {
-  if (d.K < 1) return 0;
-  const int64_t nb = (d.batch1 > 0 ? d.batch1 : 1) * (d.batch2 > 0 ? d.batch2 : 1);
-  const int64_t t128 = ((d.M + 127) / 128) * ((d.N + 127) / 128) * nb;
-  return t128 >= 192 ? 128 : 64;
 }
 
 template <int DT, int BM, int BN, int BK, int WGM, int WGN>
@@ -797,39 +779,18 @@ extern "C" int pf_gemm(const pf_gemm_desc* desc, void* stream) {
       pf_set_error("pf_gemm: unscale_by / nonfinite_flag need a 16-bit product");
       return PF_ERR_UNSUPPORTED;
     }
+    if (pf_gemm_f32_direct_ok(d)) return pf_gemm_f32_direct(d, st);
     GemmGrid g;
-    g.vec_epi = 0;
-    const int v32 = f32_variant(d);
-    if (v32 == 0) {
-      g.tiles_m = (int)tm64;
-      g.tiles_n = (int)tn64;
-      g.per_xcd = (int)((tm64 * tn64 + 7) / 8);
-      hipLaunchKernelGGL(gemm32_kernel, dim3((unsigned)(g.per_xcd * 8), (unsigned)nb, 1), dim3(256), 0, st, d, g);
-    } else {
-      g.tiles_m = (int)((d.M + v32 - 1) / v32);
-      g.tiles_n = (int)((d.N + v32 - 1) / v32);
-      g.per_xcd = (int)(((int64_t)g.tiles_m * g.tiles_n + 7) / 8);
-      g.vec_epi = epi_vec_ok(d);
-      const dim3 grid((unsigned)(g.per_xcd * 8), (unsigned)nb, 1);
-      // 16-byte loads need aligned operands whose extent along the contiguous dimension is a multiple of 4
-      const bool vec = pf_aligned(d.A, 16) && pf_aligned(d.B, 16) && d.lda % 4 == 0 && d.ldb % 4 == 0 &&
-                       d.a_stride1 % 4 == 0 && d.a_stride2 % 4 == 0 && d.b_stride1 % 4 == 0 && d.b_stride2 % 4 == 0 &&
-                       (d.a_trans ? d.M : d.K) % 4 == 0 && (d.b_trans ? d.N : d.K) % 4 == 0 && d.K >= 4 && d.M >= 4 && d.N >= 4;
-#define PF_G32(BMN, TK, AT, BT, V) hipLaunchKernelGGL((gemm32x_kernel<BMN, BMN, TK, AT, BT, V>), grid, dim3(256), 0, st, d, g)
-#define PF_G32V(BMN, TK, AT, BT) do { if (vec) PF_G32(BMN, TK, AT, BT, true); else PF_G32(BMN, TK, AT, BT, false); } while (0)
-#define PF_G32L(BMN, TK)                                   \
-  do {                                                     \
-    if (d.a_trans && d.b_trans) PF_G32V(BMN, TK, true, true);   \
-    else if (d.a_trans) PF_G32V(BMN, TK, true, false);          \
-    else if (d.b_trans) PF_G32V(BMN, TK, false, true);          \
-    else PF_G32V(BMN, TK, false, false);                        \
-  } while (0)
-      if (v32 == 128) PF_G32L(128, 16);
-      else PF_G32L(64, 64);
-#undef PF_G32L
-#undef PF_G32V
-#undef PF_G32
-    }
+    g.tiles_m = (int)tm64;
+    g.tiles_n = (int)tn64;
+    g.per_xcd = (int)((tm64 * tn64 + 7) / 8);
+    g.vec_epi = epi_vec_ok(d);
+    const dim3 grid((unsigned)(g.per_xcd * 8), (unsigned)nb, 1);
+    if (d.K == 0) hipLaunchKernelGGL(gemm32_kernel, grid, dim3(256), 0, st, d, g);
+    else if (d.a_trans && d.b_trans) hipLaunchKernelGGL((gemm32x_kernel<64, 64, 64, true, true>), grid, dim3(256), 0, st, d, g);
+    else if (d.a_trans) hipLaunchKernelGGL((gemm32x_kernel<64, 64, 64, true, false>), grid, dim3(256), 0, st, d, g);
+    else if (d.b_trans) hipLaunchKernelGGL((gemm32x_kernel<64, 64, 64, false, true>), grid, dim3(256), 0, st, d, g);
+    else hipLaunchKernelGGL((gemm32x_kernel<64, 64, 64, false, false>), grid, dim3(256), 0, st, d, g);
     PF_CHECK_LAUNCH("pf_gemm(f32)");
     return PF_OK;
   }
@@ -916,9 +877,10 @@ extern "C" int pf_gemm_variant(const pf_gemm_desc* desc, char* out, int cap) {
   if (d.batch1 <= 0) d.batch1 = 1;
   if (d.batch2 <= 0) d.batch2 = 1;
   if (d.in_dtype == PF_F32 || d.K == 0) {
-    const int v32 = (d.in_dtype == PF_F32 && d.K > 0) ? f32_variant(d) : 0;
-    if (v32) snprintf(out, (size_t)cap, "gemm32x_kernel<%d, %d, %d>", v32, v32, v32 == 128 ? 16 : 64);
-    else snprintf(out, (size_t)cap, "gemm32_kernel");
+    if (d.in_dtype != PF_F32 || d.K == 0) snprintf(out, (size_t)cap, "gemm32_kernel");
+    else if (pf_gemm_f32_direct_ok(d))
+      snprintf(out, (size_t)cap, "gemm32d_kernel<%s, %s, %s>", pf_gemm_f32_direct_shape(d), d.a_trans ? "true" : "false", d.b_trans ? "true" : "false");
+    else snprintf(out, (size_t)cap, "gemm32x_kernel<64, 64, 64>");
     return PF_OK;
   }
   const char* at = d.a_trans ? "true" : "false";

@@ -240,3 +240,8 @@ inline int epi_class(const pf_gemm_desc& d, int vec_ok) {
 }
 
 }  // namespace
+
+// pf_gemm_f32.hip: fp32 products straight from 16-byte-aligned operands
+bool pf_gemm_f32_direct_ok(const pf_gemm_desc& d);
+const char* pf_gemm_f32_direct_shape(const pf_gemm_desc& d);
+int pf_gemm_f32_direct(const pf_gemm_desc& d, hipStream_t st);

@@ -270,6 +270,44 @@ def test_gemm_small_and_ragged_direct_to_lds_tiles(hip, oracle, dtype, variant, 
     run(-1, dict(a=x, b=w, c=z16(), bias=bias, aux_out=z16()), ["c"], rt, at * 4, round_mid=1, act=3, ld_aux_out=N, **base)
 
 
+@pytest.mark.parametrize("a_trans", [0, 1])
+@pytest.mark.parametrize("b_trans", [0, 1])
+@pytest.mark.parametrize("tile,M,N,K", [("32, 32, 2, 2, 8", 3, 5, 1), ("32, 32, 2, 2, 8", 33, 197, 67), ("32, 64, 2, 4, 6", 481, 1001, 31),
+                                        ("64, 64, 4, 2, 4", 1000, 1021, 97), ("128, 128, 2, 4, 4", 2047, 2030, 129)])
+def test_gemm_fp32_direct_to_lds_tiles(hip, oracle, tile, M, N, K, a_trans, b_trans):
+    """Every tile and layout of the fp32 kernel, reductions that end inside a tile and inside a 16-byte chunk, rows
+    wider than the operand (what lies behind a row's end must not get into the products), and its epilogues."""
+    pad = lambda n: (n + 3) // 4 * 4 + 4
+    def operand(rows, cols, seed):
+        t = rnd((rows, pad(cols)), F32, seed)
+        t[:, cols:] = float("nan")
+        return t
+    a = operand(K, M, 1) if a_trans else operand(M, K, 1)
+    b = operand(K, N, 2) if b_trans else operand(N, K, 2)
+    base = dict(M=M, N=N, K=K, lda=a.shape[1], ldb=b.shape[1], ldc=N + 3, a_trans=a_trans, b_trans=b_trans)
+    name = "gemm32d_kernel<%s, %s, %s>" % (tile, "true" if a_trans else "false", "true" if b_trans else "false")
+
+    def run(what, tensors, outs, **kw):
+        print("fp32 gemm", what, M, N, K, a_trans, b_trans, flush=True)
+        dev = {k: v.cuda() for k, v in tensors.items()}
+        cpu = {k: v.clone() for k, v in tensors.items()}
+        launch = hip.gemm(**dev, **kw)
+        assert launch.variant == name, launch.variant
+        launch(torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        oracle.gemm(**cpu, **kw)()
+        for o in outs:
+            close((dev[o].cpu().float(), cpu[o].float()), 1e-2 if tensors[o].dtype == BF16 else 2e-5, 2e-3)
+
+    new = lambda seed=0: rnd((M, N + 3), F32, seed) if seed else torch.zeros(M, N + 3)
+    bias = rnd((N,), F32, 3)
+    run("store", dict(a=a, b=b, c=new()), ["c"], **base)
+    run("gelu", dict(a=a, b=b, c=new(), bias=bias, aux_out=new()), ["c", "aux_out"], act=1, ld_aux_out=N + 3, **base)
+    run("gelu'", dict(a=a, b=b, c=new(), aux_in=new(4)), ["c"], dact=1, ld_aux_in=N + 3, **base)
+    run("residual", dict(a=a, b=b, c=new(5), bias=bias, residual=new(6)), ["c"], beta=1, ld_res=N + 3, alpha=0.5, **base)
+    run("mixed", dict(a=a, b=b, c=new().to(BF16), bias=bias.to(BF16), residual=new(6).to(BF16)), ["c"], ld_res=N + 3, **base)
+
+
 @pytest.mark.parametrize("dtype", [F16, BF16])
 @pytest.mark.parametrize("rows,M,N", [(64, 8, 8), (100, 72, 136), (333, 520, 72)])
 def test_gemm_weight_gradients_on_64x64_tiles(hip, oracle, dtype, rows, M, N):
