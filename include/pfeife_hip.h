@@ -58,6 +58,28 @@ int pf_graph_capture_end(void* stream, void** graph_exec_out);
 int pf_graph_launch(void* graph_exec, void* stream);
 int pf_graph_destroy(void* graph_exec);
 
+/* Jobs issued from a thread of the library's own, in the order they are handed over, while the
+ * caller goes on: per job, `stream` waits for the events `waits`, replays `graph` and records
+ * `record` (graph and record may be null).  The arrays stay the caller's and have to live until
+ * the jobs are issued.  pf_issuer_push hands n jobs over and returns in *ticket how many have been
+ * handed over so far; pf_issuer_wait returns once the first `ticket` of them have been issued
+ * (issued, not finished), with an error if one of them failed.  One thread at a time may push.
+ * pf_issuer_destroy issues what is left and ends the thread. */
+typedef struct pf_job {
+  void* graph;
+  void* stream;
+  void* const* waits;
+  int64_t n_waits;
+  void* record;
+} pf_job;
+int pf_issuer_create(int device, void** issuer_out);
+int pf_issuer_push(void* issuer, const pf_job* jobs, int n, int64_t* ticket);
+int pf_issuer_wait(void* issuer, int64_t ticket);
+int pf_issuer_destroy(void* issuer);
+/* events that order streams (no timing) */
+int pf_event_create(void** event_out);
+int pf_event_destroy(void* event);
+
 /* ---- dense contractions (MFMA) -------------------------------------------
  * One descriptor covers every matrix product a stage executes:
  *   C[z] = epilogue( alpha * op(A[z]) . op(B[z]) )        for z in [0, batch1*batch2)

@@ -62,6 +62,12 @@ class GemmDesc(Structure):
     ]
 
 
+class Job(Structure):
+    """Mirror of `pf_job` in include/pfeife_hip.h."""
+
+    _fields_ = [("graph", c_void_p), ("stream", c_void_p), ("waits", c_void_p), ("n_waits", c_int64), ("record", c_void_p)]
+
+
 class NormBwdDesc(Structure):
     """Mirror of `pf_norm_bwd_desc` in include/pfeife_hip.h."""
 
@@ -90,6 +96,12 @@ _SIGNATURES = {
     "pf_graph_capture_end": [_P, POINTER(c_void_p)],
     "pf_graph_launch": [_P, _P],
     "pf_graph_destroy": [_P],
+    "pf_issuer_create": [_I, POINTER(c_void_p)],
+    "pf_issuer_push": [_P, _P, _I, POINTER(c_int64)],
+    "pf_issuer_wait": [_P, _L],
+    "pf_issuer_destroy": [_P],
+    "pf_event_create": [POINTER(c_void_p)],
+    "pf_event_destroy": [_P],
     "pf_gemm": [POINTER(GemmDesc), _P],
     "pf_gemm_grouped": [POINTER(GemmDesc), _I, _P],
     "pf_gemm_variant": [POINTER(GemmDesc), ctypes.c_char_p, _I],
@@ -199,6 +211,58 @@ def current_stream_ptr():
     return torch.cuda.current_stream().cuda_stream
 
 
+class Issuer:
+    """A native thread that issues jobs (graph replays and the events between their streams) in the order they are
+    handed over (`pf_issuer_*`); the calls release the interpreter."""
+
+    def __init__(self, lib, device):
+        self.lib = lib
+        h = c_void_p()
+        self._check(lib.pf_issuer_create(device, byref(h)))
+        self._h = h.value
+        self._ticket = c_int64(0)
+
+    @staticmethod
+    def _check(rc):
+        if rc != 0:
+            raise RuntimeError("pfeife_amd: %s" % last_error())
+
+    def event(self):
+        ev = c_void_p()
+        self._check(self.lib.pf_event_create(byref(ev)))
+        return ev.value
+
+    def destroy_event(self, ev):
+        self.lib.pf_event_destroy(ev)
+
+    @staticmethod
+    def jobs(jobs):
+        """[(graph replay or None, stream, [event], event or None)] -> what `push` takes."""
+        arr = (Job * len(jobs))()
+        keep = []
+        for a, (graph, stream, waits, record) in zip(arr, jobs):
+            a.graph = graph.handle if graph is not None else None
+            a.stream, a.record, a.n_waits = stream, record, len(waits)
+            if waits:
+                keep.append((c_void_p * len(waits))(*waits))
+                a.waits = ctypes.addressof(keep[-1])
+        return ctypes.addressof(arr), len(jobs), (arr, keep)
+
+    def push(self, jobs):
+        """Hands a list made by `jobs` over; it has to be kept until its jobs have been issued."""
+        if jobs[1]:
+            self._check(self.lib.pf_issuer_push(self._h, jobs[0], jobs[1], byref(self._ticket)))
+
+    def wait(self):
+        """Until everything handed over so far has been issued."""
+        self._check(self.lib.pf_issuer_wait(self._h, self._ticket.value))
+
+    def close(self):
+        if self._h:
+            self.lib.pf_issuer_destroy(self._h)
+            self._h = None
+
+
 class HipKernels:
     """Tensor-level kernel table backed by libpfeife_hip.so.
 
@@ -268,6 +332,10 @@ class HipKernels:
         if h:
             replay.handle = None
             self.lib.pf_graph_destroy(h)
+
+    def issuer(self):
+        """A thread that issues jobs in order; see `Issuer`."""
+        return Issuer(self.lib, self.device.index or 0)
 
     def colreduce_workspace(self, rows, cols):
         return int(self.lib.pf_colreduce_workspace(rows, cols))

@@ -18,6 +18,7 @@ OBJ_DIR = os.path.join(HERE, "build")
 
 SOURCES = [
     "pf_runtime.cpp",
+    "pf_issuer.cpp",
     "pf_gemm.hip",
     "pf_gemm_f32.hip",
     "pf_attention.hip",

@@ -21,7 +21,7 @@ reference's probe it contributes nothing to the gradients.
 """
 import threading
 from functools import partial
-from queue import Queue
+from queue import SimpleQueue
 from typing import List
 
 import torch
@@ -74,8 +74,8 @@ class PartialRunner:
         self.net_state = get_state()
         self._compiled = False
         self._probing = False
-        self._train_queues = [Queue() for _ in range(self.option.batch_cnt)]
-        self._return_queues = [Queue() for _ in range(self.option.batch_cnt)]
+        self._train_queues = [SimpleQueue() for _ in range(self.option.batch_cnt)]
+        self._return_queues = [SimpleQueue() for _ in range(self.option.batch_cnt)]
         self._batch_threads = []
         self.results = []
         self.worker = StageWorker(self, self.option, self.net_state.device, kernels)
@@ -142,6 +142,7 @@ class PartialRunner:
 
         # every micro-batch thread runs user code up to the compiled model, hands its
         # inputs to the worker and parks there
+        plan = worker.begin_planned_step() if pp is not None else None
         for bid in range(option.batch_cnt):
             self._train_queues[bid].put((args[bid], kwargs[bid]))
             tok = self._return_queues[bid].get()
@@ -149,6 +150,11 @@ class PartialRunner:
                 raise tok.exc
             if tok is STEP_TOKEN:
                 self._parked.add(bid)
+                if plan is not None:
+                    if worker.step_plan is plan:
+                        plan.inputs_ready(bid)
+                    else:   # a micro-batch of a new shape: its programs are new, the step starts over job by job
+                        plan = None
             else:
                 # exec_fn returned without reaching a pipelined graph: nothing to schedule for it
                 self.results.append(tok)
@@ -158,11 +164,22 @@ class PartialRunner:
         if pp is None:
             return self._take_results()
 
+        if plan is not None:
+            for jobs, mb in plan.turns:
+                plan.advance(jobs)
+                self.finalize_output(mb)
+            plan.end()
+            worker.optimizer_step()
+            worker.steps_done += 1
+            return self._take_results()
+
         worker.begin_step()
         for i, (stage, mb, is_fwd) in enumerate(worker.order):
             worker.run_job(stage, mb, is_fwd)
             if is_fwd and worker.last_forward.get(i) == mb:
+                worker.outputs_ready(mb)
                 self.finalize_output(mb)
+                worker.loss_grads_ready(mb)
         worker.end_jobs()
         worker.optimizer_step()
         worker.steps_done += 1
@@ -175,14 +192,12 @@ class PartialRunner:
     def finalize_output(self, batch_idx):
         """Wake micro-batch `batch_idx`: its outputs exist; wait until its exec_fn has
         returned (loss computed, backward hooks fired)."""
-        self.worker.outputs_ready(batch_idx)
         PartialModule._module_queues[batch_idx].put(None)
         ret = self._return_queues[batch_idx].get()
         self._parked.discard(batch_idx)
         if isinstance(ret, _ExecError):
             raise ret.exc
         self.worker.finish_micro_batch(batch_idx)
-        self.worker.loss_grads_ready(batch_idx)
         self.results.append(ret)
 
     def backward_hook(self, batch_idx, output_idx, grad):
@@ -244,7 +259,7 @@ class PartialRunner:
 
 
 class PartialModule(nn.Module):
-    _module_queues: List[Queue] = []
+    _module_queues: List[SimpleQueue] = []
     _runner: PartialRunner = None
     _all_modules: List["PartialModule"] = []
     _pp_modules: List["PartialModule"] = []
@@ -290,7 +305,7 @@ class PartialModule(nn.Module):
     def set_runner(runner: PartialRunner):
         PartialModule._runner = runner
         PartialModule._option = runner.option
-        PartialModule._module_queues = [Queue() for _ in range(runner.option.batch_cnt)]
+        PartialModule._module_queues = [SimpleQueue() for _ in range(runner.option.batch_cnt)]
         PartialModule._all_modules = []
         PartialModule._pp_modules = []
 

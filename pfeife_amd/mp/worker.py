@@ -22,6 +22,7 @@ from ..executor.values import Val
 from ..option import get_optimizer_cls
 from ..schedule.scheduler import PipeSchedParams, SingleCommScheduler, StepWork, serialize_ranks
 from ..utils import fmem, get_logger
+from .step_plan import StepPlan
 
 
 class MicroBatchPrograms:
@@ -66,6 +67,8 @@ class StageWorker:
         self.graphs_ready = False
         self.steps_done = 0
         self.begin_graph = None
+        self.issuer = None         # native thread that issues a captured step's jobs
+        self.step_plan = None      # ... and the job lists it is given
         self.plan = None           # the auto-partitioner's choice (split points + schedule variant), if it ran
         self.profile = None
         # One stream per pipeline rank ("lane"): the jobs of different ranks are independent by
@@ -225,6 +228,7 @@ class StageWorker:
         """Lower every stage for micro-batch slot `mb`; `dynamic_inputs` maps graph
         placeholder index -> the value user code passed (tensor chunk or constant)."""
         pg = part_graph if part_graph is not None else self.part_graph
+        self._drop_step_plan()     # (a step that had begun starts over)
         slot = MicroBatchPrograms()
         slot.input_sig = self._signature([dynamic_inputs[i] for i in sorted(dynamic_inputs)])
         graph_vals = {}
@@ -343,6 +347,16 @@ class StageWorker:
                 self.kernels.destroy_graph(job[1])
         self.dw_jobs = {}
 
+    def _drop_step_plan(self):
+        """Forgets the captured step's job lists, after what has been issued of them."""
+        plan, self.step_plan = self.step_plan, None
+        if plan is None:
+            return
+        self.issuer.wait()
+        for lane in {id(l): l for l in list((self.lanes or {}).values()) + [self.stream_obj]}.values():
+            lane.synchronize()
+        plan.release()
+
     def _drop_begin_graph(self):
         if self.begin_graph is not None and hasattr(self.kernels, "destroy_graph"):
             self.kernels.destroy_graph(self.begin_graph)
@@ -351,6 +365,10 @@ class StageWorker:
     def release(self):
         """Frees every captured graph and drops the stage programs and their buffers (the worker
         cannot run another step afterwards)."""
+        self._drop_step_plan()
+        if self.issuer is not None:
+            self.issuer.close()
+            self.issuer = None
         if self.stream_obj is not None:
             self.stream_obj.synchronize()
         for slot in self.mbs.values():
@@ -396,6 +414,7 @@ class StageWorker:
         self.begin_graph = self.kernels.capture(pre, s) if pre else None
         self._begin_len = (len(self.params.zero), len(self.params.refresh))
         self.graphs_ready = True
+        self._drop_step_plan()
 
     def distribute_input(self, mb, placeholder_idx, value):
         """Copy one micro-batch slab into the stage input buffer it was built for."""
@@ -409,6 +428,30 @@ class StageWorker:
             self.kernels.split_gather(value, buf, row_bytes, 0, rows)(self.stream())
         elif value.numel() > 0:
             buf.copy_(value, non_blocking=True)  # host -> device (or a layout change): PyTorch plumbing
+
+    def begin_planned_step(self):
+        """Starts a step whose jobs a native thread issues from job lists (`StepPlan`): every step after the one that
+        captured the graphs, until a micro-batch of another shape arrives.  None: the step goes job by job.
+        Decoder of four looped stages, eight micro-batches of 256 tokens: 5.9 -> 4.1 ms; two-layer ViT on four 32x32
+        images, two micro-batches: 1.78 -> 1.18 ms; ViT-S on 62 images, ragged micro-batches: 6.9 -> 6.7 ms."""
+        if not self.graphs_ready or not hasattr(self.kernels, "issuer"):
+            return None
+        if self.step_plan is None:
+            if len(self.mbs) != self.option.batch_cnt or (self.stack_dw and any(s not in self.dw_jobs for s in self.last_backward)):
+                return None
+            if any(job[1] is None and job[0] for job in self.dw_jobs.values()):
+                self.capture_graphs()      # (weight-gradient jobs that were lowered after the other graphs)
+            if self.issuer is None:
+                self.issuer = self.kernels.issuer()
+            self.step_plan = StepPlan(self)
+        elif self.step_plan.started:   # a step that failed half-way may have left lanes running
+            self.issuer.wait()
+            self.end_jobs()
+        self.params.rebind_grads()
+        for slot in self.mbs.values():
+            slot.grad_seen.clear()
+        self.step_plan.begin()
+        return self.step_plan
 
     def begin_step(self):
         s = self.stream()

@@ -945,6 +945,61 @@ def test_lanes_give_bit_identical_steps(monkeypatch):
                     assert torch.equal(a, b), mode
 
 
+@pytest.mark.parametrize("lanes", ["rankdir", "rank", "0"])
+def test_jobs_issued_by_the_native_thread_give_bit_identical_steps(monkeypatch, lanes):
+    """Steps whose jobs a native thread issues from job lists against steps issued launch by launch: in a steady
+    state, around a step whose user code raises, and where a micro-batch of another shape arrives in the middle of
+    a step that had begun."""
+    from pfeife_amd.bench_models.llama import LlamaConfig, LlamaForCausalLM
+    from pfeife_amd.mp import partial_compiler
+    from pfeife_amd.option import PipeOption
+
+    def run(no_graph):
+        monkeypatch.setenv("PFEIFE_LANES", lanes)
+        monkeypatch.setenv("PFEIFE_NO_GRAPH", no_graph)
+        torch.manual_seed(0)
+        model = LlamaForCausalLM(LlamaConfig(vocab=512, dim=128, layers=4, heads=2, ffn=344, max_seq=64))
+        ids = torch.randint(0, 512, (10, 64), generator=torch.Generator().manual_seed(1)).cuda()
+        option = PipeOption(device_cnt=2, batch_cnt=4, batch_size=2, split_points=["layers.1", "layers.2", "layers.3"],
+                            mixed_precision="bf16", optimizer=dict(type="adam", lr=1e-3))
+        runner = _fresh_runner(option)
+        model.cuda()
+        cmodel = torch.compile(model, backend=partial_compiler)
+        calls = []
+
+        def fn(tok):
+            loss = cmodel(tok, tok)
+            calls.append(0)
+            if fail and len(calls) == 2:
+                raise ValueError("user code")
+            loss.backward()
+            return loss.detach()
+
+        runner.set_exec_fn(fn)
+        out, planned = [], 0
+        for rows, fail in ((8, 0), (8, 0), (8, 0), (8, 1), (8, 0), (10, 0), (8, 0), (8, 0), (8, 0)):
+            calls.clear()
+            try:
+                losses = runner.step(ids[:rows])
+            except ValueError:
+                assert fail
+                continue
+            planned += runner.worker.step_plan is not None
+            torch.cuda.synchronize()
+            out.append(([float(l) for l in losses], [p.grad.clone() for p in model.parameters()],
+                        [p.detach().clone() for p in model.parameters()]))
+        return out, planned
+
+    want, planned = run("1")
+    assert planned == 0
+    got, planned = run("0")
+    assert planned == 4
+    for i, ((l0, g0, p0), (l1, g1, p1)) in enumerate(zip(want, got)):
+        assert l0 == l1, (i, l0, l1)
+        for a, b in zip(g0 + p0, g1 + p1):
+            assert torch.equal(a, b), i
+
+
 def test_lanes_give_bit_identical_per_micro_batch_weight_gradients(monkeypatch):
     """The same, for weight gradients added up micro-batch by micro-batch (PFEIFE_DW_STACK=0, the
     form steps with ragged micro-batches take) at ViT-S/16 size: those products run on the tile
