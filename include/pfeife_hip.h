@@ -303,7 +303,7 @@ int pf_softmax_bwd(const float* dp, int64_t ld_dp, const void* p, int p_dtype, i
  * tensors (fp16 or bf16) addressed with ELEMENT strides (batch, head, token) and unit
  * stride along hd, so that heads may sit inside a packed qkv projection.  lse: fp32
  * [B,H,Tq] (written by forward, read by backward); delta: fp32 [B,H,Tq] scratch written
- * and read by backward.  hd must be a multiple of 8 and <= 96 (PF_ERR_UNSUPPORTED
+ * and read by backward.  hd must be a multiple of 8 and <= 128 (PF_ERR_UNSUPPORTED
  * otherwise: the caller then uses pf_gemm + pf_softmax).  causal: key j is visible to
  * query i iff j <= i + (Tk - Tq) (bottom-right alignment; for Tq != Tk this is NOT
  * aten::scaled_dot_product_attention's top-left is_causal mask, so the host lowering

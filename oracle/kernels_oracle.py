@@ -136,7 +136,7 @@ class OracleKernels:
         return True       # every product of the oracle honours unscale_by / nonfinite_flag
 
     # -- fused attention -----------------------------------------------------------
-    MAX_FUSED_HEAD_DIM = 96
+    MAX_FUSED_HEAD_DIM = 128
 
     @staticmethod
     def _attn_scores(q, k, scale, causal):

@@ -139,9 +139,12 @@ __device__ __forceinline__ void attn_block(const AttnArgs& a, bool heavy_is_last
 // wavefront idles through every latency.  The register budget is set so that three (forward, head
 // dim <= 64: 152 VGPRs) or two (dQ: 240, dK/dV: 247) wavefronts share a SIMD without spilling;
 // measured on 2048 causal tokens x 64 heads: forward 76 -> 56 us, backward 280 -> 194 us.
+// Head dims above 64 hold two (forward: 204 / 248 VGPRs at 96 / 128; dQ up to 96: 251), where the compiler left to
+// itself takes registers for one: forward 577 tokens x 56 heads of 88 47 -> 28 us, 2048 causal tokens x 64 heads of
+// 128 166 -> 104 us.  dQ of 128 and dK/dV above 96 would spill (dK/dV of 128 by 307 registers: 498 -> 793 us).
 // ---------------------------------------------------------------------------------
 template <int DT, int HD>
-__global__ __launch_bounds__(256, HD <= 64 ? 3 : 1) void attn_fwd_kernel(const AttnArgs a) {
+__global__ __launch_bounds__(256, HD <= 64 ? 3 : 2) void attn_fwd_kernel(const AttnArgs a) {
   constexpr int NC = HD / 16, NO = HD / 32, KLD = HD + 8;
   __shared__ __align__(16) uint16_t sK[KT * KLD];
   __shared__ __align__(16) uint16_t sV[KT * KLD];
@@ -294,7 +297,7 @@ __global__ __launch_bounds__(256) void attn_delta_kernel(const AttnArgs a, float
 // dQ: same tiling as forward (column = query); dQ^T[hd][q] += K^T[hd][kv] dS^T[kv][q]
 // ---------------------------------------------------------------------------------
 template <int DT, int HD>
-__global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attn_dq_kernel(const AttnArgs a) {
+__global__ __launch_bounds__(256, HD <= 96 ? 2 : 1) void attn_dq_kernel(const AttnArgs a) {
   constexpr int NC = HD / 16, NO = HD / 32, KLD = HD + 8;
   __shared__ __align__(16) uint16_t sK[KT * KLD];
   __shared__ __align__(16) uint16_t sV[KT * KLD];
@@ -402,7 +405,7 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attn_dq_kernel(const At
 // accumulators are added at the end through LDS in wavefront order, so that a head's dK/dV come
 // from 4 x ceil(Tk / 32) wavefronts instead of ceil(Tk / 32).
 template <int DT, int HD, bool SPLITQ = false>
-__global__ __launch_bounds__(256, SPLITQ ? 1 : 2) void attn_dkv_kernel(const AttnArgs a) {
+__global__ __launch_bounds__(256, SPLITQ || HD > 96 ? 1 : 2) void attn_dkv_kernel(const AttnArgs a) {
   constexpr int NC = HD / 16, NO = HD / 32, QLD = HD + 8;
   constexpr int QT = SPLITQ ? 128 : KT;        // queries staged per iteration
   constexpr int NH = SPLITQ ? 1 : 2;           // 32-query halves per wavefront and iteration
@@ -1083,8 +1086,8 @@ int check_common(const pf_attn_desc* d, const char* name) {
   PF_REQUIRE(d != nullptr, "%s: null descriptor", name);
   PF_REQUIRE(d->dtype == PF_F16 || d->dtype == PF_BF16, "%s: dtype must be fp16 or bf16", name);
   PF_REQUIRE(d->B > 0 && d->H > 0 && d->Tq > 0 && d->Tk > 0 && d->hd > 0, "%s: bad shape", name);
-  if (d->hd % 8 != 0 || d->hd > 96) {
-    pf_set_error("%s: head dim %d is not supported by the fused kernels (multiple of 8, <= 96)", name, d->hd);
+  if (d->hd % 8 != 0 || d->hd > 128) {
+    pf_set_error("%s: head dim %d is not supported by the fused kernels (multiple of 8, <= 128)", name, d->hd);
     return PF_ERR_UNSUPPORTED;
   }
   PF_REQUIRE((int64_t)d->B * d->H <= 65535, "%s: B*H exceeds 65535", name);
@@ -1095,6 +1098,9 @@ int check_common(const pf_attn_desc* d, const char* name) {
   if (d->causal) PF_REQUIRE(d->Tk >= d->Tq, "%s: causal attention needs Tk >= Tq", name);
   return PF_OK;
 }
+
+// whole operands in LDS: two of them (and their padding) fit for head dims up to 96
+bool short_ok(const pf_attn_desc* d) { return d->Tq <= SHORT_T && d->Tk <= SHORT_T && d->hd <= 96; }
 
 AttnArgs make_args(const pf_attn_desc* d) {
   AttnArgs a;
@@ -1167,10 +1173,12 @@ int launch_short(K kern, dim3 grid, int threads, size_t lds, hipStream_t st, Arg
   do {                                                                                         \
     if (dt == PF_F16) {                                                                        \
       if (hd <= 64) hipLaunchKernelGGL((KERNEL<PF_F16, 64>), grid, dim3(256), 0, st, a);       \
-      else hipLaunchKernelGGL((KERNEL<PF_F16, 96>), grid, dim3(256), 0, st, a);                \
+      else if (hd <= 96) hipLaunchKernelGGL((KERNEL<PF_F16, 96>), grid, dim3(256), 0, st, a);     \
+      else hipLaunchKernelGGL((KERNEL<PF_F16, 128>), grid, dim3(256), 0, st, a);             \
     } else {                                                                                   \
       if (hd <= 64) hipLaunchKernelGGL((KERNEL<PF_BF16, 64>), grid, dim3(256), 0, st, a);      \
-      else hipLaunchKernelGGL((KERNEL<PF_BF16, 96>), grid, dim3(256), 0, st, a);               \
+      else if (hd <= 96) hipLaunchKernelGGL((KERNEL<PF_BF16, 96>), grid, dim3(256), 0, st, a);    \
+      else hipLaunchKernelGGL((KERNEL<PF_BF16, 128>), grid, dim3(256), 0, st, a);            \
     }                                                                                          \
   } while (0)
 
@@ -1181,7 +1189,7 @@ extern "C" int pf_attention_fwd(const pf_attn_desc* d, void* stream) {
              "pf_attention_fwd: bad output operand");
   AttnArgs a = make_args(d);
   const dim3 grid((unsigned)((d->Tq + 127) / 128), (unsigned)(d->B * d->H));
-  if (d->Tq <= SHORT_T && d->Tk <= SHORT_T) {
+  if (short_ok(d)) {
     const int rows = (d->Tk + 31) / 32 * 32;
     auto lds = [rows](int HD) { return (size_t)2 * rows * (HD + 8) * 2; };
     PF_ATTN_SHORT(attn_fwd_short_kernel, 512, rc, d->Tq, d->B * d->H, lds, (hipStream_t)stream, d->dtype, d->hd, a, rows);
@@ -1209,7 +1217,7 @@ extern "C" int pf_attention_bwd(const pf_attn_desc* d, void* stream) {
   if (d->dtype == PF_BF16) ad.causal |= 0x100;  // dtype flag for the delta kernel
   const dim3 gq((unsigned)((d->Tq + 127) / 128), (unsigned)(d->B * d->H));
   const dim3 gk((unsigned)((d->Tk + 127) / 128), (unsigned)(d->B * d->H));
-  if (d->Tq <= SHORT_T && d->Tk <= SHORT_T) {
+  if (short_ok(d)) {
     const int rows_k = (d->Tk + 31) / 32 * 32, rows_q = (d->Tq + 31) / 32 * 32;
     if (d->hd <= 64 && d->Tq <= 256 && d->Tk <= 256 && (d->Tq > 128 || d->Tk > 128)) {
       // one workgroup per head forms dQ, dK and dV from a single load of the head
@@ -1235,7 +1243,7 @@ extern "C" int pf_attention_bwd(const pf_attn_desc* d, void* stream) {
   hipLaunchKernelGGL(attn_delta_kernel, dim3((unsigned)((rows + 31) / 32)), dim3(256), 0, st, ad, d->delta);
   // few keys, many queries (cross attention to a short context): split each key tile's query sweep
   // over the four wavefronts of a workgroup
-  if ((int64_t)gk.x * gk.y < 200 && d->Tq >= 256) {
+  if ((int64_t)gk.x * gk.y < 200 && d->Tq >= 256 && d->hd <= 96) {   // (two 128-row tiles of more do not fit)
     const dim3 gs((unsigned)((d->Tk + 31) / 32), (unsigned)(d->B * d->H));
     if (d->dtype == PF_F16) {
       if (d->hd <= 64) hipLaunchKernelGGL((attn_dkv_kernel<PF_F16, 64, true>), gs, dim3(256), 0, st, a);

@@ -456,7 +456,7 @@ class HipKernels:
         return launch
 
     # -- fused attention -----------------------------------------------------------
-    MAX_FUSED_HEAD_DIM = 96
+    MAX_FUSED_HEAD_DIM = 128
 
     @staticmethod
     def _attn_desc(q, k, v, o, lse, scale, causal, d_o=None, dq=None, dk=None, dv=None, delta=None):

@@ -737,6 +737,9 @@ def test_deferred_reductions_match_immediate(hip):
     dict(B=1, H=2, Tq=33, Tk=250, hd=16, causal=0, packed=False),    # one-workgroup backward, two query tiles only
     dict(B=1, H=2, Tq=330, Tk=40, hd=88, causal=0, packed=False),    # the same at head dim 88, ragged query blocks
     dict(B=1, H=2, Tq=160, Tk=170, hd=96, causal=0, packed=False),   # head dim 96: six key tiles in one 4-wavefront workgroup
+    dict(B=1, H=2, Tq=301, Tk=301, hd=128, causal=1, packed=False),  # head dims above 96: tiled kernels at every length
+    dict(B=2, H=1, Tq=33, Tk=70, hd=104, causal=0, packed=False),
+    dict(B=1, H=1, Tq=300, Tk=40, hd=128, causal=0, packed=False),
 ])
 def test_fused_attention(hip, oracle, dtype, case):
     B, H, Tq, Tk, hd = case["B"], case["H"], case["Tq"], case["Tk"], case["hd"]
