@@ -886,6 +886,25 @@ def test_loss_scaler_kernels(hip, oracle):
         assert torch.equal(dev.cpu(), cpu), (found, dev.cpu(), cpu)
 
 
+@pytest.mark.parametrize("sizes", [[1], [2048, 0, 2047, 5], [3] * 300 + [70001] + [1] * 300, [5_000_000, 4096]])
+def test_adam_step_covers_every_element_of_every_tensor_once(hip, sizes):
+    """Tensors from empty to millions of elements, more of them than one pass of the work split looks at."""
+    state = [[rnd((n,), F32, 7 * i + j) if j < 3 else rnd((n,), F32, 7 * i + j).abs() for i, n in enumerate(sizes)] for j in range(4)]
+    dev = [[t.cuda() for t in ts] for ts in state]
+    params = [torch.nn.Parameter(t.clone()) for t in state[0]]
+    opt = torch.optim.Adam(params, lr=1e-2, weight_decay=0.01)
+    for p, g, m, v in zip(params, *state[1:]):
+        p.grad = g.clone()
+        opt.state[p] = dict(step=torch.tensor(4.0), exp_avg=m.clone(), exp_avg_sq=v.clone())
+    opt.step()
+    s = torch.cuda.current_stream().cuda_stream
+    hip.adam_step(*hip.adam_table(*dev), 1e-2, 0.9, 0.999, 1e-8, 0.01, 5, False, s)
+    torch.cuda.synchronize()
+    for i, p in enumerate(params):
+        for got, want in ((dev[0][i], p.detach()), (dev[2][i], opt.state[p]["exp_avg"]), (dev[3][i], opt.state[p]["exp_avg_sq"])):
+            torch.testing.assert_close(got.cpu(), want, rtol=1e-6, atol=1e-6)
+
+
 def test_adam_step_scaled_skips_on_overflow_and_counts_steps_on_device(hip):
     """pf_adam_step_scaled reads found_inf and the completed-step count from the scaler state:
     with found_inf set nothing changes; otherwise it equals pf_adam_step at step = count + 1."""
