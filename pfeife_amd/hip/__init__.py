@@ -249,13 +249,15 @@ class Issuer:
         return ctypes.addressof(arr), len(jobs), (arr, keep)
 
     def push(self, jobs):
-        """Hands a list made by `jobs` over; it has to be kept until its jobs have been issued."""
+        """Hands a list made by `jobs` over; it has to be kept until its jobs have been issued.  Returns what `wait`
+        takes."""
         if jobs[1]:
             self._check(self.lib.pf_issuer_push(self._h, jobs[0], jobs[1], byref(self._ticket)))
+        return self._ticket.value
 
-    def wait(self):
-        """Until everything handed over so far has been issued."""
-        self._check(self.lib.pf_issuer_wait(self._h, self._ticket.value))
+    def wait(self, ticket=None):
+        """Until everything handed over so far has been issued, or everything up to the `push` that returned `ticket`."""
+        self._check(self.lib.pf_issuer_wait(self._h, self._ticket.value if ticket is None else ticket))
 
     def close(self):
         if self._h:

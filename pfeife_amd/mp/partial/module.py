@@ -142,7 +142,7 @@ class PartialRunner:
 
         # every micro-batch thread runs user code up to the compiled model, hands its
         # inputs to the worker and parks there
-        plan = worker.begin_planned_step() if pp is not None else None
+        worker.settle_failed_step()
         for bid in range(option.batch_cnt):
             self._train_queues[bid].put((args[bid], kwargs[bid]))
             tok = self._return_queues[bid].get()
@@ -150,11 +150,6 @@ class PartialRunner:
                 raise tok.exc
             if tok is STEP_TOKEN:
                 self._parked.add(bid)
-                if plan is not None:
-                    if worker.step_plan is plan:
-                        plan.inputs_ready(bid)
-                    else:   # a micro-batch of a new shape: its programs are new, the step starts over job by job
-                        plan = None
             else:
                 # exec_fn returned without reaching a pipelined graph: nothing to schedule for it
                 self.results.append(tok)
@@ -164,9 +159,11 @@ class PartialRunner:
         if pp is None:
             return self._take_results()
 
+        # (not before: until here user code may still change weights and read or drop gradients)
+        plan = worker.begin_planned_step()
         if plan is not None:
-            for jobs, mb in plan.turns:
-                plan.advance(jobs)
+            for turn, mb in plan.turns:
+                plan.advance(turn)
                 self.finalize_output(mb)
             plan.end()
             worker.optimizer_step()

@@ -1,13 +1,13 @@
 """The jobs of a captured step as native job lists, worked out once per capture.
 
-A step alternates between jobs (hipGraph replays on the lanes of the pipeline ranks, with events between them) and user
-code (a micro-batch's way to the model; its loss and backward hooks).  Issuing them in one thread adds their host times
-up: in a small model's step each is about half, and the GPU waits for both.  Here a native thread issues the jobs
+A step begins when every micro-batch's user code has reached the model: until then user code may change weights, read or
+drop gradients, and nothing of the step has touched them.  From there it alternates between jobs (hipGraph replays on the
+lanes of the pipeline ranks, with events between them) and user code (a micro-batch's loss and backward hooks).  Issuing
+them in one thread adds their host times up, and the GPU waits for both.  Here a native thread issues the jobs
 (`Issuer`), and the calling thread waits for it only where user code reads a result:
 
-  * a micro-batch's forward jobs go out as soon as its inputs are in place, while the next micro-batch's user code is
-    still on its way to the model, and ahead of the user code of earlier ones: forward jobs read parameters and each
-    other only, and with lanes of their own they hold no other job up.  (Without such lanes everything keeps the
+  * with lanes of their own, forward jobs are issued up to the end of the next micro-batch while this one's user code
+    runs: they read parameters and each other only, and hold no other job up.  (Without such lanes everything keeps the
     schedule's order.)
   * backward jobs and user code keep the schedule's order among themselves, which fixes the order in which micro-batches
     are summed into a gradient.
@@ -41,12 +41,12 @@ class StepPlan:
         sources = {s.idx: {src[0] for src in s.input_source if src is not None} for s in pg.nodes.values()}
         users_of = {s: sorted(t for t in sources if s in sources[t]) for s in sources}
         out_stages = sorted({ref[0] for ref in pg.outputs if isinstance(ref[0], int)})
-        finals = {i: mb for i, mb in w.last_forward.items()}
         done = {}
+        begin = self._node(main, w.begin_graph, [])     # (after the inputs' copies, on the same stream)
 
         def job(stage, mb, is_fwd):
             prog = w.mbs[mb].stage_programs[stage]
-            deps = [done["input", mb]]
+            deps = [begin]
             if is_fwd:
                 deps += [done[s, mb, True] for s in sorted(sources[stage])]
             else:
@@ -58,29 +58,35 @@ class StepPlan:
             if not is_fwd and w.last_backward.get(stage) == mb and w.stack_dw and w.dw_jobs[stage][1] is not None:
                 self._node(st, w.dw_jobs[stage][1], [])
 
-        # the step's phases, each a list of nodes: begin, one after each micro-batch's inputs, then job lists and
-        # micro-batches ready for user code in turn
-        self._begin = [self._node(main, w.begin_graph, [])]
-        self._inputs = []
-        pending = [(s, mb) for s, mb, f in w.order if f] if early else []
-        for bid in range(len(w.mbs)):
-            first = len(self._nodes)
-            done["input", bid] = self._node(main, None, [])
-            while pending and pending[0][1] <= bid:
-                job(*pending.pop(0), True)
-            self._inputs.append(self._nodes[first:])
-        self._turns = []
-        first = len(self._nodes)
+        # the step's phases, each a list of nodes: begin, then job lists and micro-batches ready for user code in turn
+        finals = [i for i in range(len(w.order)) if i in w.last_forward]     # of each micro-batch in turn
+        ahead = [(i, s, mb) for i, (s, mb, f) in enumerate(w.order) if f] if early else []
+
+        def take():
+            nonlocal first
+            nodes, first = self._nodes[first:], len(self._nodes)
+            return nodes
+
+        def forward_through(i):
+            while ahead and ahead[0][0] <= i:
+                job(*ahead.pop(0)[1:], True)
+
+        first, turns = 0, []
+        self._begin = take()
         for i, (stage, mb, is_fwd) in enumerate(w.order):
             if not (is_fwd and early):
                 job(stage, mb, is_fwd)
-            if is_fwd and finals.get(i) == mb:
+            if is_fwd and w.last_forward.get(i) == mb:
+                forward_through(i)
                 self._node(main, None, [done[s, mb, True] for s in out_stages])
-                self._turns.append((self._nodes[first:], mb))
-                first = len(self._nodes)
+                needed = take()
+                later = finals[len(turns) + 1:]
+                if later:
+                    forward_through(later[0])
+                turns.append((needed, take(), mb))
                 done["loss", mb] = self._node(main, None, [])
         self._node(main, None, [n for s, n in self._last.items() if s is not main])
-        self._end = self._nodes[first:]
+        self._end = take()
 
         self._events = []
         for n in self._nodes:
@@ -88,9 +94,8 @@ class StepPlan:
                 n.event = self.issuer.event()
                 self._events.append(n.event)
         self._begin, self._end = self._jobs(self._begin), self._jobs(self._end)
-        self._inputs = [self._jobs(n) for n in self._inputs]
-        self.turns = [(self._jobs(n), mb) for n, mb in self._turns]
-        del self._nodes, self._last, self._known, self._turns
+        self.turns = [((self._jobs(n), self._jobs(a)), mb) for n, a, mb in turns]
+        del self._nodes, self._last, self._known
 
     def _node(self, stream, graph, deps):
         known = self._known.setdefault(stream, {})
@@ -115,21 +120,21 @@ class StepPlan:
 
     # -- one step ---------------------------------------------------------------------
     def begin(self):
+        """The inputs of all micro-batches are on their way on the main stream."""
         self.started = True
         self.issuer.push(self._begin)
 
-    def inputs_ready(self, mb):
-        """Micro-batch `mb`'s inputs are on their way on the main stream."""
-        self.issuer.push(self._inputs[mb])
-
-    def advance(self, jobs):
+    def advance(self, turn):
         """Issues a turn's jobs: the main stream may then read the outputs of the turn's micro-batch."""
-        self.issuer.push(jobs)
-        self.issuer.wait()
+        needed, ahead = turn
+        ticket = self.issuer.push(needed)
+        self.issuer.push(ahead)
+        self.issuer.wait(ticket)
 
     def end(self):
         """The rest, and the main stream after every lane."""
-        self.advance(self._end)
+        self.issuer.push(self._end)
+        self.issuer.wait()
         self.started = False
 
     def release(self):

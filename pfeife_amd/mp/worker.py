@@ -228,7 +228,7 @@ class StageWorker:
         """Lower every stage for micro-batch slot `mb`; `dynamic_inputs` maps graph
         placeholder index -> the value user code passed (tensor chunk or constant)."""
         pg = part_graph if part_graph is not None else self.part_graph
-        self._drop_step_plan()     # (a step that had begun starts over)
+        self._drop_step_plan()
         slot = MicroBatchPrograms()
         slot.input_sig = self._signature([dynamic_inputs[i] for i in sorted(dynamic_inputs)])
         graph_vals = {}
@@ -429,11 +429,18 @@ class StageWorker:
         elif value.numel() > 0:
             buf.copy_(value, non_blocking=True)  # host -> device (or a layout change): PyTorch plumbing
 
+    def settle_failed_step(self):
+        """A planned step that failed half-way may have left jobs to be issued and lanes running: the new step's user
+        code and inputs come after them."""
+        if self.step_plan is not None and self.step_plan.started:
+            self.issuer.wait()
+            self.end_jobs()
+            self.step_plan.started = False
+
     def begin_planned_step(self):
         """Starts a step whose jobs a native thread issues from job lists (`StepPlan`): every step after the one that
-        captured the graphs, until a micro-batch of another shape arrives.  None: the step goes job by job.
-        Decoder of four looped stages, eight micro-batches of 256 tokens: 5.9 -> 4.1 ms; two-layer ViT on four 32x32
-        images, two micro-batches: 1.78 -> 1.18 ms; ViT-S on 62 images, ragged micro-batches: 6.9 -> 6.7 ms."""
+        captured the graphs, until a micro-batch of another shape arrives.  Called where `begin_step` is, when every
+        micro-batch's user code has reached the model.  None: the step goes job by job."""
         if not self.graphs_ready or not hasattr(self.kernels, "issuer"):
             return None
         if self.step_plan is None:
@@ -444,9 +451,6 @@ class StageWorker:
             if self.issuer is None:
                 self.issuer = self.kernels.issuer()
             self.step_plan = StepPlan(self)
-        elif self.step_plan.started:   # a step that failed half-way may have left lanes running
-            self.issuer.wait()
-            self.end_jobs()
         self.params.rebind_grads()
         for slot in self.mbs.values():
             slot.grad_seen.clear()

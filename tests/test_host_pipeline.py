@@ -4,6 +4,7 @@ table is replaced by the CPU oracle of the kernels (a test double injected
 through PartialRunner's `kernels` argument; the product only ships the HIP
 table), so these tests check everything EXCEPT the HIP code."""
 import copy
+from types import SimpleNamespace
 
 import pytest
 import torch
@@ -510,3 +511,96 @@ def test_ragged_step_after_uniform_steps_starts_from_zeroed_gradients():
     run_unpipelined(ref, crit, x6, y6, 3)
     for (n, p), (_, q) in zip(model.named_parameters(), ref.named_parameters()):
         assert (p.grad - q.grad).abs().max() <= 1e-4 * q.grad.abs().max() + 1e-9, n
+
+
+class _HostPlan:
+    """`StepPlan` with jobs that run at once: the order of a planned step's phases without a GPU."""
+
+    def __init__(self, worker):
+        self.worker, self.started, self.turns, self.rest = worker, False, [], []
+        for i, (stage, mb, is_fwd) in enumerate(worker.order):
+            self.rest.append((stage, mb, is_fwd))
+            if is_fwd and worker.last_forward.get(i) == mb:
+                self.turns.append((self.rest, mb))
+                self.rest = []
+
+    def begin(self):
+        self.started = True
+        for launch in self.worker.params.zero_launches() + self.worker.params.refresh_launches():
+            launch(None)
+
+    def inputs_ready(self, mb):
+        pass
+
+    def advance(self, turn):
+        for job in turn:
+            self.worker.run_job(*job)
+
+    def end(self):
+        self.advance(self.rest)
+        self.started = False
+
+    def release(self):
+        pass
+
+
+@pytest.mark.parametrize("user_code", ["drops_gradients", "changes_a_weight", "reads_gradients", "raises"])
+def test_planned_steps_leave_user_code_before_the_model_alone(monkeypatch, user_code):
+    """A planned step clears and rebinds gradients and refreshes the 16-bit weights after every micro-batch's user
+    code has reached the model: what exec_fn does before it gives the same steps as job by job."""
+    from pfeife_amd.mp import partial_compiler
+    from pfeife_amd.mp import worker as worker_module
+
+    def run(planned):
+        torch.manual_seed(0)
+        model = VisionTransformer(CFG)
+        opt = torch.optim.SGD(model.parameters(), lr=0.05)
+        option = PipeOption(device_cnt=2, batch_cnt=4, batch_size=2, split_points=["blocks.2"], mixed_precision="bf16")
+        runner = make_runner(option)
+        runner.optimizer = opt
+        cmodel = torch.compile(model, backend=partial_compiler)
+        crit = nn.CrossEntropyLoss()
+        weight, seen, step = model.blocks[1].fc1.weight, [], [0]
+
+        def fn(x, y):
+            if user_code == "drops_gradients":
+                opt.zero_grad()
+            elif user_code == "changes_a_weight":
+                with torch.no_grad():
+                    weight.mul_(0.9)
+            elif user_code == "reads_gradients":
+                seen.extend(p.grad.clone() for p in model.parameters() if p.grad is not None)
+            elif step[0] == 3 and int(y[0]) == int(ys[-2]):
+                raise ValueError("user code")
+            loss = crit(cmodel(x).float(), y)
+            loss.backward()
+            return loss.detach()
+
+        runner.set_exec_fn(fn)
+        g = torch.Generator().manual_seed(42)
+        x, ys = torch.randn(8, 3, 32, 32, generator=g), torch.arange(8)
+        w, out, plans = runner.worker, [], 0
+        for step[0] in range(5):
+            if planned and step[0] == 2:
+                monkeypatch.setattr(worker_module, "StepPlan", _HostPlan)
+                w.kernels.issuer = lambda: SimpleNamespace(wait=lambda: None)
+                w.capture_graphs = lambda: None
+                w.graphs_ready = True
+            try:
+                losses = [float(l) for l in runner.step(x, ys)]
+            except ValueError:
+                losses = "raised"
+            plans += w.step_plan is not None
+            out.append((losses, [p.grad.clone() for p in model.parameters()], [p.detach().clone() for p in model.parameters()]))
+        w.step_plan = None
+        assert plans == (3 if planned else 0)
+        return out, seen
+
+    (want, seen0), (got, seen1) = run(False), run(True)
+    if user_code == "raises":
+        assert want[3][0] == "raised"
+    for i, ((l0, g0, p0), (l1, g1, p1)) in enumerate(zip(want, got)):
+        assert l0 == l1, (i, l0, l1)
+        for a, b in zip(g0 + p0, g1 + p1):
+            assert torch.equal(a, b), i
+    assert len(seen0) == len(seen1) and all(torch.equal(a, b) for a, b in zip(seen0, seen1))

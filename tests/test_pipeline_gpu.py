@@ -1000,6 +1000,66 @@ def test_jobs_issued_by_the_native_thread_give_bit_identical_steps(monkeypatch, 
             assert torch.equal(a, b), i
 
 
+@pytest.mark.parametrize("lanes", ["0", "rankdir"])
+@pytest.mark.parametrize("user_code", ["drops_gradients", "changes_a_weight", "raises"])
+def test_planned_steps_leave_user_code_before_the_model_alone(monkeypatch, lanes, user_code):
+    """exec_fn drops the gradients, changes a weight or raises before the model is called: steps issued from job lists
+    give the bits of steps issued launch by launch."""
+    from pfeife_amd.bench_models.llama import LlamaConfig, LlamaForCausalLM
+    from pfeife_amd.mp import partial_compiler
+    from pfeife_amd.option import PipeOption
+
+    def run(no_graph):
+        monkeypatch.setenv("PFEIFE_LANES", lanes)
+        monkeypatch.setenv("PFEIFE_NO_GRAPH", no_graph)
+        torch.manual_seed(0)
+        model = LlamaForCausalLM(LlamaConfig(vocab=512, dim=128, layers=4, heads=2, ffn=344, max_seq=64)).cuda()
+        ids = torch.randint(0, 512, (8, 64), generator=torch.Generator().manual_seed(1)).cuda()
+        opt = torch.optim.Adam(model.parameters(), lr=1e-3)
+        option = PipeOption(device_cnt=2, batch_cnt=4, batch_size=2, split_points=["layers.1", "layers.2", "layers.3"],
+                            mixed_precision="bf16")
+        runner = _fresh_runner(option)
+        runner.optimizer = opt
+        cmodel = torch.compile(model, backend=partial_compiler)
+        weight, calls, step = list(model.parameters())[3], [], [0]
+
+        def fn(tok):
+            calls.append(0)
+            if user_code == "drops_gradients":
+                opt.zero_grad()
+            elif user_code == "changes_a_weight":
+                with torch.no_grad():
+                    weight.mul_(0.99)
+            elif step[0] == 4 and len(calls) == 3:
+                raise ValueError("user code")
+            loss = cmodel(tok, tok)
+            loss.backward()
+            return loss.detach()
+
+        runner.set_exec_fn(fn)
+        out, planned = [], 0
+        for step[0] in range(6):
+            calls.clear()
+            try:
+                losses = [float(l) for l in runner.step(ids)]
+            except ValueError:
+                losses = "raised"
+            planned += runner.worker.step_plan is not None
+            torch.cuda.synchronize()
+            out.append((losses, [p.grad.clone() for p in model.parameters()],
+                        [p.detach().clone() for p in model.parameters()]))
+        return out, planned
+
+    want, planned = run("1")
+    assert planned == 0 and (want[4][0] == "raised") == (user_code == "raises")
+    got, planned = run("0")
+    assert planned == 4
+    for i, ((l0, g0, p0), (l1, g1, p1)) in enumerate(zip(want, got)):
+        assert l0 == l1, (i, l0, l1)
+        for a, b in zip(g0 + p0, g1 + p1):
+            assert torch.equal(a, b), i
+
+
 def test_lanes_give_bit_identical_per_micro_batch_weight_gradients(monkeypatch):
     """The same, for weight gradients added up micro-batch by micro-batch (PFEIFE_DW_STACK=0, the
     form steps with ragged micro-batches take) at ViT-S/16 size: those products run on the tile
