@@ -18,9 +18,6 @@
 // Q, K, V, O and their gradients are [B, H, T, hd] tensors addressed with element
 // strides (batch, head, token) and unit stride along hd, so heads can live inside a
 // packed qkv projection and the output can be token-major.
-#include <mutex>
-#include <set>
-#include <utility>
 
 #include "pf_common.h"
 
@@ -1120,25 +1117,11 @@ AttnArgs make_args(const pf_attn_desc* d) {
 
 }  // namespace
 
-// Launch of a short-sequence kernel with `lds` bytes of dynamic LDS (above 64 KB the kernel is
-// opted in once per kernel and device).
+// Launch of a short-sequence kernel with `lds` bytes of dynamic LDS.
 template <typename K, typename... Args>
 int launch_short(K kern, dim3 grid, int threads, size_t lds, hipStream_t st, Args... args) {
-  if (lds > 64 * 1024) {
-    static std::mutex mu;
-    static std::set<std::pair<const void*, int>> raised;   // instantiations share this function's type
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) dev = 0;
-    std::lock_guard<std::mutex> lock(mu);
-    if (!raised.count({(const void*)kern, dev})) {
-      const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-      if (e != hipSuccess) {
-        pf_set_error("pf_attention: cannot raise dynamic LDS: %s", hipGetErrorString(e));
-        return PF_ERR_HIP;
-      }
-      raised.insert({(const void*)kern, dev});
-    }
-  }
+  const int rc = pf_allow_lds((const void*)kern, lds > 64 * 1024 ? 160 * 1024 : lds, "pf_attention");
+  if (rc != PF_OK) return rc;
   hipLaunchKernelGGL(kern, grid, dim3((unsigned)threads), lds, st, args...);
   return PF_OK;
 }

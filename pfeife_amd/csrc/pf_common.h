@@ -26,6 +26,10 @@ typedef float float16_t __attribute__((ext_vector_type(16)));
 // ---------------------------------------------------------------------------
 void pf_set_error(const char* fmt, ...);
 
+// Opts `kernel` into `bytes` of dynamic LDS on the current device, where the kernel needs more than the 64 KB every
+// kernel may have; remembered per kernel and device.  Any thread.
+int pf_allow_lds(const void* kernel, size_t bytes, const char* who);
+
 #define PF_REQUIRE(cond, ...)            \
   do {                                   \
     if (!(cond)) {                       \

@@ -570,24 +570,13 @@ int launch16(const pf_gemm_desc& d, hipStream_t st) {
   size_t lds = 2 * (size_t)(BM + BN) * (BK + 8) * sizeof(uint16_t);
   const size_t lds_epi = (size_t)(WGM * WGN) * (BN / WGN / 32) * 32 * EPI_LD * sizeof(float);
   if (lds < lds_epi) lds = lds_epi;
-  if (lds > 64 * 1024) {  // opt in to the large LDS carve-out once per instantiation
-    static bool raised[4] = {false, false, false, false};
-    const int v = (d.a_trans ? 2 : 0) + (d.b_trans ? 1 : 0);
-    if (!raised[v]) {
-      hipError_t e = hipSuccess;
-      if (v == 0) e = hipFuncSetAttribute((const void*)gemm16_kernel<DT, BM, BN, BK, WGM, WGN, false, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      if (v == 1) e = hipFuncSetAttribute((const void*)gemm16_kernel<DT, BM, BN, BK, WGM, WGN, false, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      if (v == 2) e = hipFuncSetAttribute((const void*)gemm16_kernel<DT, BM, BN, BK, WGM, WGN, true, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      if (v == 3) e = hipFuncSetAttribute((const void*)gemm16_kernel<DT, BM, BN, BK, WGM, WGN, true, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      if (e != hipSuccess) {
-        pf_set_error("pf_gemm: cannot raise dynamic LDS to %zu bytes: %s", lds, hipGetErrorString(e));
-        return PF_ERR_HIP;
-      }
-      raised[v] = true;
-    }
-  }
 #define PF_LAUNCH16(AT, BT)                                                                           \
-  hipLaunchKernelGGL((gemm16_kernel<DT, BM, BN, BK, WGM, WGN, AT, BT>), grid, dim3(NT), lds, st, d, g)
+  do {                                                                                                \
+    auto kern = gemm16_kernel<DT, BM, BN, BK, WGM, WGN, AT, BT>;                                      \
+    const int rc = pf_allow_lds((const void*)kern, lds, "pf_gemm");                                   \
+    if (rc != PF_OK) return rc;                                                                       \
+    hipLaunchKernelGGL(kern, grid, dim3(NT), lds, st, d, g);                                          \
+  } while (0)
   if (!d.a_trans && !d.b_trans) PF_LAUNCH16(false, false);
   else if (!d.a_trans && d.b_trans) PF_LAUNCH16(false, true);
   else if (d.a_trans && !d.b_trans) PF_LAUNCH16(true, false);

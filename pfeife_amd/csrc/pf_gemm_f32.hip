@@ -328,19 +328,18 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm32d_kernel(const pf_gemm_d
 }
 
 template <int BM, int BN, int WGM, int WGN, int ST, bool AT, bool BT>
-void launch_one(const pf_gemm_desc& d, const GemmGrid& g, dim3 grid, hipStream_t st) {
+int launch_one(const pf_gemm_desc& d, const GemmGrid& g, dim3 grid, hipStream_t st) {
   constexpr size_t lds = (size_t)ST * (BM + BN) * FK * 4;
-  if constexpr (lds > 64 * 1024) {   // opt in to the large LDS carve-out once per instantiation
-    static std::once_flag once;
-    std::call_once(once, [] {
-      (void)hipFuncSetAttribute((const void*)gemm32d_kernel<BM, BN, WGM, WGN, ST, AT, BT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    });
-  }
-  hipLaunchKernelGGL((gemm32d_kernel<BM, BN, WGM, WGN, ST, AT, BT>), grid, dim3(64 * WGM * WGN), lds, st, d, g);
+  auto kern = gemm32d_kernel<BM, BN, WGM, WGN, ST, AT, BT>;
+  const int rc = pf_allow_lds((const void*)kern, lds, "pf_gemm(f32)");
+  if (rc != PF_OK) return rc;
+  hipLaunchKernelGGL(kern, grid, dim3(64 * WGM * WGN), lds, st, d, g);
+  PF_CHECK_LAUNCH("pf_gemm(f32)");
+  return PF_OK;
 }
 
 template <int BM, int BN, int WGM, int WGN, int ST>
-void launch(const pf_gemm_desc& d, hipStream_t st) {
+int launch(const pf_gemm_desc& d, hipStream_t st) {
   GemmGrid g;
   g.tiles_m = (int)((d.M + BM - 1) / BM);
   g.tiles_n = (int)((d.N + BN - 1) / BN);
@@ -349,10 +348,10 @@ void launch(const pf_gemm_desc& d, hipStream_t st) {
   g.vec_epi = d.c_dtype == PF_F32 && (!d.bias || d.bias_dtype == PF_F32) && (!d.residual || d.res_dtype == PF_F32) && d.ldc < lim &&
               (!d.residual || d.ld_res < lim) && (!d.aux_in || d.ld_aux_in < lim) && (!d.aux_out || d.ld_aux_out < lim);
   const dim3 grid((unsigned)(g.per_xcd * 8), (unsigned)(d.batch1 * d.batch2), 1);
-  if (d.a_trans && d.b_trans) launch_one<BM, BN, WGM, WGN, ST, true, true>(d, g, grid, st);
-  else if (d.a_trans) launch_one<BM, BN, WGM, WGN, ST, true, false>(d, g, grid, st);
-  else if (d.b_trans) launch_one<BM, BN, WGM, WGN, ST, false, true>(d, g, grid, st);
-  else launch_one<BM, BN, WGM, WGN, ST, false, false>(d, g, grid, st);
+  if (d.a_trans && d.b_trans) return launch_one<BM, BN, WGM, WGN, ST, true, true>(d, g, grid, st);
+  if (d.a_trans) return launch_one<BM, BN, WGM, WGN, ST, true, false>(d, g, grid, st);
+  if (d.b_trans) return launch_one<BM, BN, WGM, WGN, ST, false, true>(d, g, grid, st);
+  return launch_one<BM, BN, WGM, WGN, ST, false, false>(d, g, grid, st);
 }
 
 // Tiles.  ST so that a microsecond or more of loads is in flight and (but for the largest) two or more workgroups fit
@@ -395,11 +394,9 @@ const char* pf_gemm_f32_direct_shape(const pf_gemm_desc& d) { return TILES[choos
 
 int pf_gemm_f32_direct(const pf_gemm_desc& d, hipStream_t st) {
   switch (choose(d)) {
-    case 0: launch<128, 128, 2, 4, 4>(d, st); break;
-    case 1: launch<64, 64, 4, 2, 4>(d, st); break;
-    case 2: launch<32, 64, 2, 4, 6>(d, st); break;
-    default: launch<32, 32, 2, 2, 8>(d, st); break;
+    case 0: return launch<128, 128, 2, 4, 4>(d, st);
+    case 1: return launch<64, 64, 4, 2, 4>(d, st);
+    case 2: return launch<32, 64, 2, 4, 6>(d, st);
+    default: return launch<32, 32, 2, 2, 8>(d, st);
   }
-  PF_CHECK_LAUNCH("pf_gemm(f32)");
-  return PF_OK;
 }

@@ -747,21 +747,8 @@ int launch16x_t(const pf_gemm_desc& d, const GemmGrid& g, hipStream_t st) {
   void (*kern)(const pf_gemm_desc, const GemmGrid);
   if constexpr (RAG) kern = gemm16x_ragged_kernel<DT, BM, BN, BK, WGM, WGN, KS, ST, AT, BT, EC>;
   else kern = gemm16x_kernel<DT, BM, BN, BK, WGM, WGN, KS, ST, AT, BT, EC>;
-  if (lds > 64 * 1024) {  // opt in to the large LDS carve-out once per instantiation and device
-    static std::mutex mu;
-    static bool raised[64] = {};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-    std::lock_guard<std::mutex> lock(mu);
-    if (!raised[dev]) {
-      const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      if (e != hipSuccess) {
-        pf_set_error("pf_gemm: cannot raise dynamic LDS to %zu bytes: %s", lds, hipGetErrorString(e));
-        return PF_ERR_HIP;
-      }
-      raised[dev] = true;
-    }
-  }
+  const int rc = pf_allow_lds((const void*)kern, lds, "pf_gemm");
+  if (rc != PF_OK) return rc;
   const dim3 grid((unsigned)(g.per_xcd * 8), (unsigned)(d.batch1 * d.batch2), 1);
   hipLaunchKernelGGL(kern, grid, dim3(NT), lds, st, d, g);
   PF_CHECK_LAUNCH("pf_gemm");
@@ -857,21 +844,8 @@ int launch16x_group(const pf_gemm_desc* d, int n, hipStream_t st) {
     }
     ga.n = n;
     auto kern = gemm16x_group_kernel<DT, BM, BN, BK, WGM, WGN, KS, ST, true, true, EC_ACC32>;
-    if (lds > 64 * 1024) {
-      static std::mutex mu;
-      static bool raised[64] = {};
-      int dev = 0;
-      if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-      std::lock_guard<std::mutex> lock(mu);
-      if (!raised[dev]) {
-        const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) {
-          pf_set_error("pf_gemm_grouped: cannot raise dynamic LDS to %zu bytes: %s", lds, hipGetErrorString(e));
-          return PF_ERR_HIP;
-        }
-        raised[dev] = true;
-      }
-    }
+    const int rc = pf_allow_lds((const void*)kern, lds, "pf_gemm_grouped");
+    if (rc != PF_OK) return rc;
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks, 1, 1), dim3(NT), lds, st, ga);
     PF_CHECK_LAUNCH("pf_gemm_grouped");
     return PF_OK;

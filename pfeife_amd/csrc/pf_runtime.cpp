@@ -2,6 +2,10 @@
 #include <stdarg.h>
 #include <string.h>
 
+#include <map>
+#include <mutex>
+#include <utility>
+
 #include "pf_common.h"
 
 int pf_norm_init_device();   // pf_norm.hip
@@ -15,6 +19,24 @@ void pf_set_error(const char* fmt, ...) {
   va_start(ap, fmt);
   vsnprintf(g_err, sizeof(g_err), fmt, ap);
   va_end(ap);
+}
+
+int pf_allow_lds(const void* kernel, size_t bytes, const char* who) {
+  static std::mutex mu;
+  static std::map<std::pair<const void*, int>, size_t> allowed;
+  if (bytes <= 64 * 1024) return PF_OK;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e == hipSuccess) {
+    std::lock_guard<std::mutex> lock(mu);
+    size_t& have = allowed[{kernel, dev}];
+    if (have >= bytes) return PF_OK;
+    e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (e == hipSuccess) have = bytes;
+  }
+  if (e == hipSuccess) return PF_OK;
+  pf_set_error("%s: cannot raise dynamic LDS to %zu bytes: %s", who, bytes, hipGetErrorString(e));
+  return PF_ERR_HIP;
 }
 
 extern "C" const char* pf_last_error(void) { return g_err; }

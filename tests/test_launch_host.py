@@ -1,0 +1,101 @@
+"""What the library's launchers do on the host, without a GPU: a stand-in for the HIP runtime's launch calls, loaded
+ahead of the library in a child process, checks and counts launches and runs none."""
+import subprocess
+import sys
+
+import pytest
+
+STUB = r"""
+#include <cstddef>
+#include <cstdio>
+#include <map>
+#include <utility>
+struct Dim3 { unsigned x, y, z; };
+static int device = 0, fail_attribute = 0, launches = 0, last_error = 0;
+static std::map<std::pair<const void*, int>, int> allowed;
+static struct { Dim3 grid, block; size_t lds; void* stream; } config;
+extern "C" {
+void stub_device(int d) { device = d; }
+void stub_fail_attribute(int on) { fail_attribute = on; }
+int stub_launches() { const int n = launches; launches = 0; return n; }
+int hipGetDevice(int* d) { *d = device; return 0; }
+int hipFuncSetAttribute(const void* f, int, int value) {
+  if (fail_attribute) return 1;
+  allowed[{f, device}] = value;
+  return 0;
+}
+unsigned __hipPushCallConfiguration(Dim3 g, Dim3 b, size_t lds, void* s) { config = {g, b, lds, s}; return 0; }
+int __hipPopCallConfiguration(Dim3* g, Dim3* b, size_t* lds, void** s) {
+  *g = config.grid; *b = config.block; *lds = config.lds; *s = config.stream; return 0;
+}
+int hipLaunchKernel(const void* f, Dim3, Dim3, void**, size_t lds, void*) {
+  if (lds > 65536 && (size_t)allowed[{f, device}] < lds) return last_error = 1;   // as the runtime refuses it
+  ++launches;
+  return 0;
+}
+int hipGetLastError() { const int e = last_error; last_error = 0; return e; }
+}
+"""
+
+CHILD = r"""
+import ctypes, sys
+stub = ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)     # before anything else that brings the HIP runtime in
+from pfeife_amd import hip
+lib = hip.load(*sys.argv[2:3])
+
+def gemm(M, N, K, at=0, bt=0, dtype=hip.PF_F32, variant=0, **kw):
+    d = hip.GemmDesc()
+    d.in_dtype, d.c_dtype, d.M, d.N, d.K = dtype, hip.PF_F32, M, N, K
+    d.a_trans, d.b_trans, d.variant = at, bt, variant
+    d.lda, d.ldb, d.ldc = (M if at else K), (N if bt else K), N
+    d.batch1, d.batch2, d.alpha = 1, 1, 1.0
+    d.A, d.B, d.C = 1 << 20, 1 << 21, 1 << 22           # (nothing reads them)
+    for k, v in kw.items():
+        setattr(d, k, v)
+    return d
+
+def run(d):
+    return lib.pf_gemm(ctypes.byref(d), None), stub.stub_launches()
+"""
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    path = tmp_path_factory.mktemp("stub")
+    src, so = path / "stub.cpp", path / "libstub.so"
+    src.write_text(STUB)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", str(src), "-o", str(so)], check=True)
+    return str(so)
+
+
+def child(stub, code):
+    res = subprocess.run([sys.executable, "-c", CHILD + code, stub], capture_output=True, text=True, timeout=300)
+    assert res.returncode == 0, res.stdout + res.stderr
+
+
+def test_dynamic_lds_is_allowed_on_every_device_a_kernel_runs_on(stub):
+    """Tiles that need more than 64 KB of LDS, on two devices of one process: every launch is allowed its LDS on the
+    device it goes to; where that fails the call is an error and nothing is launched."""
+    child(stub, r"""
+calls = []
+for at in (0, 1):
+    for bt in (0, 1):
+        calls += [gemm(2048, 2048, 64, at, bt), gemm(1024, 384, 64, at, bt), gemm(256, 192, 64, at, bt), gemm(64, 64, 64, at, bt)]
+        for dt in (hip.PF_F16, hip.PF_BF16):
+            calls += [gemm(512, 512, 128, at, bt, dt, v) for v in (11, 12, 13, 14)]
+            if at == bt:
+                calls += [gemm(512, 512, 128, at, bt, dt, v) for v in list(range(1, 11)) + [15] if not (at and v in (4, 10))]
+stub.stub_fail_attribute(1)
+refused = [run(d) for d in calls]
+assert all((rc == 0) == (n == 1) for rc, n in refused) and sum(rc != 0 for rc, _ in refused) >= 30, refused
+stub.stub_fail_attribute(0)
+for device in (0, 1, 0, 5):
+    stub.stub_device(device)
+    for d in calls:
+        got = run(d)
+        assert got == (0, 1), (device, d.M, d.N, d.a_trans, d.b_trans, d.in_dtype, d.variant, got, lib.pf_last_error())
+group = (hip.GemmDesc * 2)(*[gemm(512, 512, 128, 1, 1, hip.PF_F16, 8, beta=1)] * 2)
+for device in (0, 1):
+    stub.stub_device(device)
+    assert (lib.pf_gemm_grouped(group, 2, None), stub.stub_launches()) == (0, 1), device
+""")
