@@ -705,10 +705,10 @@ int dispatch16(const pf_gemm_desc& d, hipStream_t st) {
       return PF_ERR_UNSUPPORTED;
     }
   }
-  if (d.nonfinite_flag != nullptr) {   // only the fp32 classes of the direct-to-LDS kernel check what they write
+  if (d.nonfinite_flag != nullptr) {   // only plain fp32 results (and these with a bias) of the direct-to-LDS kernel are checked
     const int ec = epi_class(d, epi_vec_ok(d));
     if (!is_x_variant(v) || !x_supports(d, v) || (ec != EC_STORE32 && ec != EC_ACC32) ||
-        (d.a_trans != d.b_trans) || (d.a_trans && d.bias != nullptr)) {
+        (d.a_trans != d.b_trans)) {
       pf_set_error("pf_gemm: nonfinite_flag needs a 16-bit product with fp32 C (stored or accumulated) on the direct-to-LDS kernel");
       return PF_ERR_UNSUPPORTED;
     }
@@ -887,8 +887,7 @@ extern "C" int pf_gemm_variant(const pf_gemm_desc* desc, char* out, int cap) {
                      "reduction-strided) K a multiple of %d", v, x_tile_bk(x_tile_of(v)), x_tile_bk(x_tile_of(v)));
         return PF_ERR_INVALID;
       }
-      int ec = epi_class(d, epi_vec_ok(d));
-      if (d.a_trans && ((ec != EC_ACC32 && ec != EC_STORE32) || d.bias != nullptr)) ec = EC_GENERIC;
+      const int ec = x_epi_class(d, epi_vec_ok(d));
       const bool ragged = !d.a_trans && d.K % x_tile_bk(x_tile_of(v)) != 0;
       snprintf(out, (size_t)cap, "gemm16x_%skernel<%d, %s, %s, %s, %d>", ragged ? "ragged_" : "", d.in_dtype, shapes[x_tile_of(v)], at, bt, ec);
       return PF_OK;

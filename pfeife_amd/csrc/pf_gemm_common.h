@@ -42,8 +42,8 @@ __device__ __forceinline__ Epi make_epi(const pf_gemm_desc& p) {
   return e;
 }
 
-// one element (scalar path: fp32 kernel and ragged / unaligned tails)
-__device__ __forceinline__ void epilogue_scalar(const Epi& e, int64_t c_base, int64_t row, int64_t col, float acc) {
+// one element (scalar path: fp32 kernel and ragged / unaligned tails); returns what is stored, before its rounding
+__device__ __forceinline__ float epilogue_scalar(const Epi& e, int64_t c_base, int64_t row, int64_t col, float acc) {
   float v = e.alpha * acc;
   if (e.bias) v += pf_load_as_f32(e.bias, col, e.bias_dtype);
   if (e.round_mid) v = pf_round_to(e.in_dtype, v);
@@ -54,6 +54,7 @@ __device__ __forceinline__ void epilogue_scalar(const Epi& e, int64_t c_base, in
   const int64_t ci = c_base + row * e.ldc + col;
   if (e.beta) v += pf_load_as_f32(e.C, ci, e.c_dtype);
   pf_store_from_f32(e.C, ci, e.c_dtype, v);
+  return v;
 }
 
 // 8 consecutive columns of one row (vector path)
@@ -237,6 +238,13 @@ inline int epi_class(const pf_gemm_desc& d, int vec_ok) {
   if (dact) return (c16 && d.dact == PF_ACT_GELU) ? EC_DACT16 : EC_GENERIC;
   if (res) return (c32 && d.res_dtype == PF_F32) ? EC_RES32 : ((c16 && d.res_dtype == d.in_dtype) ? EC_RES16 : EC_GENERIC);
   return c32 ? EC_ACC32 : EC_ACC16;
+}
+// ... and the class the direct-to-LDS kernel runs it as: reduction-strided products have straight-line code for a
+// plain fp32 result only
+inline int x_epi_class(const pf_gemm_desc& d, int vec_ok) {
+  const int ec = epi_class(d, vec_ok);
+  const bool plain = (ec == EC_STORE32 || ec == EC_ACC32) && d.bias == nullptr;
+  return d.a_trans && d.b_trans && !plain ? EC_GENERIC : ec;
 }
 
 }  // namespace

@@ -506,6 +506,7 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
   static_assert(BT || TN == 2 || TN == 4 || TN == 8, "whole vectors per lane and row");
   if constexpr (EC == EC_GENERIC) {
     // one rolled loop over 16-row blocks (unrolled, the run-time switches of this class fill the instruction cache)
+    float worst = 0.f;   // sum of v * 0 over the values written: 0 if all are finite, NaN otherwise
 #pragma nounroll
     for (int h = 0; h < TM; ++h) {
       float4_t x[TN];
@@ -522,10 +523,11 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
           const int64_t col = c0 + (BT ? 16 : 1) * j;
-          if (row < M && col < N) epilogue_scalar(epi, c_base, row, col, x[j][r]);
+          if (row < M && col < N) worst = fmaf(epilogue_scalar(epi, c_base, row, col, x[j][r]), 0.f, worst);
         }
       }
     }
+    if (epi.nonfinite != nullptr && worst != 0.f) *epi.nonfinite = 1.f;
     return;
   } else {
     // Straight-line classes.  All global accesses are raw buffer operations whose range check drops rows
@@ -771,7 +773,7 @@ int launch16x(const pf_gemm_desc& d, hipStream_t st) {
     pf_set_error("pf_gemm: this variant needs K %% %d == 0 unless both operands are transposed", BK);
     return PF_ERR_INVALID;
   }
-  const int ec = epi_class(d, g.vec_epi);
+  const int ec = x_epi_class(d, g.vec_epi);
 #define PF_X(AT, BT, EC) launch16x_t<DT, BM, BN, BK, WGM, WGN, KS, ST, AT, BT, EC, false>(d, g, st)
 #define PF_XR(EC) launch16x_t<DT, BM, BN, BK, WGM, WGN, KS, ST, false, false, EC, HAS_RAGGED>(d, g, st)
   if constexpr (HAS_RAGGED) {
@@ -806,8 +808,8 @@ int launch16x(const pf_gemm_desc& d, hipStream_t st) {
   // transposed (reduction-strided) tiles exist for 128 and 256 rows only
   if constexpr (BM != 192) {
     if (d.a_trans && d.b_trans) {   // weight-gradient products
-      if (ec == EC_ACC32 && d.bias == nullptr) return PF_X(true, true, EC_ACC32);
-      if (ec == EC_STORE32 && d.bias == nullptr) return PF_X(true, true, EC_STORE32);
+      if (ec == EC_ACC32) return PF_X(true, true, EC_ACC32);
+      if (ec == EC_STORE32) return PF_X(true, true, EC_STORE32);
       return PF_X(true, true, EC_GENERIC);
     }
   }

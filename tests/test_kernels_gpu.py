@@ -1193,3 +1193,28 @@ def test_weight_gradient_product_unscales_checks_and_stores_inside_a_group(hip, 
                    nonfinite_flag=flag)
     with pytest.raises(RuntimeError, match="nonfinite_flag"):
         bad(torch.cuda.current_stream().cuda_stream)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("beta", [0, 1])
+def test_transposed_product_with_bias_checks_what_it_writes(hip, oracle, dtype, beta):
+    """Both operands transposed, fp32 C, bias, loss scale and overflow flag in one call, at ragged sizes of every tile;
+    a non-finite operand in the last row and column raises the flag."""
+    for i, (variant, M, N, K) in enumerate([(0, 72, 40, 72), (7, 264, 520, 96), (8, 264, 136, 200), (9, 264, 392, 64),
+                                            (15, 72, 136, 136)]):
+        a, b, c = rnd((K, M), dtype, 40 + i), rnd((K, N), dtype, 50 + i, 0.1), rnd((M, N), F32, 60 + i)
+        bias, scale = rnd((N,), dtype, 70 + i), torch.tensor([64.0])
+        kw = dict(M=M, N=N, K=K, lda=M, ldb=N, ldc=N, a_trans=1, b_trans=1, beta=beta)
+        want = c.clone()
+        oracle.gemm(a=a, b=b, c=want, bias=bias, unscale_by=scale, **kw)()
+        flag = torch.zeros(1, device="cuda")
+        for plant in (False, True):
+            if plant:
+                a[K - 1, M - 1] = float("inf")
+            dev = c.cuda()
+            hip.gemm(a=a.cuda(), b=b.cuda(), c=dev, bias=bias.cuda(), unscale_by=scale.cuda(), nonfinite_flag=flag,
+                     variant=variant, **kw)(torch.cuda.current_stream().cuda_stream)
+            torch.cuda.synchronize()
+            assert float(flag) == float(plant), (variant, plant)
+            # fp32 sums of K products of order 0.1 / 64 in another order
+            torch.testing.assert_close(dev.cpu()[:M - plant], want[:M - plant], rtol=1e-4, atol=1e-5)

@@ -99,3 +99,18 @@ for device in (0, 1):
     stub.stub_device(device)
     assert (lib.pf_gemm_grouped(group, 2, None), stub.stub_launches()) == (0, 1), device
 """)
+
+
+def test_transposed_product_with_bias_and_overflow_flag_is_accepted(stub):
+    """Both operands transposed, fp32 C stored or accumulated, a bias and `nonfinite_flag`, on every tile with such a
+    kernel; the flag stays refused with an activation and where no tile checks what it writes."""
+    child(stub, r"""
+for dt in (hip.PF_F16, hip.PF_BF16):
+    for beta in (0, 1):
+        for v in (0, 1, 2, 3, 5, 6, 7, 8, 9, 15):
+            d = gemm(512, 512, 128, 1, 1, dt, v, beta=beta, bias=1 << 23, nonfinite_flag=1 << 24)
+            assert run(d) == (0, 1), (dt, beta, v, lib.pf_last_error())
+    assert run(gemm(512, 512, 128, 1, 1, dt, act=1, aux_out=1 << 23, ld_aux_out=512, nonfinite_flag=1 << 24)) == (-2, 0)
+    assert run(gemm(512, 512, 128, 1, 0, dt, nonfinite_flag=1 << 24)) == (-2, 0)
+    assert run(gemm(512, 512, 128, 1, 1, dt, 11, nonfinite_flag=1 << 24)) == (-2, 0)
+""")
