@@ -170,7 +170,7 @@ typedef struct pf_gemm_desc {
   float* nonfinite_flag; /* optional: set to 1.0f when a value written to C is not finite (the overflow check of
                        the same unscale_); only where the direct-to-LDS kernel stores or accumulates an fp32 C without
                        activation or residual (pf_gemm_variant ends in ", 1>" or ", 4>", or in ", -1>" for such a
-                       product with both operands transposed and a bias), PF_ERR_UNSUPPORTED elsewhere */
+                       product with both operands transposed and a bias or round_mid), PF_ERR_UNSUPPORTED elsewhere */
 } pf_gemm_desc;
 
 int pf_gemm(const pf_gemm_desc* desc, void* stream);

@@ -824,7 +824,7 @@ bool groupable(const pf_gemm_desc& d, int& variant) {
   if (!is_x_variant(variant)) return false;
   if (!x_supports(d, variant)) return false;
   // (a product that stores rides in the accumulate launch: its old C reads as zeros)
-  const int ec = epi_class(d, epi_vec_ok(d));
+  const int ec = x_epi_class(d, epi_vec_ok(d));
   return ec == EC_ACC32 || ec == EC_STORE32;
 }
 }  // namespace

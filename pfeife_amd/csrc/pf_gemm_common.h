@@ -240,10 +240,10 @@ inline int epi_class(const pf_gemm_desc& d, int vec_ok) {
   return c32 ? EC_ACC32 : EC_ACC16;
 }
 // ... and the class the direct-to-LDS kernel runs it as: reduction-strided products have straight-line code for a
-// plain fp32 result only
+// plain fp32 result only (no bias, no rounding to the operands' type before it is stored or added)
 inline int x_epi_class(const pf_gemm_desc& d, int vec_ok) {
   const int ec = epi_class(d, vec_ok);
-  const bool plain = (ec == EC_STORE32 || ec == EC_ACC32) && d.bias == nullptr;
+  const bool plain = (ec == EC_STORE32 || ec == EC_ACC32) && d.bias == nullptr && !d.round_mid;
   return d.a_trans && d.b_trans && !plain ? EC_GENERIC : ec;
 }
 

@@ -309,7 +309,7 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
     }
   };
   // Fetched before the K loop, which hides the latency; after it in the GELU' class, which hardly ever has a
-  // bias and has no registers to spare for one.  Weight-gradient products with a bias take the generic class.
+  // bias and has no registers to spare for one.  (Weight-gradient products with a bias take the generic class.)
   constexpr bool HAS_BIAS = EC != EC_GENERIC && !AT;
   constexpr bool BIAS_EARLY = HAS_BIAS && EC != EC_DACT16;
   if constexpr (BIAS_EARLY) load_bias();

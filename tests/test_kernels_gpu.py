@@ -1218,3 +1218,23 @@ def test_transposed_product_with_bias_checks_what_it_writes(hip, oracle, dtype, 
             assert float(flag) == float(plant), (variant, plant)
             # fp32 sums of K products of order 0.1 / 64 in another order
             torch.testing.assert_close(dev.cpu()[:M - plant], want[:M - plant], rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("beta", [0, 1])
+def test_transposed_product_rounds_before_it_stores_or_adds(hip, oracle, dtype, beta):
+    """`round_mid` with both operands transposed and an fp32 C.  Integer-valued operands: every sum is exact in fp32, so
+    what is stored is exactly the sum rounded to the operands' type (many sums are not representable there)."""
+    for i, (variant, M, N, K) in enumerate([(0, 72, 40, 72), (7, 264, 520, 96), (8, 264, 136, 200), (9, 264, 392, 64),
+                                            (15, 72, 136, 136)]):
+        g = torch.Generator().manual_seed(i)
+        a = torch.randint(-30, 31, (K, M), generator=g).to(dtype)
+        b = torch.randint(-30, 31, (K, N), generator=g).to(dtype)
+        c = torch.randint(-30, 31, (M, N), generator=g).to(F32)
+        kw = dict(M=M, N=N, K=K, lda=M, ldb=N, ldc=N, a_trans=1, b_trans=1, beta=beta, round_mid=1)
+        want, dev = c.clone(), c.cuda()
+        oracle.gemm(a=a, b=b, c=want, **kw)()
+        assert not torch.equal(want - (c if beta else 0), a.float().t() @ b.float())
+        hip.gemm(a=a.cuda(), b=b.cuda(), c=dev, variant=variant, **kw)(torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert torch.equal(dev.cpu(), want), variant

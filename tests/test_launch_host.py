@@ -114,3 +114,20 @@ for dt in (hip.PF_F16, hip.PF_BF16):
     assert run(gemm(512, 512, 128, 1, 0, dt, nonfinite_flag=1 << 24)) == (-2, 0)
     assert run(gemm(512, 512, 128, 1, 1, dt, 11, nonfinite_flag=1 << 24)) == (-2, 0)
 """)
+
+
+def test_transposed_product_that_rounds_before_it_stores_runs_where_that_is_done(stub):
+    """round_mid of a product with both operands transposed: not on the straight-line kernels (no rounding there), and
+    not as a member of a grouped launch."""
+    child(stub, r"""
+name = ctypes.create_string_buffer(128)
+for dt in (hip.PF_F16, hip.PF_BF16):
+    for beta in (0, 1):
+        for v in (0, 1, 2, 3, 5, 6, 7, 8, 9, 15):
+            for flag in (None, 1 << 24):
+                d = gemm(512, 512, 128, 1, 1, dt, v, beta=beta, round_mid=1, nonfinite_flag=flag)
+                assert run(d) == (0, 1), (dt, beta, v, lib.pf_last_error())
+                assert lib.pf_gemm_variant(ctypes.byref(d), name, 128) == 0 and name.value.endswith(b", true, true, -1>"), name.value
+                group = (hip.GemmDesc * 2)(d, d)
+                assert (lib.pf_gemm_grouped(group, 2, None), stub.stub_launches()) == (0, 2)
+""")
