@@ -334,6 +334,7 @@ class StageWorker:
         """Frees the captured hipGraphs of a micro-batch slot that is being replaced or released."""
         if slot is None or not hasattr(self.kernels, "destroy_graph"):
             return
+        self._drain()
         for prog in slot.stage_programs.values():
             for attr in ("fwd_graph", "bwd_graph"):
                 g = getattr(prog, attr, None)
@@ -342,9 +343,11 @@ class StageWorker:
                     setattr(prog, attr, None)
 
     def _drop_dw_jobs(self):
-        for job in self.dw_jobs.values():
-            if job[1] is not None and hasattr(self.kernels, "destroy_graph"):
-                self.kernels.destroy_graph(job[1])
+        graphs = [job[1] for job in self.dw_jobs.values() if job[1] is not None]
+        if graphs and hasattr(self.kernels, "destroy_graph"):
+            self._drain()
+            for graph in graphs:
+                self.kernels.destroy_graph(graph)
         self.dw_jobs = {}
 
     def _drop_step_plan(self):
@@ -353,12 +356,19 @@ class StageWorker:
         if plan is None:
             return
         self.issuer.wait()
-        for lane in {id(l): l for l in list((self.lanes or {}).values()) + [self.stream_obj]}.values():
-            lane.synchronize()
+        self._drain()
         plan.release()
+
+    def _drain(self):
+        """What has been issued has run, on every lane (a failed step leaves lanes running): graphs, events and
+        buffers it uses may go."""
+        for lane in list((self.lanes or {}).values()) + [self.stream_obj]:
+            if lane is not None:
+                lane.synchronize()
 
     def _drop_begin_graph(self):
         if self.begin_graph is not None and hasattr(self.kernels, "destroy_graph"):
+            self._drain()      # (the step before may still be running it)
             self.kernels.destroy_graph(self.begin_graph)
         self.begin_graph = None
 
@@ -369,8 +379,7 @@ class StageWorker:
         if self.issuer is not None:
             self.issuer.close()
             self.issuer = None
-        if self.stream_obj is not None:
-            self.stream_obj.synchronize()
+        self._drain()
         for slot in self.mbs.values():
             self._drop_graphs(slot)
         self._drop_begin_graph()

@@ -604,3 +604,42 @@ def test_planned_steps_leave_user_code_before_the_model_alone(monkeypatch, user_
         for a, b in zip(g0 + p0, g1 + p1):
             assert torch.equal(a, b), i
     assert len(seen0) == len(seen1) and all(torch.equal(a, b) for a, b in zip(seen0, seen1))
+
+
+@pytest.mark.parametrize("drop", ["begin", "capture", "slot", "weight_gradients"])
+def test_a_graph_is_destroyed_after_every_lane_has_run_what_was_issued(drop):
+    """Replays of a step may still be running when its graphs are captured anew or dropped, on the main stream and,
+    after a failed step, on any lane."""
+    from pfeife_amd.mp.worker import StageWorker
+
+    log = []
+
+    class Stream:
+        cuda_stream = 0
+
+        def synchronize(self):
+            log.append(self)
+
+    class Kernels:
+        def capture(self, launches, stream):
+            return "graph"
+
+        def destroy_graph(self, graph):
+            log.append("destroy")
+
+    w = StageWorker.__new__(StageWorker)
+    w.kernels, w.stream_obj, w.lanes = Kernels(), Stream(), {0: Stream(), 1: Stream()}
+    w.mbs, w.dw_jobs, w.step_plan, w.issuer, w.begin_graph = {}, {}, None, None, "graph"
+    w.params = SimpleNamespace(zero_launches=lambda: [0], refresh_launches=lambda: [], zero=[], refresh=[])
+    if drop == "begin":
+        w._drop_begin_graph()
+    elif drop == "capture":
+        w.capture_graphs()
+        assert w.begin_graph == "graph"
+    elif drop == "slot":
+        w._drop_graphs(SimpleNamespace(stage_programs={0: SimpleNamespace(fwd_graph="graph", bwd_graph="graph")}))
+    else:
+        w.dw_jobs = {0: [[], "graph"], 1: [[], None]}
+        w._drop_dw_jobs()
+    assert "destroy" in log
+    assert set(log[:log.index("destroy")]) == {w.stream_obj, *w.lanes.values()}
