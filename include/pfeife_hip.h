@@ -323,6 +323,9 @@ typedef struct pf_attn_desc {
   float* delta;
   int64_t q_sb, q_sh, q_st, k_sb, k_sh, k_st, v_sb, v_sh, v_st, o_sb, o_sh, o_st;
   int64_t do_sb, do_sh, do_st, dq_sb, dq_sh, dq_st, dk_sb, dk_sh, dk_st, dv_sb, dv_sh, dv_st;
+  void* o_lo;         /* optional, hd > 96 only (PF_ERR_INVALID otherwise): 2048 times what O lost when it was rounded
+                         to `dtype`, laid out as o; forward: written; backward: read, delta = rowsum(dO * O) is then
+                         formed from O to twice its digits */
 } pf_attn_desc;
 int pf_attention_fwd(const pf_attn_desc* desc, void* stream);
 int pf_attention_bwd(const pf_attn_desc* desc, void* stream);

@@ -137,6 +137,7 @@ class OracleKernels:
 
     # -- fused attention -----------------------------------------------------------
     MAX_FUSED_HEAD_DIM = 128
+    O_LO_HEAD_DIM = 96
 
     @staticmethod
     def _attn_scores(q, k, scale, causal):
@@ -148,22 +149,25 @@ class OracleKernels:
             s = s.masked_fill(j > i + (Tk - Tq), float("-inf"))
         return s
 
-    def attention_fwd(self, q, k, v, o, lse, scale, causal):
+    def attention_fwd(self, q, k, v, o, lse, scale, causal, o_lo=None):
         def launch(stream=None):
             s = self._attn_scores(q, k, scale, causal)
             l = torch.logsumexp(s, dim=-1)
             p = torch.exp(s - l[..., None]).to(q.dtype).float()   # probabilities enter the PV product in 16 bits
-            o.copy_(torch.matmul(p, v.float()).to(o.dtype))
+            out = torch.matmul(p, v.float())
+            o.copy_(out.to(o.dtype))
             lse.copy_(l)
+            if o_lo is not None:     # what the rounding lost, scaled into the type's range
+                o_lo.copy_(((out - o.float()) * 2048.0).to(o.dtype))
 
         return launch
 
-    def attention_bwd(self, q, k, v, o, d_o, lse, delta, dq, dk, dv, scale, causal):
+    def attention_bwd(self, q, k, v, o, d_o, lse, delta, dq, dk, dv, scale, causal, o_lo=None):
         def launch(stream=None):
             s = self._attn_scores(q, k, scale, causal)
             p = torch.exp(s - lse[..., None].float())
             do = d_o.float()
-            dlt = (do * o.float()).sum(dim=-1)
+            dlt = (do * (o.float() if o_lo is None else o.float() + o_lo.float() / 2048.0)).sum(dim=-1)
             delta.copy_(dlt)
             dp = torch.matmul(do, v.float().transpose(-1, -2))
             ds = (p * (dp - dlt[..., None]) * scale).to(q.dtype).float()

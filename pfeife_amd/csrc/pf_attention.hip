@@ -25,10 +25,11 @@ namespace {
 
 constexpr int KT = 64;        // keys (forward/dQ) or queries (dK/dV) per LDS tile
 constexpr float LOG2E = 1.4426950408889634f;
+constexpr float O_LO = 2048.f;   // scale of what rounding O lost: at most as large as O itself, in fp16 too
 
 struct AttnArgs {
   const uint16_t* q; const uint16_t* k; const uint16_t* v; const uint16_t* o; const uint16_t* d_o;
-  uint16_t* out; uint16_t* dq; uint16_t* dk; uint16_t* dv;
+  uint16_t* out; uint16_t* o_lo; uint16_t* dq; uint16_t* dk; uint16_t* dv;
   float* lse; const float* delta;
   int64_t q_sb, q_sh, q_st, k_sb, k_sh, k_st, v_sb, v_sh, v_st, o_sb, o_sh, o_st;
   int64_t do_sb, do_sh, do_st, dq_sb, dq_sh, dq_st, dk_sb, dk_sh, dk_st, dv_sb, dv_sh, dv_st;
@@ -43,6 +44,8 @@ template <> struct M32<PF_F16> {
                                                   0, 0);
   }
   static __device__ __forceinline__ uint32_t pack(float lo, float hi) { return pf_pack2_f16(lo, hi); }
+  static __device__ __forceinline__ float lo(uint32_t w) { return pf_f16_bits_to_f32((uint16_t)(w & 0xffffu)); }
+  static __device__ __forceinline__ float hi(uint32_t w) { return pf_f16_bits_to_f32((uint16_t)(w >> 16)); }
 };
 template <> struct M32<PF_BF16> {
   static __device__ __forceinline__ float16_t run(uint4 a, uint4 b, float16_t c) {
@@ -50,6 +53,8 @@ template <> struct M32<PF_BF16> {
                                                    0, 0, 0);
   }
   static __device__ __forceinline__ uint32_t pack(float lo, float hi) { return pf_pack2_bf16(lo, hi); }
+  static __device__ __forceinline__ float lo(uint32_t w) { return __uint_as_float(w << 16); }
+  static __device__ __forceinline__ float hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 };
 
 // registers r..r+7 of an accumulator tile -> one 16-byte MFMA operand (8 x 16-bit)
@@ -258,13 +263,23 @@ __global__ __launch_bounds__(256, HD <= 64 ? 3 : 2) void attn_fwd_kernel(const A
           const uint2 w = make_uint2(M32<DT>::pack(oacc[o][4 * g] * inv, oacc[o][4 * g + 1] * inv),
                                      M32<DT>::pack(oacc[o][4 * g + 2] * inv, oacc[o][4 * g + 3] * inv));
           *(uint2*)(O + h0) = w;
+          if constexpr (HD > 96) {
+            if (a.o_lo != nullptr) {
+              auto rest = [&](float v, float kept) { return (v * inv - kept) * O_LO; };
+              *(uint2*)(a.o_lo + (O - a.out) + h0) =
+                  make_uint2(M32<DT>::pack(rest(oacc[o][4 * g], M32<DT>::lo(w.x)), rest(oacc[o][4 * g + 1], M32<DT>::hi(w.x))),
+                             M32<DT>::pack(rest(oacc[o][4 * g + 2], M32<DT>::lo(w.y)), rest(oacc[o][4 * g + 3], M32<DT>::hi(w.y))));
+            }
+          }
         }
       }
     if ((lane >> 5) == 0) a.lse[((int64_t)bh) * a.Tq + qi] = (l > 0.f) ? (m * sc + log2f(l)) / LOG2E : -INFINITY;
   }
 }
 
-// delta[b,h,q] = sum_hd dO * O : 8 lanes per row (16-byte loads), 8 rows per wavefront
+// delta[b,h,q] = sum_hd dO * O : 8 lanes per row (16-byte loads), 8 rows per wavefront.  With o_lo, from O to twice its
+// digits: where one key has most of a query's weight, dP - delta is a small difference, and the rounding of O is the
+// largest error in it.
 __global__ __launch_bounds__(256) void attn_delta_kernel(const AttnArgs a, float* delta) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t rows = (int64_t)a.B * a.H * a.Tq;
@@ -280,6 +295,13 @@ __global__ __launch_bounds__(256) void attn_delta_kernel(const AttnArgs a, float
       float x[8], y[8];
       if (bf) { Vec8<PF_BF16>::load(O, c, x); Vec8<PF_BF16>::load(D, c, y); }
       else { Vec8<PF_F16>::load(O, c, x); Vec8<PF_F16>::load(D, c, y); }
+      if (a.o_lo != nullptr) {
+        float z[8];
+        if (bf) Vec8<PF_BF16>::load(a.o_lo + (O - a.o), c, z);
+        else Vec8<PF_F16>::load(a.o_lo + (O - a.o), c, z);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) x[k] += z[k] * (1.f / O_LO);
+      }
 #pragma unroll
       for (int k = 0; k < 8; ++k) s += x[k] * y[k];
     }
@@ -1092,6 +1114,7 @@ int check_common(const pf_attn_desc* d, const char* name) {
   PF_REQUIRE(strides_ok(d->q, d->q_sb, d->q_sh, d->q_st) && strides_ok(d->k, d->k_sb, d->k_sh, d->k_st) &&
                  strides_ok(d->v, d->v_sb, d->v_sh, d->v_st),
              "%s: q/k/v must be 16-byte aligned with strides that are multiples of 8", name);
+  if (d->o_lo) PF_REQUIRE(d->hd > 96 && pf_aligned(d->o_lo, 16), "%s: o_lo needs a head dim above 96 and 16-byte alignment", name);
   if (d->causal) PF_REQUIRE(d->Tk >= d->Tq, "%s: causal attention needs Tk >= Tq", name);
   return PF_OK;
 }
@@ -1104,7 +1127,7 @@ AttnArgs make_args(const pf_attn_desc* d) {
   a.q = (const uint16_t*)d->q; a.k = (const uint16_t*)d->k; a.v = (const uint16_t*)d->v;
   a.o = (const uint16_t*)d->o; a.d_o = (const uint16_t*)d->d_o; a.out = (uint16_t*)d->o;
   a.dq = (uint16_t*)d->dq; a.dk = (uint16_t*)d->dk; a.dv = (uint16_t*)d->dv;
-  a.lse = d->lse; a.delta = d->delta;
+  a.o_lo = (uint16_t*)d->o_lo; a.lse = d->lse; a.delta = d->delta;
   a.q_sb = d->q_sb; a.q_sh = d->q_sh; a.q_st = d->q_st; a.k_sb = d->k_sb; a.k_sh = d->k_sh; a.k_st = d->k_st;
   a.v_sb = d->v_sb; a.v_sh = d->v_sh; a.v_st = d->v_st; a.o_sb = d->o_sb; a.o_sh = d->o_sh; a.o_st = d->o_st;
   a.do_sb = d->do_sb; a.do_sh = d->do_sh; a.do_st = d->do_st; a.dq_sb = d->dq_sb; a.dq_sh = d->dq_sh;

@@ -10,7 +10,7 @@
 
 int pf_norm_init_device();   // pf_norm.hip
 
-#define PF_ABI_VERSION 4
+#define PF_ABI_VERSION 5
 
 static thread_local char g_err[512] = "";
 

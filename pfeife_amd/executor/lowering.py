@@ -1394,7 +1394,9 @@ def _lower_sdpa_fused(L, vals, tensors, dims, scale, causal, req):
     O = L.alloc((Bn, Tq, H, hd), cd)            # token-major, so that transpose(1,2).reshape is a view
     Ov = O.permute(0, 2, 1, 3)
     lse = L.alloc((Bn, H, Tq), torch.float32)
-    L.emit(L.kernels.attention_fwd(qt, kt, vt, Ov, lse, scale, causal))
+    # (wide heads keep O to twice its digits for the backward pass, see attn_delta_kernel)
+    o_lo = L.alloc((Bn, Tq, H, hd), cd).permute(0, 2, 1, 3) if req and hd > L.kernels.O_LO_HEAD_DIM else None
+    L.emit(L.kernels.attention_fwd(qt, kt, vt, Ov, lse, scale, causal, o_lo))
     outv = Val(Ov, req_grad=req)
 
     def bwd(B):
@@ -1418,7 +1420,7 @@ def _lower_sdpa_fused(L, vals, tensors, dims, scale, causal, req):
             else:
                 buf = B.temp(val.shape, cd)
             outs.append(buf)
-        B.emit(B.k.attention_bwd(qt, kt, vt, Ov, g, lse, delta, outs[0], outs[1], outs[2], scale, causal))
+        B.emit(B.k.attention_bwd(qt, kt, vt, Ov, g, lse, delta, outs[0], outs[1], outs[2], scale, causal, o_lo))
         for val, dst, prev, buf, direct in plan:
             if not direct:
                 B.merge(buf, dst, prev)

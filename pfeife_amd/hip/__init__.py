@@ -16,7 +16,7 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libpfeife_hip.so")
-ABI_VERSION = 4
+ABI_VERSION = 5
 
 PF_F32, PF_F16, PF_BF16, PF_I64, PF_I32, PF_U8 = 0, 1, 2, 3, 4, 5
 ACT_NONE, ACT_GELU, ACT_GELU_TANH, ACT_SILU, ACT_RELU = 0, 1, 2, 3, 4
@@ -85,7 +85,8 @@ class AttnDesc(Structure):
                 + [(n, c_void_p) for n in ("q", "k", "v", "o", "d_o", "dq", "dk", "dv", "lse", "delta")]
                 + [(n, c_int64) for n in ("q_sb", "q_sh", "q_st", "k_sb", "k_sh", "k_st", "v_sb", "v_sh", "v_st",
                                           "o_sb", "o_sh", "o_st", "do_sb", "do_sh", "do_st", "dq_sb", "dq_sh",
-                                          "dq_st", "dk_sb", "dk_sh", "dk_st", "dv_sb", "dv_sh", "dv_st")])
+                                          "dq_st", "dk_sb", "dk_sh", "dk_st", "dv_sb", "dv_sh", "dv_st")]
+                + [("o_lo", c_void_p)])
 
 
 # name -> argtypes (every function returns int unless listed in _RET_I64)
@@ -459,9 +460,10 @@ class HipKernels:
 
     # -- fused attention -----------------------------------------------------------
     MAX_FUSED_HEAD_DIM = 128
+    O_LO_HEAD_DIM = 96     # above it the forward pass may keep what rounding O lost, for the backward pass
 
     @staticmethod
-    def _attn_desc(q, k, v, o, lse, scale, causal, d_o=None, dq=None, dk=None, dv=None, delta=None):
+    def _attn_desc(q, k, v, o, lse, scale, causal, d_o=None, dq=None, dk=None, dv=None, delta=None, o_lo=None):
         d = AttnDesc()
         Bn, H, Tq, hd = q.shape
         d.dtype, d.B, d.H, d.Tq, d.Tk, d.hd, d.causal = dtype_code(q.dtype), Bn, H, Tq, k.shape[2], hd, int(causal)
@@ -476,15 +478,19 @@ class HipKernels:
             setattr(d, name + "_sb", t.stride(0))
             setattr(d, name + "_sh", t.stride(1))
             setattr(d, name + "_st", t.stride(2))
+        if o_lo is not None:
+            if o_lo.shape != o.shape or o_lo.stride() != o.stride() or o_lo.dtype != o.dtype:
+                raise RuntimeError("attention operand o_lo must be laid out as o")
+            d.o_lo = _ptr(o_lo)
         return d
 
-    def attention_fwd(self, q, k, v, o, lse, scale, causal):
-        d = self._attn_desc(q, k, v, o, lse, scale, causal)
-        return self._prep("pf_attention_fwd", (byref(d),), (d, q, k, v, o, lse))
+    def attention_fwd(self, q, k, v, o, lse, scale, causal, o_lo=None):
+        d = self._attn_desc(q, k, v, o, lse, scale, causal, o_lo=o_lo)
+        return self._prep("pf_attention_fwd", (byref(d),), (d, q, k, v, o, lse, o_lo))
 
-    def attention_bwd(self, q, k, v, o, d_o, lse, delta, dq, dk, dv, scale, causal):
-        d = self._attn_desc(q, k, v, o, lse, scale, causal, d_o, dq, dk, dv, delta)
-        return self._prep("pf_attention_bwd", (byref(d),), (d, q, k, v, o, d_o, lse, delta, dq, dk, dv))
+    def attention_bwd(self, q, k, v, o, d_o, lse, delta, dq, dk, dv, scale, causal, o_lo=None):
+        d = self._attn_desc(q, k, v, o, lse, scale, causal, d_o, dq, dk, dv, delta, o_lo)
+        return self._prep("pf_attention_bwd", (byref(d),), (d, q, k, v, o, d_o, lse, delta, dq, dk, dv, o_lo))
 
     # -- normalisation -----------------------------------------------------------
     def layernorm_fwd(self, x, gamma, beta, y, mean, rstd, rows, d, eps):

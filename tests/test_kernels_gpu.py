@@ -1238,3 +1238,41 @@ def test_transposed_product_rounds_before_it_stores_or_adds(hip, oracle, dtype, 
         hip.gemm(a=a.cuda(), b=b.cuda(), c=dev, variant=variant, **kw)(torch.cuda.current_stream().cuda_stream)
         torch.cuda.synchronize()
         assert torch.equal(dev.cpu(), want), variant
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("hd,T,causal", [(104, 131, 0), (112, 509, 1), (128, 1021, 1), (128, 33, 0)])
+def test_wide_head_gradients_are_no_further_off_than_with_stored_probabilities(hip, dtype, hd, T, causal):
+    """Head dims above 96 where single keys hold most of a query's weight (scores of standard deviation 4 to 6): dQ and
+    dK against 64 bits, no further off than the route that stores 16-bit probabilities and forms the row sums of
+    dP * P in fp32, here with 64 bits in place of its fp32 (with delta from the rounded O alone they are)."""
+    B, H, scale = 1, 4, hd ** -0.5
+    for spread in (2.0, 2.5):
+        g = torch.Generator().manual_seed(hd + T)
+        q, k, v, do = ((torch.randn(B, T, H, hd, generator=g) * s).to(dtype).permute(0, 2, 1, 3)
+                       for s in (spread, spread, spread, 1.0))
+        qd, kd, vd, dod = (t.cuda() for t in (q, k, v, do))
+        o = torch.zeros(B, T, H, hd, dtype=dtype, device="cuda").permute(0, 2, 1, 3)
+        o_lo, dq, dk, dv = (torch.zeros_like(o) for _ in range(4))
+        lse, delta = (torch.zeros(B, H, T, device="cuda") for _ in range(2))
+        hip.run("attention_fwd", qd, kd, vd, o, lse, scale, causal, o_lo)
+        hip.run("attention_bwd", qd, kd, vd, o, dod, lse, delta, dq, dk, dv, scale, causal, o_lo)
+        torch.cuda.synchronize()
+        q, k, v, do = (t.double() for t in (q, k, v, do))
+        s = q @ k.transpose(2, 3) * scale
+        if causal:
+            s = s.masked_fill(torch.ones(T, T, dtype=torch.bool).triu(1), float("-inf"))
+        p, dp = torch.softmax(s, -1), do @ v.transpose(2, 3)
+        p16 = p.to(dtype).double()
+
+        def grads(ds):
+            return ds @ k * scale, ds.transpose(2, 3) @ q * scale
+
+        def err(got, want):
+            return float((got - want).norm() / want.norm())
+
+        want = grads(p * (dp - (dp * p).sum(-1, keepdim=True)))
+        stored = grads((p16 * (dp - (dp * p16).sum(-1, keepdim=True))).to(dtype).double())
+        for nm, got, ref, w in (("dq", dq, stored[0], want[0]), ("dk", dk, stored[1], want[1])):
+            # (rounding the gradient itself to 16 bits is in `got` only)
+            assert err(got.cpu().double(), w) <= err(ref.to(dtype).double(), w), (nm, spread)
