@@ -821,6 +821,51 @@ def test_llama_style_four_stages_looped(mixed):
     _check_grads(model, ref, mixed)
 
 
+@pytest.mark.parametrize("mixed", ["bf16", "fp16"])
+@pytest.mark.parametrize("hd,seq", [(104, 77), (128, 131)])
+def test_decoder_with_wide_heads_matches_pytorch(mixed, hd, seq):
+    """Whole steps of a decoder whose head dims (above 96) run on the fused kernels that keep O's lost digits: odd
+    sequence lengths, two looped stages, captured steps included, against the oracle's stage executor."""
+    import torch.nn.functional as F
+
+    from oracle.stage_oracle import run_pipeline_step
+    from pfeife_amd.bench_models.llama import LlamaConfig, LlamaForCausalLM, split_stages
+    from pfeife_amd.mp import partial_compiler
+    from pfeife_amd.option import PipeOption
+
+    cfg = LlamaConfig(vocab=512, dim=2 * hd, layers=2, heads=2, ffn=688, max_seq=seq)
+    torch.manual_seed(0)
+    model = LlamaForCausalLM(cfg)
+    ref = copy.deepcopy(model)
+    ids = torch.randint(0, cfg.vocab, (4, seq), generator=torch.Generator().manual_seed(42))
+    option = PipeOption(device_cnt=2, batch_cnt=2, batch_size=2, split_points=["layers.1"], mixed_precision=mixed,
+                        optimizer=dict(type="sgd", lr=0.0))
+    runner = _fresh_runner(option)
+    model.cuda()
+    cmodel = torch.compile(model, backend=partial_compiler)
+
+    def fn(tok):
+        loss = cmodel(tok, tok)
+        loss.backward()
+        return loss.detach()
+
+    runner.set_exec_fn(fn)
+
+    def shifted_ce(logits, tok):
+        return F.cross_entropy(logits[:, :-1, :].reshape(-1, logits.shape[-1]).float(), tok[:, 1:].reshape(-1))
+
+    adt = {"bf16": torch.bfloat16, "fp16": torch.float16}[mixed]
+    want = run_pipeline_step(split_stages(ref, [1]), shifted_ce, ids, ids, 2, device_cnt=2, autocast_dtype=adt)
+    for _ in range(3):      # job by job, captured, from job lists
+        losses = runner.step(ids.cuda())
+        torch.cuda.synchronize()
+        for a, b in zip(losses, want):
+            assert abs(float(a) - float(b)) <= 2e-2 * abs(float(b)), (float(a), float(b))
+        _check_grads(model, ref, mixed)
+    launches = [l for slot in runner.worker.mbs.values() for p in slot.stage_programs.values() for l in list(p.fwd) + list(p.bwd)]
+    assert {"pf_attention_fwd", "pf_attention_bwd"} <= {getattr(l, "kernel", "") for l in launches}
+
+
 @pytest.mark.parametrize("loop_batch,prefetch_fwd", [(2, 1), (4, 0), (4, 1), (8, 0)])
 def test_llama_style_four_stages_schedule_variants(loop_batch, prefetch_fwd):
     """`prefetch_fwd` and `loop_batch` on the HIP path (pfeife/schedule/scheduler.py:89-100): the
