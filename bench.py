@@ -110,16 +110,32 @@ def build_workload(name, device):
     return runner, tuple(t.to(device) for t in inputs), info
 
 
+def gemm_source_digest():
+    """Names the matrix-product kernels' source code; the traffic summary says which it was measured on."""
+    import hashlib
+
+    h = hashlib.sha256()
+    csrc = os.path.join(ROOT, "pfeife_amd", "csrc")
+    for name in sorted(os.listdir(csrc)):
+        if name.startswith("pf_gemm") or name == "pf_common.h":
+            h.update(open(os.path.join(csrc, name), "rb").read())
+    return h.hexdigest()[:16]
+
+
 def measured_traffic(workload):
     """HBM bytes per launch (FETCH_SIZE + WRITE_SIZE, each scaled by the same counter's reading
     for a copy kernel of known size) per kernel name, parsed from the committed rocprofv3 --pmc
     summary `profiles/<workload>_pmc_traffic.md` (table rows `| `kernel` | ... | bytes |`, last
-    column = bytes per launch).  Kernels that are not in the file have no figure."""
+    column = bytes per launch).  Kernels that are not in the file have no figure, and none has one
+    after the kernels' sources have changed (the summary names the sources it was taken from)."""
     path = os.path.join(ROOT, "profiles", "%s_pmc_traffic.md" % workload)
     out = {}
     if not os.path.exists(path):
         return out
-    for line in open(path):
+    text = open(path).read()
+    if "GEMM sources `%s`" % gemm_source_digest() not in text:
+        return out      # the counters were read from other kernels than today's, whatever their names
+    for line in text.splitlines():
         cells = [c.strip() for c in line.strip().strip("|").split("|")]
         if len(cells) < 2 or not cells[0].startswith("`"):
             continue
@@ -276,10 +292,11 @@ def gemm_ceiling(kernels, mixed, reps=20):
     products ([3152 x 1024] . [1024 x 4096], the MLP's first layer, plain 16-bit store) and the same
     product with a four times longer reduction, plus the 128x128 tile on the step's dominant
     shape ([3152 x 4096] . [4096 x 1024]) and on that shape with 16 times the rows.  The first entry
-    is no product at all: the tile's matrix-instruction stream alone on register-resident fragments
-    of the same random data (`pf_mfma_rate`, no loads, LDS or barriers), on every CU for about as
-    long as the 8192^3 product runs: what the MFMA pipes sustain under the board's power limit, the
-    attainable ceiling the published peak (full boost clock) overstates."""
+    is no product at all: the tile's matrix-instruction stream (16x16x32) alone on register-resident
+    fragments of the same random data (`pf_mfma16_rate`, no loads, LDS or barriers), on every CU for
+    about as long as the 8192^3 product runs: what the MFMA pipes sustain under the board's power
+    limit, the attainable ceiling the published peak (full boost clock) overstates.  The second is
+    the same for 32x32x16 instructions, the shape of the attention kernels (`pf_mfma_rate`)."""
     import torch
 
     dt = {"fp16": torch.float16, "bf16": torch.bfloat16}.get(mixed)
@@ -289,22 +306,26 @@ def gemm_ceiling(kernels, mixed, reps=20):
     s = st.cuda_stream
     out = []
     ev0, ev1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-    frags = torch.cat([torch.randn(2048, device="cuda"), torch.randn(2048, device="cuda") * 0.03]).to(dt)
-    wgs, iters = 1024, 512          # 4 workgroups per CU in turn, 8192 MFMAs per wavefront: the 8192^3 product's count
-    sink = torch.empty(256 * wgs, device="cuda", dtype=torch.float32)
-    rate = kernels.mfma_rate(frags, iters, wgs, sink)
-    torch.cuda.synchronize()        # operands were made on the current stream, the launches go to `st`
-    rate(s)
-    ev0.record(st)
-    for _ in range(reps):
-        rate(s)
-    ev1.record(st)
-    ev1.synchronize()
-    us = 1e3 * ev0.elapsed_time(ev1) / reps
-    tf = wgs * 4 * iters * 16 * 2.0 * 32 * 32 * 16 / us / 1e6
-    out.append(dict(shape="MFMA instruction stream only (no operand traffic), %d workgroups x 4 wavefronts x %d MFMAs" % (wgs, iters * 16),
-                    kernel="mfma_rate_kernel<%d>" % {"fp16": 1, "bf16": 2}[mixed], avg_launch_us=round(us, 2),
-                    tflops=round(tf, 1), frac=round(tf / PEAK_TFLOPS[mixed], 4)))
+    # 4 rounds of workgroups per CU; as many FLOPs per wavefront, and in all, as the 8192^3 product
+    for name, probe, n_a, wgs, waves, iters, per, flop in (
+            ("mfma16_rate_kernel", kernels.mfma16_rate, 4096, 1024, 8, 256, 32, 2.0 * 16 * 16 * 32),
+            ("mfma_rate_kernel", kernels.mfma_rate, 2048, 1024, 4, 512, 16, 2.0 * 32 * 32 * 16)):
+        frags = torch.cat([torch.randn(n_a, device="cuda"), torch.randn(2048, device="cuda") * 0.03]).to(dt)
+        sink = torch.empty(64 * waves * wgs, device="cuda", dtype=torch.float32)
+        rate = probe(frags, iters, wgs, sink)
+        torch.cuda.synchronize()        # operands were made on the current stream, the launches go to `st`
+        for _ in range(4 * reps):       # until the clock has settled under the load
+            rate(s)
+        ev0.record(st)
+        for _ in range(reps):
+            rate(s)
+        ev1.record(st)
+        ev1.synchronize()
+        us = 1e3 * ev0.elapsed_time(ev1) / reps
+        tf = wgs * waves * iters * per * flop / us / 1e6
+        out.append(dict(shape="MFMA instruction stream only (no operand traffic), %d workgroups x %d wavefronts x %d MFMAs"
+                        % (wgs, waves, iters * per), kernel="%s<%d>" % (name, {"fp16": 1, "bf16": 2}[mixed]),
+                        avg_launch_us=round(us, 2), tflops=round(tf, 1), frac=round(tf / PEAK_TFLOPS[mixed], 4)))
     for label, M, N, K, variant in (("8192^3, 256x256 tile", 8192, 8192, 8192, 7),
                                     ("step shape 3152x4096x1024, 256x256 tile", 3152, 4096, 1024, 7),
                                     ("same with K x4 (3152x4096x4096), 256x256 tile", 3152, 4096, 4096, 7),

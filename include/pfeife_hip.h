@@ -189,6 +189,10 @@ int pf_gemm_grouped(const pf_gemm_desc* descs, int n, void* stream);
  * 4 B fragments), with no loads, LDS traffic or barriers in the loop: the rate the matrix pipes
  * sustain under the board's power limit, the ceiling of any GEMM K loop.  sink: 256 * workgroups floats (per-lane checksums). */
 int pf_mfma_rate(int dtype, const void* operands, int64_t iters, int workgroups, float* sink, void* stream);
+/* The same for the direct-to-LDS kernel's instruction stream: workgroups of 8 wavefronts, iters * 32
+ * v_mfma_f32_16x16x32 (2 * 16 * 16 * 32 FLOP each) per wavefront.  operands: 12 KiB, 8 A fragments of 64 lanes x 8
+ * values, then 4 B fragments; sink: 512 * workgroups floats. */
+int pf_mfma16_rate(int dtype, const void* operands, int64_t iters, int workgroups, float* sink, void* stream);
 /* Name of the kernel instantiation pf_gemm would launch for `desc`, spelled the
  * way a profiler prints it, e.g. "gemm16x_kernel<1, 256, 256, 32, 2, 4, 1, 5, false, false, 0>"
  * (dtype, tile M, tile N, stage depth, wavefront rows, columns, reduction split, stages, a_trans,

@@ -86,3 +86,18 @@ def test_the_product_package_never_imports_the_checker_or_scratch_files():
             if any(m == "oracle" or m.startswith("oracle.") for m in mods):
                 users.add(fn.name)
     assert users <= {"smoke", "build"}, users
+
+
+def test_traffic_figures_are_reported_for_the_measured_kernels_only(tmp_path, monkeypatch):
+    sys.path.insert(0, ROOT)
+    import bench
+
+    csrc, profiles = tmp_path / "pfeife_amd" / "csrc", tmp_path / "profiles"
+    csrc.mkdir(parents=True)
+    profiles.mkdir()
+    monkeypatch.setattr(bench, "ROOT", str(tmp_path))
+    (csrc / "pf_gemm.hip").write_text("one")
+    (profiles / "w_pmc_traffic.md").write_text("GEMM sources `%s`\n\n| `gemm<1>` | 3 | 8.5e+07 |\n" % bench.gemm_source_digest())
+    assert bench.measured_traffic("w") == {"gemm<1>": 8.5e7}
+    (csrc / "pf_gemm.hip").write_text("two")
+    assert bench.measured_traffic("w") == {}

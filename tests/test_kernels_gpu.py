@@ -1108,6 +1108,21 @@ def test_mfma_rate_probe_multiplies_what_it_is_given(hip, dtype):
     assert sink.cpu().double().reshape(4 * wgs, 64).sum(1).tolist() == [want] * (4 * wgs)
 
 
+@pytest.mark.parametrize("dtype", [F16, BF16])
+def test_mfma16_rate_probe_multiplies_what_it_is_given(hip, dtype):
+    """The same for v_mfma_f32_16x16x32 (lane l holds row or column l % 16 and reduction indices 8 * (l / 16) + 0..7),
+    iters * 32 of them on 8 + 4 fragments per wavefront, 8 wavefronts to a workgroup."""
+    g = torch.Generator().manual_seed(6)
+    frags = torch.randint(-2, 3, (12, 64, 8), generator=g).to(dtype)
+    iters, wgs = 7, 3
+    sink = torch.full((512 * wgs,), float("nan"), device="cuda")
+    hip.mfma16_rate(frags.cuda(), iters, wgs, sink)(torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    per_k = frags.double().reshape(12, 4, 16, 8).sum(2).reshape(12, 32)   # [fragment][k]: sum over its 16 rows / columns
+    want = iters * float((per_k[:8].sum(0) * per_k[8:].sum(0)).sum())
+    assert sink.cpu().double().reshape(8 * wgs, 64).sum(1).tolist() == [want] * (8 * wgs)
+
+
 @pytest.mark.parametrize("variant", [0, 7, 8, 9])
 def test_accumulating_products_stay_exact_next_to_other_streams(hip, variant):
     """Weight-gradient products (both operands reduction-strided, fp32 accumulate) on one stream while
