@@ -182,9 +182,11 @@ __device__ __forceinline__ uint4 buf_load16(__amdgpu_buffer_rsrc_t r, uint32_t b
 //   256x256 (32 deep, 5 stages): one 128x128 block per wavefront, the least operand traffic per FLOP
 //   256x128 (64 deep, 3 stages), 128x128 (64 deep, 3 stages): more workgroups for smaller outputs
 //   192x256 (32 deep, 5 stages): for outputs that 256-row blocks cover badly
-//   ids 1-4: four wavefronts (2 x 2); ids 7-10: the same tiles shared by EIGHT wavefronts (2 x 4 or 4 x 2,
-//   two per SIMD); id 11: 64x64 by four wavefronts, two workgroups to a CU, for small outputs; ids 5, 6: 128x128 and 256x128 with eight wavefronts as TWO 2 x 2 grids that
-//   split every tile's reduction depth between them ("k2")
+//   ids 1-4: four wavefronts (2 x 2); ids 7-10: the same tiles shared by EIGHT wavefronts (2 x 4 or 4 x 2, two per SIMD)
+//   ids 5, 6: 128x128 and 256x128 with eight wavefronts as TWO 2 x 2 grids that split every tile's reduction depth
+//   between them ("k2")
+//   id 11: 64x64 by four wavefronts, two workgroups to a CU, for small outputs
+//   (ids 1-6 run where a descriptor pins them; the automatic choice takes 7-11, which were faster wherever measured)
 enum { PF_XT_256x256 = 1, PF_XT_256x128 = 2, PF_XT_128x128 = 3, PF_XT_192x256 = 4, PF_XT_128x128k2 = 5,
        PF_XT_256x128k2 = 6, PF_XT_256x256w8 = 7, PF_XT_128x128w8 = 8, PF_XT_256x128w8 = 9, PF_XT_192x256w8 = 10, PF_XT_64x64 = 11, PF_XT_COUNT = 12 };
 // BM, BN, reduction depth per stage, stages, wavefront grid (rows x columns x reduction split) of each tile id

@@ -21,9 +21,9 @@ namespace {
 //                                           the transposing LDS read, which hands a lane
 //                                           four consecutive k of one row.
 // Each wavefront owns a (BM/WGM) x (BN/WGN) block of accumulators, computed with v_mfma_f32_16x16x32.  That
-// shape instead of 32x32x16 because of power: at the same peak rate the matrix pipes of the whole chip sustain
-// 1.99 against 1.72 PFLOP/s (fp16, random data; bf16 2.15 / 1.89), and a large product is bound by the board's
-// power.  The price is twice as many instructions of half the length, so the K loop deals out its LDS reads and
+// shape instead of 32x32x16 because of power: at the same peak rate (on zeros 2.4 PFLOP/s either way) the matrix pipes
+// of the whole chip sustain 1.87 against 1.63 PFLOP/s (fp16, random data; bf16 1.99 / 1.76; pf_mfma_rate.hip), and a
+// large product is bound by the board's power.  The price is twice as many instructions of half the length, so the K loop deals out its LDS reads and
 // loads one at a time between them.  The K loop has ONE barrier per tile, before the tile's last MFMA group: by
 // then the group's fragments are in registers, so the buffer can be refilled at once, and the first fragments
 // of the next tile are read under that last group's MFMAs (no LDS latency exposed at the barrier).
@@ -500,7 +500,7 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j) acc[i][j] += xch[(i * TN + j) * 64];
-    lds_barrier();  // all partial sums are read before the epilogue patches overwrite them
+    lds_barrier();  // all partial sums are read before the epilogue uses the LDS (column sums)
   }
   if constexpr (HAS_BIAS && !BIAS_EARLY) load_bias();
   static_assert(BT || TN == 2 || TN == 4 || TN == 8, "whole vectors per lane and row");

@@ -429,9 +429,12 @@ class BwdCtx:
         return ((launch.desc.M + 127) // 128) * ((launch.desc.N + 127) // 128)
 
     def _retile_held(self, launches):
-        """The held products on the tile that suits how many there are.  On 64x64 tiles a step of 64 rows costs
-        0.2 us while the device has room and grows with the number of tiles, on 128x128 tiles 0.37-0.54 us
-        (measured): the small tile is ahead up to about 112 tiles of 128x128 in all."""
+        """The held products on the tile that suits how many there are, whatever each would run on alone.  One launch
+        on 64x64 / 128x128 / 256x128 tiles, us, by tiles of 128x128 in all: over 788 rows 36: 6.6 / 9.7 / 13.9,
+        72: 8.9 / 11.0 / 15.4, 108: 11.0 / 12.2 / 16.6, 144: 14.5 / 13.0 / 17.2, 192: 13.8 / 12.3 / 16.5; over 3152 rows
+        36: 15.8 / 25.3 / 37.4, 72: 26.9 / 25.9 / 37.7, 108: 27.3 / 27.1 / 38.9, 144: 34.8 / 28.2 / 38.6.  64x64 is ahead
+        until it fills the device twice over (two workgroups to a CU: 128), over long reductions until about 100;
+        256x128 never is below 256."""
         retile = getattr(self.k, "gemm_retiled", None)
         if retile is None:
             return launches

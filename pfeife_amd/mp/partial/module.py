@@ -10,8 +10,12 @@ Same contract as pfeife/mp/partial/module.py:37-438:
 `step` splits the batch (pfeife/batch.py), runs `fn` once per micro-batch on a
 helper thread that parks inside the compiled model until the schedule has
 produced that micro-batch's outputs (module.py:161-166, 417-433), and executes
-the stage jobs on the calling thread in the schedule's order.  Exactly one
-thread is runnable at any time, as in the reference (module.py:87-89, 145-159).
+the stage jobs in the schedule's order.  Of the calling thread and the helper
+threads exactly one is runnable at any time, as in the reference
+(module.py:87-89, 145-159).  The first steps issue their jobs from the calling
+thread; once the jobs are captured, a native thread issues them from job lists
+and runs beside user code (mp/step_plan.py).  A step's work on gradients, 16-bit
+weight copies and stage jobs begins when every micro-batch has parked.
 
 What differs: the first `step` does not profile the model.  The probe call of
 `fn` (module.py:168-170) only records the captured graph and the micro-batch's

@@ -13,6 +13,10 @@ them in one thread adds their host times up, and the GPU waits for both.  Here a
     are summed into a gradient.
   * an event is waited for only if nothing the stream has waited for before implies it, and recorded only if some job
     waits for it.
+
+Against the same graphs issued job by job in the calling thread: two-layer ViT on four 32x32 images, two micro-batches
+1.14 -> 0.88 ms; decoder of four looped stages, eight micro-batches of 256 tokens 5.3 -> 3.85 ms; ViT-S on 62 images in
+bf16 6.76 -> 6.69 ms, on 16 in fp32 9.83 -> 9.77 ms.
 """
 
 
