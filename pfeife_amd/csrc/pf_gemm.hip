@@ -699,7 +699,8 @@ template <int DT>
 int dispatch16(const pf_gemm_desc& d, hipStream_t st) {
   const int v = resolve_variant(d);
   if (d.colsum_ws != nullptr) {   // only the GELU' class of the direct-to-LDS kernel sums its columns
-    if (!is_x_variant(v) || d.a_trans || d.b_trans || !x_supports(d, v) || epi_class(d, epi_vec_ok(d)) != EC_DACT16 ||
+    if (!is_x_variant(v) || d.a_trans || d.b_trans || !x_supports(d, v) ||
+        x_epi_class(d, epi_vec_ok(d), x_tile_bm(x_tile_of(v))) != EC_DACT16 ||
         !pf_aligned(d.colsum_ws, 16)) {
       pf_set_error("pf_gemm: colsum_ws needs a 16-bit product with the GELU' epilogue on the direct-to-LDS kernel");
       return PF_ERR_UNSUPPORTED;
@@ -824,7 +825,7 @@ bool groupable(const pf_gemm_desc& d, int& variant) {
   if (!is_x_variant(variant)) return false;
   if (!x_supports(d, variant)) return false;
   // (a product that stores rides in the accumulate launch: its old C reads as zeros)
-  const int ec = x_epi_class(d, epi_vec_ok(d));
+  const int ec = x_epi_class(d, epi_vec_ok(d), x_tile_bm(x_tile_of(variant)));
   return ec == EC_ACC32 || ec == EC_STORE32;
 }
 }  // namespace
@@ -887,7 +888,7 @@ extern "C" int pf_gemm_variant(const pf_gemm_desc* desc, char* out, int cap) {
                      "reduction-strided) K a multiple of %d", v, x_tile_bk(x_tile_of(v)), x_tile_bk(x_tile_of(v)));
         return PF_ERR_INVALID;
       }
-      const int ec = x_epi_class(d, epi_vec_ok(d));
+      const int ec = x_epi_class(d, epi_vec_ok(d), x_tile_bm(x_tile_of(v)));
       const bool ragged = !d.a_trans && d.K % x_tile_bk(x_tile_of(v)) != 0;
       snprintf(out, (size_t)cap, "gemm16x_%skernel<%d, %s, %s, %s, %d>", ragged ? "ragged_" : "", d.in_dtype, shapes[x_tile_of(v)], at, bt, ec);
       return PF_OK;

@@ -205,6 +205,10 @@ template <> struct XTile<PF_XT_64x64> { static constexpr int BM = 64, BN = 64, B
 // tiles with a kernel for row-major products whose reduction length is no multiple of the stage depth: the
 // eight-wavefront 128x128 and 256x128 tiles and 64x64
 constexpr bool x_tile_ragged(int bm, int bn, int nw) { return (nw == 8 && bn == 128) || (bm == 64 && bn == 64); }
+constexpr int x_tile_bm(int xt) {
+  return xt == PF_XT_64x64 ? 64 : (xt == PF_XT_128x128 || xt == PF_XT_128x128k2 || xt == PF_XT_128x128w8) ? 128
+         : (xt == PF_XT_192x256 || xt == PF_XT_192x256w8) ? 192 : 256;
+}
 inline int x_tile_bk(int xt) { return (xt == PF_XT_256x256 || xt == PF_XT_192x256 || xt == PF_XT_256x256w8 || xt == PF_XT_192x256w8) ? 32 : 64; }
 
 // Epilogue classes with straight-line code (which operands exist, and their dtypes, fixed at
@@ -242,9 +246,14 @@ inline int epi_class(const pf_gemm_desc& d, int vec_ok) {
   return c32 ? EC_ACC32 : EC_ACC16;
 }
 // ... and the class the direct-to-LDS kernel runs it as: reduction-strided products have straight-line code for a
-// plain fp32 result only (no bias, no rounding to the operands' type before it is stored or added)
-inline int x_epi_class(const pf_gemm_desc& d, int vec_ok) {
+// plain fp32 result only (no bias, no rounding to the operands' type before it is stored or added).  Their rows past M
+// (the last of the tiles' bm rows) are dropped by the range check of a buffer: an offset that wrapped at 2^32 would pass it.
+inline int x_epi_class(const pf_gemm_desc& d, int vec_ok, int bm) {
   const int ec = epi_class(d, vec_ok);
+  const int64_t rows = (d.M + bm - 1) / bm * bm, es = d.c_dtype == PF_F32 ? 4 : 2;
+  auto wraps = [&](const void* p, int64_t ld, int64_t size) { return p != nullptr && rows * ld * size >= (1ll << 32); };
+  if (wraps(d.C, d.ldc, es) || wraps(d.residual, d.ld_res, es) || wraps(d.aux_out, d.ld_aux_out, 2) || wraps(d.aux_in, d.ld_aux_in, 2))
+    return EC_GENERIC;
   const bool plain = (ec == EC_STORE32 || ec == EC_ACC32) && d.bias == nullptr && !d.round_mid;
   return d.a_trans && d.b_trans && !plain ? EC_GENERIC : ec;
 }

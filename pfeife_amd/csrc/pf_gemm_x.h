@@ -773,7 +773,7 @@ int launch16x(const pf_gemm_desc& d, hipStream_t st) {
     pf_set_error("pf_gemm: this variant needs K %% %d == 0 unless both operands are transposed", BK);
     return PF_ERR_INVALID;
   }
-  const int ec = x_epi_class(d, g.vec_epi);
+  const int ec = x_epi_class(d, g.vec_epi, BM);
 #define PF_X(AT, BT, EC) launch16x_t<DT, BM, BN, BK, WGM, WGN, KS, ST, AT, BT, EC, false>(d, g, st)
 #define PF_XR(EC) launch16x_t<DT, BM, BN, BK, WGM, WGN, KS, ST, false, false, EC, HAS_RAGGED>(d, g, st)
   if constexpr (HAS_RAGGED) {
@@ -865,6 +865,7 @@ int gemm_x_group_launch(const pf_gemm_desc* d, int n, hipStream_t st) {
 template <int DT, int XT>
 int gemm_x_launch(const pf_gemm_desc& d, hipStream_t st) {
   using T = XTile<XT>;
+  static_assert(x_tile_bm(XT) == T::BM, "x_tile_bm");
   return launch16x<DT, T::BM, T::BN, T::BK, T::WGM, T::WGN, T::KS, T::ST>(d, st);
 }
 

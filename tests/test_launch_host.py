@@ -131,3 +131,28 @@ for dt in (hip.PF_F16, hip.PF_BF16):
                 group = (hip.GemmDesc * 2)(d, d)
                 assert (lib.pf_gemm_grouped(group, 2, None), stub.stub_launches()) == (0, 2)
 """)
+
+
+def test_rows_so_wide_that_a_tiles_last_rows_wrap_a_32_bit_offset_take_the_generic_epilogue(stub):
+    """The straight-line epilogues drop rows past M by the range check of a buffer: for every tile, class and operand
+    the byte offset of any row of the last tile stays below 2^32, and nothing else changes its class."""
+    child(stub, r"""
+name = ctypes.create_string_buffer(128)
+def straight(M, fits, **kw):
+    d = gemm(M, 64, 64, dtype=hip.PF_F16, **kw)
+    assert lib.pf_gemm_variant(ctypes.byref(d), name, 128) == 0 and run(d) == (0, 1)
+    d.nonfinite_flag = 1 << 24
+    plain = d.c_dtype == hip.PF_F32 and not d.residual and fits
+    assert (run(d) == (0, 1)) == plain, lib.pf_last_error()      # what took the flag takes it on either epilogue
+    return not name.value.endswith(b", -1>")
+for variant, bm in ((7, 256), (8, 128), (9, 256), (10, 192), (15, 64), (1, 256), (3, 128), (4, 192), (5, 128)):
+    for M in (1, 8, 63, 128, 300):
+        rows = (M + bm - 1) // bm * bm
+        for ld in (64, 1 << 16, 1 << 20, (1 << 21) - 8, 1 << 21, 1 << 22, 1 << 23, 1 << 24, 1 << 26):
+            for kw, size in ((dict(ldc=ld), 4), (dict(ldc=ld, c_dtype=hip.PF_F16), 2), (dict(ldc=ld, beta=1), 4),
+                             (dict(residual=1 << 23, ld_res=ld), 4),
+                             (dict(c_dtype=hip.PF_F16, act=1, aux_out=1 << 23, ld_aux_out=ld), 2),
+                             (dict(c_dtype=hip.PF_F16, dact=1, aux_in=1 << 23, ld_aux_in=ld), 2)):
+                fits = M * ld * (4 if "ldc" in kw or "ld_res" in kw else 2) < (1 << 31) - 64
+                assert straight(M, fits, variant=variant, **kw) == (fits and rows * ld * size < 1 << 32), (variant, M, ld, kw)
+""")
