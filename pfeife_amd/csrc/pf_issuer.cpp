@@ -7,8 +7,8 @@
 #include <atomic>
 #include <condition_variable>
 #include <deque>
+#include <exception>
 #include <mutex>
-#include <new>
 #include <string>
 #include <thread>
 
@@ -112,8 +112,13 @@ struct Issuer {
 
 extern "C" int pf_issuer_create(int device, void** out) {
   PF_REQUIRE(out != nullptr, "pf_issuer_create: null result pointer");
-  *out = new (std::nothrow) Issuer(device);
-  PF_REQUIRE(*out != nullptr, "pf_issuer_create: out of memory");
+  try {
+    *out = new Issuer(device);
+  } catch (const std::exception& e) {   // no memory, or no thread to be had
+    *out = nullptr;
+    pf_set_error("pf_issuer_create: %s", e.what());
+    return PF_ERR_HIP;
+  }
   return PF_OK;
 }
 
@@ -121,7 +126,12 @@ extern "C" int pf_issuer_push(void* issuer, const pf_job* jobs, int n, int64_t* 
   PF_REQUIRE(issuer && ticket && n >= 0 && (jobs || n == 0), "pf_issuer_push: bad arguments");
   for (int i = 0; i < n; ++i)
     PF_REQUIRE(jobs[i].stream && jobs[i].n_waits >= 0 && (jobs[i].waits || jobs[i].n_waits == 0), "pf_issuer_push: bad job %d", i);
-  *ticket = ((Issuer*)issuer)->push(jobs, n);
+  try {
+    *ticket = ((Issuer*)issuer)->push(jobs, n);
+  } catch (const std::exception& e) {
+    pf_set_error("pf_issuer_push: %s", e.what());
+    return PF_ERR_HIP;
+  }
   return PF_OK;
 }
 

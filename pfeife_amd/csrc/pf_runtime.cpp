@@ -2,6 +2,7 @@
 #include <stdarg.h>
 #include <string.h>
 
+#include <exception>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -28,11 +29,15 @@ int pf_allow_lds(const void* kernel, size_t bytes, const char* who) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e == hipSuccess) {
-    std::lock_guard<std::mutex> lock(mu);
-    size_t& have = allowed[{kernel, dev}];
-    if (have >= bytes) return PF_OK;
-    e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-    if (e == hipSuccess) have = bytes;
+    try {
+      std::lock_guard<std::mutex> lock(mu);
+      size_t& have = allowed[{kernel, dev}];
+      if (have >= bytes) return PF_OK;
+      e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+      if (e == hipSuccess) have = bytes;
+    } catch (const std::exception&) {
+      e = hipErrorOutOfMemory;
+    }
   }
   if (e == hipSuccess) return PF_OK;
   pf_set_error("%s: cannot raise dynamic LDS to %zu bytes: %s", who, bytes, hipGetErrorString(e));

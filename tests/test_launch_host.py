@@ -156,3 +156,20 @@ for variant, bm in ((7, 256), (8, 128), (9, 256), (10, 192), (15, 64), (1, 256),
                 fits = M * ld * (4 if "ldc" in kw or "ld_res" in kw else 2) < (1 << 31) - 64
                 assert straight(M, fits, variant=variant, **kw) == (fits and rows * ld * size < 1 << 32), (variant, M, ld, kw)
 """)
+
+
+def test_an_issuer_without_a_thread_is_an_error(stub):
+    """No room for another thread's stack: pf_issuer_create reports it (an exception that left a C entry point would end
+    the process) and works once there is room."""
+    child(stub, r"""
+import resource
+out = ctypes.c_void_p()
+size = 1024 * int(next(l for l in open("/proc/self/status") if l.startswith("VmSize")).split()[1])
+before = resource.getrlimit(resource.RLIMIT_AS)
+resource.setrlimit(resource.RLIMIT_AS, (size + (2 << 20), before[1]))
+rc, text = lib.pf_issuer_create(0, ctypes.byref(out)), lib.pf_last_error()
+resource.setrlimit(resource.RLIMIT_AS, before)
+assert rc != 0 and b"pf_issuer_create" in text and not out.value, (rc, text)
+assert lib.pf_issuer_create(0, ctypes.byref(out)) == 0 and out.value
+assert lib.pf_issuer_destroy(out) == 0
+""")
