@@ -710,7 +710,8 @@ class StageWorker:
                     st["step"] = torch.tensor(0.0, dtype=torch.float32)
                     st["exp_avg"] = torch.zeros_like(p, memory_format=torch.preserve_format)
                     st["exp_avg_sq"] = torch.zeros_like(p, memory_format=torch.preserve_format)
-            sig = tuple((p.data_ptr(), p.grad.data_ptr(), opt.state[p]["exp_avg"].data_ptr()) for p in params)
+            sig = tuple((p.numel(), p.data_ptr(), p.grad.data_ptr(), opt.state[p]["exp_avg"].data_ptr(),
+                         opt.state[p]["exp_avg_sq"].data_ptr()) for p in params)   # (all that the table holds)
             ent = cache.get(gi)
             if ent is None or ent[0] != sig:
                 table = self.kernels.adam_table([p.data for p in params], [p.grad for p in params],

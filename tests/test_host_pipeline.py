@@ -643,3 +643,46 @@ def test_a_graph_is_destroyed_after_every_lane_has_run_what_was_issued(drop):
         w._drop_dw_jobs()
     assert "destroy" in log
     assert set(log[:log.index("destroy")]) == {w.stream_obj, *w.lanes.values()}
+
+
+@pytest.mark.parametrize("replaced", ["data", "grad", "exp_avg", "exp_avg_sq", "smaller"])
+def test_the_adam_table_follows_every_tensor_it_points_to(replaced):
+    """A parameter, gradient or moment that user code replaces between steps: the next fused step runs on a table with
+    its address and size."""
+    from pfeife_amd.mp.worker import StageWorker
+
+    tables = []
+
+    class Kernels:
+        def adam_table(self, params, grads, exp_avgs, exp_avg_sqs):
+            tables.append([(t.numel(), t.data_ptr()) for ts in (params, grads, exp_avgs, exp_avg_sqs) for t in ts])
+            return object(), len(params), max(p.numel() for p in params)
+
+        def adam_step(self, *args):
+            pass
+
+    w = StageWorker.__new__(StageWorker)
+    w.kernels, w.stream_obj = Kernels(), None
+    params = [torch.nn.Parameter(torch.randn(8)) for _ in range(2)]
+    for p in params:
+        p.grad = torch.randn(8)
+    opt = torch.optim.Adam(params, lr=0.1)
+    w._fused_adam_step(opt)
+    w._fused_adam_step(opt)
+    assert len(tables) == 1
+    p, st = params[1], opt.state[params[1]]
+    if replaced == "data":
+        p.data = p.data.clone()
+    elif replaced == "grad":
+        p.grad = p.grad.clone()
+    elif replaced == "smaller":
+        keep = p.data, p.grad, st["exp_avg"], st["exp_avg_sq"]
+        p.grad = None
+        p.data, p.grad, st["exp_avg"], st["exp_avg_sq"] = (t[:4] for t in keep)
+    else:
+        old, st[replaced] = st[replaced], st[replaced].clone()
+    w._fused_adam_step(opt)
+    assert len(tables) == 2
+    assert tables[1] == [(t.numel(), t.data_ptr()) for ts in (params, [q.grad for q in params],
+                                                            [opt.state[q]["exp_avg"] for q in params],
+                                                            [opt.state[q]["exp_avg_sq"] for q in params]) for t in ts]
