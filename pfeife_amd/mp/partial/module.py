@@ -104,10 +104,11 @@ class PartialRunner:
             return self._step(*args, **kwargs)
         outer = torch.cuda.current_stream(so.device)
         so.wait_stream(outer)
-        with torch.cuda.stream(so):
-            out = self._step(*args, **kwargs)
-        outer.wait_stream(so)
-        return out
+        try:
+            with torch.cuda.stream(so):
+                return self._step(*args, **kwargs)
+        finally:
+            outer.wait_stream(so)    # (after a failed step too: its caller may touch weights and gradients)
 
     def _step(self, *args, **kwargs):
         if self.exec_fn is None:
@@ -128,6 +129,7 @@ class PartialRunner:
             return self._run_step(args, kwargs)
         except BaseException:
             self._abort_parked()
+            self.worker.settle_failed_step()
             raise
 
     def _abort_parked(self):
@@ -146,7 +148,6 @@ class PartialRunner:
 
         # every micro-batch thread runs user code up to the compiled model, hands its
         # inputs to the worker and parks there
-        worker.settle_failed_step()
         for bid in range(option.batch_cnt):
             self._train_queues[bid].put((args[bid], kwargs[bid]))
             tok = self._return_queues[bid].get()

@@ -439,12 +439,12 @@ class StageWorker:
             buf.copy_(value, non_blocking=True)  # host -> device (or a layout change): PyTorch plumbing
 
     def settle_failed_step(self):
-        """A planned step that failed half-way may have left jobs to be issued and lanes running: the new step's user
-        code and inputs come after them."""
+        """A step that failed half-way may have left jobs to be issued and lanes running: what its caller does next, and
+        the next step's user code and inputs, come after them."""
         if self.step_plan is not None and self.step_plan.started:
-            self.issuer.wait()
-            self.end_jobs()
             self.step_plan.started = False
+            self.issuer.wait()
+        self.end_jobs()
 
     def begin_planned_step(self):
         """Starts a step whose jobs a native thread issues from job lists (`StepPlan`): every step after the one that
@@ -468,7 +468,6 @@ class StageWorker:
 
     def begin_step(self):
         s = self.stream()
-        self.end_jobs()   # a step that failed half-way may have left lanes running
         self.params.rebind_grads()
         if self.use_graphs and not self.graphs_ready and self.steps_done >= 1 and len(self.mbs) == self.option.batch_cnt:
             self.capture_graphs()

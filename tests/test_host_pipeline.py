@@ -686,3 +686,46 @@ def test_the_adam_table_follows_every_tensor_it_points_to(replaced):
     assert tables[1] == [(t.numel(), t.data_ptr()) for ts in (params, [q.grad for q in params],
                                                             [opt.state[q]["exp_avg"] for q in params],
                                                             [opt.state[q]["exp_avg_sq"] for q in params]) for t in ts]
+
+
+@pytest.mark.parametrize("planned", [False, True])
+def test_a_failed_step_is_settled_before_its_error_reaches_the_caller(monkeypatch, planned):
+    """exec_fn raises after the model has returned: when step() raises, everything of the step has been issued and the
+    main stream comes after every lane, so that the caller may touch weights and gradients."""
+    from pfeife_amd.mp import partial_compiler
+    from pfeife_amd.mp import worker as worker_module
+
+    torch.manual_seed(0)
+    model = VisionTransformer(CFG)
+    runner = make_runner(PipeOption(device_cnt=2, batch_cnt=2, batch_size=2, split_points=["blocks.2"],
+                                    optimizer=dict(type="sgd", lr=0.0)))
+    cmodel = torch.compile(model, backend=partial_compiler)
+    crit, fail, log = nn.CrossEntropyLoss(), [False], []
+
+    def fn(x, y):
+        loss = crit(cmodel(x).float(), y)
+        if fail[0]:
+            log.append("raise")
+            raise ValueError("user code")
+        loss.backward()
+        return loss.detach()
+
+    runner.set_exec_fn(fn)
+    x, y = torch.randn(4, 3, 32, 32), torch.arange(4)
+    w = runner.worker
+    good = [[float(l) for l in runner.step(x, y)] for _ in range(2)][1]
+    if planned:
+        monkeypatch.setattr(worker_module, "StepPlan", _HostPlan)
+        w.kernels.issuer = lambda: SimpleNamespace(wait=lambda: log.append("issued"))
+        w.capture_graphs = lambda: None
+        w.graphs_ready = True
+    end_jobs = w.end_jobs
+    w.end_jobs = lambda: (log.append("lanes"), end_jobs())
+    fail[0] = True
+    with pytest.raises(ValueError):
+        runner.step(x, y)
+    assert log[log.index("raise"):] == (["raise", "issued", "lanes"] if planned else ["raise", "lanes"])
+    assert w.step_plan is None or not w.step_plan.started
+    fail[0] = False
+    assert [float(l) for l in runner.step(x, y)] == good
+    w.step_plan = None
