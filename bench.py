@@ -147,10 +147,9 @@ def measured_traffic(workload):
 
 
 def _step_launches(runner):
-    for slot in runner.worker.mbs.values():
-        for prog in slot.stage_programs.values():
-            for launch in list(prog.fwd) + list(prog.bwd):
-                yield launch
+    for prog in runner.worker.step_programs():
+        for launch in list(prog.fwd) + list(prog.bwd):
+            yield launch
     for launches, _ in runner.worker.dw_jobs.values():   # the once-per-step weight-gradient job of each stage
         for launch in launches:
             yield launch

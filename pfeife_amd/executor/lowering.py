@@ -27,6 +27,7 @@ import os
 import torch
 import torch.nn.functional as F
 
+from .merge import CallRecorder, Merger
 from .values import Val, as_matrix, collapse_for_copy, dense_like, is_dense
 
 ACT_NONE, ACT_GELU, ACT_GELU_TANH, ACT_SILU, ACT_RELU = 0, 1, 2, 3, 4
@@ -316,25 +317,34 @@ class BufferPool:
         self.bytes += t.numel() * t.element_size()
         return t
 
-    def stacked(self, key, shape, dtype, mb, count):
-        """Buffer `key` of micro-batch `mb`, one of `count` equal buffers laid end to end in one
-        allocation: what the micro-batches of a step write at the same place of the same stage
-        (an activation, the gradient of a layer's output) then forms ONE matrix with `count` times
-        the rows, which the weight-gradient product of the whole step reads in a single launch."""
+    def stacked(self, key, shape, dtype, place, strides=None, aligned=False):
+        """Buffer `key` of the micro-batch at `place` (`MicroBatchLayout.place`): the buffers of all of them lie
+        end to end in one allocation.  What the micro-batches of a step write at the same place of the same stage
+        (an activation, the gradient of a layer's output) then forms ONE matrix over all their rows, which one
+        launch works on.  Micro-batches of different sizes lie end to end where a buffer's extent goes with the
+        number of samples, and have buffers of their own otherwise.  aligned: also where a 16-byte boundary would
+        be lost."""
         shape = tuple(int(x) for x in shape)
-        if mb is None or not 0 <= mb < count:
-            return torch.empty(shape, dtype=dtype, device=self.device)
-        key = (key, shape, dtype, count)
+        numel = 1
+        for x in shape:
+            numel *= x
+        offset, total = place.span(numel)
+        es = torch.empty((), dtype=dtype).element_size()
+        if offset is None or (aligned and offset * es % 16):
+            key, offset, total = (key, "own", place.index), 0, numel
+        key = (key, numel if place.uniform else shape[1:], dtype, total)
         slab = self._stacked.get(key)
         if slab is None:
-            slab = self._stacked[key] = torch.empty((count,) + shape, dtype=dtype, device=self.device)
+            slab = self._stacked[key] = torch.empty((total,), dtype=dtype, device=self.device)
             self.bytes += slab.numel() * slab.element_size()
-        return slab[mb]
+        flat = slab[offset:offset + numel]
+        return flat.view(shape) if strides is None else torch.as_strided(flat, shape, strides, offset)
 
     def prune_stacked(self, live_tags):
         """Forget the stacked allocations made under tags no micro-batch slot uses any more (their
         memory goes when the programs that hold slices of them do)."""
-        self._stacked = {k: v for k, v in self._stacked.items() if k[0][0] in live_tags}
+        tag = lambda k: k[0][0][0] if k[0][1:2] == ("own",) else k[0][0]
+        self._stacked = {k: v for k, v in self._stacked.items() if tag(k) in live_tags}
 
 
 class StageProgram:
@@ -361,6 +371,9 @@ class StageProgram:
         # output gradients they read, and per product (dy, x, accumulator, gemm arguments)
         self.dw_sigs = set()
         self.dw_deferred = []
+        # the tail of the backward list finishes these column reductions
+        self.reduces = []
+        self.n_tail = 0
 
     def run_forward(self, stream):
         if self.fwd_graph is not None:
@@ -391,6 +404,7 @@ class BwdCtx:
         self.program = program
         self.out = program.bwd
         self._seq = 0
+        self._private = 0
         self._pending = {}
         self.reduces = []   # deferred column reductions, finished by one batched launch at the end
         self._dw = []       # held-back weight-gradient products: (launch, accumulator, tiles)
@@ -417,8 +431,8 @@ class BwdCtx:
         if (n, dtype) not in sigs:
             return None
         i = self._kept[(n, dtype)] = self._kept.get((n, dtype), 0) + 1
-        return self.L.pool.stacked((self.L.stack_tag, "g", self.program.stage, i, n), shape, dtype, self.program.mb,
-                                   self.L.stack_mbs)
+        return self.L.pool.stacked((self.L.layout.tag, "g", self.program.stage, i, n), shape, dtype,
+                                   self.L.layout.place(self.program.mb))
 
     # -- weight-gradient products that share a launch ---------------------------------------------
     FULL_GRID = 256     # workgroups that fill the device (one tile per CU)
@@ -604,18 +618,29 @@ class BwdCtx:
             kept = self._kept_for_dw(like.shape, like.dtype)
             if kept is not None:
                 return kept
+        shared = self.L.shares_jobs(self.program.mb)
         if private:
             # gradients that outlive this job (they cross a stage boundary) get their own storage
+            if shared and is_dense(like):
+                self._private += 1
+                return self.L.pool.stacked((self.L.layout.tag, "b", self.program.stage, self._private), like.shape,
+                                           like.dtype, self.L.layout.place(self.program.mb), like.stride(), aligned=True)
             return self.L.pool.fresh_like(like)
+        return self._job_buffer(like.shape, like.dtype, like.stride() if is_dense(like) else None)
+
+    def _job_buffer(self, shape, dtype, strides=None):
         self._seq += 1
+        if self.L.shares_jobs(self.program.mb):
+            return self.L.job_buffer(("t", self._seq), self.program.mb, shape, dtype, strides)
+        like = (torch.empty(tuple(shape), dtype=dtype, device="meta") if strides is None else
+                torch.empty_strided(tuple(shape), tuple(strides), dtype=dtype, device="meta"))
         return self.L.pool.bwd_like(self._seq, like)
 
     def temp(self, shape, dtype):
         kept = self._kept_for_dw(shape, dtype)
         if kept is not None:
             return kept
-        self._seq += 1
-        return self.L.pool.bwd_like(self._seq, torch.empty(tuple(shape), dtype=dtype, device="meta"))
+        return self._job_buffer(shape, dtype)
 
     # -- reading -------------------------------------------------------------
     def grad_of(self, val):
@@ -772,7 +797,7 @@ class BwdCtx:
 # ---------------------------------------------------------------------------
 class Lowerer:
     def __init__(self, kernels, device, compute_dtype=None, params=None, pool=None):
-        self.kernels = kernels
+        self.kernels = CallRecorder(kernels)
         self.device = torch.device(device)
         self.cd = compute_dtype or torch.float32
         self.mixed = self.cd != torch.float32
@@ -780,25 +805,51 @@ class Lowerer:
         self.pool = pool or BufferPool(self.device)
         self._ws = None
         # defer_dw: weight-gradient products of linear layers are left out of the backward jobs and run
-        # once per step over all `stack_mbs` micro-batches (the worker builds that job); forward buffers
-        # and the gradients those products read are then laid end to end across micro-batches
+        # once per step over all micro-batches (the worker builds that job)
         self.defer_dw = False
-        self.stack_mbs = 1
-        self.stack_tag = None   # micro-batch slots lowered under the same tag (input shapes) share stacked allocations
+        # layout (`MicroBatchLayout`): the micro-batches' forward buffers and the gradients that those products or
+        # jobs over several micro-batches read are laid end to end; None: buffers of their own
+        self.layout = None
         # loss scaling as the once-per-step weight-gradient products see it: (device scale or None,
         # device overflow flag or None, constant factor); set by the worker
         self.dw_unscale = (None, None, 1.0)
 
     # -- buffers -------------------------------------------------------------
-    def alloc(self, shape, dtype):
-        if self.defer_dw:
+    def alloc(self, shape, dtype, strides=None):
+        if self.layout is not None:
             self.cur.alloc_seq += 1
-            t = self.pool.stacked((self.stack_tag, "f", self.cur.stage, self.cur.alloc_seq), shape, dtype, self.cur.mb,
-                                  self.stack_mbs)
-        else:
+            t = self.pool.stacked((self.layout.tag, "f", self.cur.stage, self.cur.alloc_seq), shape, dtype,
+                                  self.layout.place(self.cur.mb), strides)
+        elif strides is None:
             t = torch.empty(tuple(int(s) for s in shape), dtype=dtype, device=self.device)
+        else:
+            t = torch.empty_strided(tuple(shape), tuple(strides), dtype=dtype, device=self.device)
         self.cur.fwd_bytes += t.numel() * t.element_size()
         return t
+
+    def alloc_like(self, like, dtype=None):
+        """A buffer laid out as the dense tensor `like`."""
+        return self.alloc(like.shape, dtype or like.dtype, None if like.is_contiguous() else like.stride())
+
+    def shares_jobs(self, mb):
+        """Does a job of this micro-batch work on other micro-batches too?  What it leaves for a later launch of the
+        job must then lie in a buffer of the micro-batch's own."""
+        if self.layout is None or mb is None:
+            return False
+        first, end = self.layout.group(mb)
+        return end - first > 1
+
+    def job_buffer(self, key, mb, shape, dtype, strides=None):
+        """Such a buffer; jobs of one lane never overlap in time and share them."""
+        return self.pool.stacked((self.layout.tag, "j", self.pool.lane, key, tuple(shape[1:])), shape, dtype,
+                                 self.layout.place(mb, in_group=True), strides, aligned=True)
+
+    def scratch(self, slot, mb, shape, dtype):
+        """Scratch that several launches of a job use (forward jobs: their groups are not known yet)."""
+        if self.layout is None or mb is None:
+            return self.pool.scratch(slot, shape, dtype)
+        return self.pool.stacked((self.layout.tag, "s", self.pool.lane, slot, tuple(shape[1:])), shape, dtype,
+                                 self.layout.place(mb))
 
     def workspace(self, rows, cols):
         """fp32 scratch for the two-stage column reductions (shared by every launch of that size)."""
@@ -868,7 +919,9 @@ class Lowerer:
             prog.bwd_ranges.append((name, first, len(prog.bwd)))
         first = len(prog.bwd)
         B.close_dw()
-        prog.bwd.extend(B.finish_reduces())
+        tail = B.finish_reduces()
+        prog.bwd.extend(tail)
+        prog.reduces, prog.n_tail = B.reduces, len(tail)
         if prog.bwd_ranges and len(prog.bwd) > first:   # held-back tail: charged to the job's last node
             prog.bwd_ranges.append((prog.bwd_ranges[-1][0], first, len(prog.bwd)))
         B.compact(prog.bwd_ranges)
@@ -885,6 +938,27 @@ class Lowerer:
                                    "the unwritten region would hold garbage" % prog.stage)
         prog.backward_fns = []  # closures keep build-time state alive; not needed any more
         return prog
+
+    def merge_programs(self, progs):
+        """One program that does the work of the programs of consecutive micro-batches of a stage, or None if their
+        launch lists do not correspond."""
+        bufs = []
+
+        def workspace(n):
+            bufs.append(self.pool.scratch(("merged", len(bufs)), (n,), torch.float32))
+            return bufs[-1]
+
+        m = Merger(self.kernels, workspace)
+        fwd = m.lists([p.fwd for p in progs])
+        bwd = m.lists([p.bwd[:len(p.bwd) - p.n_tail] for p in progs])
+        reduces = m.reduces([p.reduces for p in progs])
+        if fwd is None or bwd is None or reduces is None:
+            return None
+        job = StageProgram(progs[0].stage, progs[0].mb)
+        B = BwdCtx(self, job)
+        B.reduces = reduces
+        job.fwd, job.bwd = fwd, bwd + B.finish_reduces()
+        return job
 
     def lower_deferred_dw(self, progs):
         """The once-per-step weight-gradient job of one stage.  `progs`: the stage's programs, one
@@ -1331,7 +1405,7 @@ def lower_sdpa(L, node):
     kern = L.kernels
     if L.mixed and hv == hd and hd % 8 == 0 and hd <= getattr(kern, "MAX_FUSED_HEAD_DIM", 0):
         return _lower_sdpa_fused(L, (q, k, v), (qt, kt, vt), (Bn, H, Tq, Tk, hd), scale, causal, req)
-    S = L.pool.scratch("attn_s", (Bn, H, Tq, Tkp), torch.float32)
+    S = L.scratch("attn_s", L.cur.mb, (Bn, H, Tq, Tkp), torch.float32)
     P = L.alloc((Bn, H, Tq, Tkp), cd)
     O = L.alloc((Bn, Tq, H, hv), cd)           # token-major, so that transpose(1,2).reshape is a view
     Ov = O.permute(0, 2, 1, 3)
@@ -1351,8 +1425,8 @@ def lower_sdpa(L, node):
             t = B.new_like(Ov)
             B.copy(g, t)
             g = t
-        dP = L.pool.scratch("attn_dp", (Bn, H, Tq, Tkp), torch.float32)
-        dS = L.pool.scratch("attn_ds", (Bn, H, Tq, Tkp), cd)
+        dP = L.scratch("attn_dp", B.program.mb, (Bn, H, Tq, Tkp), torch.float32)
+        dS = L.scratch("attn_ds", B.program.mb, (Bn, H, Tq, Tkp), cd)
         kb = B.k
         B.emit(kb.gemm(g, vt, dP, M=Tq, N=Tk, K=hv, lda=g.stride(2), ldb=vt.stride(2), ldc=Tkp, batch=(Bn, H),
                        sa=bs(g), sb=bs(vt), sc=bs(dP)))
@@ -1410,7 +1484,7 @@ def _lower_sdpa_fused(L, vals, tensors, dims, scale, causal, req):
             t = B.new_like(Ov)
             B.copy(g, t)
             g = t
-        delta = L.pool.scratch("attn_delta", (Bn, H, Tq), torch.float32)
+        delta = L.scratch("attn_delta", B.program.mb, (Bn, H, Tq), torch.float32)
         plan = []
         outs = []
         for val, like in ((q, qt), (k, kt), (v, vt)):
@@ -1537,8 +1611,7 @@ def _lower_conv_same(L, x, w, b, k):
         w_cd = L.params.shadow(w.buf, cd).reshape(O, C)
     else:
         Kc = 9 * C
-        padded = torch.zeros((Bn, H + 2, W + 2, C), dtype=cd, device=L.device)  # border stays zero for good
-        L.cur.fwd_bytes += padded.numel() * padded.element_size()
+        padded = L.alloc((Bn, H + 2, W + 2, C), cd).zero_()  # border stays zero for good
         L.copy(xn, padded[:, 1:H + 1, 1:W + 1, :])
         cols = L.alloc((M, Kc), cd)
         ps = padded.stride()
@@ -1884,8 +1957,7 @@ def lower_add(L, node):
     if a.shape == b.shape:
         if not (is_dense(a.buf) and is_dense(b.buf) and a.buf.stride() == b.buf.stride()):
             raise Unsupported("add of differently laid out tensors")
-        out = torch.empty_like(a.buf, dtype=out_dtype)
-        L.cur.fwd_bytes += out.numel() * out.element_size()
+        out = L.alloc_like(a.buf, out_dtype)
         L.emit(L.kernels.axpby(a.buf, 1.0, b.buf, 1.0, out, out.numel()))
         outv = Val(out, req_grad=req)
 
@@ -1963,8 +2035,7 @@ def lower_unary_act(L, node):
     x = L.arg(node.args[0])
     if not is_dense(x.buf):
         raise Unsupported("activation on a non-dense tensor")
-    y = torch.empty_like(x.buf)   # same (possibly permuted) dense layout: the kernel walks flat memory
-    L.cur.fwd_bytes += y.numel() * y.element_size()
+    y = L.alloc_like(x.buf)   # same (possibly permuted) dense layout: the kernel walks flat memory
     L.emit(L.kernels.act_fwd(x.buf, y, act, y.numel()))
     outv = Val(y, req_grad=x.req_grad)
 
@@ -2018,8 +2089,7 @@ def lower_pad(L, node):
         dim = x.buf.dim() - 1 - i
         shape[dim] += pad[2 * i] + pad[2 * i + 1]
         region.append((dim, pad[2 * i], x.shape[dim]))
-    out = torch.full(shape, 0 if value is None else value, dtype=x.dtype, device=L.device)
-    L.cur.fwd_bytes += out.numel() * out.element_size()
+    out = L.alloc(shape, x.dtype).fill_(0 if value is None else value)
     inner = out
     for dim, start, n in region:
         inner = inner.narrow(dim, start, n)
@@ -2082,7 +2152,7 @@ def lower_float(L, node):
 def _lower_cast(L, x, dtype):
     if x.dtype == dtype:
         return Val(x.buf, req_grad=x.req_grad, kind="view", base=x, view_fn=lambda t: t)
-    out = torch.empty_like(x.buf, dtype=dtype) if is_dense(x.buf) else L.alloc(x.shape, dtype)
+    out = L.alloc_like(x.buf, dtype) if is_dense(x.buf) else L.alloc(x.shape, dtype)
     L.copy(x.buf, out)
     outv = Val(out, req_grad=x.req_grad)
 
@@ -2153,8 +2223,7 @@ def lower_mul(L, node):
         raise Unsupported("mul operands %s" % (node.format_node(),))
     if not is_dense(v.buf):
         raise Unsupported("scaling a non-dense tensor")
-    out = torch.empty_like(v.buf)
-    L.cur.fwd_bytes += out.numel() * out.element_size()
+    out = L.alloc_like(v.buf)
     L.emit(L.kernels.axpby(v.buf, float(s), None, 0.0, out, out.numel()))
     outv = Val(out, req_grad=v.req_grad)
 

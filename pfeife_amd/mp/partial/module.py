@@ -56,6 +56,13 @@ def _same_shapes(args, kwargs):
     return len(sigs) <= 1
 
 
+def _samples(args, kwargs):
+    """How many samples a micro-batch has: the rows of its first tensor."""
+    from torch.utils._pytree import tree_flatten
+
+    return next((int(t.shape[0]) for t in tree_flatten((args, kwargs))[0] if torch.is_tensor(t) and t.dim() > 0), 1)
+
+
 class _ExecError:
     def __init__(self, exc):
         self.exc = exc
@@ -116,6 +123,7 @@ class PartialRunner:
         option = self.option
         args, kwargs = split_args_kwargs(args, kwargs, option.batch_cnt)
         self.worker.uniform_mbs = _same_shapes(args, kwargs)
+        self.worker.mb_sizes = [_samples(a, k) for a, k in zip(args, kwargs)]
 
         if not self._compiled:
             self._probe_forward(args[0], kwargs[0])

@@ -49,16 +49,20 @@ class StepPlan:
         begin = self._node(main, w.begin_graph, [])     # (after the inputs' copies, on the same stream)
 
         def job(stage, mb, is_fwd):
-            prog = w.mbs[mb].stage_programs[stage]
+            j = w.jobs[stage, mb]
+            if mb != (j.first if is_fwd else j.last):
+                return           # part of the job that runs at another place
             deps = [begin]
-            if is_fwd:
-                deps += [done[s, mb, True] for s in sorted(sources[stage])]
-            else:
-                deps += [done[t, mb, False] for t in users_of[stage]] + [done[stage, mb, True]]
-                if stage in out_stages:
-                    deps.append(done["loss", mb])
+            for m in j.mbs:
+                if is_fwd:
+                    deps += [done[s, m, True] for s in sorted(sources[stage])]
+                else:
+                    deps += [done[t, m, False] for t in users_of[stage]] + [done[stage, m, True]]
+                    if stage in out_stages:
+                        deps.append(done["loss", m])
             st = lane(stage, is_fwd)
-            done[stage, mb, is_fwd] = self._node(st, prog.fwd_graph if is_fwd else prog.bwd_graph, deps)
+            node = self._node(st, j.prog.fwd_graph if is_fwd else j.prog.bwd_graph, deps)
+            done.update({(stage, m, is_fwd): node for m in j.mbs})
             if not is_fwd and w.last_backward.get(stage) == mb and w.stack_dw and w.dw_jobs[stage][1] is not None:
                 self._node(st, w.dw_jobs[stage][1], [])
 

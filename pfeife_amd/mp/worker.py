@@ -14,15 +14,20 @@ every stage:
   * `_init_optimizer` / `optimizer_step` (worker.py:583-597, 1432-1436).
 """
 import os
+from types import SimpleNamespace
 
 import torch
 
 from ..executor.lowering import BufferPool, Lowerer, ParamStore, Unsupported
+from ..executor.merge import MicroBatchLayout
 from ..executor.values import Val
 from ..option import get_optimizer_cls
 from ..schedule.scheduler import PipeSchedParams, SingleCommScheduler, StepWork, serialize_ranks
 from ..utils import fmem, get_logger
 from .step_plan import StepPlan
+
+
+JOB_ROWS = 8192    # (measured: executor/merge.py)
 
 
 class MicroBatchPrograms:
@@ -35,10 +40,24 @@ class MicroBatchPrograms:
         self.outputs = []          # per graph output: Val | python constant
         self.loss_grads = {}       # graph output index -> static gradient buffer
         self.graph = None          # the partition graph the programs were lowered from
+        self.layout = None         # MicroBatchLayout of the step the programs were lowered for
         self.grad_seen = set()
 
 
+class StageJob:
+    """What runs a stage's forward (or backward) of consecutive micro-batches: the stage program of one, or one
+    made of several."""
+
+    def __init__(self, prog, mbs, first, last):
+        self.prog = prog
+        self.mbs = mbs           # the micro-batches it covers
+        self.first = first       # the forward runs where the schedule has the forward of this one,
+        self.last = last         # the backward where it has the backward of this one
+
+
 class StageWorker:
+    jobs = None                # (stage, micro-batch) -> StageJob; None: to be formed from the slots
+
     def __init__(self, runner, option, device, kernels=None):
         self.runner = runner
         self.option = option
@@ -96,6 +115,11 @@ class StageWorker:
         # shapes stack their buffers (`uniform_mbs`, set by the runner before the step's first job)
         self.stack_dw = os.environ.get("PFEIFE_DW_STACK", "1") != "0"
         self.uniform_mbs = getattr(self, "uniform_mbs", True)
+        # Consecutive micro-batches share a stage's jobs until these have this many rows (PFEIFE_JOB_ROWS; 0: every
+        # micro-batch has jobs of its own)
+        self.job_rows = int(os.environ.get("PFEIFE_JOB_ROWS", str(JOB_ROWS)))
+        self.mb_sizes = getattr(self, "mb_sizes", [1] * self.option.batch_cnt)    # samples, set by the runner
+        self._layouts = {}         # tag -> MicroBatchLayout
         return Lowerer(self.kernels, self.device, self.option.mixed_precision, self.params, self.pool)
 
     # -- graph ---------------------------------------------------------------------
@@ -234,12 +258,13 @@ class StageWorker:
         graph_vals = {}
         L = self.lowerer
         L.defer_dw = self.stack_dw and self.uniform_mbs
-        L.stack_mbs = self.option.batch_cnt
-        L.stack_tag = slot.input_sig
+        L.layout = slot.layout = self._layout(mb, slot.input_sig)
+        if L.layout is not None and mb >= len(L.layout.sizes):
+            raise RuntimeError("micro-batch %d of a step of %d" % (mb, len(L.layout.sizes)))
         for i, v in dynamic_inputs.items():
             if torch.is_tensor(v):
-                if L.defer_dw:   # (a layer that reads a graph input directly: its rows of all micro-batches in one matrix)
-                    buf = self.pool.stacked((L.stack_tag, "in", i), v.shape, v.dtype, mb, L.stack_mbs)
+                if L.layout is not None:   # (a layer that reads a graph input directly: its rows of all micro-batches in one matrix)
+                    buf = self.pool.stacked((L.layout.tag, "in", i), v.shape, v.dtype, L.layout.place(mb), aligned=v.dtype.is_floating_point)
                 else:
                     buf = torch.empty(v.shape, dtype=v.dtype, device=self.device)
                 slot.input_buffers[i] = buf
@@ -279,6 +304,8 @@ class StageWorker:
             prog = L.lower_forward(st, mb, ins)
             slot.stage_programs[sid] = prog
             stage_out[sid] = prog.outputs
+        if L.layout is not None and not L.layout.formed:
+            self._form_groups(L.layout, mb, slot.stage_programs.values())
         # graph outputs and the buffers their loss gradients arrive in
         for oi, ref in enumerate(pg.outputs):
             if ref[0] == "const":
@@ -289,10 +316,10 @@ class StageWorker:
                 v = stage_out[ref[0]][ref[1]]
                 slot.outputs.append(v)
                 if isinstance(v, Val) and v.req_grad:
-                    if L.defer_dw and v.buf.is_contiguous():
+                    if L.layout is not None and v.buf.is_contiguous():
                         # (the last layer's weight gradient reads these across micro-batches as one matrix)
-                        slot.loss_grads[oi] = self.pool.stacked((L.stack_tag, "loss", oi), v.buf.shape, v.buf.dtype, mb,
-                                                                L.stack_mbs).zero_()
+                        slot.loss_grads[oi] = self.pool.stacked((L.layout.tag, "loss", oi), v.buf.shape, v.buf.dtype,
+                                                                L.layout.place(mb)).zero_()
                     else:
                         slot.loss_grads[oi] = torch.zeros_like(v.buf)
         # backward, last stage first: a stage's output gradients are its consumers' input gradients
@@ -322,13 +349,86 @@ class StageWorker:
             # that read them run on the lanes
             self.stream_obj.synchronize()
             torch.cuda.current_stream(self.device).synchronize()
+        self._drop_jobs()
         self._drop_graphs(self.mbs.get(mb))   # a slot rebuilt for another micro-batch shape
         self._drop_dw_jobs()
         self.mbs[mb] = slot
-        self.pool.prune_stacked({s.input_sig for s in self.mbs.values()})
+        self._layouts = {s.layout.tag: s.layout for s in self.mbs.values() if s.layout is not None}
+        self.pool.prune_stacked(set(self._layouts))
         self.graphs_ready = False   # new programs (and possibly new parameters): capture again
         self._drop_begin_graph()
         return slot
+
+    def _layout(self, mb, sig):
+        """How the buffers of the step's micro-batches lie, for a micro-batch whose inputs have the signature `sig`;
+        None: each has buffers of its own."""
+        uniform = self.uniform_mbs
+        if not (self.stack_dw and uniform) and not self.job_rows:
+            return None
+        n = self.option.batch_cnt
+        if uniform:
+            tag, sizes = sig, [1] * n
+        else:
+            # the same graph over other numbers of samples: one tag, if the inputs' extents follow the number
+            sizes = list(self.mb_sizes)
+            own = sizes[mb]
+            tag = ("ragged", tuple(sizes)) + tuple(
+                x if x[0] == "const" or not x[0] or not own or x[0][0] % own else
+                (("samples", x[0][0] // own) + tuple(x[0][1:]), x[1]) for x in sig)
+        layout = self._layouts.get(tag)
+        if layout is None:
+            layout = MicroBatchLayout(sizes, tag)
+        return layout
+
+    def _form_groups(self, layout, mb, progs):
+        """Which micro-batches share jobs: by the rows of the longest matrix product of a forward job."""
+        layout.formed = True
+        rows = max([l.call[1]["M"] for p in progs for l in p.fwd
+                    if getattr(l, "call", ("",))[0] == "gemm" and tuple(l.call[1]["batch"]) == (1, 1)] + [0])
+        if self.job_rows and rows and layout.sizes[mb]:
+            layout.form_groups(rows / layout.sizes[mb], self.job_rows)
+
+    def form_jobs(self):
+        """The jobs of a step from the micro-batches' programs: consecutive micro-batches of one layout and group whose
+        launch lists correspond run as one.  A job's forward runs where the schedule has its first micro-batch, its
+        backward where it has its last: every order that the schedule allows stays one."""
+        runs, self.jobs = [], {}
+        for mb in sorted(self.mbs):
+            lay = self.mbs[mb].layout
+            key = None if lay is None else (lay.tag, lay.group(mb))
+            if runs and key is not None and runs[-1][0] == key and runs[-1][1][-1] == mb - 1:
+                runs[-1][1].append(mb)
+            else:
+                runs.append((key, [mb]))
+        at = {job: i for i, job in enumerate(self.order)} if runs else {}
+        for _, mbs in runs:
+            for sid in self.part_graph.nodes:
+                progs = [self.mbs[m].stage_programs[sid] for m in mbs]
+                prog = None
+                if len(mbs) > 1:
+                    self.pool.lane = self._lane_key(sid, False) if self.lanes is not None else 0
+                    prog = self.lowerer.merge_programs(progs)
+                    self.pool.lane = 0
+                for part in ([mbs] if prog is not None else [[m] for m in mbs]):
+                    job = StageJob(prog if prog is not None else self.mbs[part[0]].stage_programs[sid], part,
+                                   min(part, key=lambda m: at[sid, m, True]), max(part, key=lambda m: at[sid, m, False]))
+                    for m in part:
+                        self.jobs[sid, m] = job
+        if runs and self.stream_obj is not None:     # (tables of batched reductions)
+            torch.cuda.current_stream(self.device).synchronize()
+
+    def step_programs(self):
+        """The programs whose launches a step issues, each once."""
+        if self.jobs is None:
+            self.form_jobs()
+        return list({id(j.prog): j.prog for j in self.jobs.values()}.values())
+
+    def _drop_jobs(self):
+        """Forgets the jobs, after what has been issued of them; frees the graphs of those over several micro-batches."""
+        jobs, self.jobs = self.jobs, None
+        for job in {id(j): j for j in (jobs or {}).values()}.values():
+            if len(job.mbs) > 1:
+                self._drop_graphs(SimpleNamespace(stage_programs={0: job.prog}))
 
     def _drop_graphs(self, slot):
         """Frees the captured hipGraphs of a micro-batch slot that is being replaced or released."""
@@ -380,6 +480,7 @@ class StageWorker:
             self.issuer.close()
             self.issuer = None
         self._drain()
+        self._drop_jobs()
         for slot in self.mbs.values():
             self._drop_graphs(slot)
         self._drop_begin_graph()
@@ -409,12 +510,11 @@ class StageWorker:
         Called after one complete eager step, when every program exists and every kernel has
         run once (so one-time function attributes are set)."""
         s = self.stream()
-        for slot in self.mbs.values():
-            for prog in slot.stage_programs.values():
-                if prog.fwd_graph is None and prog.fwd:
-                    prog.fwd_graph = self.kernels.capture(prog.fwd, s)
-                if prog.bwd_graph is None and prog.bwd:
-                    prog.bwd_graph = self.kernels.capture(prog.bwd, s)
+        for prog in self.step_programs():
+            if prog.fwd_graph is None and prog.fwd:
+                prog.fwd_graph = self.kernels.capture(prog.fwd, s)
+            if prog.bwd_graph is None and prog.bwd:
+                prog.bwd_graph = self.kernels.capture(prog.bwd, s)
         for job in self.dw_jobs.values():
             if job[1] is None and job[0]:
                 job[1] = self.kernels.capture(job[0], s)
@@ -459,6 +559,8 @@ class StageWorker:
                 self.capture_graphs()      # (weight-gradient jobs that were lowered after the other graphs)
             if self.issuer is None:
                 self.issuer = self.kernels.issuer()
+            if self.jobs is None:
+                self.form_jobs()
             self.step_plan = StepPlan(self)
         self.params.rebind_grads()
         for slot in self.mbs.values():
@@ -468,6 +570,8 @@ class StageWorker:
 
     def begin_step(self):
         s = self.stream()
+        if self.jobs is None:
+            self.form_jobs()
         self.params.rebind_grads()
         if self.use_graphs and not self.graphs_ready and self.steps_done >= 1 and len(self.mbs) == self.option.batch_cnt:
             self.capture_graphs()
@@ -498,7 +602,7 @@ class StageWorker:
             return
         for sid in self._output_stages:
             if self.lanes[self._lane_key(sid, True)] is not self.stream_obj:
-                ev = self._job_events.get((sid, mb, True))
+                ev = self._job_events.get((sid, self.jobs[sid, mb].first, True))
                 if ev is not None:
                     self.stream_obj.wait_event(ev)
 
@@ -586,7 +690,12 @@ class StageWorker:
                 launch(stream)
 
     def run_job(self, stage, mb, is_fwd):
-        prog = self.mbs[mb].stage_programs[stage]
+        if self.jobs is None:
+            self.form_jobs()
+        job = self.jobs[stage, mb]
+        if mb != (job.first if is_fwd else job.last):
+            return               # part of the job that runs at another place
+        prog = job.prog
         if self.lanes is None:
             if is_fwd:
                 prog.run_forward(self.stream())
@@ -608,15 +717,17 @@ class StageWorker:
             deps.add((stage, True))    # its own forward (which followed the producers of its inputs)
         for other, d in sorted(deps):
             if self.lanes[self._lane_key(other, d)] is not lane:
-                ev = self._job_events.get((other, mb, d))
-                if ev is None:
-                    raise RuntimeError("job order: stage %d of micro-batch %d runs before stage %d (%s)"
-                                       % (stage, mb, other, "forward" if is_fwd else "backward"))
-                lane.wait_event(ev)
+                for m in sorted({self._runs_at(other, m, d) for m in job.mbs}):
+                    ev = self._job_events.get((other, m, d))
+                    if ev is None:
+                        raise RuntimeError("job order: stage %d of micro-batch %d runs before stage %d (%s)"
+                                           % (stage, mb, other, "forward" if is_fwd else "backward"))
+                    lane.wait_event(ev)
         if not is_fwd and lane is not self.stream_obj and stage in self._output_stages:
-            ev = self._loss_events.get(mb)
-            if ev is not None:
-                lane.wait_event(ev)
+            for m in job.mbs:
+                ev = self._loss_events.get(m)
+                if ev is not None:
+                    lane.wait_event(ev)
         if is_fwd:
             prog.run_forward(lane.cuda_stream)
         else:
@@ -624,6 +735,11 @@ class StageWorker:
         self._event(self._job_events, (stage, mb, is_fwd)).record(lane)   # (the weight-gradient job feeds no other job)
         if not is_fwd and self.last_backward.get(stage) == mb and self.stack_dw:
             self._run_dw_job(stage, lane.cuda_stream)
+
+    def _runs_at(self, stage, mb, is_fwd):
+        """The micro-batch at whose place in the schedule a micro-batch's job of a stage runs."""
+        job = self.jobs[stage, mb]
+        return job.first if is_fwd else job.last
 
     def init_optimizer(self, optimizer):
         if optimizer is not None:

@@ -1,0 +1,160 @@
+"""Stage jobs over several micro-batches (pfeife_amd/executor/merge.py) on the kernel oracle: a step whose jobs are
+merged against the same step with one job per micro-batch."""
+import copy
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from pfeife_amd.bench_models.llama import LlamaConfig, LlamaForCausalLM
+from pfeife_amd.bench_models.unet_stage import UNetStage, UNetStageConfig
+from pfeife_amd.bench_models.vit import ViTConfig, VisionTransformer
+from pfeife_amd.executor.merge import MicroBatchLayout
+from pfeife_amd.option import PipeOption
+from test_host_pipeline import make_runner
+
+
+def _model(family):
+    torch.manual_seed(0)
+    if family == "vit":
+        return VisionTransformer(ViTConfig(image_size=32, patch_size=16, dim=64, depth=2, heads=2, mlp_dim=128, num_classes=16))
+    if family == "decoder":
+        return LlamaForCausalLM(LlamaConfig(vocab=64, dim=64, layers=2, heads=2, ffn=88, max_seq=9))
+    return UNetStage(UNetStageConfig(in_channels=32, channels=64, temb_dim=32, context_dim=24, heads=2, layers=1))
+
+
+def _gpu_runner(option):
+    from pfeife_amd.mp import PartialRunner, initialize_pfeife, net_states
+
+    torch._dynamo.reset()
+    net_states._reset_state_for_tests()
+    initialize_pfeife()
+    return PartialRunner(option)
+
+
+def _steps(family, mixed, batch, micro, rows, steps, monkeypatch, device="cpu"):
+    """[(results, gradients)] of some steps, and the worker.  `batch`: samples of each step."""
+    from pfeife_amd.mp import partial_compiler
+
+    monkeypatch.setenv("PFEIFE_JOB_ROWS", str(rows))
+    model = _model(family).to(device)
+    make = make_runner if device == "cpu" else _gpu_runner
+    splits = {"vit": ["blocks.1"], "decoder": ["layers.1"], "unet": None}[family]
+    runner = make(PipeOption(device_cnt=2 if splits else 1, batch_cnt=micro, batch_size=1, split_points=splits,
+                                    mixed_precision=mixed, optimizer=dict(type="sgd", lr=0.01)))
+    cmodel = torch.compile(model, backend=partial_compiler, dynamic=False)
+
+    def fn(*a):
+        if family == "vit":
+            loss = F.cross_entropy(cmodel(a[0]).float(), a[1])
+        elif family == "decoder":
+            loss = cmodel(a[0], a[0])
+        else:
+            loss = F.mse_loss(cmodel(*a[:3]).float(), a[3])
+        loss.backward()
+        return loss.detach()
+
+    runner.set_exec_fn(fn)
+    out = []
+    for n in (batch if isinstance(batch, tuple) else (batch,) * steps):
+        g = torch.Generator().manual_seed(n)
+        if family == "vit":
+            args = (torch.randn(n, 3, 32, 32, generator=g), torch.randint(0, 10, (n,), generator=g))
+        elif family == "decoder":
+            args = (torch.randint(0, 64, (n, 9), generator=g),)
+        else:
+            args = (torch.randn(n, 32, 6, 6, generator=g), torch.randn(n, 32, generator=g),
+                    torch.randn(n, 5, 24, generator=g), torch.randn(n, 64, 6, 6, generator=g))
+        losses = [float(l) for l in runner.step(*(a.to(device) for a in args))]
+        out.append((losses, {k: p.grad.cpu().clone() for k, p in model.named_parameters()}))
+    return out, runner.worker
+
+
+@pytest.mark.parametrize("mixed", [None, "bf16"])
+@pytest.mark.parametrize("family,batch,micro,rows,jobs", [
+    ("vit", 8, 4, 10 ** 6, [[0, 1, 2, 3]]), ("vit", 8, 4, 20, [[0, 1], [2, 3]]), ("vit", 10, 5, 25, [[0, 1, 2], [3, 4]]),
+    ("vit", 7, 3, 10 ** 6, [[0, 1, 2]]), ("vit", 3, 3, 10 ** 6, [[0, 1, 2]]), ("vit", 11, 4, 27, [[0, 1], [2, 3]]),
+    ("vit", (8, 8, 10, 8, 7), 4, 10 ** 6, None),
+    ("decoder", 4, 4, 10 ** 6, [[0, 1, 2, 3]]), ("decoder", 5, 3, 10 ** 6, [[0, 1, 2]]),
+    ("unet", 4, 2, 10 ** 6, [[0, 1]]), ("unet", 3, 2, 10 ** 6, [[0], [1]]),    # (its channel bias sums sample by sample: other lists)
+])
+def test_merged_jobs_equal_jobs_per_micro_batch(monkeypatch, family, batch, micro, rows, jobs, mixed):
+    """Losses bit for bit (every row is computed from the same operands by the same arithmetic); gradients to the
+    rounding of fp32 sums in another order (2e-6 of their norm: sums of at most 700 rows), in the second and later
+    steps to what an update with such gradients changes."""
+    want, w0 = _steps(family, mixed, batch, micro, 0, 2, monkeypatch)
+    got, w = _steps(family, mixed, batch, micro, rows, 2, monkeypatch)
+    assert all(len(j.mbs) == 1 for j in w0.jobs.values())
+    if jobs is not None:
+        assert [sorted(j.mbs) for (s, m), j in sorted(w.jobs.items()) if s == 0 and m == j.mbs[0]] == jobs
+        assert all(j.first == min(j.mbs) and j.last == max(j.mbs) for j in w.jobs.values())
+    tol = 2e-6 if mixed is None else 2e-2
+    for i, ((l0, g0), (l1, g1)) in enumerate(zip(want, got)):
+        assert all(abs(a - b) <= (0 if i == 0 and mixed else max(tol, 1e-6) * abs(a)) for a, b in zip(l0, l1)), (i, l0, l1)
+        for k in g0:
+            d = float((g0[k].double() - g1[k].double()).norm() / (g0[k].double().norm() + 1e-30))
+            assert d <= (tol if i else 2e-6 if mixed is None else tol), (i, k, d)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mixed", [None, "bf16"])
+@pytest.mark.parametrize("family,batch,micro,rows", [
+    ("vit", 8, 4, 10 ** 6), ("vit", 8, 4, 20), ("vit", 7, 3, 10 ** 6), ("vit", (8, 8, 8, 10, 8, 8, 7), 4, 10 ** 6),
+    ("decoder", 5, 5, 10 ** 6), ("decoder", 5, 3, 10 ** 6), ("unet", 4, 2, 10 ** 6)])
+def test_merged_jobs_on_the_device(monkeypatch, family, batch, micro, rows, mixed):
+    """Launch by launch, captured and from job lists (four steps): gradients to the rounding of fp32 sums, with 16-bit
+    operands to that of a dozen layers (2.5e-2, as every whole-step test here)."""
+    if family == "unet" and mixed is None:
+        pytest.skip("a stage that runs in 16 bits")
+    want, _ = _steps(family, mixed, batch, micro, 0, 4, monkeypatch, "cuda")
+    got, w = _steps(family, mixed, batch, micro, rows, 4, monkeypatch, "cuda")
+    assert any(len(j.mbs) > 1 for j in w.jobs.values())
+    tol = 1e-4 if mixed is None else 2.5e-2
+    for i, ((l0, g0), (l1, g1)) in enumerate(zip(want, got)):
+        assert all(abs(a - b) <= tol * abs(a) for a, b in zip(l0, l1)), (i, l0, l1)
+        for k in g0:
+            d = float((g0[k].double() - g1[k].double()).norm() / (g0[k].double().norm() + 1e-30))
+            assert d <= tol, (i, k, d)
+
+
+def test_merged_lists_are_as_short_as_one_micro_batchs(monkeypatch):
+    """Nothing but a loss inside the model stays per micro-batch."""
+    for family, per_mb in (("vit", 0), ("decoder", 2 * 3)):    # cross entropy forward and backward of the last stage
+        _, w = _steps(family, "bf16", 8, 4, 10 ** 6, 1, monkeypatch)
+        one = sum(len(p.fwd) + len(p.bwd) for p in w.mbs[0].stage_programs.values())
+        assert sum(len(p.fwd) + len(p.bwd) for p in w.step_programs()) == one + per_mb
+
+
+def test_a_micro_batch_that_differs_keeps_its_own_launches(monkeypatch):
+    """Operands that do not follow each other: the launches stay as they are, in order."""
+    from oracle.kernels_oracle import OracleKernels
+    from pfeife_amd.executor.merge import CallRecorder, Merger
+
+    k = CallRecorder(OracleKernels("cpu"))
+    x, y, z = torch.arange(12.0), torch.zeros(12), torch.zeros(12)
+    m = Merger(k, torch.empty)
+    calls = [k.cast(x[0:4], y[0:4], 4), k.cast(x[4:8], y[4:8], 4), k.cast(x[8:12], z[0:4], 4)]
+    out = m.lists([[c] for c in calls])
+    assert len(out) == 2 and out[1] is calls[2]
+    for l in out:
+        l(None)
+    assert torch.equal(y[:8], x[:8]) and torch.equal(z[:4], x[8:])
+    assert m.lists([[calls[0]], [k.cast(x[4:8], y[6:10], 4)]])[0] is calls[0]      # a gap
+    assert m.lists([[calls[0]], [k.fill(y[4:8], 0.0, 4)]])[0] is calls[0]         # another kernel
+    assert m.lists([[calls[0]], []]) is None                                       # another structure
+
+
+@pytest.mark.parametrize("sizes", [[2] * 5, [3, 3, 2, 2], [1, 1, 0, 0], [4]])
+@pytest.mark.parametrize("rows", [1, 7, 10 ** 6])
+def test_layout_places_do_not_overlap(sizes, rows):
+    lay = MicroBatchLayout(sizes, "t")
+    lay.form_groups(3, rows)
+    assert [m for a, b in lay.groups for m in range(a, b)] == list(range(len(sizes)))
+    for in_group in (False, True):
+        for per in (1, 6):
+            spans = [(m, lay.place(m, in_group).span(per * n)) for m, n in enumerate(sizes) if n]
+            for m, (off, total) in spans:
+                assert 0 <= off and off + per * sizes[m] <= total == spans[0][1][1]
+            for (m, (a, _)), (m2, (b, _)) in zip(spans, spans[1:]):
+                if not in_group or lay.group(m) == lay.group(m2):
+                    assert b == a + per * sizes[m]
