@@ -80,20 +80,20 @@ def _steps(family, mixed, batch, micro, rows, steps, monkeypatch, device="cpu"):
 ])
 def test_merged_jobs_equal_jobs_per_micro_batch(monkeypatch, family, batch, micro, rows, jobs, mixed):
     """Losses bit for bit (every row is computed from the same operands by the same arithmetic); gradients to the
-    rounding of fp32 sums in another order (2e-6 of their norm: sums of at most 700 rows), in the second and later
-    steps to what an update with such gradients changes."""
+    rounding of fp32 sums in another order: at most 144 rows (four images of 36 pixels), 144 * 2^-24 = 8.6e-6; in
+    16 bits, after an update, to what it changes in the weights' rounding."""
     want, w0 = _steps(family, mixed, batch, micro, 0, 2, monkeypatch)
     got, w = _steps(family, mixed, batch, micro, rows, 2, monkeypatch)
     assert all(len(j.mbs) == 1 for j in w0.jobs.values())
     if jobs is not None:
         assert [sorted(j.mbs) for (s, m), j in sorted(w.jobs.items()) if s == 0 and m == j.mbs[0]] == jobs
         assert all(j.first == min(j.mbs) and j.last == max(j.mbs) for j in w.jobs.values())
-    tol = 2e-6 if mixed is None else 2e-2
+    tol = 8.6e-6 if mixed is None else 2e-2
     for i, ((l0, g0), (l1, g1)) in enumerate(zip(want, got)):
-        assert all(abs(a - b) <= (0 if i == 0 and mixed else max(tol, 1e-6) * abs(a)) for a, b in zip(l0, l1)), (i, l0, l1)
+        assert all(abs(a - b) <= (0 if i == 0 and mixed else tol * abs(a)) for a, b in zip(l0, l1)), (i, l0, l1)
         for k in g0:
             d = float((g0[k].double() - g1[k].double()).norm() / (g0[k].double().norm() + 1e-30))
-            assert d <= (tol if i else 2e-6 if mixed is None else tol), (i, k, d)
+            assert d <= tol, (i, k, d)
 
 
 @pytest.mark.gpu
