@@ -69,13 +69,16 @@ static inline bool pf_aligned(const void* p, size_t a) { return (reinterpret_cas
 
 // bf16 <-> f32 with round-to-nearest-even (matches torch's .to(torch.bfloat16))
 __device__ __forceinline__ float pf_bf16_bits_to_f32(uint16_t b) { return __uint_as_float(((uint32_t)b) << 16); }
-__device__ __forceinline__ uint16_t pf_f32_to_bf16_bits(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x0040u);  // quiet NaN
-  uint32_t lsb = (u >> 16) & 1u;
-  u += 0x7fffu + lsb;
-  return (uint16_t)(u >> 16);
+typedef __bf16 pf_bf16x2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 pf_f16x2_t __attribute__((ext_vector_type(2)));
+typedef float pf_f32x2_t __attribute__((ext_vector_type(2)));
+// two fp32 -> one packed pair of 16-bit values (low half = first argument), round to nearest
+// even: single v_cvt_pk_{bf16,f16}_f32 instructions on gfx950
+__device__ __forceinline__ uint32_t pf_pack2_bf16(float lo, float hi) {
+  const pf_f32x2_t v = {lo, hi};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, pf_bf16x2_t));
 }
+__device__ __forceinline__ uint16_t pf_f32_to_bf16_bits(float f) { return (uint16_t)pf_pack2_bf16(f, f); }
 __device__ __forceinline__ float pf_f16_bits_to_f32(uint16_t b) {
   union { uint16_t u; _Float16 h; } c;
   c.u = b;
@@ -87,15 +90,6 @@ __device__ __forceinline__ uint16_t pf_f32_to_f16_bits(float f) {
   return c.u;
 }
 
-// two fp32 -> one packed pair of 16-bit values (low half = first argument), round to nearest
-// even: single v_cvt_pk_{bf16,f16}_f32 instructions on gfx950
-typedef __bf16 pf_bf16x2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 pf_f16x2_t __attribute__((ext_vector_type(2)));
-typedef float pf_f32x2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t pf_pack2_bf16(float lo, float hi) {
-  const pf_f32x2_t v = {lo, hi};
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, pf_bf16x2_t));
-}
 __device__ __forceinline__ uint32_t pf_pack2_f16(float lo, float hi) {
   const pf_f32x2_t v = {lo, hi};
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, pf_f16x2_t));
@@ -286,8 +280,8 @@ __device__ __forceinline__ float pf_erf_fast(float u, float& e2) {
 }
 // GELU (erf form) without the reciprocal: the upper tail of the normal distribution is
 // 1 - Phi(a) = 2^-g(a) with g a degree-5 polynomial on [0, 5.5] (weighted minimax fit; beyond 5.5 the
-// tail is below 2e-8), and x * Phi(x) = x - x * tail(|x|) for x >= 0, x * tail(|x|) for x < 0.
-// |error| <= 9e-7 in fp32 arithmetic over [-8, 8]: five FMAs, one v_exp_f32, a multiply, a subtract, a select.
+// tail is below 2e-8), and x * Phi(x) = max(x, 0) - |x| * tail(|x|).
+// |error| <= 9e-7 in fp32 arithmetic over [-8, 8]: six FMAs, one v_exp_f32, a minimum, a maximum.
 __device__ __forceinline__ float pf_gelu_erf(float x) {
   const float a = fminf(fabsf(x), 5.5f);
   float g = fmaf(0.00049698935f, a, -0.007244379f);
@@ -295,8 +289,7 @@ __device__ __forceinline__ float pf_gelu_erf(float x) {
   g = fmaf(g, a, 0.45959195f);
   g = fmaf(g, a, 1.1509614f);
   g = fmaf(g, a, 1.0000144f);
-  const float xq = x * __builtin_amdgcn_exp2f(-g);
-  return x >= 0.f ? x - xq : xq;
+  return fmaf(-fabsf(x), __builtin_amdgcn_exp2f(-g), fmaxf(x, 0.f));
 }
 __device__ __forceinline__ float pf_gelu_erf_grad(float x) {
   float e2;   // = exp(-x*x/2)

@@ -20,15 +20,15 @@
   int pf_gemm_x_##DT##_##XT(const pf_gemm_desc& d, hipStream_t st);    \
   int pf_gemm_xgroup_##DT##_##XT(const pf_gemm_desc* d, int n, hipStream_t st);
 #define PF_X_DECL_DT(DT) \
-  PF_X_DECL(DT, 1) PF_X_DECL(DT, 2) PF_X_DECL(DT, 3) PF_X_DECL(DT, 4) PF_X_DECL(DT, 5) PF_X_DECL(DT, 6) PF_X_DECL(DT, 7) PF_X_DECL(DT, 8) PF_X_DECL(DT, 9) PF_X_DECL(DT, 10) PF_X_DECL(DT, 11)
+  PF_X_DECL(DT, 1) PF_X_DECL(DT, 2) PF_X_DECL(DT, 3) PF_X_DECL(DT, 4) PF_X_DECL(DT, 5) PF_X_DECL(DT, 6) PF_X_DECL(DT, 7) PF_X_DECL(DT, 8) PF_X_DECL(DT, 9) PF_X_DECL(DT, 10) PF_X_DECL(DT, 11) PF_X_DECL(DT, 12)
 PF_X_DECL_DT(1)
 PF_X_DECL_DT(2)
 #undef PF_X_DECL_DT
 #undef PF_X_DECL
-static_assert(PF_F16 == 1 && PF_BF16 == 2 && PF_XT_COUNT == 12, "the table below is written out for these ids");
+static_assert(PF_F16 == 1 && PF_BF16 == 2 && PF_XT_COUNT == 13, "the table below is written out for these ids");
 typedef int (*pf_x_fn)(const pf_gemm_desc&, hipStream_t);
 typedef int (*pf_xgroup_fn)(const pf_gemm_desc*, int, hipStream_t);
-#define PF_X_ROW(P, DT) {nullptr, P##DT##_1, P##DT##_2, P##DT##_3, P##DT##_4, P##DT##_5, P##DT##_6, P##DT##_7, P##DT##_8, P##DT##_9, P##DT##_10, P##DT##_11}
+#define PF_X_ROW(P, DT) {nullptr, P##DT##_1, P##DT##_2, P##DT##_3, P##DT##_4, P##DT##_5, P##DT##_6, P##DT##_7, P##DT##_8, P##DT##_9, P##DT##_10, P##DT##_11, P##DT##_12}
 static const pf_x_fn pf_x_table[3][PF_XT_COUNT] = {{}, PF_X_ROW(pf_gemm_x_, 1), PF_X_ROW(pf_gemm_x_, 2)};
 static const pf_xgroup_fn pf_xgroup_table[3][PF_XT_COUNT] = {{}, PF_X_ROW(pf_gemm_xgroup_, 1), PF_X_ROW(pf_gemm_xgroup_, 2)};
 #undef PF_X_ROW
@@ -589,15 +589,16 @@ int launch16(const pf_gemm_desc& d, hipStream_t st) {
 // Variant ids (pf_gemm_desc.variant; 0 = automatic):
 //   1..10  direct-to-LDS kernel, tiles PF_XT_256x256 / 256x128 / 128x128 / 192x256 / 128x128k2 / 256x128k2 /
 //          256x256w8 / 128x128w8 / 256x128w8 / 192x256w8
+//   18     direct-to-LDS kernel, tile PF_XT_256x256w4
 //   15     direct-to-LDS kernel, tile PF_XT_64x64; 16, 17: 128x128w8 and 256x128w8 for row-major products whose
 //          K is a multiple of 8 only (15 takes these too)
 //   11..14 register-staged kernel: 128x128 by 8 wavefronts, 128x128, 128x64, 64x64 by 4
 enum { V_AUTO = 0, V_X256 = 1, V_X256x128 = 2, V_X128 = 3, V_X192x256 = 4, V_X128K2 = 5, V_X256x128K2 = 6, V_X256W8 = 7, V_X128W8 = 8, V_X256x128W8 = 9, V_X192x256W8 = 10,
-       V_X64 = 15, V_X128W8R = 16, V_X256x128W8R = 17, V_R128W8 = 11, V_R128 = 12, V_R128x64 = 13, V_R64 = 14 };
-inline bool is_x_variant(int v) { return (v >= V_X256 && v <= V_X192x256W8) || (v >= V_X64 && v <= V_X256x128W8R); }
+       V_X64 = 15, V_X128W8R = 16, V_X256x128W8R = 17, V_X256W4 = 18, V_R128W8 = 11, V_R128 = 12, V_R128x64 = 13, V_R64 = 14 };
+inline bool is_x_variant(int v) { return (v >= V_X256 && v <= V_X192x256W8) || (v >= V_X64 && v <= V_X256W4); }
 // tile id (PF_XT_*) of a direct-to-LDS variant
 inline int x_tile_of(int v) {
-  return v == V_X64 ? (int)PF_XT_64x64 : v == V_X128W8R ? (int)PF_XT_128x128w8 : v == V_X256x128W8R ? (int)PF_XT_256x128w8 : v;
+  return v == V_X64 ? (int)PF_XT_64x64 : v == V_X128W8R ? (int)PF_XT_128x128w8 : v == V_X256x128W8R ? (int)PF_XT_256x128w8 : v == V_X256W4 ? (int)PF_XT_256x256w4 : v;
 }
 
 // Register-staged tiles: 128x128 with two workgroups resident per CU is the largest that keeps
@@ -623,27 +624,30 @@ bool x_supports(const pf_gemm_desc& d, int v) {
   const int xt = x_tile_of(v), bk = x_tile_bk(xt);
   if ((xt == PF_XT_192x256 || xt == PF_XT_192x256w8) && d.a_trans) return false;   // no reduction-strided 192-row tile
   if (d.a_trans != d.b_trans) return false;
-  if (!d.a_trans && d.K % bk != 0 && !(v >= V_X64 && d.K % 8 == 0)) return false;
+  if (!d.a_trans && d.K % bk != 0 && !(v >= V_X64 && v != V_X256W4 && d.K % 8 == 0)) return false;
   return d.K >= bk;
 }
 
-// Automatic choice: a cost model fitted to measurements on MI355X (microseconds; sweeps of 32 row-major and 21
-// reduction-strided shapes, 16 to 8192 rows).  A workgroup's fixed cost (dispatch, first tile, epilogue) plus, per
-// round of 256 workgroups, K / 64 tile steps; a step gets slower the more CUs stream operands at the same time, so
-// a step costs t0 in an empty device and t0 + t1 in a full one.  The 64x64 tile runs two workgroups to a CU
-// and its cost grows with their number.  On the sweeps the choice is the fastest variant or within 8 % of it.
+// Automatic choice: a cost model fitted to measurements on MI355X (microseconds; a sweep of 162 row-major shapes, 256 to
+// 16384 rows and 256 to 10240 columns, and 21 reduction-strided ones).  A workgroup's fixed cost (dispatch, first tile, epilogue)
+// plus, per round of 256 workgroups, K / 64 tile steps and an epilogue that nothing hides; a step gets slower the more CUs
+// stream operands at the same time, so a step costs t0 in an empty device and t0 + t1 in a full one.  The 64x64 tile
+// runs two workgroups to a CU and its cost grows with their number.  On the row-major sweep the choice is on average
+// 0.4 % off the fastest tile, 16 % at most (8192 x 1280 over 5120: 117.6 on 192x256 against 101.1 us); the constants and tiles
+// before the four-wavefront 256x256 tile were 2.9 % and 23 % off.
 // (The tiles whose eight wavefronts split every tile step's depth, variants 5 and 6, are no candidates: inside a
 // pipeline step, next to other streams' kernels, they lost what they gain alone.)
 int choose_variant(const pf_gemm_desc& d) {
   const int64_t nb = d.batch1 * d.batch2;
   struct Cand { int v, bm, bn; double fixed, t0, t1, again; };
-  static const Cand nn[7] = {{V_X256W8, 256, 256, 6.3, 1.05, 0.50, 3.5},
-                             {V_X192x256W8, 192, 256, 5.5, 0.90, 0.40, 3.0},
-                             {V_X256x128W8, 256, 128, 4.5, 0.50, 0.35, 2.0},
-                             {V_X128W8, 128, 128, 3.4, 0.26, 0.27, 1.0},
-                             {V_X256x128W8R, 256, 128, 4.7, 0.52, 0.36, 2.0},   // (ragged K: only where the two above cannot)
-                             {V_X128W8R, 128, 128, 3.5, 0.27, 0.28, 1.0},
-                             {V_X64, 64, 64, 3.0, 0.16, 0.0, 0.6}};
+  static const Cand nn[8] = {{V_X256W4, 256, 256, 6.7, 0.95, 0.43, 6.3},
+                             {V_X256W8, 256, 256, 6.5, 0.95, 0.64, 6.2},
+                             {V_X192x256W8, 192, 256, 5.6, 0.78, 0.47, 5.8},
+                             {V_X256x128W8, 256, 128, 4.9, 0.47, 0.33, 4.4},
+                             {V_X128W8, 128, 128, 3.6, 0.295, 0.176, 2.2},
+                             {V_X256x128W8R, 256, 128, 5.1, 0.49, 0.34, 4.4},   // (ragged K: only where the two above cannot)
+                             {V_X128W8R, 128, 128, 3.7, 0.305, 0.18, 2.2},
+                             {V_X64, 64, 64, 3.2, 0.165, 0.0, 0.73}};
   static const Cand tt[4] = {{V_X256W8, 256, 256, 6.9, 1.10, 0.55, 3.5},
                              {V_X256x128W8, 256, 128, 4.8, 0.58, 0.20, 2.0},
                              {V_X128W8, 128, 128, 3.7, 0.37, 0.17, 1.0},
@@ -654,15 +658,19 @@ int choose_variant(const pf_gemm_desc& d) {
   const int64_t t64 = ((d.M + 63) / 64) * ((d.N + 63) / 64) * nb;
   int best = -1;
   double best_t = 0;
-  for (int i = 0; i < (strided ? 4 : 7); ++i) {
+  for (int i = 0; i < (strided ? 4 : 8); ++i) {
     const Cand& c = strided ? tt[i] : nn[i];
     if (!x_supports(d, c.v)) continue;
     if (strided && c.v == V_X64 && t64 > 160) continue;
     const int64_t tiles = ((d.M + c.bm - 1) / c.bm) * ((d.N + c.bn - 1) / c.bn) * nb;
+    // One round over a short depth whose epilogue is GELU's arithmetic: the four wavefronts gain over the depth what their
+    // longer epilogue costs.  us on eight / four wavefronts, fp16, GELU and GELU': [3072 x 768] . [768 x 4096] 29.9 / 30.4, 34.2 /
+    // 33.7; [4096 x 1024] . [1024 x 3152] 35.2 / 35.2, 39.7 / 38.9; over 2048 55.9 / 54.5, 60.6 / 57.8
+    if (c.v == V_X256W4 && tiles <= 256 && d.K <= 1024 && (d.act != PF_ACT_NONE || d.dact != PF_ACT_NONE)) continue;
     const int64_t full = tiles / 256, rest = tiles % 256;
     double step;
     if (c.v == V_X64) {
-      step = 0.05 + 0.19 * (double)tiles / 256.0;
+      step = strided ? 0.05 + 0.19 * (double)tiles / 256.0 : 0.08 + 0.171 * (double)tiles / 256.0;
       if (step < c.t0) step = c.t0;
     } else {
       step = (double)full * (c.t0 + c.t1) + (rest ? c.t0 + c.t1 * (double)rest / 256.0 : 0.0);
@@ -715,7 +723,7 @@ int dispatch16(const pf_gemm_desc& d, hipStream_t st) {
     }
   }
   switch (v) {
-    case V_X256: case V_X256x128: case V_X128: case V_X192x256: case V_X128K2: case V_X256x128K2: case V_X256W8: case V_X128W8: case V_X256x128W8: case V_X192x256W8: case V_X64: case V_X128W8R: case V_X256x128W8R: {
+    case V_X256: case V_X256x128: case V_X128: case V_X192x256: case V_X128K2: case V_X256x128K2: case V_X256W8: case V_X128W8: case V_X256x128W8: case V_X192x256W8: case V_X64: case V_X128W8R: case V_X256x128W8R: case V_X256W4: {
       const int xt = x_tile_of(v);
       if (!x_supports(d, v)) {
         pf_set_error("pf_gemm: variant %d needs both operands stored alike and (unless transposed) K a multiple of the stage depth", v);
@@ -877,12 +885,12 @@ extern "C" int pf_gemm_variant(const pf_gemm_desc* desc, char* out, int cap) {
   const char* bt = d.b_trans ? "true" : "false";
   const int v = resolve_variant(d);
   switch (v) {
-    case V_X256: case V_X256x128: case V_X128: case V_X192x256: case V_X128K2: case V_X256x128K2: case V_X256W8: case V_X128W8: case V_X256x128W8: case V_X192x256W8: case V_X64: case V_X128W8R: case V_X256x128W8R: {
+    case V_X256: case V_X256x128: case V_X128: case V_X192x256: case V_X128K2: case V_X256x128K2: case V_X256W8: case V_X128W8: case V_X256x128W8: case V_X192x256W8: case V_X64: case V_X128W8R: case V_X256x128W8R: case V_X256W4: {
       // BM, BN, BK, wavefront rows, columns, reduction split, stages: as rocprofv3 prints the instantiation
       static const char* shapes[PF_XT_COUNT] = {"", "256, 256, 32, 2, 2, 1, 5", "256, 128, 64, 2, 2, 1, 3", "128, 128, 64, 2, 2, 1, 3",
                                                 "192, 256, 32, 2, 2, 1, 5", "128, 128, 64, 2, 2, 2, 3", "256, 128, 64, 2, 2, 2, 3",
                                                 "256, 256, 32, 2, 4, 1, 5", "128, 128, 64, 2, 4, 1, 3", "256, 128, 64, 4, 2, 1, 3",
-                                                "192, 256, 32, 2, 4, 1, 5", "64, 64, 64, 2, 2, 1, 5"};
+                                                "192, 256, 32, 2, 4, 1, 5", "64, 64, 64, 2, 2, 1, 5", "256, 256, 64, 2, 2, 1, 2"};
       if (!x_supports(d, v)) {   // a pinned tile that cannot run this product: say so here, not at launch time
         pf_set_error("pf_gemm_variant: variant %d needs both operands stored alike, K >= %d and (unless both are "
                      "reduction-strided) K a multiple of %d", v, x_tile_bk(x_tile_of(v)), x_tile_bk(x_tile_of(v)));

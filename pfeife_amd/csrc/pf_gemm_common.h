@@ -141,6 +141,10 @@ __device__ __forceinline__ void static_for(F&& f) {
 
 template <int DT> struct Mfma;
 template <> struct Mfma<PF_F16> {
+  // accumulates in place in accumulation registers; hazards with other instructions' accesses to `c` are the caller's
+  static __device__ __forceinline__ void run16_agpr(short __attribute__((ext_vector_type(8))) a, short __attribute__((ext_vector_type(8))) b, float4_t& c) {
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+  }
   static __device__ __forceinline__ float4_t run16(short __attribute__((ext_vector_type(8))) a, short __attribute__((ext_vector_type(8))) b, float4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), c, 0, 0, 0);
   }
@@ -150,6 +154,10 @@ template <> struct Mfma<PF_F16> {
   }
 };
 template <> struct Mfma<PF_BF16> {
+  // accumulates in place in accumulation registers; hazards with other instructions' accesses to `c` are the caller's
+  static __device__ __forceinline__ void run16_agpr(short __attribute__((ext_vector_type(8))) a, short __attribute__((ext_vector_type(8))) b, float4_t& c) {
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+  }
   static __device__ __forceinline__ float4_t run16(short __attribute__((ext_vector_type(8))) a, short __attribute__((ext_vector_type(8))) b, float4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
   }
@@ -186,9 +194,11 @@ __device__ __forceinline__ uint4 buf_load16(__amdgpu_buffer_rsrc_t r, uint32_t b
 //   ids 5, 6: 128x128 and 256x128 with eight wavefronts as TWO 2 x 2 grids that split every tile's reduction depth
 //   between them ("k2")
 //   id 11: 64x64 by four wavefronts, two workgroups to a CU, for small outputs
-//   (ids 1-6 run where a descriptor pins them; the automatic choice takes 7-11, which were faster wherever measured)
+//   id 12: 256x256 (64 deep, 2 stages, 3 of the right-hand operand) by four wavefronts with their accumulators in
+//   accumulation registers: the fastest per tile wherever K is a multiple of 64
+//   (ids 1-6 run where a descriptor pins them; the automatic choice takes 7-12, which were faster wherever measured)
 enum { PF_XT_256x256 = 1, PF_XT_256x128 = 2, PF_XT_128x128 = 3, PF_XT_192x256 = 4, PF_XT_128x128k2 = 5,
-       PF_XT_256x128k2 = 6, PF_XT_256x256w8 = 7, PF_XT_128x128w8 = 8, PF_XT_256x128w8 = 9, PF_XT_192x256w8 = 10, PF_XT_64x64 = 11, PF_XT_COUNT = 12 };
+       PF_XT_256x128k2 = 6, PF_XT_256x256w8 = 7, PF_XT_128x128w8 = 8, PF_XT_256x128w8 = 9, PF_XT_192x256w8 = 10, PF_XT_64x64 = 11, PF_XT_256x256w4 = 12, PF_XT_COUNT = 13 };
 // BM, BN, reduction depth per stage, stages, wavefront grid (rows x columns x reduction split) of each tile id
 template <int XT> struct XTile;
 template <> struct XTile<PF_XT_256x256> { static constexpr int BM = 256, BN = 256, BK = 32, ST = 5, WGM = 2, WGN = 2, KS = 1; };
@@ -201,6 +211,7 @@ template <> struct XTile<PF_XT_256x256w8> { static constexpr int BM = 256, BN = 
 template <> struct XTile<PF_XT_128x128w8> { static constexpr int BM = 128, BN = 128, BK = 64, ST = 3, WGM = 2, WGN = 4, KS = 1; };
 template <> struct XTile<PF_XT_256x128w8> { static constexpr int BM = 256, BN = 128, BK = 64, ST = 3, WGM = 4, WGN = 2, KS = 1; };
 template <> struct XTile<PF_XT_192x256w8> { static constexpr int BM = 192, BN = 256, BK = 32, ST = 5, WGM = 2, WGN = 4, KS = 1; };
+template <> struct XTile<PF_XT_256x256w4> { static constexpr int BM = 256, BN = 256, BK = 64, ST = 2, WGM = 2, WGN = 2, KS = 1; };
 template <> struct XTile<PF_XT_64x64> { static constexpr int BM = 64, BN = 64, BK = 64, ST = 5, WGM = 2, WGN = 2, KS = 1; };
 // tiles with a kernel for row-major products whose reduction length is no multiple of the stage depth: the
 // eight-wavefront 128x128 and 256x128 tiles and 64x64

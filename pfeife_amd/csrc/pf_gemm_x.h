@@ -216,6 +216,24 @@ template <int N> struct Words {
   }
 };
 
+// A 16-row block's accumulators for the epilogue; out of the accumulation registers by hand, where they are used (left
+// to itself the compiler moves all of them at once, and spills)
+template <bool AGPR, int TN> __device__ __forceinline__ void acc_read(float4_t (&x)[TN], const float4_t (&acc)[TN]) {
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    if constexpr (AGPR) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float v;
+        asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(acc[j][r]));
+        x[j][r] = v;
+      }
+    } else {
+      x[j] = acc[j];
+    }
+  }
+}
+
 // `pid`: index of this workgroup among the workgroups of its problem (the launch may hold several
 // problems, see gemm16x_group_kernel)
 template <int DT, int BM, int BN, int BK, int WGM, int WGN, int KS, int ST, bool AT, bool BT, int EC, bool RAG = false>
@@ -243,6 +261,9 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
   // are bound by instruction issue)
   constexpr int NFA = AT ? (TM * TN <= 16 ? TM : 1) : KK, NFB = BT ? (TM * TN <= 16 ? TN : 1) : KK;
   static_assert((!AT || (WM & (WM - 1)) == 0) && (!BT || (WN & (WN - 1)) == 0), "tile_xor");
+  // Two stages (three of the right-hand operand): four wavefronts with 128x128 blocks, one to a SIMD, see below
+  constexpr bool TWO = ST == 2;
+  static_assert(!TWO || (NW == 4 && TM * TN == 64 && KS == 1 && BK == 64 && !RAG), "the two-stage pipeline's tile");
   extern __shared__ __align__(16) uint16_t smem[];
 
   const int t = gemm_tile_id(pid, g.tiles_m * g.tiles_n, g.per_xcd);
@@ -319,7 +340,7 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
   // straight-line code with the same number of loads in flight.
   // The loads of one tile are dealt over the sub-groups of one MFMA group: a burst of them would fill the
   // memory pipeline's queue and stall the wavefront for as long as the tile takes to stream in.
-  static_assert(ST >= 3, "a stage is refilled while the next tile is multiplied");
+  static_assert(ST >= 3 || TWO, "a stage is refilled while the next tile is multiplied");
   auto adv_of = [&](int kt, uint32_t step) { return kt < nk ? (uint32_t)kt * step : 0x80000000u; };
   auto sel_of = [&](int kt) { return RAG && kt == nk - 1 ? 0xffffffffu : 0u; };
   auto issue_all = [&](int kt, uint32_t sb) {
@@ -335,7 +356,7 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
   // Blocks of more than 128 accumulator registers (the four-wavefront 256x256 and 192x256 tiles), and those that exchange
   // half their sums with another wavefront, have no room for two sets of fragments: they read a phase's fragments at its start (SINGLE).
   constexpr int NM = TM * TN;
-  constexpr bool SINGLE = NM > 32 || (KS == 2 && NM == 32);
+  constexpr bool SINGLE = !TWO && (NM > 32 || (KS == 2 && NM == 32));
   constexpr int NREADS = TM * TA::NRD + TN * TB::NRD;
   Frag<AT> fa[SINGLE ? 1 : 2][TM];
   Frag<BT> fb[SINGLE ? 1 : 2][TN];
@@ -400,6 +421,77 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
       __builtin_amdgcn_sched_barrier(0);
     });
   };
+  if constexpr (TWO) {
+    // What bounds the tiles above is the way of the operands, not the matrix pipes: eight 128x64 blocks of a 256x256 tile
+    // read 96 KB of fragments per 32 of depth and 32 KB arrive, together all that the LDS port moves while the MFMAs run, and a
+    // tile step 32 deep takes half of every 128-byte line it requests.  Four wavefronts with 128x128 blocks read a
+    // third less, steps 64 deep request whole lines (half the requests to the L2), and there is one barrier per 128
+    // MFMAs.  One wavefront to a SIMD has the registers for it: 256 accumulators (AGPRs, named in the MFMAs by hand:
+    // the compiler's own choice moves them about inside the loop) and two sets of fragments, so that a phase's reads
+    // run under the phase before.  160 KB are two stages of A and THREE of B: B's tile kt + 2 is requested during
+    // the first phase of tile kt, A's during the second, when the last fragments of tile kt are in registers; at even
+    // spacing, as four wavefronts that all load at once stall each other.  Each load has a tile's time, 2048 cycles, to arrive.
+    // 8192^3 926 -> 775 us (bf16; 1.42 PFLOP/s), [8192 x 5632] . [5632 x 2048] 160 -> 140, 4096 x 4096 over 32768 977 -> 766,
+    // [12608 x 4096] . [4096 x 1024] 111 -> 97, over 1024 30 -> 28 (eight wavefronts -> four, one card).
+    auto mm = [&](auto curc, auto lac, uint32_t ra, uint32_t rb, int ktl, uint32_t dst) {
+      constexpr int cur = decltype(curc)::value, slot = cur ^ 1, kkn = cur ^ 1;
+      constexpr bool LA = decltype(lac)::value;           // this phase requests A's tile (else B's)
+      constexpr int NL = LA ? TA::IPW : TB::IPW, NS = NM * 7 / 8;
+      const uint32_t adv = adv_of(ktl, LA ? step_a : step_b);
+      static_for<NM>([&](auto mc) {
+        constexpr int m = decltype(mc)::value;
+        static_for<NL>([&](auto ec) {
+          constexpr int l = decltype(ec)::value;
+          if constexpr (l * NS / NL == m) {
+            if constexpr (LA) TA::template issue<l, l + 1, false>(rs_a, offa, taila, adv, 0u, dst, wave);
+            else TB::template issue<l, l + 1, false>(rs_b, offb, tailb, adv, 0u, dst, wave);
+          }
+        });
+        static_for<NREADS>([&](auto ec) {
+          constexpr int r = decltype(ec)::value;
+          if constexpr (r * NS / NREADS == m) {
+            if constexpr (r < TN * TB::NRD) TB::template read<NFB, r / TB::NRD, kkn, r % TB::NRD>(fb[slot][r / TB::NRD], rb, fob);
+            else {
+              constexpr int q = r - TN * TB::NRD;
+              TA::template read<NFA, q / TA::NRD, kkn, q % TA::NRD>(fa[slot][q / TA::NRD], ra, foa);
+            }
+          }
+        });
+        if constexpr (AT && BT && m % TN == 0) {   // (as in `phase`)
+          constexpr int need = TN * TB::NRD + (m / TN + 1) * TA::NRD;
+          constexpr int up = ((m + 1) * NREADS + NS - 1) / NS, issued = up < NREADS ? up : NREADS;
+          constexpr int later = NREADS - need + issued;
+          asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(later < 15 ? later : 15) : "memory");
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        constexpr int i = m / TN, j = (i & 1) ? TN - 1 - m % TN : m % TN;
+        Mfma<DT>::run16_agpr(fa[cur][i].get(), fb[cur][j].get(), acc[i][j]);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    };
+    uint32_t a0 = lds0, a1 = lds0 + TA::BYTES, b0 = lds0 + 2 * TA::BYTES, b1 = b0 + TB::BYTES, b2 = b1 + TB::BYTES;
+    TA::template issue<0, TA::IPW, false>(rs_a, offa, taila, adv_of(0, step_a), 0u, a0, wave);
+    TB::template issue<0, TB::IPW, false>(rs_b, offb, tailb, adv_of(0, step_b), 0u, b0, wave);
+    TB::template issue<0, TB::IPW, false>(rs_b, offb, tailb, adv_of(1, step_b), 0u, b1, wave);
+    TA::template issue<0, TA::IPW, false>(rs_a, offa, taila, adv_of(1, step_a), 0u, a1, wave);
+    wait_vm<LPW>();
+    lds_barrier();
+    static_for<TN>([&](auto jc) { TB::template read_first<NFB, decltype(jc)::value>(fb[0][decltype(jc)::value], b0, fob); });
+    static_for<TM>([&](auto ic) { TA::template read_first<NFA, decltype(ic)::value>(fa[0][decltype(ic)::value], a0, foa); });
+    asm volatile("s_nop 7" ::: "memory");   // (the compiler sees no MFMA: the distance to the zeros written to AGPRs is kept by hand)
+    __builtin_amdgcn_sched_barrier(0);
+    int kt = 0;
+    do {
+      mm(std::integral_constant<int, 0>{}, std::false_type{}, a0, b0, kt + 2, b2);
+      wait_vm<TB::IPW>();
+      lds_barrier();       // tile kt + 1 landed everywhere, stage a0 and (since the barrier before) b2 no longer read
+      mm(std::integral_constant<int, 1>{}, std::true_type{}, a1, b1, kt + 2, a0);
+      const uint32_t ta = a0, tb = b0;
+      a0 = a1; a1 = ta;
+      b0 = b1; b1 = b2; b2 = tb;
+    } while (++kt < nk);
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // (and the distance from the last MFMA to the first read of its result)
+  } else {
   // A tile's fragments are in registers at the barrier that opens its last phase: from there on its stage is
   // refilled with the tile ST further on, the first part in that phase, the others in the next tile's
   // phases but its last (one part per phase keeps the stream of loads even).  With one phase per tile the
@@ -460,6 +552,7 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
     }
     if (kt < nk) tile(kt, std::integral_constant<int, 0>{});
   }
+  }
   // The last tile's last phase has read fragments of a tile that does not exist, and nothing
   // consumes them: the reads issued by inline assembly may still be in flight here, and the
   // compiler, which knows nothing of that, would hand their registers to the epilogue's first
@@ -512,10 +605,7 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
       float4_t x[TN];
       static_for<TM>([&](auto hc) {
         constexpr int c = decltype(hc)::value;
-        if (h == c) {
-#pragma unroll
-          for (int j = 0; j < TN; ++j) x[j] = acc[c][j];
-        }
+        if (h == c) acc_read<TWO>(x, acc[c]);
       });
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -583,11 +673,15 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
             if constexpr (HAS_BIAS) v[k] += bias[k];
           }
           // (the plain 16-bit store rounds once, when it packs: rounding to the same format before
-          // that changes nothing)
-          if constexpr (EC != EC_STORE16 && !BT) {
+          // that changes nothing.  The GELU class rounds by packing what it keeps, below.)
+          if constexpr (EC != EC_STORE16 && EC != EC_ACT16 && !BT) {
             if (round_mid) {
 #pragma unroll
-              for (int k = 0; k < GW; ++k) v[k] = Codec<DT>::round(v[k]);
+              for (int k = 0; k < GW; k += 2) {
+                const uint32_t w = pack2<DT>(v[k], v[k + 1]);
+                v[k] = unpack1<DT>(w, 0);
+                v[k + 1] = unpack1<DT>(w, 1);
+              }
             }
           }
           const uint32_t oc = off_c[g] + (h * 16 + (uint32_t)r) * step_c;
@@ -608,6 +702,10 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
 #pragma unroll
               for (int k = 0; k < NV; ++k) o.w[k] = (int)pack2<DT>(v[2 * k], v[2 * k + 1]);
               o.store(rs_x, off_x[g] + (h * 16 + (uint32_t)r) * step_x);
+              if (round_mid) {
+#pragma unroll
+                for (int k = 0; k < GW; ++k) v[k] = unpack1<DT>((uint32_t)o.w[k / 2], k % 2);
+              }
 #pragma unroll
               for (int k = 0; k < GW; ++k) v[k] = pf_gelu_erf(v[k]);
             }
@@ -651,10 +749,7 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
         float4_t x[TN];
         static_for<TM>([&](auto cc) {
           constexpr int c = decltype(cc)::value;
-          if (h == c) {
-#pragma unroll
-            for (int j = 0; j < TN; ++j) x[j] = acc[c][j];
-          }
+          if (h == c) acc_read<TWO>(x, acc[c]);
         });
         block((uint32_t)h, x, old);
 #pragma unroll
@@ -667,7 +762,9 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
       static_for<DEPTH>([&](auto hc) { fetch((uint32_t)decltype(hc)::value, old[decltype(hc)::value]); });
       static_for<TM>([&](auto hc) {
         constexpr int h = decltype(hc)::value;
-        block((uint32_t)h, acc[h], old[h % DEPTH]);
+        float4_t x[TN];
+        acc_read<TWO>(x, acc[h]);
+        block((uint32_t)h, x, old[h % DEPTH]);
         if constexpr (LOADS && h + DEPTH < TM) fetch((uint32_t)(h + DEPTH), old[h % DEPTH]);
         __builtin_amdgcn_sched_barrier(0);   // (left alone, the scheduler starts every block at once and spills)
       });
@@ -744,7 +841,7 @@ int launch16x_t(const pf_gemm_desc& d, const GemmGrid& g, hipStream_t st) {
   constexpr int NT = 64 * WGM * WGN * KS;
   constexpr size_t lds_xch = KS == 2 ? (size_t)BM * BN * 4 : 0;   // one grid's partial sums on their way to the other
   constexpr size_t lds_main = ((size_t)ST * (BM + BN) * BK * 2 > lds_xch) ? (size_t)ST * (BM + BN) * BK * 2 : lds_xch;
-  constexpr size_t lds = lds_main;
+  constexpr size_t lds = lds_main + (ST == 2 ? (size_t)BN * BK * 2 : 0);   // (the third stage of B)
   static_assert(lds <= 160 * 1024, "tile pipeline exceeds the 160 KB of LDS");
   void (*kern)(const pf_gemm_desc, const GemmGrid);
   if constexpr (RAG) kern = gemm16x_ragged_kernel<DT, BM, BN, BK, WGM, WGN, KS, ST, AT, BT, EC>;
@@ -827,7 +924,7 @@ int launch16x_group(const pf_gemm_desc* d, int n, hipStream_t st) {
     constexpr int NT = 64 * WGM * WGN * KS;
     constexpr size_t lds_xch = KS == 2 ? (size_t)BM * BN * 4 : 0;
     constexpr size_t lds_main = ((size_t)ST * (BM + BN) * BK * 2 > lds_xch) ? (size_t)ST * (BM + BN) * BK * 2 : lds_xch;
-    constexpr size_t lds = lds_main;
+    constexpr size_t lds = lds_main + (ST == 2 ? (size_t)BN * BK * 2 : 0);
     GemmGroup ga;
     int blocks = 0;
     for (int i = 0; i < n; ++i) {

@@ -1,0 +1,101 @@
+"""The four-wavefront 256x256 tile of the direct-to-LDS kernel (variant 18) at its edges, against the kernel oracle and,
+bit for bit, against the eight-wavefront tile (variant 7), which adds up in the same order."""
+import pytest
+import torch
+
+from test_kernels_gpu import BF16, F16, F32, TOL, close, rnd
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hip():
+    from pfeife_amd.hip import HipKernels
+
+    return HipKernels(0)
+
+
+@pytest.fixture(scope="module")
+def oracle():
+    from oracle.kernels_oracle import OracleKernels
+
+    return OracleKernels("cpu")
+
+
+def _run(hip, oracle, tensors, outs, variant_name, **kw):
+    cpu = {k: (None if v is None else v.clone()) for k, v in tensors.items()}
+    got = {}
+    for variant in (7, 18):
+        dev = {k: (None if v is None else v.cuda()) for k, v in tensors.items()}
+        launch = hip.gemm(**dev, variant=variant, **kw)
+        if variant == 18:
+            assert launch.variant.endswith(variant_name), launch.variant
+        launch(torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        got[variant] = {o: dev[o].cpu() for o in outs}
+    oracle.gemm(**cpu, **kw)()
+    for o in outs:
+        assert torch.equal(got[7][o], got[18][o]), o
+    return {o: (got[18][o], cpu[o]) for o in outs}
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("M,N,K", [(256, 256, 64), (1, 8, 128), (257, 264, 192), (511, 520, 320), (300, 1160, 2048)])
+def test_row_major_classes(hip, oracle, dtype, M, N, K):
+    """One, two, three stages and more; one tile, ragged tiles, tiles with one row or eight columns."""
+    x, w, bias = rnd((M, K), dtype, 1), rnd((N, K), dtype, 2, 0.1), rnd((N,), dtype, 3)
+    rt, at = TOL[dtype]
+    z16 = lambda: torch.zeros(M, N, dtype=dtype)
+    base = dict(M=M, N=N, K=K, lda=K, ldb=K, ldc=N)
+    cls = lambda ec: "256, 256, 64, 2, 2, 1, 2, false, false, %d>" % ec
+    close(_run(hip, oracle, dict(a=x, b=w, c=z16(), bias=bias), ["c"], cls(0), round_mid=1, **base)["c"], rt, at)
+    close(_run(hip, oracle, dict(a=x, b=w, c=torch.zeros(M, N, dtype=F32), bias=bias), ["c"], cls(1), **base)["c"], 1e-3, 1e-2)
+    r = _run(hip, oracle, dict(a=x, b=w, c=z16(), bias=bias, aux_out=z16()), ["c", "aux_out"], cls(2), round_mid=1, act=1,
+             ld_aux_out=N, **base)
+    close(r["c"], rt, at)
+    close(r["aux_out"], rt, at)
+    close(_run(hip, oracle, dict(a=x, b=w, c=torch.zeros(M, N, dtype=F32), bias=bias, residual=rnd((M, N), F32, 4)), ["c"], cls(3),
+               round_mid=1, ld_res=N, **base)["c"], rt, at)
+    close(_run(hip, oracle, dict(a=x, b=w, c=z16(), aux_in=rnd((M, N), dtype, 6)), ["c"], cls(5), dact=1, ld_aux_in=N, **base)["c"],
+          rt, at * 4)
+    close(_run(hip, oracle, dict(a=x, b=w, c=rnd((M, N), dtype, 7)), ["c"], cls(6), beta=1, **base)["c"], rt, at * 2)
+    close(_run(hip, oracle, dict(a=x, b=w, c=z16(), bias=bias, residual=rnd((M, N + 8), dtype, 8)), ["c"], cls(7), round_mid=1,
+               ld_res=N + 8, **base)["c"], rt, at * 2)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("M,N,K", [(256, 256, 64), (264, 520, 72), (304, 256, 1021), (512, 8, 200)])
+def test_weight_gradients(hip, oracle, dtype, M, N, K):
+    """Both operands reduction-strided; depths that are no multiple of a stage."""
+    a, b = rnd((K, M), dtype, 1), rnd((K, N), dtype, 2)
+    for beta, ec in ((0, 1), (1, 4)):
+        r = _run(hip, oracle, dict(a=a, b=b, c=rnd((M, N), F32, 3)), ["c"], "true, true, %d>" % ec, M=M, N=N, K=K, lda=M, ldb=N,
+                 ldc=N, a_trans=1, b_trans=1, beta=beta)
+        close(r["c"], 1e-4, 2e-3)
+
+
+def test_column_sums(hip):
+    """GELU' with the column sums of what is stored, as partial rows: equal to sums over the stored values."""
+    M, N, K = 700, 520, 128
+    dy, w, h = rnd((M, K), BF16, 1).cuda(), rnd((N, K), BF16, 2, 0.1).cuda(), rnd((M, N), BF16, 3).cuda()
+    c = torch.zeros(M, N, dtype=BF16, device="cuda")
+    launch = hip.gemm(dy, w, c, M=M, N=N, K=K, lda=K, ldb=K, ldc=N, dact=1, aux_in=h, ld_aux_in=N, variant=18)
+    ws, _, nb, _ = hip.gemm_attach_colsum(launch, lambda shape, dtype: torch.full(shape, float("nan"), dtype=dtype, device="cuda"))
+    launch(torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    want = c.double().sum(0)
+    # (fp32 sums of at most 256 values each)
+    assert nb == 3 and float((ws.double().sum(0) - want).abs().max()) <= 256 * 2.0 ** -24 * float(c.double().abs().sum(0).max())
+
+
+def test_automatic_choice(hip):
+    """Long rows in whole rounds take the tile; depths that are no multiple of 64, small outputs and weight gradients do not."""
+    def name(M, N, K, t=0):
+        a = torch.empty(K if t else M, M if t else K, dtype=BF16, device="cuda")
+        b = torch.empty(K if t else N, N if t else K, dtype=BF16, device="cuda")
+        c = torch.empty(M, N, dtype=F32 if t else BF16, device="cuda")
+        return hip.gemm(a, b, c, M=M, N=N, K=K, lda=a.shape[1], ldb=b.shape[1], ldc=N, a_trans=t, b_trans=t).variant
+
+    w4 = "256, 256, 64, 2, 2, 1, 2"
+    assert w4 in name(8192, 2048, 2048) and w4 in name(12608, 1024, 4096)
+    assert w4 not in name(8192, 2048, 2048 + 32) and w4 not in name(788, 384, 1536) and w4 not in name(2048, 2048, 8192, 1)
