@@ -626,6 +626,117 @@ __global__ __launch_bounds__(256) void groupnorm_bwd_apply_kernel(const void* dy
   }
 }
 
+// Rows of 513 to 2048 columns, dtypes known: NWV wavefronts (a team) share a row, eight columns to a lane, TEAMS rows
+// to a workgroup at a time.  A wavefront that owns a whole row of 2048 holds 32 columns in each of ten operands and sums, more
+// registers than leave a second wavefront on its SIMD, and then waits out every memory round trip (measured: 143 MB
+// in 58 us).  Here a lane keeps 8 columns of everything, four wavefronts fit a SIMD, and the next row is on its way
+// while this one is reduced.  Two sums per row cross the team through LDS, one barrier per row (two slots in turn).
+// The column sums of a lane's columns need no other lane but those of the other teams.
+template <int NWV, int TEAMS, int IODT, int LPDT, int DYDT>
+__global__ __launch_bounds__(64 * NWV * TEAMS, 4) void norm_bwd_team_kernel(
+    const void* dy, const void* x, const float* gamma, const float* mean, const float* rstd, const void* dx_add, void* dx,
+    float* ws, int64_t rows, int64_t d, int rms, int want_wgrad, void* dx_lp, int want_colsum) {
+  constexpr int W = 8;
+  __shared__ float part[2][TEAMS][NWV][2];
+  __shared__ __align__(16) float red[TEAMS > 1 ? (TEAMS - 1) * NWV * 64 * W : 1];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int team = wave / NWV, tw = wave % NWV;
+  const int64_t c = (int64_t)(tw * 64 + lane) * W;
+  const bool ok = c < d, has_add = dx_add != nullptr;
+  const int64_t col = ok ? c : 0;
+  float g[W], pg[W], pb[W], ps[W];
+  ld_vec_c<W, PF_F32>(gamma, col, PF_F32, g);
+#pragma unroll
+  for (int k = 0; k < W; ++k) pg[k] = pb[k] = ps[k] = 0.f;
+  const int64_t stride = (int64_t)gridDim.x * TEAMS;
+  float ndy[W], nx[W], nadd[W], nmu, nrs;
+  auto fetch = [&](int64_t r) {
+    const int64_t rr = r < rows ? r : rows - 1;
+    ld_vec_c<W, DYDT>(dy, rr * d + col, DYDT, ndy);
+    ld_vec_c<W, IODT>(x, rr * d + col, IODT, nx);
+    if (has_add) ld_vec_c<W, IODT>(dx_add, rr * d + col, IODT, nadd);
+    nmu = rms ? 0.f : mean[rr];
+    nrs = rstd[rr];
+  };
+  int64_t row = (int64_t)blockIdx.x * TEAMS + team;
+  fetch(row);
+  int slot = 0;
+  // (the same number of rounds for every team: a team without a row takes part in the barriers only)
+  for (int64_t first = (int64_t)blockIdx.x * TEAMS; first < rows; first += stride, row += stride, slot ^= 1) {
+    const bool mine = row < rows && ok;
+    const float mu = nmu, rs = nrs;
+    float gg[W], xh[W], cdy[W], cadd[W];
+    float c1 = 0.f, c2 = 0.f;
+#pragma unroll
+    for (int k = 0; k < W; ++k) {
+      cdy[k] = mine ? ndy[k] : 0.f;
+      cadd[k] = has_add ? nadd[k] : 0.f;
+      gg[k] = cdy[k] * g[k];
+      xh[k] = mine ? (nx[k] - mu) * rs : 0.f;
+      c1 += gg[k];
+      c2 += gg[k] * xh[k];
+    }
+    fetch(row + stride);
+    c1 = rms ? 0.f : pf_wave_sum(c1);
+    c2 = pf_wave_sum(c2);
+    if (lane == 0) {
+      part[slot][team][tw][0] = c1;
+      part[slot][team][tw][1] = c2;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // (LDS only: the next row's loads stay in flight)
+    c1 = c2 = 0.f;
+#pragma unroll
+    for (int w = 0; w < NWV; ++w) {
+      c1 += part[slot][team][w][0];
+      c2 += part[slot][team][w][1];
+    }
+    c1 /= (float)d;
+    c2 /= (float)d;
+    if (mine) {
+      float o[W];
+#pragma unroll
+      for (int k = 0; k < W; ++k) {
+        o[k] = rs * (gg[k] - c1 - xh[k] * c2) + cadd[k];
+        pg[k] += cdy[k] * xh[k];
+        pb[k] += cdy[k];
+      }
+      st_vec_c<W, IODT>(dx, row * d + c, IODT, o);
+      if (dx_lp) {
+        st_vec_c<W, LPDT>(dx_lp, row * d + c, LPDT, o);
+        if (want_colsum) {
+#pragma unroll
+          for (int k = 0; k < W; ++k) ps[k] += pf_round_to(LPDT, o[k]);
+        }
+      }
+    }
+  }
+  // one partial row of each kind per workgroup: ws [gridDim.x][2 or 3][d]
+  const int nrows = want_colsum ? 3 : 2;
+  float* wrow = ws + (int64_t)blockIdx.x * nrows * d;
+#pragma unroll
+  for (int which = 0; which < 3; ++which) {
+    if (which < 2 ? !want_wgrad : !want_colsum) continue;   // uniform over the block
+    float s[W];
+#pragma unroll
+    for (int k = 0; k < W; ++k) s[k] = which == 0 ? pg[k] : (which == 1 ? pb[k] : ps[k]);
+    if constexpr (TEAMS > 1) {
+      __syncthreads();
+      if (team > 0) {
+#pragma unroll
+        for (int k = 0; k < W; ++k) red[(((team - 1) * NWV + tw) * W + k) * 64 + lane] = s[k];
+      }
+      __syncthreads();
+      if (team == 0) {
+#pragma unroll
+        for (int q = 0; q < TEAMS - 1; ++q)
+#pragma unroll
+          for (int k = 0; k < W; ++k) s[k] += red[((q * NWV + tw) * W + k) * 64 + lane];
+      }
+    }
+    if (team == 0 && ok) st_vec_c<W, PF_F32>(wrow, which * d + c, PF_F32, s);
+  }
+}
+
 inline int64_t colsum_chunks(int64_t rows) {
   int64_t chunks = (rows + 31) / 32;
   if (chunks > 256) chunks = 256;
@@ -718,6 +829,17 @@ int norm_bwd(const void* dy, int dy_dt, const void* x, int x_dt, const float* ga
 #define PF_NBI(NV, IO, LP, DY)                                                                                       \
   hipLaunchKernelGGL((norm_bwd_kernel<8, NV, IO, LP, DY>), dim3(blocks), dim3(256), 0, st, dy, dy_dt, x, x_dt, gamma, \
                      mean, rstd, dx_add, add_dt, dx, dx_dt, ws, rows, d, rms, want, dx_lp, lp_dt, want_colsum)
+#define PF_NBT(NWV, TEAMS, IO, LP, DY)                                                                                       \
+  hipLaunchKernelGGL((norm_bwd_team_kernel<NWV, TEAMS, IO, LP, DY>), dim3(blocks), dim3(64 * NWV * TEAMS), 0, st, dy, x, gamma, mean, \
+                     rstd, dx_add, dx, ws, rows, d, rms, want, dx_lp, want_colsum)
+#define PF_NBTD(NWV, TEAMS, ELSE)                                                           \
+  if (io32 && dy_dt == PF_F16 && (!dx_lp || lp_dt == PF_F16)) PF_NBT(NWV, TEAMS, PF_F32, PF_F16, PF_F16);    \
+  else if (io32 && dy_dt == PF_BF16 && (!dx_lp || lp_dt == PF_BF16)) PF_NBT(NWV, TEAMS, PF_F32, PF_BF16, PF_BF16); \
+  else if (io32 && dy_dt == PF_F32 && (!dx_lp || lp_dt == PF_F16)) PF_NBT(NWV, TEAMS, PF_F32, PF_F16, PF_F32);    \
+  else if (io32 && dy_dt == PF_F32 && lp_dt == PF_BF16) PF_NBT(NWV, TEAMS, PF_F32, PF_BF16, PF_F32);         \
+  else if (io16 && x_dt == PF_F16) PF_NBT(NWV, TEAMS, PF_F16, PF_F16, PF_F16);               \
+  else if (io16 && x_dt == PF_BF16) PF_NBT(NWV, TEAMS, PF_BF16, PF_BF16, PF_BF16);           \
+  else ELSE
 #define PF_NBD(NV)                                                                          \
   if (io32 && dy_dt == PF_F16 && (!dx_lp || lp_dt == PF_F16)) PF_NBC(NV, PF_F16, PF_F16);    \
   else if (io32 && dy_dt == PF_BF16 && (!dx_lp || lp_dt == PF_BF16)) PF_NBC(NV, PF_BF16, PF_BF16); \
@@ -727,9 +849,10 @@ int norm_bwd(const void* dy, int dy_dt, const void* x, int x_dt, const float* ga
   else if (io16 && x_dt == PF_BF16) PF_NBI(NV, PF_BF16, PF_BF16, PF_BF16);                   \
   else PF_NB(8, NV)
   if (v) {
-    if (d <= 64 * 8 * 2) { PF_NBD(2); }
-    else if (d <= 64 * 8 * 3) { PF_NBD(3); }
-    else if (d <= 64 * 8 * 4) { PF_NBD(4); }
+    if (d <= 64 * 8) { PF_NBD(2); }
+    else if (d <= 64 * 8 * 2) { PF_NBTD(2, 4, PF_NB(8, 2)); }
+    else if (d <= 64 * 8 * 3) { PF_NBTD(3, 2, PF_NB(8, 3)); }
+    else if (d <= 64 * 8 * 4) { PF_NBTD(4, 2, PF_NB(8, 4)); }
     else if (d <= 64 * 8 * 8) PF_NB(8, 8);
     else if (d <= 64 * 8 * 16) PF_NB(8, 16);
     else { pf_set_error("%s: d=%lld exceeds 8192", name, (long long)d); return PF_ERR_UNSUPPORTED; }
@@ -739,6 +862,8 @@ int norm_bwd(const void* dy, int dy_dt, const void* x, int x_dt, const float* ga
     else { pf_set_error("%s: unaligned d=%lld exceeds 4096", name, (long long)d); return PF_ERR_UNSUPPORTED; }
   }
 #undef PF_NBD
+#undef PF_NBTD
+#undef PF_NBT
 #undef PF_NBC
 #undef PF_NBI
 #undef PF_NB
