@@ -629,12 +629,13 @@ bool x_supports(const pf_gemm_desc& d, int v) {
 }
 
 // Automatic choice: a cost model fitted to measurements on MI355X (microseconds; a sweep of 162 row-major shapes, 256 to
-// 16384 rows and 256 to 10240 columns, and 21 reduction-strided ones).  A workgroup's fixed cost (dispatch, first tile, epilogue)
+// 16384 rows and 256 to 10240 columns, and 118 reduction-strided ones).  A workgroup's fixed cost (dispatch, first tile, epilogue)
 // plus, per round of 256 workgroups, K / 64 tile steps and an epilogue that nothing hides; a step gets slower the more CUs
 // stream operands at the same time, so a step costs t0 in an empty device and t0 + t1 in a full one.  The 64x64 tile
 // runs two workgroups to a CU and its cost grows with their number.  On the row-major sweep the choice is on average
 // 0.4 % off the fastest tile, 16 % at most (8192 x 1280 over 5120: 117.6 on 192x256 against 101.1 us); the constants and tiles
-// before the four-wavefront 256x256 tile were 2.9 % and 23 % off.
+// before the four-wavefront 256x256 tile were 2.9 % and 23 % off.  Among the tiles of 128 rows and more the reduction-strided
+// choice is 0.1 % off, 5 % at most; before that refit 4.9 % and 43 % (6144 x 1408 over 32768: 873 us on 256x128, 609 on 256x256).
 // (The tiles whose eight wavefronts split every tile step's depth, variants 5 and 6, are no candidates: inside a
 // pipeline step, next to other streams' kernels, they lost what they gain alone.)
 int choose_variant(const pf_gemm_desc& d) {
@@ -648,9 +649,10 @@ int choose_variant(const pf_gemm_desc& d) {
                              {V_X256x128W8R, 256, 128, 5.1, 0.49, 0.34, 4.4},   // (ragged K: only where the two above cannot)
                              {V_X128W8R, 128, 128, 3.7, 0.305, 0.18, 2.2},
                              {V_X64, 64, 64, 3.2, 0.165, 0.0, 0.73}};
-  static const Cand tt[4] = {{V_X256W8, 256, 256, 6.9, 1.10, 0.55, 3.5},
-                             {V_X256x128W8, 256, 128, 4.8, 0.58, 0.20, 2.0},
-                             {V_X128W8, 128, 128, 3.7, 0.37, 0.17, 1.0},
+  static const Cand tt[5] = {{V_X256W4, 256, 256, 12.5, 1.09, 0.41, 28.0},
+                             {V_X256W8, 256, 256, 12.7, 1.04, 0.49, 32.5},
+                             {V_X256x128W8, 256, 128, 7.2, 0.573, 0.30, 11.7},
+                             {V_X128W8, 128, 128, 5.1, 0.354, 0.216, 5.4},
                              {V_X64, 64, 64, 3.0, 0.20, 0.0, 0.6}};
   const bool strided = d.a_trans && d.b_trans;
   // A weight gradient rarely runs alone: the lowering puts several into one launch once it knows how many
@@ -658,11 +660,14 @@ int choose_variant(const pf_gemm_desc& d) {
   const int64_t t64 = ((d.M + 63) / 64) * ((d.N + 63) / 64) * nb;
   int best = -1;
   double best_t = 0;
-  for (int i = 0; i < (strided ? 4 : 8); ++i) {
+  for (int i = 0; i < (strided ? 5 : 8); ++i) {
     const Cand& c = strided ? tt[i] : nn[i];
     if (!x_supports(d, c.v)) continue;
     if (strided && c.v == V_X64 && t64 > 160) continue;
     const int64_t tiles = ((d.M + c.bm - 1) / c.bm) * ((d.N + c.bn - 1) / c.bn) * nb;
+    // (four wavefronts: the transposing reads move half as much per cycle and bound both 256x256 tiles; over several rounds
+    // four are ahead, 5632 x 2048 over 32768 671 / 646 us, 32000 x 2048 over 788 183 / 170, in one round 4096 x 1024 over 12608 240 / 249)
+    if (strided && c.v == V_X256W4 && tiles <= 256) continue;
     // One round over a short depth whose epilogue is GELU's arithmetic: the four wavefronts gain over the depth what their
     // longer epilogue costs.  us on eight / four wavefronts, fp16, GELU and GELU': [3072 x 768] . [768 x 4096] 29.9 / 30.4, 34.2 /
     // 33.7; [4096 x 1024] . [1024 x 3152] 35.2 / 35.2, 39.7 / 38.9; over 2048 55.9 / 54.5, 60.6 / 57.8
