@@ -638,52 +638,98 @@ bool x_supports(const pf_gemm_desc& d, int v) {
 // choice is 0.1 % off, 5 % at most; before that refit 4.9 % and 43 % (6144 x 1408 over 32768: 873 us on 256x128, 609 on 256x256).
 // (The tiles whose eight wavefronts split every tile step's depth, variants 5 and 6, are no candidates: inside a
 // pipeline step, next to other streams' kernels, they lost what they gain alone.)
-int choose_variant(const pf_gemm_desc& d) {
+struct TileCost { int v, bm, bn; double fixed, t0, t1, again; };
+constexpr TileCost ROW_MAJOR[] = {{V_X256W4, 256, 256, 6.7, 0.95, 0.43, 6.3},
+                                  {V_X256W8, 256, 256, 6.5, 0.95, 0.64, 6.2},
+                                  {V_X192x256W8, 192, 256, 5.6, 0.78, 0.47, 5.8},
+                                  {V_X256x128W8, 256, 128, 4.9, 0.47, 0.33, 4.4},
+                                  {V_X128W8, 128, 128, 3.6, 0.295, 0.176, 2.2},
+                                  {V_X256x128W8R, 256, 128, 5.1, 0.49, 0.34, 4.4},   // (ragged K: only where the two above cannot)
+                                  {V_X128W8R, 128, 128, 3.7, 0.305, 0.18, 2.2},
+                                  {V_X64, 64, 64, 3.2, 0.165, 0.0, 0.73}};
+constexpr TileCost STRIDED[] = {{V_X256W4, 256, 256, 12.5, 1.09, 0.41, 28.0},
+                                {V_X256W8, 256, 256, 12.7, 1.04, 0.49, 32.5},
+                                {V_X256x128W8, 256, 128, 7.2, 0.573, 0.30, 11.7},
+                                {V_X128W8, 128, 128, 5.1, 0.354, 0.216, 5.4},
+                                {V_X64, 64, 64, 3.0, 0.20, 0.0, 0.6}};
+
+double tile_cost(const TileCost& c, int64_t tiles, int64_t K, bool strided) {
+  const int64_t full = tiles / 256, rest = tiles % 256;
+  double step;
+  if (c.v == V_X64) {
+    step = strided ? 0.05 + 0.19 * (double)tiles / 256.0 : 0.08 + 0.171 * (double)tiles / 256.0;
+    if (step < c.t0) step = c.t0;
+  } else {
+    step = (double)full * (c.t0 + c.t1) + (rest ? c.t0 + c.t1 * (double)rest / 256.0 : 0.0);
+  }
+  return c.fixed + (double)K / 64.0 * step + c.again * (double)(full - (rest ? 0 : 1));
+}
+
+// The cheapest tile for `M` rows of the product (-1: none), among tiles of `bm` rows unless 0
+int choose_tile(const pf_gemm_desc& d, int64_t M, int bm, double& best_t) {
   const int64_t nb = d.batch1 * d.batch2;
-  struct Cand { int v, bm, bn; double fixed, t0, t1, again; };
-  static const Cand nn[8] = {{V_X256W4, 256, 256, 6.7, 0.95, 0.43, 6.3},
-                             {V_X256W8, 256, 256, 6.5, 0.95, 0.64, 6.2},
-                             {V_X192x256W8, 192, 256, 5.6, 0.78, 0.47, 5.8},
-                             {V_X256x128W8, 256, 128, 4.9, 0.47, 0.33, 4.4},
-                             {V_X128W8, 128, 128, 3.6, 0.295, 0.176, 2.2},
-                             {V_X256x128W8R, 256, 128, 5.1, 0.49, 0.34, 4.4},   // (ragged K: only where the two above cannot)
-                             {V_X128W8R, 128, 128, 3.7, 0.305, 0.18, 2.2},
-                             {V_X64, 64, 64, 3.2, 0.165, 0.0, 0.73}};
-  static const Cand tt[5] = {{V_X256W4, 256, 256, 12.5, 1.09, 0.41, 28.0},
-                             {V_X256W8, 256, 256, 12.7, 1.04, 0.49, 32.5},
-                             {V_X256x128W8, 256, 128, 7.2, 0.573, 0.30, 11.7},
-                             {V_X128W8, 128, 128, 5.1, 0.354, 0.216, 5.4},
-                             {V_X64, 64, 64, 3.0, 0.20, 0.0, 0.6}};
   const bool strided = d.a_trans && d.b_trans;
   // A weight gradient rarely runs alone: the lowering puts several into one launch once it knows how many
   // there are, and then the larger tile moves half the bytes.  Alone, 64x64 pays while it fills less than the device.
-  const int64_t t64 = ((d.M + 63) / 64) * ((d.N + 63) / 64) * nb;
+  const int64_t t64 = ((M + 63) / 64) * ((d.N + 63) / 64) * nb;
   int best = -1;
-  double best_t = 0;
-  for (int i = 0; i < (strided ? 5 : 8); ++i) {
-    const Cand& c = strided ? tt[i] : nn[i];
-    if (!x_supports(d, c.v)) continue;
-    if (strided && c.v == V_X64 && t64 > 160) continue;
-    const int64_t tiles = ((d.M + c.bm - 1) / c.bm) * ((d.N + c.bn - 1) / c.bn) * nb;
+  auto consider = [&](const TileCost& c) {
+    if (!x_supports(d, c.v) || (bm != 0 && c.bm != bm)) return;
+    if (strided && c.v == V_X64 && t64 > 160) return;
+    const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((d.N + c.bn - 1) / c.bn) * nb;
     // (four wavefronts: the transposing reads move half as much per cycle and bound both 256x256 tiles; over several rounds
     // four are ahead, 5632 x 2048 over 32768 671 / 646 us, 32000 x 2048 over 788 183 / 170, in one round 4096 x 1024 over 12608 240 / 249)
-    if (strided && c.v == V_X256W4 && tiles <= 256) continue;
+    if (strided && c.v == V_X256W4 && tiles <= 256) return;
     // One round over a short depth whose epilogue is GELU's arithmetic: the four wavefronts gain over the depth what their
     // longer epilogue costs.  us on eight / four wavefronts, fp16, GELU and GELU': [3072 x 768] . [768 x 4096] 29.9 / 30.4, 34.2 /
     // 33.7; [4096 x 1024] . [1024 x 3152] 35.2 / 35.2, 39.7 / 38.9; over 2048 55.9 / 54.5, 60.6 / 57.8
-    if (c.v == V_X256W4 && tiles <= 256 && d.K <= 1024 && (d.act != PF_ACT_NONE || d.dact != PF_ACT_NONE)) continue;
-    const int64_t full = tiles / 256, rest = tiles % 256;
-    double step;
-    if (c.v == V_X64) {
-      step = strided ? 0.05 + 0.19 * (double)tiles / 256.0 : 0.08 + 0.171 * (double)tiles / 256.0;
-      if (step < c.t0) step = c.t0;
-    } else {
-      step = (double)full * (c.t0 + c.t1) + (rest ? c.t0 + c.t1 * (double)rest / 256.0 : 0.0);
-    }
-    const double t = c.fixed + (double)d.K / 64.0 * step + c.again * (double)(full - (rest ? 0 : 1));
+    if (c.v == V_X256W4 && tiles <= 256 && d.K <= 1024 && (d.act != PF_ACT_NONE || d.dact != PF_ACT_NONE)) return;
+    const double t = tile_cost(c, tiles, d.K, strided);
     if (best < 0 || t < best_t) { best = c.v; best_t = t; }
+  };
+  if (strided) for (const TileCost& c : STRIDED) consider(c);
+  else for (const TileCost& c : ROW_MAJOR) consider(c);
+  return best;
+}
+
+int choose_variant(const pf_gemm_desc& d) {
+  double t = 0;
+  const int v = choose_tile(d, d.M, 0, t);
+  return v < 0 ? choose_staged(d) : v;
+}
+
+// Row-major products in two launches: the rows that fill whole rounds of 256 workgroups on one tile, and the rest on the
+// tile that suits what is left.  A round of large tiles costs the same however few of them it holds (12336 x 1408: 294
+// tiles of 256x256, the last 38 in a round of their own; the next smaller tile moves half again as many bytes).  Each row's sums
+// are those of either tile, bit for bit.
+int remap_variant(const pf_gemm_desc& d, int v);
+struct Split { int64_t rows; int v1, v2; };   // rows of the first launch, its tile, the second's
+bool plan_split(const pf_gemm_desc& d, Split& s) {
+  if (d.variant != V_AUTO || d.in_dtype == PF_F32 || d.a_trans || d.b_trans || d.batch1 * d.batch2 != 1) return false;
+  double single = 0;
+  if (choose_tile(d, d.M, 0, single) < 0) return false;
+  double best_t = 0.96 * single - 0.5;   // (less is within the model's error and a launch's)
+  bool found = false;
+  for (const TileCost& c : ROW_MAJOR) {
+    if (c.v == V_X64 || !x_supports(d, c.v)) continue;
+    const int64_t tn = (d.N + c.bn - 1) / c.bn;
+    for (int64_t round = 1;; ++round) {
+      const int64_t blocks = 256 * round / tn, rows = blocks * c.bm;
+      if (rows >= d.M) break;
+      if (rows == 0) continue;
+      const double t1 = tile_cost(c, blocks * tn, d.K, false);
+      if (t1 >= best_t) break;
+      // (column sums leave one partial row per tile row: both tiles of one height)
+      double t2 = 0;
+      const int v2 = choose_tile(d, d.M - rows, d.dact != PF_ACT_NONE ? c.bm : 0, t2);
+      if (v2 >= 0 && t1 + t2 < best_t) {
+        best_t = t1 + t2;
+        s = {rows, c.v, v2};
+        found = true;
+      }
+    }
   }
-  return best < 0 ? choose_staged(d) : best;
+  return found && remap_variant(d, s.v1) == s.v1;
 }
 
 // PF_GEMM_TILE_MAP="3:5,1:6": the automatic choice's tile 3 runs as tile 5, tile 1 as tile 6 (where the
@@ -706,10 +752,32 @@ int remap_variant(const pf_gemm_desc& d, int v) {
   return (w != v && x_supports(d, w)) ? w : v;
 }
 
-int resolve_variant(const pf_gemm_desc& d) { return d.variant == V_AUTO ? remap_variant(d, choose_variant(d)) : d.variant; }
+// (a product in two launches: the first one's)
+int resolve_variant(const pf_gemm_desc& d) {
+  Split s;
+  return d.variant != V_AUTO ? d.variant : remap_variant(d, plan_split(d, s) ? s.v1 : choose_variant(d));
+}
 
 template <int DT>
 int dispatch16(const pf_gemm_desc& d, hipStream_t st) {
+  Split sp;
+  if (plan_split(d, sp)) {
+    pf_gemm_desc part = d;
+    part.M = sp.rows;
+    part.variant = sp.v1;
+    const int rc = dispatch16<DT>(part, st);
+    if (rc != PF_OK) return rc;
+    auto below = [&](const void* p, int64_t ld, int64_t size) { return p == nullptr ? nullptr : (char*)p + sp.rows * ld * size; };
+    part.M = d.M - sp.rows;
+    part.variant = sp.v2;
+    part.A = below(d.A, d.lda, 2);
+    part.C = below(d.C, d.ldc, d.c_dtype == PF_F32 ? 4 : 2);
+    part.aux_out = below(d.aux_out, d.ld_aux_out, 2);
+    part.aux_in = below(d.aux_in, d.ld_aux_in, 2);
+    part.residual = below(d.residual, d.ld_res, d.res_dtype == PF_F32 ? 4 : 2);
+    if (d.colsum_ws) part.colsum_ws = d.colsum_ws + sp.rows / x_tile_bm(x_tile_of(sp.v1)) * d.N;
+    return dispatch16<DT>(part, st);
+  }
   const int v = resolve_variant(d);
   if (d.colsum_ws != nullptr) {   // only the GELU' class of the direct-to-LDS kernel sums its columns
     if (!is_x_variant(v) || d.a_trans || d.b_trans || !x_supports(d, v) ||

@@ -99,3 +99,38 @@ def test_automatic_choice(hip):
     w4 = "256, 256, 64, 2, 2, 1, 2"
     assert w4 in name(8192, 2048, 2048) and w4 in name(12608, 1024, 4096)
     assert w4 not in name(8192, 2048, 2048 + 32) and w4 not in name(788, 384, 1536) and w4 not in name(2048, 2048, 8192, 1)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("M,N,K", [(12336, 1408, 256), (6000, 3072, 192), (8200, 4096, 128), (20001, 1024, 128)])
+def test_products_in_two_launches(hip, dtype, M, N, K):
+    """Rows past the last whole round of large tiles go to a launch of their own: the bits of one launch, for every operand
+    that has a row of its own, with row strides wider than N; the column sums to fp32 sums in another order."""
+    x, w, bias = rnd((M, K), dtype, 1).cuda(), rnd((N, K), dtype, 2, 0.1).cuda(), rnd((N,), dtype, 3).cuda()
+    s = torch.cuda.current_stream().cuda_stream
+    wide = lambda dt, seed: rnd((M, N + 8), dt, seed).cuda()
+    for kind in ("store", "act", "res32", "acc16", "dact"):
+        got = []
+        for variant in (0, 9):
+            c = wide(F32 if kind == "res32" else dtype, 4)
+            aux, ws = wide(dtype, 5), None
+            kw = dict(M=M, N=N, K=K, lda=K, ldb=K, ldc=N + 8, round_mid=1, variant=variant)
+            if kind == "act":
+                kw.update(act=1, aux_out=aux, ld_aux_out=N + 8)
+            elif kind == "dact":
+                kw.update(dact=1, aux_in=aux, ld_aux_in=N + 8)
+            elif kind == "res32":
+                kw.update(residual=wide(F32, 6), ld_res=N + 8)
+            elif kind == "acc16":
+                kw.update(beta=1)
+            launch = hip.gemm(x, w, c, bias=None if kind in ("dact", "acc16") else bias, **kw)
+            if kind == "dact":
+                ws = hip.gemm_attach_colsum(launch, lambda shape, dt: torch.full(shape, float("nan"), dtype=dt, device="cuda"))[0]
+            launch(s)
+            torch.cuda.synchronize()
+            got.append((c, aux, ws))
+        (c0, a0, w0), (c1, a1, w1) = got
+        assert torch.equal(c0, c1) and torch.equal(a0, a1), kind
+        if w0 is not None:
+            want = c0[:, :N].double().sum(0)
+            assert float((w0.double().sum(0) - want).abs().max()) <= 256 * 2.0 ** -24 * float(c0[:, :N].double().abs().sum(0).max())
