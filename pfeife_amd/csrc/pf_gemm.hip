@@ -636,6 +636,7 @@ bool x_supports(const pf_gemm_desc& d, int v) {
 // 0.4 % off the fastest tile, 16 % at most (8192 x 1280 over 5120: 117.6 on 192x256 against 101.1 us); the constants and tiles
 // before the four-wavefront 256x256 tile were 2.9 % and 23 % off.  Among the tiles of 128 rows and more the reduction-strided
 // choice is 0.1 % off, 5 % at most; before that refit 4.9 % and 43 % (6144 x 1408 over 32768: 873 us on 256x128, 609 on 256x256).
+// (Four wavefronts are ahead of eight at every reduction-strided size measured, by 1 to 8 %; eight stay for depths below 64.)
 // (The tiles whose eight wavefronts split every tile step's depth, variants 5 and 6, are no candidates: inside a
 // pipeline step, next to other streams' kernels, they lost what they gain alone.)
 struct TileCost { int v, bm, bn; double fixed, t0, t1, again; };
@@ -647,7 +648,7 @@ constexpr TileCost ROW_MAJOR[] = {{V_X256W4, 256, 256, 6.7, 0.95, 0.43, 6.3},
                                   {V_X256x128W8R, 256, 128, 5.1, 0.49, 0.34, 4.4},   // (ragged K: only where the two above cannot)
                                   {V_X128W8R, 128, 128, 3.7, 0.305, 0.18, 2.2},
                                   {V_X64, 64, 64, 3.2, 0.165, 0.0, 0.73}};
-constexpr TileCost STRIDED[] = {{V_X256W4, 256, 256, 12.5, 1.09, 0.41, 28.0},
+constexpr TileCost STRIDED[] = {{V_X256W4, 256, 256, 12.5, 0.98, 0.47, 28.0},
                                 {V_X256W8, 256, 256, 12.7, 1.04, 0.49, 32.5},
                                 {V_X256x128W8, 256, 128, 7.2, 0.573, 0.30, 11.7},
                                 {V_X128W8, 128, 128, 5.1, 0.354, 0.216, 5.4},
@@ -677,9 +678,6 @@ int choose_tile(const pf_gemm_desc& d, int64_t M, int bm, double& best_t) {
     if (!x_supports(d, c.v) || (bm != 0 && c.bm != bm)) return;
     if (strided && c.v == V_X64 && t64 > 160) return;
     const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((d.N + c.bn - 1) / c.bn) * nb;
-    // (four wavefronts: the transposing reads move half as much per cycle and bound both 256x256 tiles; over several rounds
-    // four are ahead, 5632 x 2048 over 32768 671 / 646 us, 32000 x 2048 over 788 183 / 170, in one round 4096 x 1024 over 12608 240 / 249)
-    if (strided && c.v == V_X256W4 && tiles <= 256) return;
     // One round over a short depth whose epilogue is GELU's arithmetic: the four wavefronts gain over the depth what their
     // longer epilogue costs.  us on eight / four wavefronts, fp16, GELU and GELU': [3072 x 768] . [768 x 4096] 29.9 / 30.4, 34.2 /
     // 33.7; [4096 x 1024] . [1024 x 3152] 35.2 / 35.2, 39.7 / 38.9; over 2048 55.9 / 54.5, 60.6 / 57.8

@@ -306,8 +306,12 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
   // row-major product (see DTile's PW), c0 + 16 j of a reduction-strided one (the transposing LDS reads fix
   // the order of its columns).  16 neighbouring lanes cover 16 * TN (or 16) consecutive columns of a row:
   // neighbouring lanes have to, the address coalescer joins the accesses of lanes 4 k .. 4 k + 3 only.
-  const int64_t row0 = m0 + wm0 + (lane >> 4) * 4;
-  const int64_t c0 = n0 + wn0 + (lane & 15) * (BT ? 1 : TN);
+  // (The two-stage pipeline's transposed operands go to the MFMA tiles eight rows to a lane: rows row0 + 8 r + i, and
+  // again TN consecutive columns.)
+  constexpr bool RUNS = !BT || TWO;        // a lane keeps runs of TN columns
+  const int64_t row0 = m0 + wm0 + (lane >> 4) * (AT && TWO ? 32 : 4);
+  const int64_t c0 = n0 + wn0 + (lane & 15) * (RUNS ? TN : 1);
+  auto row_in = [](uint32_t h, uint32_t r) { return AT && TWO ? 8 * r + h : 16 * h + r; };
   float bias[TN];
   // One branch on the dtype around all of the bias loads; a missing bias, and columns past N, read as zeros
   // through the buffer's extent.
@@ -433,23 +437,42 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
     // spacing, as four wavefronts that all load at once stall each other.  Each load has a tile's time, 2048 cycles, to arrive.
     // 8192^3 926 -> 775 us (bf16; 1.42 PFLOP/s), [8192 x 5632] . [5632 x 2048] 160 -> 140, 4096 x 4096 over 32768 977 -> 766,
     // [12608 x 4096] . [4096 x 1024] 111 -> 97, over 1024 30 -> 28 (eight wavefronts -> four, one card).
+    // A lone wavefront has no other to issue under its MFMAs: whatever stands between two of them beyond two or three
+    // instructions is time.  So a tile's place in memory is in the descriptor, two scalar sums and a clamp of its extent per tile in
+    // place of an addition per load (past the end of K nothing is left of the extent and the loads are dropped), four loads share one
+    // LDS base, and loads and fragment reads take turns: 245 -> 202 instructions per 128 MFMAs beside them, 8192^3
+    // 716 -> 698 us, 4096 x 4096 over 12608 281 -> 275, [8192 x 5632] . [5632 x 2048] 149 -> 145.
+    static_assert(TA::IPW == 8 && TB::IPW == 8, "eight loads of 1 KB per wavefront and operand tile");
+    constexpr int LEAD = 3072;      // four loads share an LDS base: their distance is in the instruction, which moves both addresses
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      offa[q] += LEAD - (q & 3) * 1024;
+      offb[q] += LEAD - (q & 3) * 1024;
+    }
+    const uint32_t ext_a = TA::extent(M, K, lda), ext_b = TB::extent(N, K, ldb);
+    auto tile_rsrc = [&](const uint16_t* base, uint32_t ext, uint32_t adv) {
+      const int left = (int)(ext + LEAD - adv);
+      return make_rsrc((const char*)base - LEAD + adv, (uint32_t)(left > 0 ? left : 0));
+    };
+    auto fetch = [&](__amdgpu_buffer_rsrc_t rs, const uint32_t (&off)[8], uint32_t dst, auto qc) {
+      constexpr int q = decltype(qc)::value;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (PF_LDS(void))(uintptr_t)(dst + (uint32_t)wave * 8192u + (q / 4) * 4096u), 16, (int)off[q], 0, (q & 3) * 1024, 0);
+    };
+    auto fetch_a = [&](int kt, uint32_t dst) { static_for<8>([&](auto qc) { fetch(tile_rsrc(A, ext_a, (uint32_t)kt * step_a), offa, dst, qc); }); };
+    auto fetch_b = [&](int kt, uint32_t dst) { static_for<8>([&](auto qc) { fetch(tile_rsrc(B, ext_b, (uint32_t)kt * step_b), offb, dst, qc); }); };
     auto mm = [&](auto curc, auto lac, uint32_t ra, uint32_t rb, int ktl, uint32_t dst) {
       constexpr int cur = decltype(curc)::value, slot = cur ^ 1, kkn = cur ^ 1;
       constexpr bool LA = decltype(lac)::value;           // this phase requests A's tile (else B's)
-      constexpr int NL = LA ? TA::IPW : TB::IPW, NS = NM * 7 / 8;
-      const uint32_t adv = adv_of(ktl, LA ? step_a : step_b);
+      const __amdgpu_buffer_rsrc_t rs = LA ? tile_rsrc(A, ext_a, (uint32_t)ktl * step_a) : tile_rsrc(B, ext_b, (uint32_t)ktl * step_b);
       static_for<NM>([&](auto mc) {
         constexpr int m = decltype(mc)::value;
-        static_for<NL>([&](auto ec) {
+        static_for<8>([&](auto ec) {
           constexpr int l = decltype(ec)::value;
-          if constexpr (l * NS / NL == m) {
-            if constexpr (LA) TA::template issue<l, l + 1, false>(rs_a, offa, taila, adv, 0u, dst, wave);
-            else TB::template issue<l, l + 1, false>(rs_b, offb, tailb, adv, 0u, dst, wave);
-          }
+          if constexpr (7 * l + 2 == m) fetch(rs, LA ? offa : offb, dst, ec);
         });
         static_for<NREADS>([&](auto ec) {
           constexpr int r = decltype(ec)::value;
-          if constexpr (r * NS / NREADS == m) {
+          if constexpr (r * 7 / 2 == m) {   // (never beside a load: each slot takes one more instruction or two)
             if constexpr (r < TN * TB::NRD) TB::template read<NFB, r / TB::NRD, kkn, r % TB::NRD>(fb[slot][r / TB::NRD], rb, fob);
             else {
               constexpr int q = r - TN * TB::NRD;
@@ -457,35 +480,101 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
             }
           }
         });
-        if constexpr (AT && BT && m % TN == 0) {   // (as in `phase`)
-          constexpr int need = TN * TB::NRD + (m / TN + 1) * TA::NRD;
-          constexpr int up = ((m + 1) * NREADS + NS - 1) / NS, issued = up < NREADS ? up : NREADS;
-          constexpr int later = NREADS - need + issued;
-          asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(later < 15 ? later : 15) : "memory");
-          __builtin_amdgcn_sched_barrier(0);
-        }
         constexpr int i = m / TN, j = (i & 1) ? TN - 1 - m % TN : m % TN;
         Mfma<DT>::run16_agpr(fa[cur][i].get(), fb[cur][j].get(), acc[i][j]);
         __builtin_amdgcn_sched_barrier(0);
       });
     };
+    // Reduction-strided operands lie in LDS as they do in memory, [k][row].  ds_read_b64_tr_b16 moves 64 bytes a cycle, half of what
+    // ds_read_b128 does, and bounds these products on the other tiles.  Here a lane reads eight whole 16-byte chunks, eight rows
+    // of one k each, and puts its eight fragments together in registers, one byte permutation per pair of k: lane i's rows
+    // 8 i + t are row i of MFMA tile t.  32 permutations per operand and phase run between the MFMAs: A's tile t + 1 while
+    // tile t is multiplied, B's for the next phase as its chunks arrive, none beside two others.  bf16, eight wavefronts
+    // with transposing reads / this: 4096 x 4096 over 12608 323 / 312 us, over 3152 104 / 100, 4096 x 1024 over 12608 239 / 226,
+    // 2048 x 5632 over 32768 655 / 637, 32000 x 2048 over 788 184 / 175 (the permutations keep it 5 % behind row-major
+    // products of these sizes).
+    short8_t rwa[AT ? 2 : 1][8], rwb[8];
+    u32x4_t fpa[2], fpb[2][8];
+    uint32_t fta[4], ftb[4];
+    if constexpr (AT && BT) {
+      const int g8 = (lane >> 4) * 8, c = (lane & 15) ^ (((lane >> 4) & 1) << 1);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        fta[q] = (uint32_t)(g8 * TA::ROWB + (wm0 / 8 + (c ^ (q << 2))) * 16);
+        ftb[q] = (uint32_t)(g8 * TB::ROWB + (wn0 / 8 + (c ^ (q << 2))) * 16);
+      }
+    }
+    auto raw_a = [&](short8_t& f, uint32_t lds, auto ec, auto kkc) {
+      constexpr int e = decltype(ec)::value, kk = decltype(kkc)::value;
+      f = *(PF_LDS(const short8_t))(uintptr_t)(lds + fta[e & 3] + (uint32_t)((kk * 32 + e) * TA::ROWB));
+    };
+    auto raw_b = [&](short8_t& f, uint32_t lds, auto ec, auto kkc) {
+      constexpr int e = decltype(ec)::value, kk = decltype(kkc)::value;
+      f = *(PF_LDS(const short8_t))(uintptr_t)(lds + ftb[e & 3] + (uint32_t)((kk * 32 + e) * TB::ROWB));
+    };
+    // dword P of tile T's fragment: k 2 P and 2 P + 1 of row T of the lane's eight
+    auto join = [](u32x4_t& f, const short8_t (&raw)[8], auto tc, auto pc) {
+      constexpr int T = decltype(tc)::value, P = decltype(pc)::value;
+      const u32x4_t lo = __builtin_bit_cast(u32x4_t, raw[2 * P]), hi = __builtin_bit_cast(u32x4_t, raw[2 * P + 1]);
+      f[P] = __builtin_amdgcn_perm(hi[T / 2], lo[T / 2], T % 2 ? 0x07060302u : 0x05040100u);
+    };
+    auto mt = [&](auto curc, auto lac, uint32_t ra, uint32_t rb, int ktl, uint32_t dst) {
+      constexpr int cur = decltype(curc)::value, kkn = cur ^ 1;
+      constexpr bool LA = decltype(lac)::value;
+      constexpr std::integral_constant<int, kkn> kknc{};
+      const __amdgpu_buffer_rsrc_t rs = LA ? tile_rsrc(A, ext_a, (uint32_t)ktl * step_a) : tile_rsrc(B, ext_b, (uint32_t)ktl * step_b);
+      static_for<NM>([&](auto mc) {
+        constexpr int m = decltype(mc)::value, i = m / TN, j = (i & 1) ? TN - 1 - m % TN : m % TN;
+        static_for<8>([&](auto ec) {
+          constexpr int l = decltype(ec)::value;
+          if constexpr (7 * l + 2 == m) fetch(rs, LA ? offa : offb, dst, ec);
+        });
+        // the next phase's chunks: B's first
+        if constexpr (m < 16 && m % 2 == 1) raw_b(rwb[m / 2], rb, std::integral_constant<int, m / 2>{}, kknc);
+        if constexpr (m >= 16 && m < 48 && m % 4 == 0) raw_a(rwa[cur ^ 1][m / 4 - 4], ra, std::integral_constant<int, m / 4 - 4>{}, kknc);
+        // A's next fragment (after the last row of MFMAs, the next phase's first); its last part two MFMAs before its first
+        // use, the distance that the matrix instructions ask of a register written by another
+        if constexpr (m % 2 == 0) {
+          constexpr std::integral_constant<int, (i + 1) & 7> tc{};
+          constexpr std::integral_constant<int, (m % TN) / 2> pc{};
+          join(fpa[(i + 1) & 1], rwa[i == TM - 1 ? (cur ^ 1) : cur], tc, pc);
+        }
+        // B's for the next phase, in the order in which its chunks arrive
+        static_for<32>([&](auto nc) {
+          constexpr int n = decltype(nc)::value;
+          if constexpr ((n < 26 ? 13 + 2 * n : 34 + 4 * (n - 26)) == m)
+            join(fpb[cur ^ 1][n % 8], rwb, std::integral_constant<int, n % 8>{}, std::integral_constant<int, n / 8>{});
+        });
+        Mfma<DT>::run16_agpr(__builtin_bit_cast(short8_t, fpa[i & 1]), __builtin_bit_cast(short8_t, fpb[cur][j]), acc[i][j]);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    };
     uint32_t a0 = lds0, a1 = lds0 + TA::BYTES, b0 = lds0 + 2 * TA::BYTES, b1 = b0 + TB::BYTES, b2 = b1 + TB::BYTES;
-    TA::template issue<0, TA::IPW, false>(rs_a, offa, taila, adv_of(0, step_a), 0u, a0, wave);
-    TB::template issue<0, TB::IPW, false>(rs_b, offb, tailb, adv_of(0, step_b), 0u, b0, wave);
-    TB::template issue<0, TB::IPW, false>(rs_b, offb, tailb, adv_of(1, step_b), 0u, b1, wave);
-    TA::template issue<0, TA::IPW, false>(rs_a, offa, taila, adv_of(1, step_a), 0u, a1, wave);
+    fetch_a(0, a0);
+    fetch_b(0, b0);
+    fetch_b(1, b1);
+    fetch_a(1, a1);
     wait_vm<LPW>();
     lds_barrier();
-    static_for<TN>([&](auto jc) { TB::template read_first<NFB, decltype(jc)::value>(fb[0][decltype(jc)::value], b0, fob); });
-    static_for<TM>([&](auto ic) { TA::template read_first<NFA, decltype(ic)::value>(fa[0][decltype(ic)::value], a0, foa); });
+    if constexpr (AT && BT) {
+      static_for<8>([&](auto ec) { raw_b(rwb[decltype(ec)::value], b0, ec, std::integral_constant<int, 0>{}); });
+      static_for<8>([&](auto ec) { raw_a(rwa[0][decltype(ec)::value], a0, ec, std::integral_constant<int, 0>{}); });
+      static_for<8>([&](auto tc) { static_for<4>([&](auto pc) { join(fpb[0][decltype(tc)::value], rwb, tc, pc); }); });
+      static_for<4>([&](auto pc) { join(fpa[0], rwa[0], std::integral_constant<int, 0>{}, pc); });
+    } else {
+      static_for<TN>([&](auto jc) { TB::template read_first<NFB, decltype(jc)::value>(fb[0][decltype(jc)::value], b0, fob); });
+      static_for<TM>([&](auto ic) { TA::template read_first<NFA, decltype(ic)::value>(fa[0][decltype(ic)::value], a0, foa); });
+    }
     asm volatile("s_nop 7" ::: "memory");   // (the compiler sees no MFMA: the distance to the zeros written to AGPRs is kept by hand)
     __builtin_amdgcn_sched_barrier(0);
     int kt = 0;
     do {
-      mm(std::integral_constant<int, 0>{}, std::false_type{}, a0, b0, kt + 2, b2);
+      if constexpr (AT && BT) mt(std::integral_constant<int, 0>{}, std::false_type{}, a0, b0, kt + 2, b2);
+      else mm(std::integral_constant<int, 0>{}, std::false_type{}, a0, b0, kt + 2, b2);
       wait_vm<TB::IPW>();
       lds_barrier();       // tile kt + 1 landed everywhere, stage a0 and (since the barrier before) b2 no longer read
-      mm(std::integral_constant<int, 1>{}, std::true_type{}, a1, b1, kt + 2, a0);
+      if constexpr (AT && BT) mt(std::integral_constant<int, 1>{}, std::true_type{}, a1, b1, kt + 2, a0);
+      else mm(std::integral_constant<int, 1>{}, std::true_type{}, a1, b1, kt + 2, a0);
       const uint32_t ta = a0, tb = b0;
       a0 = a1; a1 = ta;
       b0 = b1; b1 = b2; b2 = tb;
@@ -563,9 +652,9 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
 #pragma unroll
   for (int sl = 0; sl < (SINGLE ? 1 : 2); ++sl) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i) frag_hold(fa[sl][i]);
+    for (int i = 0; i < TM; ++i) if constexpr (!(AT && TWO)) frag_hold(fa[sl][i]);
 #pragma unroll
-    for (int j = 0; j < TN; ++j) frag_hold(fb[sl][j]);
+    for (int j = 0; j < TN; ++j) if constexpr (!(BT && TWO)) frag_hold(fb[sl][j]);
   }
   // (the dropped requests past K are counted too)  The builtin, not inline assembly: the compiler
   // tracks the LDS-writing loads itself and, unless it sees them retired here, makes every LDS
@@ -609,10 +698,10 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
       });
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int64_t row = row0 + h * 16 + r;
+        const int64_t row = row0 + row_in((uint32_t)h, (uint32_t)r);
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-          const int64_t col = c0 + (BT ? 16 : 1) * j;
+          const int64_t col = c0 + (RUNS ? 1 : 16) * j;
           if (row < M && col < N) worst = fmaf(epilogue_scalar(epi, c_base, row, col, x[j][r]), 0.f, worst);
         }
       }
@@ -626,8 +715,8 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
     // aux_in) is requested DEPTH row blocks ahead, into the registers the operand fragments have left.
     constexpr bool LOADS = EC == EC_RES32 || EC == EC_ACC32 || EC == EC_DACT16 || EC == EC_ACC16 || EC == EC_RES16;
     constexpr int ESC = C32 ? 4 : 2;       // (the operand read has the element size of C in every class)
-    constexpr int NG = BT ? TN : 1;        // runs of columns per lane and row
-    constexpr int GW = BT ? 1 : TN;        // columns per run
+    constexpr int NG = RUNS ? 1 : TN;      // runs of columns per lane and row
+    constexpr int GW = RUNS ? TN : 1;      // columns per run
     constexpr int NV = GW * ESC / 4;       // 32-bit words per run
     static_assert(!BT || C32, "reduction-strided products have fp32 results");
     constexpr int DEPTH = !LOADS ? 1 : (TM * NG * NV <= 16 ? TM : (16 / (NG * NV) > 0 ? 16 / (NG * NV) : 1));
@@ -662,14 +751,14 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
     auto block = [&](uint32_t h, const float4_t (&x)[TN], const Words<NV> (&old)[4][NG]) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const bool row_ok = row0 + (int64_t)(h * 16 + r) < M;
+        const bool row_ok = row0 + (int64_t)row_in(h, (uint32_t)r) < M;
         float bad = 0.f;
 #pragma unroll
         for (int g = 0; g < NG; ++g) {
           float v[GW];
 #pragma unroll
           for (int k = 0; k < GW; ++k) {
-            v[k] = x[BT ? g : k][r] * alpha;
+            v[k] = x[RUNS ? k : g][r] * alpha;
             if constexpr (HAS_BIAS) v[k] += bias[k];
           }
           // (the plain 16-bit store rounds once, when it packs: rounding to the same format before
@@ -684,7 +773,7 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
               }
             }
           }
-          const uint32_t oc = off_c[g] + (h * 16 + (uint32_t)r) * step_c;
+          const uint32_t oc = off_c[g] + row_in(h, (uint32_t)r) * step_c;
           Words<NV> o;
           if constexpr (C32) {
             if constexpr (LOADS) {
@@ -701,7 +790,7 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
             if constexpr (EC == EC_ACT16) {   // GELU only (other activations take the generic class)
 #pragma unroll
               for (int k = 0; k < NV; ++k) o.w[k] = (int)pack2<DT>(v[2 * k], v[2 * k + 1]);
-              o.store(rs_x, off_x[g] + (h * 16 + (uint32_t)r) * step_x);
+              o.store(rs_x, off_x[g] + row_in(h, (uint32_t)r) * step_x);
               if (round_mid) {
 #pragma unroll
                 for (int k = 0; k < GW; ++k) v[k] = unpack1<DT>((uint32_t)o.w[k / 2], k % 2);
@@ -735,7 +824,7 @@ __device__ __forceinline__ void gemm16x_body(const pf_gemm_desc& p, const GemmGr
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll
-          for (int g = 0; g < NG; ++g) old[r][g].load(rs_l, off_l[g] + (h * 16 + (uint32_t)r) * step_l);
+          for (int g = 0; g < NG; ++g) old[r][g].load(rs_l, off_l[g] + row_in(h, (uint32_t)r) * step_l);
       }
     };
     if constexpr (EC == EC_ACT16 || EC == EC_DACT16) {

@@ -31,10 +31,10 @@ from .merge import CallRecorder, Merger
 from .values import Val, as_matrix, collapse_for_copy, dense_like, is_dense
 
 ACT_NONE, ACT_GELU, ACT_GELU_TANH, ACT_SILU, ACT_RELU = 0, 1, 2, 3, 4
-# kernel variant (pf_gemm_desc.variant) that regrouped weight-gradient products are pinned to: the 256x256
-# tile the automatic choice itself uses (eight wavefronts), so that products that chose it on their own and
-# products moved onto it share launches
+# kernel variants (pf_gemm_desc.variant) that regrouped weight-gradient products are pinned to: 256x256 tiles by eight
+# wavefronts, and by four for sets that fill the device
 BIG_TILE_VARIANT = int(os.environ.get("PFEIFE_BIG_TILE", "7"))
+FULL_TILE_VARIANT = 18
 MID_TILE_VARIANT, SMALL_TILE_VARIANT = 8, 15    # 128x128 and 64x64
 
 
@@ -499,7 +499,7 @@ class BwdCtx:
         bigs, t256 = [], 0
         for launch, _ in members:
             d = launch.desc
-            big = launch if launch.variant.startswith("gemm16x_kernel<%d, 256, 256" % d.in_dtype) else retile(launch, BIG_TILE_VARIANT)
+            big = retile(launch, BIG_TILE_VARIANT)
             if d.M < 256 or d.N < 256 or big is None or not self.k.gemm_groupable(big):
                 return               # less than one full tile either way: stays on the small tile
             bigs.append(big)
@@ -526,12 +526,19 @@ class BwdCtx:
 
     def _close_set(self, entries):
         """Two or more remembered launches that cover half the device or more on 256x256 tiles give way to
-        one launch on that tile, here; anything less stays as it was issued."""
+        one launch on that tile, here; anything less stays as it was issued.  A set that nearly fills the device
+        takes the four-wavefront form: five of ViT-L's weights over 12608 rows 356 us on
+        eight wavefronts, 350 on four, 5632 x 2048 + 2048 x 2048 over 32768 782 / 771 (bf16), 3 x 64 tiles over 12608
+        247 / 243.  (Half a set, closed at the job's end, stays on eight: 236 / 228, once per stage and step.)"""
         self._dw_big.remove(entries)
         if len(entries) >= 2 and sum(t for _, _, _, t in entries) >= self.FULL_GRID // 2:
+            bigs = [b for _, bs, _, _ in entries for b in bs]
+            if sum(t for _, _, _, t in entries) >= self.FULL_GRID - 56:
+                full = [self.k.gemm_retiled(b, FULL_TILE_VARIANT) for b in bigs]
+                bigs = bigs if any(b is None for b in full) else full
             for old, _, _, _ in entries:   # blanked, not deleted: positions in the list stay valid until compact()
                 self.out[next(i for i in range(len(self.out) - 1, -1, -1) if self.out[i] is old)] = None
-            self.emit(self.k.gemm_group([b for _, bs, _, _ in entries for b in bs]))
+            self.emit(self.k.gemm_group(bigs))
 
     def compact(self, ranges):
         """Drop the blanked launches; `ranges` ((name, first, end) over the list) follow."""

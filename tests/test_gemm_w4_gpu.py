@@ -74,6 +74,30 @@ def test_weight_gradients(hip, oracle, dtype, M, N, K):
         close(r["c"], 1e-4, 2e-3)
 
 
+@pytest.mark.parametrize("dtype", [F16, BF16])
+def test_grouped_weight_gradients(hip, dtype):
+    """Products of different sizes, depths and betas in one launch: what each gives alone on the eight-wavefront tile."""
+    outs = {}
+    for variant in (7, 18):
+        members, outs[variant] = [], []
+        for i, (M, N, K, beta) in enumerate([(512, 264, 200, 0), (256, 520, 64, 1), (264, 256, 1021, 0)]):
+            a, b, c = rnd((K, M + 8), dtype, i).cuda(), rnd((K, N + 16), dtype, i + 3).cuda(), rnd((M, N + 8), F32, i + 6).cuda()
+            members.append(hip.gemm(a, b, c, M=M, N=N, K=K, lda=M + 8, ldb=N + 16, ldc=N + 8, a_trans=1, b_trans=1, beta=beta,
+                                    variant=variant))
+            outs[variant].append(c)
+        stream = torch.cuda.current_stream().cuda_stream
+        if variant == 18:
+            group = hip.gemm_group(members)
+            assert group.variant == "gemm16x_group_kernel<%d, 256, 256, 64, 2, 2, 1, 2, true, true, 4>" % (1 if dtype == F16 else 2)
+            group(stream)
+        else:
+            for m in members:
+                m(stream)
+        torch.cuda.synchronize()
+    for x, y in zip(outs[7], outs[18]):
+        assert torch.equal(x, y)
+
+
 def test_column_sums(hip):
     """GELU' with the column sums of what is stored, as partial rows: equal to sums over the stored values."""
     M, N, K = 700, 520, 128
@@ -89,7 +113,7 @@ def test_column_sums(hip):
 
 
 def test_automatic_choice(hip):
-    """Long rows in whole rounds take the tile; depths that are no multiple of 64, small outputs and weight gradients do not."""
+    """Long rows and large weight gradients take the tile; depths that are no multiple of 64 and small outputs do not."""
     def name(M, N, K, t=0):
         a = torch.empty(K if t else M, M if t else K, dtype=BF16, device="cuda")
         b = torch.empty(K if t else N, N if t else K, dtype=BF16, device="cuda")
@@ -97,7 +121,7 @@ def test_automatic_choice(hip):
         return hip.gemm(a, b, c, M=M, N=N, K=K, lda=a.shape[1], ldb=b.shape[1], ldc=N, a_trans=t, b_trans=t).variant
 
     w4 = "256, 256, 64, 2, 2, 1, 2"
-    assert w4 in name(8192, 2048, 2048) and w4 in name(12608, 1024, 4096)
+    assert w4 in name(8192, 2048, 2048) and w4 in name(12608, 1024, 4096) and w4 in name(4096, 4096, 12608, 1)
     assert w4 not in name(8192, 2048, 2048 + 32) and w4 not in name(788, 384, 1536) and w4 not in name(2048, 2048, 8192, 1)
 
 
