@@ -487,8 +487,10 @@ __global__ __launch_bounds__(256, SPLITQ || HD > 96 ? 1 : 2) void attn_dkv_kerne
     }
     if (q0 + QT < a.Tq) prefetch(q0 + QT);
     __syncthreads();
-    // causal: the tile needs element masks only where it crosses the diagonal
-    const bool masked = a.causal && (kw0 + 31 > q0 + qoff + shift);
+    // causal: rows before `first` (of this lane's) do not see its key; a constant against a threshold, 32 sums less per step
+    // than key against query: 2048 tokens x 128 heads backward 354 -> 350 us.  (Lighter still without the `causal` in every
+    // compare, or with vector loads of lse and delta: four registers spill, whose reloads wait for the next tile's loads, 392.)
+    const int first = a.causal ? kj - (q0 + qoff + 4 * (lane >> 5) + shift) : 0;
     float16_t s[NH], dp[NH];
 #pragma unroll
     for (int t = 0; t < NH; ++t) {
@@ -504,7 +506,7 @@ __global__ __launch_bounds__(256, SPLITQ || HD > 96 ? 1 : 2) void attn_dkv_kerne
       for (int r = 0; r < 16; ++r) {
         const int ql = qoff + t * 32 + acc_row(r, lane);
         float p = __builtin_amdgcn_exp2f(s[t][r] * sc - sLse[ql]);
-        if (masked && kj > q0 + ql + shift) p = 0.f;
+        if (t * 32 + 8 * (r >> 2) + (r & 3) < first) p = 0.f;
         s[t][r] = p;                                         // P
         dp[t][r] = p * (dp[t][r] - sDelta[ql]);              // dS / scale (applied to dK at the end)
       }
@@ -592,24 +594,42 @@ __device__ __forceinline__ void unpack8(const uint4& r, float (&v)[8]) {
   }
 }
 
-// Two whole [T][hd] operands of one head -> LDS [rows][HD + 8] each (rows past T and hd
-// chunks past hd are zero); NT threads, eight 16-byte loads in flight per thread
-template <int HD, int NT>
-__device__ __forceinline__ void load_heads(const uint16_t* x, int64_t x_st, const uint16_t* y, int64_t y_st, int T,
-                                           int hd, int rows, uint16_t* sx, uint16_t* sy, int tid) {
-  constexpr int VPR = HD / 8, LD = HD + 8;
-  const int n = rows * VPR;
-  for (int e0 = 0; e0 < n; e0 += NT * 4) {
-    uint4 vx[4], vy[4];
+// One head's [T][hd] operand for 16-byte loads without a branch: rows past T and chunks past hd get an offset out of the
+// buffer's range, which reads zeros.  (T * st * 2 bytes are below 2 GiB, see short_ok.)
+struct HeadRows {
+  __amdgpu_buffer_rsrc_t rs;
+  uint32_t st2;
+  int T, hd;
+  __device__ __forceinline__ HeadRows(const uint16_t* x, int64_t st, int T_, int hd_) : st2((uint32_t)(st * 2)), T(T_), hd(hd_) {
+    rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x), 0, (int)((uint32_t)(T - 1) * st2 + (uint32_t)hd_ * 2u), 0x00020000);
+  }
+  __device__ __forceinline__ uint4 load(int t, int c) const {
+    typedef int v4 __attribute__((ext_vector_type(4)));
+    const v4 x = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(t < T && c < hd ? (uint32_t)t * st2 + (uint32_t)c * 2u : 0x80000000u), 0, 0);
+    return make_uint4((uint32_t)x.x, (uint32_t)x.y, (uint32_t)x.z, (uint32_t)x.w);
+  }
+};
+
+// Two whole [T][hd] operands of one head on their way to LDS, [rows][HD + 8] each (rows past T and hd chunks past hd are
+// zero); NT threads.  Nothing else runs on a compute unit whose LDS one head fills, so a workgroup's loads go out
+// together, up to the largest head of eight wavefronts in one batch, next to those of the rows that a wavefront keeps in
+// registers: 257 tokens x 384 heads of 64 30.1 -> 28.6 us, 65 tokens x 256 heads 6.5 -> 5.7, in two batches behind the rows -> this.
+template <int HD, int NT> struct HeadPair {
+  static constexpr int VPR = HD / 8, LD = HD + 8, U = NT == 512 ? (HD == 64 ? 5 : 7) : (HD == 64 ? 4 : 6);
+  uint4 vx[U], vy[U];
+  __device__ __forceinline__ void issue(const HeadRows& x, const HeadRows& y, int rows, int tid, int e0 = 0) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < U; ++i) {
       const int e = e0 + i * NT + tid;
-      const int t = e / VPR, c = (e % VPR) * 8;
-      vx[i] = e < n ? load_row8(x, x_st, t, T, c, hd) : make_uint4(0, 0, 0, 0);
-      vy[i] = e < n ? load_row8(y, y_st, t, T, c, hd) : make_uint4(0, 0, 0, 0);
+      if (e0 + i * NT < rows * VPR) {
+        vx[i] = x.load(e / VPR, (e % VPR) * 8);
+        vy[i] = y.load(e / VPR, (e % VPR) * 8);
+      }
     }
+  }
+  __device__ __forceinline__ void store(uint16_t* sx, uint16_t* sy, int n, int tid, int e0 = 0) const {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < U; ++i) {
       const int e = e0 + i * NT + tid;
       if (e < n) {
         *(uint4*)(sx + (e / VPR) * LD + (e % VPR) * 8) = vx[i];
@@ -617,19 +637,30 @@ __device__ __forceinline__ void load_heads(const uint16_t* x, int64_t x_st, cons
       }
     }
   }
-}
+  // the first batch, issued before, and whatever it did not hold
+  __device__ __forceinline__ void finish(const HeadRows& x, const HeadRows& y, uint16_t* sx, uint16_t* sy, int rows, int tid) {
+    const int n = rows * VPR;
+    store(sx, sy, n, tid);
+    for (int e0 = NT * U; e0 < n; e0 += NT * U) {
+      issue(x, y, rows, tid, e0);
+      store(sx, sy, n, tid, e0);
+    }
+  }
+};
 
 // forward: workgroup = NT / 2 queries of one (batch, head) at a time, wavefront = 32 of them; keys in
-// steps of 32.  A wavefront whose tile lies past what the grid covers at once (gridDim.x * NT / 2
-// queries) takes it in a second pass.  NT = 512 (eight wavefronts) lets ONE workgroup cover a whole head,
-// so that the head's K and V are fetched once instead of once per 128 queries; NT = 256 otherwise.
+// steps of 32.  NT = 512 (eight wavefronts): ONE workgroup covers a whole head, so that the head's K and V are fetched
+// once instead of once per 128 queries.  With `share` its ninth tile (257 to 288 tokens) is everybody's: each wavefront sweeps an
+// eighth of the keys, and the eight partial results meet in LDS, where one wavefront would sweep all keys with the other
+// seven gone.  257 tokens x 384 heads of 64: 32.2 -> 30.1 us, backward 89 -> 78; x 16 heads of 88 17.7 -> 16.9.
+// NT = 256: a wavefront whose tile lies past what the grid covers at once takes it in a second pass.
 template <int DT, int HD, int NT>
-__global__ __launch_bounds__(NT) void attn_fwd_short_kernel(const AttnArgs a, int rows) {
+__global__ __launch_bounds__(NT) void attn_fwd_short_kernel(const AttnArgs a, int rows, int share) {
   constexpr int NC = HD / 16, NO = HD / 32, LD = HD + 8;
   extern __shared__ __align__(16) uint16_t smem[];
   uint16_t* sK = smem;
   uint16_t* sV = smem + rows * LD;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int bh = blockIdx.y, b = bh / a.H, h = bh % a.H;
   const int q_step = (int)gridDim.x * (NT / 2);
   int q0 = blockIdx.x * (NT / 2) + wave * 32;
@@ -637,15 +668,26 @@ __global__ __launch_bounds__(NT) void attn_fwd_short_kernel(const AttnArgs a, in
   const float sc = a.scale * LOG2E;
   const int shift = a.Tk - a.Tq;
 
-  uint4 qf[NC];   // the first tile's queries are requested before the head is loaded
+  const HeadRows rq(Q, a.q_st, a.Tq, a.hd);
+  const HeadRows rk(a.k + b * a.k_sb + h * a.k_sh, a.k_st, a.Tk, a.hd), rv(a.v + b * a.v_sb + h * a.v_sh, a.v_st, a.Tk, a.hd);
+  uint4 qf[NC];
+  auto load_q = [&](int qs) {
 #pragma unroll
-  for (int c = 0; c < NC; ++c) qf[c] = load_row8(Q, a.q_st, q0 + (lane & 31), a.Tq, c * 16 + (lane >> 5) * 8, a.hd);
-  load_heads<HD, NT>(a.k + b * a.k_sb + h * a.k_sh, a.k_st, a.v + b * a.v_sb + h * a.v_sh, a.v_st, a.Tk, a.hd, rows, sK,
-                 sV, tid);
+    for (int c = 0; c < NC; ++c) qf[c] = rq.load(qs + (lane & 31), c * 16 + (lane >> 5) * 8);
+  };
+  {
+    HeadPair<HD, NT> kv;
+    kv.issue(rk, rv, rows, tid);
+    load_q(q0);
+    kv.finish(rk, rv, sK, sV, rows, tid);
+  }
   __syncthreads();
-  // no barrier follows: a wavefront without a query tile leaves, one with several (the tiles past
-  // what the grid covers at once, e.g. the 257th token of a 256-token-wide grid) loops
-  for (; q0 < a.Tq; q0 += q_step) {
+  // no barrier follows but for a shared tile: a wavefront without a query tile leaves, one with several loops
+  constexpr int SHARED = NT / 2;             // the tile from here on is shared by all wavefronts where they share one
+  const bool sharing = NT == 512 && share;
+  for (; q0 < a.Tq; q0 = sharing ? (q0 < SHARED ? SHARED : a.Tq) : q0 + q_step) {
+  const bool shared = sharing && q0 >= SHARED;
+  const int k_first = shared ? wave * 32 : 0, k_step = shared ? NT / 2 : 32;
   const int qi = q0 + (lane & 31);
   float16_t oacc[NO];
 #pragma unroll
@@ -654,7 +696,7 @@ __global__ __launch_bounds__(NT) void attn_fwd_short_kernel(const AttnArgs a, in
     for (int r = 0; r < 16; ++r) oacc[o][r] = 0.f;
   float m = -INFINITY, l = 0.f;
   const int k_end = a.causal ? min(a.Tk, min(q0 + 31, a.Tq - 1) + shift + 1) : a.Tk;
-  for (int k0 = 0; k0 < k_end; k0 += 32) {
+  for (int k0 = k_first; k0 < k_end; k0 += k_step) {
     float16_t s;
 #pragma unroll
     for (int r = 0; r < 16; ++r) s[r] = 0.f;
@@ -704,36 +746,92 @@ __global__ __launch_bounds__(NT) void attn_fwd_short_kernel(const AttnArgs a, in
     }
   }
   l += __shfl_xor(l, 32, 64);
-  const float inv = l > 0.f ? 1.f / l : 0.f;
-  if (qi < a.Tq) {
-    uint16_t* O = a.out + b * a.o_sb + h * a.o_sh + (int64_t)qi * a.o_st;
+  if (!shared) {
+    const int qn = sharing ? SHARED : q0 + q_step;
+    if (qn < a.Tq) load_q(qn);
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    if (qi < a.Tq) {
+      uint16_t* O = a.out + b * a.o_sb + h * a.o_sh + (int64_t)qi * a.o_st;
+#pragma unroll
+      for (int o = 0; o < NO; ++o)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int h0 = o * 32 + 8 * g + 4 * (lane >> 5);
+          if (h0 < a.hd)
+            *(uint2*)(O + h0) = make_uint2(M32<DT>::pack(oacc[o][4 * g] * inv, oacc[o][4 * g + 1] * inv),
+                                           M32<DT>::pack(oacc[o][4 * g + 2] * inv, oacc[o][4 * g + 3] * inv));
+        }
+      if ((lane >> 5) == 0) a.lse[((int64_t)bh) * a.Tq + qi] = (l > 0.f) ? (m * sc + log2f(l)) / LOG2E : -INFINITY;
+    }
+  } else if constexpr (NT == 512) {
+    // each wavefront's maxima meet first, then its sums on the scale of the largest; wavefront w finishes registers
+    // 2 w and 2 w + 1 of every tile of the head dimension
+    float* xm = (float*)smem;             // [8][32]
+    float* xl = xm + 256;                 // [8][32]
+    float* xo = xl + 256;                 // [8][NO][16][64]
+    __syncthreads();                      // K and V are no longer read
+    if (lane < 32) xm[wave * 32 + lane] = m;
+    __syncthreads();
+    float top = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) top = fmaxf(top, xm[w * 32 + (lane & 31)]);
+    const float f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m - top) * sc);
+    if (lane < 32) xl[wave * 32 + lane] = l * f;
 #pragma unroll
     for (int o = 0; o < NO; ++o)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int h0 = o * 32 + 8 * g + 4 * (lane >> 5);
-        if (h0 < a.hd)
-          *(uint2*)(O + h0) = make_uint2(M32<DT>::pack(oacc[o][4 * g] * inv, oacc[o][4 * g + 1] * inv),
-                                         M32<DT>::pack(oacc[o][4 * g + 2] * inv, oacc[o][4 * g + 3] * inv));
-      }
-    if ((lane >> 5) == 0) a.lse[((int64_t)bh) * a.Tq + qi] = (l > 0.f) ? (m * sc + log2f(l)) / LOG2E : -INFINITY;
-  }
-  if (q0 + q_step < a.Tq) {
+      for (int r = 0; r < 16; ++r) xo[((wave * NO + o) * 16 + r) * 64 + lane] = oacc[o][r] * f;
+    __syncthreads();
+    l = 0.f;
 #pragma unroll
-    for (int c = 0; c < NC; ++c)
-      qf[c] = load_row8(Q, a.q_st, q0 + q_step + (lane & 31), a.Tq, c * 16 + (lane >> 5) * 8, a.hd);
+    for (int w = 0; w < 8; ++w) l += xl[w * 32 + (lane & 31)];
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    float x[2 * NO];
+#pragma unroll
+    for (int e = 0; e < 2 * NO; ++e) x[e] = 0.f;
+#pragma unroll
+    for (int w = 0; w < 8; ++w)
+#pragma unroll
+      for (int e = 0; e < 2 * NO; ++e) x[e] += xo[((w * NO + e / 2) * 16 + 2 * wave + e % 2) * 64 + lane];
+    if (qi < a.Tq) {
+      uint16_t* O = a.out + b * a.o_sb + h * a.o_sh + (int64_t)qi * a.o_st;
+#pragma unroll
+      for (int o = 0; o < NO; ++o) {
+        const int h0 = o * 32 + acc_row(2 * wave, lane);
+        if (h0 < a.hd) *(uint32_t*)(O + h0) = M32<DT>::pack(x[2 * o] * inv, x[2 * o + 1] * inv);
+      }
+      if (wave == 0 && lane < 32) a.lse[((int64_t)bh) * a.Tq + qi] = (l > 0.f) ? (top * sc + log2f(l)) / LOG2E : -INFINITY;
+    }
   }
   }
 }
 
+// The sum over eight wavefronts of a tile's accumulators: wavefront w gets registers 2 w and 2 w + 1 of each of the
+// NO tiles.  (All wavefronts call; `red` may hold what they have read until now.)
+template <int NO>
+__device__ __forceinline__ void sum_waves(const float16_t (&acc)[NO], float* red, int wave, int lane, float (&x)[2 * NO]) {
+  __syncthreads();
+#pragma unroll
+  for (int o = 0; o < NO; ++o)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) red[((wave * NO + o) * 16 + r) * 64 + lane] = acc[o][r];
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < 2 * NO; ++e) x[e] = 0.f;
+#pragma unroll
+  for (int w = 0; w < 8; ++w)
+#pragma unroll
+    for (int e = 0; e < 2 * NO; ++e) x[e] += red[((w * NO + e / 2) * 16 + 2 * wave + e % 2) * 64 + lane];
+}
+
 // dQ (and delta = rowsum(dO * O), which the dK/dV kernel launched after this one reads)
 template <int DT, int HD, int NT>
-__global__ __launch_bounds__(NT) void attn_dq_short_kernel(const AttnArgs a, float* delta_out, int rows) {
+__global__ __launch_bounds__(NT) void attn_dq_short_kernel(const AttnArgs a, float* delta_out, int rows, int share) {
   constexpr int NC = HD / 16, NO = HD / 32, LD = HD + 8;
   extern __shared__ __align__(16) uint16_t smem[];
   uint16_t* sK = smem;
   uint16_t* sV = smem + rows * LD;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int bh = blockIdx.y, b = bh / a.H, h = bh % a.H;
   const int q_step = (int)gridDim.x * (NT / 2);
   int q0 = blockIdx.x * (NT / 2) + wave * 32;
@@ -743,34 +841,51 @@ __global__ __launch_bounds__(NT) void attn_dq_short_kernel(const AttnArgs a, flo
   const float sc = a.scale * LOG2E;
   const int shift = a.Tk - a.Tq;
 
-  uint4 qf[NC], dof[NC];
+  constexpr int SHARED = NT / 2;             // the tile from here on is shared by all wavefronts where they share one
+  const bool sharing = NT == 512 && share;
+  const HeadRows rq(Q, a.q_st, a.Tq, a.hd), rdo(DO, a.do_st, a.Tq, a.hd), ro(OO, a.o_st, a.Tq, a.hd);
+  const HeadRows rk(a.k + b * a.k_sb + h * a.k_sh, a.k_st, a.Tk, a.hd), rv(a.v + b * a.v_sb + h * a.v_sh, a.v_st, a.Tk, a.hd);
+  uint4 qf[NC], dof[NC], of[NC];
   float dlt, lse2;
-  // this lane's query row of the tile at `qs`: Q, dO, delta (also written out) and the row's lse
+  // this lane's query row of the tile at `qs`: Q, dO, O and the row's lse
   auto load_rows = [&](int qs) {
+    const int qr = qs + (lane & 31);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int h0 = c * 16 + (lane >> 5) * 8;
+      qf[c] = rq.load(qr, h0);
+      dof[c] = rdo.load(qr, h0);
+      of[c] = ro.load(qr, h0);
+    }
+    lse2 = qr < a.Tq ? a.lse[(int64_t)bh * a.Tq + qr] * LOG2E : INFINITY;
+  };
+  // ... and its delta (also written out)
+  auto row_delta = [&](int qs) {
     const int qr = qs + (lane & 31);
     dlt = 0.f;
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-      const int h0 = c * 16 + (lane >> 5) * 8;
-      qf[c] = load_row8(Q, a.q_st, qr, a.Tq, h0, a.hd);
-      dof[c] = load_row8(DO, a.do_st, qr, a.Tq, h0, a.hd);
-      const uint4 of = load_row8(OO, a.o_st, qr, a.Tq, h0, a.hd);
       float x[8], y[8];
       unpack8<DT>(dof[c], x);
-      unpack8<DT>(of, y);
+      unpack8<DT>(of[c], y);
 #pragma unroll
       for (int k = 0; k < 8; ++k) dlt += x[k] * y[k];
     }
     dlt += __shfl_xor(dlt, 32, 64);
-    if (qr < a.Tq && (lane >> 5) == 0) delta_out[(int64_t)bh * a.Tq + qr] = dlt;
-    lse2 = qr < a.Tq ? a.lse[(int64_t)bh * a.Tq + qr] * LOG2E : INFINITY;
+    if (qr < a.Tq && (lane >> 5) == 0 && (wave == 0 || !sharing || qs < SHARED)) delta_out[(int64_t)bh * a.Tq + qr] = dlt;
   };
-  load_rows(q0);   // the first tile's rows are requested before the head is loaded
-  load_heads<HD, NT>(a.k + b * a.k_sb + h * a.k_sh, a.k_st, a.v + b * a.v_sb + h * a.v_sh, a.v_st, a.Tk, a.hd, rows, sK,
-                 sV, tid);
+  {
+    HeadPair<HD, NT> kv;
+    load_rows(q0);
+    kv.issue(rk, rv, rows, tid);
+    row_delta(q0);
+    kv.finish(rk, rv, sK, sV, rows, tid);
+  }
   __syncthreads();
-  // no barrier follows: a wavefront without a query tile leaves, one with several loops
-  for (; q0 < a.Tq; q0 += q_step) {
+  // no barrier follows but for a shared tile: a wavefront without a query tile leaves, one with several loops
+  for (; q0 < a.Tq; q0 = sharing ? (q0 < SHARED ? SHARED : a.Tq) : q0 + q_step) {
+  const bool shared = sharing && q0 >= SHARED;
+  const int k_first = shared ? wave * 32 : 0, k_step = shared ? NT / 2 : 32;
   const int qi = q0 + (lane & 31);
   const bool qok = qi < a.Tq;
   float16_t acc[NO];
@@ -779,7 +894,7 @@ __global__ __launch_bounds__(NT) void attn_dq_short_kernel(const AttnArgs a, flo
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[o][r] = 0.f;
   const int k_end = a.causal ? min(a.Tk, min(q0 + 31, a.Tq - 1) + shift + 1) : a.Tk;
-  for (int k0 = 0; k0 < k_end; k0 += 32) {
+  for (int k0 = k_first; k0 < k_end; k0 += k_step) {
     float16_t s, dp;
 #pragma unroll
     for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
@@ -809,32 +924,67 @@ __global__ __launch_bounds__(NT) void attn_dq_short_kernel(const AttnArgs a, flo
       for (int o = 0; o < NO; ++o) acc[o] = M32<DT>::run(frag_tr<LD>(sK, k0 + 16 * j, o * 32, lane), dsf, acc[o]);
     }
   }
-  if (qok) {
-    uint16_t* DQ = a.dq + b * a.dq_sb + h * a.dq_sh + (int64_t)qi * a.dq_st;
+  if (!shared) {
+    const int qn = sharing ? SHARED : q0 + q_step;
+    if (qn < a.Tq) {
+      load_rows(qn);
+      row_delta(qn);
+    }
+    if (qok) {
+      uint16_t* DQ = a.dq + b * a.dq_sb + h * a.dq_sh + (int64_t)qi * a.dq_st;
 #pragma unroll
-    for (int o = 0; o < NO; ++o)
+      for (int o = 0; o < NO; ++o)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int h0 = o * 32 + 8 * g + 4 * (lane >> 5);
-        if (h0 < a.hd)
-          *(uint2*)(DQ + h0) = make_uint2(M32<DT>::pack(acc[o][4 * g] * a.scale, acc[o][4 * g + 1] * a.scale),
-                                          M32<DT>::pack(acc[o][4 * g + 2] * a.scale, acc[o][4 * g + 3] * a.scale));
+        for (int g = 0; g < 4; ++g) {
+          const int h0 = o * 32 + 8 * g + 4 * (lane >> 5);
+          if (h0 < a.hd)
+            *(uint2*)(DQ + h0) = make_uint2(M32<DT>::pack(acc[o][4 * g] * a.scale, acc[o][4 * g + 1] * a.scale),
+                                            M32<DT>::pack(acc[o][4 * g + 2] * a.scale, acc[o][4 * g + 3] * a.scale));
+        }
+    }
+  } else if constexpr (NT == 512) {
+    float x[2 * NO];
+    sum_waves<NO>(acc, (float*)smem, wave, lane, x);
+    if (qok) {
+      uint16_t* DQ = a.dq + b * a.dq_sb + h * a.dq_sh + (int64_t)qi * a.dq_st;
+#pragma unroll
+      for (int o = 0; o < NO; ++o) {
+        const int h0 = o * 32 + acc_row(2 * wave, lane);
+        if (h0 < a.hd) *(uint32_t*)(DQ + h0) = M32<DT>::pack(x[2 * o] * a.scale, x[2 * o + 1] * a.scale);
       }
+    }
   }
-  if (q0 + q_step < a.Tq) load_rows(q0 + q_step);
+  }
+}
+
+// A tile of scores and of dP, [query][key], into P and dS / scale = P * (dP - delta) (the scale is applied to dK at the
+// end).  lse (times log2 e), delta: this lane's first query's (a lane's are 8 (r / 4) + r % 4 rows on); rows before
+// `first` do not see this lane's key.  The row of a register is a constant beside a lane's threshold, and lse and delta come four at a time:
+// 281 -> 241 instructions per step of 32 x 32 x 96, 197 tokens x 1024 heads of 64 100 -> 94 us (whole backward).
+__device__ __forceinline__ void p_and_ds(float16_t& s, float16_t& dp, const float* lse, const float* delta, float sc, int first) {
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const float4_t l = *(const float4_t*)(lse + 8 * g), d = *(const float4_t*)(delta + 8 * g);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int r = 4 * g + e;
+      const float p = __builtin_amdgcn_exp2f(s[r] * sc - l[e]);
+      s[r] = 8 * g + e < first ? 0.f : p;
+      dp[r] = s[r] * (dp[r] - d[e]);
+    }
   }
 }
 
 // dK/dV: workgroup = NT / 2 keys, wavefront = 32 of them; queries in steps of 32
 template <int DT, int HD, int NT>
-__global__ __launch_bounds__(NT) void attn_dkv_short_kernel(const AttnArgs a, int rows) {
+__global__ __launch_bounds__(NT) void attn_dkv_short_kernel(const AttnArgs a, int rows, int share) {
   constexpr int NC = HD / 16, NO = HD / 32, LD = HD + 8;
   extern __shared__ __align__(16) uint16_t smem[];
   uint16_t* sQ = smem;
   uint16_t* sDO = smem + rows * LD;
   float* sLse = (float*)(smem + 2 * rows * LD);
   float* sDelta = sLse + rows;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int bh = blockIdx.y, b = bh / a.H, h = bh % a.H;
   const int k_step = (int)gridDim.x * (NT / 2);
   int kw0 = blockIdx.x * (NT / 2) + wave * 32;
@@ -843,25 +993,34 @@ __global__ __launch_bounds__(NT) void attn_dkv_short_kernel(const AttnArgs a, in
   const float sc = a.scale * LOG2E;
   const int shift = a.Tk - a.Tq;
 
+  const HeadRows rk(K, a.k_st, a.Tk, a.hd), rv(V, a.v_st, a.Tk, a.hd);
+  const HeadRows rq(a.q + b * a.q_sb + h * a.q_sh, a.q_st, a.Tq, a.hd), rdo(a.d_o + b * a.do_sb + h * a.do_sh, a.do_st, a.Tq, a.hd);
   uint4 kf[NC], vf[NC];
   auto load_rows = [&](int ks) {   // this lane's key row of the tile at `ks`
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-      kf[c] = load_row8(K, a.k_st, ks + (lane & 31), a.Tk, c * 16 + (lane >> 5) * 8, a.hd);
-      vf[c] = load_row8(V, a.v_st, ks + (lane & 31), a.Tk, c * 16 + (lane >> 5) * 8, a.hd);
+      kf[c] = rk.load(ks + (lane & 31), c * 16 + (lane >> 5) * 8);
+      vf[c] = rv.load(ks + (lane & 31), c * 16 + (lane >> 5) * 8);
     }
   };
-  load_rows(kw0);   // the first tile's rows are requested before the head is loaded
-  for (int i = tid; i < rows; i += NT) {
-    // rows past the end: Q and dO rows are zero, lse = +inf makes their P exactly zero
-    sLse[i] = i < a.Tq ? a.lse[(int64_t)bh * a.Tq + i] * LOG2E : INFINITY;
-    sDelta[i] = i < a.Tq ? a.delta[(int64_t)bh * a.Tq + i] : 0.f;
+  {
+    HeadPair<HD, NT> qd;
+    qd.issue(rq, rdo, rows, tid);
+    load_rows(kw0);
+    for (int i = tid; i < rows; i += NT) {
+      // rows past the end: Q and dO rows are zero, lse = +inf makes their P exactly zero
+      sLse[i] = i < a.Tq ? a.lse[(int64_t)bh * a.Tq + i] * LOG2E : INFINITY;
+      sDelta[i] = i < a.Tq ? a.delta[(int64_t)bh * a.Tq + i] : 0.f;
+    }
+    qd.finish(rq, rdo, sQ, sDO, rows, tid);
   }
-  load_heads<HD, NT>(a.q + b * a.q_sb + h * a.q_sh, a.q_st, a.d_o + b * a.do_sb + h * a.do_sh, a.do_st, a.Tq, a.hd, rows,
-                 sQ, sDO, tid);
   __syncthreads();
-  // no barrier follows: a wavefront without a key tile leaves, one with several loops
-  for (; kw0 < a.Tk; kw0 += k_step) {
+  // no barrier follows but for a shared tile: a wavefront without a key tile leaves, one with several loops
+  constexpr int SHARED = NT / 2;             // the tile from here on is shared by all wavefronts where they share one
+  const bool sharing = NT == 512 && share;
+  for (; kw0 < a.Tk; kw0 = sharing ? (kw0 < SHARED ? SHARED : a.Tk) : kw0 + k_step) {
+  const bool shared = sharing && kw0 >= SHARED;
+  const int q_step = shared ? NT / 2 : 32;
   const int kj = kw0 + (lane & 31);
   const bool kok = kj < a.Tk;
   float16_t dk[NO], dv[NO];
@@ -871,8 +1030,7 @@ __global__ __launch_bounds__(NT) void attn_dkv_short_kernel(const AttnArgs a, in
     for (int r = 0; r < 16; ++r) dk[o][r] = dv[o][r] = 0.f;
   int q_begin = 0;
   if (a.causal) q_begin = max(0, kw0 - shift) / 32 * 32;   // queries i with i + shift >= kw0 see this wavefront's keys
-  for (int q0 = q_begin; q0 < a.Tq; q0 += 32) {
-    const bool masked = a.causal && (kw0 + 31 > q0 + shift);
+  for (int q0 = q_begin + (shared ? wave * 32 : 0); q0 < a.Tq; q0 += q_step) {
     float16_t s, dp;
 #pragma unroll
     for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
@@ -882,14 +1040,8 @@ __global__ __launch_bounds__(NT) void attn_dkv_short_kernel(const AttnArgs a, in
       s = M32<DT>::run(*(const uint4*)(sQ + off), kf[c], s);
       dp = M32<DT>::run(*(const uint4*)(sDO + off), vf[c], dp);
     }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int ql = q0 + acc_row(r, lane);
-      float p = __builtin_amdgcn_exp2f(s[r] * sc - sLse[ql]);
-      if (masked && kj > ql + shift) p = 0.f;
-      s[r] = p;
-      dp[r] = p * (dp[r] - sDelta[ql]);
-    }
+    const int ql = q0 + 4 * (lane >> 5);
+    p_and_ds(s, dp, sLse + ql, sDelta + ql, sc, a.causal ? kj - (ql + shift) : 0);
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const uint4 pf = pack8<DT>(s, 8 * j);
@@ -901,23 +1053,42 @@ __global__ __launch_bounds__(NT) void attn_dkv_short_kernel(const AttnArgs a, in
       }
     }
   }
-  if (kok) {
-    uint16_t* DK = a.dk + b * a.dk_sb + h * a.dk_sh + (int64_t)kj * a.dk_st;
-    uint16_t* DV = a.dv + b * a.dv_sb + h * a.dv_sh + (int64_t)kj * a.dv_st;
+  if (!shared) {
+    const int kn = sharing ? SHARED : kw0 + k_step;
+    if (kn < a.Tk) load_rows(kn);
+    if (kok) {
+      uint16_t* DK = a.dk + b * a.dk_sb + h * a.dk_sh + (int64_t)kj * a.dk_st;
+      uint16_t* DV = a.dv + b * a.dv_sb + h * a.dv_sh + (int64_t)kj * a.dv_st;
 #pragma unroll
-    for (int o = 0; o < NO; ++o)
+      for (int o = 0; o < NO; ++o)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int h0 = o * 32 + 8 * g + 4 * (lane >> 5);
+        for (int g = 0; g < 4; ++g) {
+          const int h0 = o * 32 + 8 * g + 4 * (lane >> 5);
+          if (h0 < a.hd) {
+            *(uint2*)(DK + h0) = make_uint2(M32<DT>::pack(dk[o][4 * g] * a.scale, dk[o][4 * g + 1] * a.scale),
+                                            M32<DT>::pack(dk[o][4 * g + 2] * a.scale, dk[o][4 * g + 3] * a.scale));
+            *(uint2*)(DV + h0) = make_uint2(M32<DT>::pack(dv[o][4 * g], dv[o][4 * g + 1]),
+                                            M32<DT>::pack(dv[o][4 * g + 2], dv[o][4 * g + 3]));
+          }
+        }
+    }
+  } else if constexpr (NT == 512) {
+    float xk[2 * NO], xv[2 * NO];
+    sum_waves<NO>(dk, (float*)smem, wave, lane, xk);
+    sum_waves<NO>(dv, (float*)smem, wave, lane, xv);
+    if (kok) {
+      uint16_t* DK = a.dk + b * a.dk_sb + h * a.dk_sh + (int64_t)kj * a.dk_st;
+      uint16_t* DV = a.dv + b * a.dv_sb + h * a.dv_sh + (int64_t)kj * a.dv_st;
+#pragma unroll
+      for (int o = 0; o < NO; ++o) {
+        const int h0 = o * 32 + acc_row(2 * wave, lane);
         if (h0 < a.hd) {
-          *(uint2*)(DK + h0) = make_uint2(M32<DT>::pack(dk[o][4 * g] * a.scale, dk[o][4 * g + 1] * a.scale),
-                                          M32<DT>::pack(dk[o][4 * g + 2] * a.scale, dk[o][4 * g + 3] * a.scale));
-          *(uint2*)(DV + h0) = make_uint2(M32<DT>::pack(dv[o][4 * g], dv[o][4 * g + 1]),
-                                          M32<DT>::pack(dv[o][4 * g + 2], dv[o][4 * g + 3]));
+          *(uint32_t*)(DK + h0) = M32<DT>::pack(xk[2 * o] * a.scale, xk[2 * o + 1] * a.scale);
+          *(uint32_t*)(DV + h0) = M32<DT>::pack(xv[2 * o], xv[2 * o + 1]);
         }
       }
+    }
   }
-  if (kw0 + k_step < a.Tk) load_rows(kw0 + k_step);
   }
 }
 
@@ -937,33 +1108,42 @@ __global__ __launch_bounds__(512) void attn_bwd_short_fused_kernel(const AttnArg
   uint16_t* sDO = sQ + rows_q * LD;
   float* sLse = (float*)(sDO + rows_q * LD);
   float* sDelta = sLse + rows_q;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int bh = blockIdx.y, b = bh / a.H, h = bh % a.H;
   const uint16_t* OO = a.o + b * a.o_sb + h * a.o_sh;
   const float sc = a.scale * LOG2E;
   const int shift = a.Tk - a.Tq;
 
-  // delta = rowsum(dO * O) and lse of this lane's query row: requested before the head is loaded
+  // delta = rowsum(dO * O) and lse of this lane's query row
   const int q0 = wave * 32, qi = q0 + (lane & 31);
   const bool qok = qi < a.Tq;
-  const uint16_t* DOg = a.d_o + b * a.do_sb + h * a.do_sh;
+  const HeadRows rdo(a.d_o + b * a.do_sb + h * a.do_sh, a.do_st, a.Tq, a.hd), ro(OO, a.o_st, a.Tq, a.hd);
+  const HeadRows rq(a.q + b * a.q_sb + h * a.q_sh, a.q_st, a.Tq, a.hd);
+  const HeadRows rk(a.k + b * a.k_sb + h * a.k_sh, a.k_st, a.Tk, a.hd), rv(a.v + b * a.v_sb + h * a.v_sh, a.v_st, a.Tk, a.hd);
   float dlt = 0.f;
-#pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    const int h0 = c * 16 + (lane >> 5) * 8;
-    const uint4 dof = load_row8(DOg, a.do_st, qi, a.Tq, h0, a.hd);
-    const uint4 of = load_row8(OO, a.o_st, qi, a.Tq, h0, a.hd);
-    float x[8], y[8];
-    unpack8<DT>(dof, x);
-    unpack8<DT>(of, y);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) dlt += x[k] * y[k];
-  }
-  dlt += __shfl_xor(dlt, 32, 64);
   const float lse2 = qok ? a.lse[(int64_t)bh * a.Tq + qi] * LOG2E : INFINITY;
-  load_heads<HD, NT>(a.k + b * a.k_sb + h * a.k_sh, a.k_st, a.v + b * a.v_sb + h * a.v_sh, a.v_st, a.Tk, a.hd, rows_k, sK,
-                     sV, tid);
-  load_heads<HD, NT>(a.q + b * a.q_sb + h * a.q_sh, a.q_st, DOg, a.do_st, a.Tq, a.hd, rows_q, sQ, sDO, tid);
+  {
+    HeadPair<HD, NT> kv, qd;
+    uint4 dof[NC], of[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      dof[c] = rdo.load(qi, c * 16 + (lane >> 5) * 8);
+      of[c] = ro.load(qi, c * 16 + (lane >> 5) * 8);
+    }
+    kv.issue(rk, rv, rows_k, tid);
+    qd.issue(rq, rdo, rows_q, tid);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      float x[8], y[8];
+      unpack8<DT>(dof[c], x);
+      unpack8<DT>(of[c], y);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) dlt += x[k] * y[k];
+    }
+    dlt += __shfl_xor(dlt, 32, 64);
+    kv.finish(rk, rv, sK, sV, rows_k, tid);
+    qd.finish(rq, rdo, sQ, sDO, rows_q, tid);
+  }
   if (q0 < rows_q && (lane >> 5) == 0) {
     // rows past the end: Q and dO rows are zero, lse = +inf makes their P exactly zero
     sLse[qi] = lse2;
@@ -1050,7 +1230,6 @@ __global__ __launch_bounds__(512) void attn_bwd_short_fused_kernel(const AttnArg
   int q_begin = 0;
   if (a.causal) q_begin = max(0, kw0 - shift) / 32 * 32;
   for (int qs = q_begin; qs < a.Tq; qs += 32) {
-    const bool masked = a.causal && (kw0 + 31 > qs + shift);
     float16_t s, dp;
 #pragma unroll
     for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
@@ -1060,14 +1239,8 @@ __global__ __launch_bounds__(512) void attn_bwd_short_fused_kernel(const AttnArg
       s = M32<DT>::run(*(const uint4*)(sQ + off), kf[c], s);
       dp = M32<DT>::run(*(const uint4*)(sDO + off), vf[c], dp);
     }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int ql = qs + acc_row(r, lane);
-      float p = __builtin_amdgcn_exp2f(s[r] * sc - sLse[ql]);
-      if (masked && kj > ql + shift) p = 0.f;
-      s[r] = p;
-      dp[r] = p * (dp[r] - sDelta[ql]);
-    }
+    const int ql = qs + 4 * (lane >> 5);
+    p_and_ds(s, dp, sLse + ql, sDelta + ql, sc, a.causal ? kj - (ql + shift) : 0);
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const uint4 pf = pack8<DT>(s, 8 * j);
@@ -1120,7 +1293,11 @@ int check_common(const pf_attn_desc* d, const char* name) {
 }
 
 // whole operands in LDS: two of them (and their padding) fit for head dims up to 96
-bool short_ok(const pf_attn_desc* d) { return d->Tq <= SHORT_T && d->Tk <= SHORT_T && d->hd <= 96; }
+bool short_ok(const pf_attn_desc* d, bool bwd) {
+  auto near = [](int64_t st) { return st >= 0 && st < (1 << 30) / SHORT_T; };   // (a head's rows within 2 GiB)
+  return d->Tq <= SHORT_T && d->Tk <= SHORT_T && d->hd <= 96 && near(d->q_st) && near(d->k_st) && near(d->v_st) &&
+         (!bwd || (near(d->o_st) && near(d->do_st)));
+}
 
 AttnArgs make_args(const pf_attn_desc* d) {
   AttnArgs a;
@@ -1149,28 +1326,39 @@ int launch_short(K kern, dim3 grid, int threads, size_t lds, hipStream_t st, Arg
   return PF_OK;
 }
 
+// Does a workgroup of eight wavefronts share the ninth tile of the T tokens along its axis?  Not under a mask
+// (the wavefronts' own tiles differ in work, and all have to wait for the last: 275 causal tokens x 128 heads of 88 16.5 ->
+// 18.1 us, backward 45.6 -> 50.5), and not over a sweep of few tiles, which costs less than the exchange (288 queries of
+// 77 keys, backward 36.9 -> 45.6; 257 of 257 57 -> 49).
+bool shares_tile(const pf_attn_desc* d, int64_t T, int64_t sweep) { return !d->causal && T > 256 && sweep > 192; }
+
+// LDS of a short-sequence kernel whose operands take `operands` bytes; the partial results of a shared tile (eight
+// accumulator tiles, and maxima and sums) take their place.
+inline size_t lds_with_shared_tile(size_t operands, int share, int HD) {
+  const size_t partial = 2048 + (size_t)8 * (HD / 32) * 16 * 64 * 4;
+  return share && partial > operands ? partial : operands;
+}
+
 // T: tokens along the axis the workgroups divide (queries, or keys for dK/dV), in tiles of 32 per
-// wavefront.  A head of more than 128 tokens takes ONE workgroup of eight wavefronts (its two LDS
-// operands are fetched once; the tiles past the eighth, e.g. the 257th token's, are a second pass of
-// the first wavefronts).  NT96: workgroup size for head dims above 64, 512 where the kernel's
-// registers allow two wavefronts per SIMD (forward, dQ), else 256: then every workgroup takes four
+// wavefront.  A head of more than 128 tokens takes ONE workgroup of eight wavefronts, its two LDS
+// operands are fetched once.  WIDE96 false, at head dims above 64: workgroups of four; each takes four
 // tiles and a remainder of one or two tiles becomes a second pass instead of a workgroup (and a
 // load of the whole head) of its own.
-#define PF_ATTN_SHORT(KERNEL, NT96, rc, T, BH, lds, st, dt, hd, ...)                                            \
+#define PF_ATTN_SHORT(KERNEL, WIDE96, rc, T, BH, lds, st, dt, hd, ...)                                          \
   do {                                                                                                         \
     const int tiles_ = ((T) + 31) / 32;                                                                        \
-    const bool w64_ = (hd) <= 64 && (T) > 128, w96_ = (hd) > 64 && (NT96) == 512 && (T) > 128;                  \
+    const bool w64_ = (hd) <= 64 && (T) > 128, w96_ = (hd) > 64 && (WIDE96) && (T) > 128;                       \
     const int gx_ = (w64_ || w96_) ? 1 : ((tiles_ + 1) / 4 > 1 ? (tiles_ + 1) / 4 : 1);                         \
     const dim3 grid_((unsigned)gx_, (unsigned)(BH));                                                           \
     if (dt == PF_F16) {                                                                                        \
       if (w64_) rc = launch_short(KERNEL<PF_F16, 64, 512>, grid_, 512, (lds)(64), st, __VA_ARGS__);             \
       else if (hd <= 64) rc = launch_short(KERNEL<PF_F16, 64, 256>, grid_, 256, (lds)(64), st, __VA_ARGS__);    \
-      else if (w96_) rc = launch_short(KERNEL<PF_F16, 96, NT96>, grid_, NT96, (lds)(96), st, __VA_ARGS__);      \
+      else if (w96_) rc = launch_short(KERNEL<PF_F16, 96, 512>, grid_, 512, (lds)(96), st, __VA_ARGS__);        \
       else rc = launch_short(KERNEL<PF_F16, 96, 256>, grid_, 256, (lds)(96), st, __VA_ARGS__);                  \
     } else {                                                                                                   \
       if (w64_) rc = launch_short(KERNEL<PF_BF16, 64, 512>, grid_, 512, (lds)(64), st, __VA_ARGS__);            \
       else if (hd <= 64) rc = launch_short(KERNEL<PF_BF16, 64, 256>, grid_, 256, (lds)(64), st, __VA_ARGS__);   \
-      else if (w96_) rc = launch_short(KERNEL<PF_BF16, 96, NT96>, grid_, NT96, (lds)(96), st, __VA_ARGS__);     \
+      else if (w96_) rc = launch_short(KERNEL<PF_BF16, 96, 512>, grid_, 512, (lds)(96), st, __VA_ARGS__);       \
       else rc = launch_short(KERNEL<PF_BF16, 96, 256>, grid_, 256, (lds)(96), st, __VA_ARGS__);                 \
     }                                                                                                          \
   } while (0)
@@ -1195,10 +1383,11 @@ extern "C" int pf_attention_fwd(const pf_attn_desc* d, void* stream) {
              "pf_attention_fwd: bad output operand");
   AttnArgs a = make_args(d);
   const dim3 grid((unsigned)((d->Tq + 127) / 128), (unsigned)(d->B * d->H));
-  if (short_ok(d)) {
+  if (short_ok(d, false)) {
     const int rows = (d->Tk + 31) / 32 * 32;
-    auto lds = [rows](int HD) { return (size_t)2 * rows * (HD + 8) * 2; };
-    PF_ATTN_SHORT(attn_fwd_short_kernel, 512, rc, d->Tq, d->B * d->H, lds, (hipStream_t)stream, d->dtype, d->hd, a, rows);
+    const int share = shares_tile(d, d->Tq, d->Tk);
+    auto lds = [rows, share](int HD) { return lds_with_shared_tile((size_t)2 * rows * (HD + 8) * 2, share, HD); };
+    PF_ATTN_SHORT(attn_fwd_short_kernel, true, rc, d->Tq, d->B * d->H, lds, (hipStream_t)stream, d->dtype, d->hd, a, rows, share);
     if (rc != PF_OK) return rc;
   } else {
     PF_ATTN_DISPATCH(attn_fwd_kernel, grid, (hipStream_t)stream, a, d->dtype, d->hd);
@@ -1223,7 +1412,7 @@ extern "C" int pf_attention_bwd(const pf_attn_desc* d, void* stream) {
   if (d->dtype == PF_BF16) ad.causal |= 0x100;  // dtype flag for the delta kernel
   const dim3 gq((unsigned)((d->Tq + 127) / 128), (unsigned)(d->B * d->H));
   const dim3 gk((unsigned)((d->Tk + 127) / 128), (unsigned)(d->B * d->H));
-  if (short_ok(d)) {
+  if (short_ok(d, true)) {
     const int rows_k = (d->Tk + 31) / 32 * 32, rows_q = (d->Tq + 31) / 32 * 32;
     if (d->hd <= 64 && d->Tq <= 256 && d->Tk <= 256 && (d->Tq > 128 || d->Tk > 128)) {
       // one workgroup per head forms dQ, dK and dV from a single load of the head
@@ -1236,11 +1425,19 @@ extern "C" int pf_attention_bwd(const pf_attn_desc* d, void* stream) {
       return PF_OK;
     }
     // dQ first: it also leaves delta = rowsum(dO * O) for the dK/dV kernel
-    auto lds_q = [rows_k](int HD) { return (size_t)2 * rows_k * (HD + 8) * 2; };
-    auto lds_k = [rows_q](int HD) { return (size_t)2 * rows_q * (HD + 8) * 2 + (size_t)rows_q * 8; };
-    PF_ATTN_SHORT(attn_dq_short_kernel, 512, rc, d->Tq, d->B * d->H, lds_q, st, d->dtype, d->hd, a, d->delta, rows_k);
+    const int share_q = shares_tile(d, d->Tq, d->Tk), share_k = shares_tile(d, d->Tk, d->Tq);
+    auto lds_q = [rows_k, share_q](int HD) { return lds_with_shared_tile((size_t)2 * rows_k * (HD + 8) * 2, share_q, HD); };
+    auto lds_k = [rows_q, share_k](int HD) {
+      return lds_with_shared_tile((size_t)2 * rows_q * (HD + 8) * 2 + (size_t)rows_q * 8, share_k, HD);
+    };
+    PF_ATTN_SHORT(attn_dq_short_kernel, true, rc, d->Tq, d->B * d->H, lds_q, st, d->dtype, d->hd, a, d->delta, rows_k, share_q);
     if (rc != PF_OK) return rc;
-    PF_ATTN_SHORT(attn_dkv_short_kernel, 256, rc, d->Tk, d->B * d->H, lds_k, st, d->dtype, d->hd, a, rows_q);
+    // dK/dV above head dim 64: one workgroup of eight wavefronts per head, or two of four, which fill more of the chip while
+    // there are few heads (two -> one, us of backward: 197 tokens x 64 heads of 80 31.0 -> 33.8, x 128 of 88 37.6 -> 39.4, x 192
+    // 53 -> 41, x 384 91 -> 82; 257 tokens x 768 261 -> 206).  Up to six tiles the second form is one workgroup too (145
+    // tokens x 96 heads: 28.5 -> 25.9 on eight).
+    const bool wide = d->B * d->H > 128 || d->Tk <= 192;
+    PF_ATTN_SHORT(attn_dkv_short_kernel, wide, rc, d->Tk, d->B * d->H, lds_k, st, d->dtype, d->hd, a, rows_q, share_k);
     if (rc != PF_OK) return rc;
     PF_CHECK_LAUNCH("pf_attention_bwd");
     return PF_OK;
