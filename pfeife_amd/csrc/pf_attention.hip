@@ -76,14 +76,30 @@ __device__ __forceinline__ uint4 load_row8(const uint16_t* base, int64_t st, int
 
 // One [ROWS tokens][HD] tile in flight: NV 16-byte vectors per thread, loaded from global into
 // registers while the previous tile is being multiplied, stored to LDS ([KT][HD + 8]) afterwards.
-template <int HD, int ROWS = KT> struct Tile {
+// The loads go through a buffer descriptor at the tile's first row: an offset out of its range reads zeros, where a test in front of
+// each load was a branch and a 64-bit product (2048 causal tokens x 128 heads of 64: forward 112 -> 106 us, backward 350 -> 332;
+// 577 x 32 heads of 88: forward 23.0 -> 19.2).  FAR: tokens so far apart that a tile spans 2 GiB keep that form.
+template <int HD, int ROWS = KT, bool FAR = false> struct Tile {
   static constexpr int LD = HD + 8, VPR = HD / 8, NV = (ROWS * VPR + 255) / 256;
   uint4 v[NV];
   __device__ __forceinline__ void load(const uint16_t* base, int64_t st, int t0, int T, int hd, int tid) {
+    if constexpr (FAR) {
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int e = tid + i * 256;
-      v[i] = (e < ROWS * VPR) ? load_row8(base, st, t0 + e / VPR, T, (e % VPR) * 8, hd) : make_uint4(0, 0, 0, 0);
+      for (int i = 0; i < NV; ++i) {
+        const int e = tid + i * 256;
+        v[i] = (e < ROWS * VPR) ? load_row8(base, st, t0 + e / VPR, T, (e % VPR) * 8, hd) : make_uint4(0, 0, 0, 0);
+      }
+    } else {
+      typedef int v4 __attribute__((ext_vector_type(4)));
+      const __amdgpu_buffer_rsrc_t rs =
+          __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base + (int64_t)t0 * st), 0, 0x7fffffff, 0x00020000);
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const int e = tid + i * 256, t = e / VPR, c = (e % VPR) * 8;
+        const bool ok = e < ROWS * VPR && t0 + t < T && c < hd;
+        const v4 x = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(ok ? (uint32_t)(t * (int)st + c) * 2u : 0x80000000u), 0, 0);
+        v[i] = make_uint4((uint32_t)x.x, (uint32_t)x.y, (uint32_t)x.z, (uint32_t)x.w);
+      }
     }
   }
   __device__ __forceinline__ void store(uint16_t* s, int tid) const {
@@ -145,12 +161,12 @@ __device__ __forceinline__ void attn_block(const AttnArgs& a, bool heavy_is_last
 // itself takes registers for one: forward 577 tokens x 56 heads of 88 47 -> 28 us, 2048 causal tokens x 64 heads of
 // 128 166 -> 104 us.  dQ of 128 and dK/dV above 96 would spill (dK/dV of 128 by 307 registers: 498 -> 793 us).
 // ---------------------------------------------------------------------------------
-template <int DT, int HD>
+template <int DT, int HD, bool FAR = false>
 __global__ __launch_bounds__(256, HD <= 64 ? 3 : 2) void attn_fwd_kernel(const AttnArgs a) {
   constexpr int NC = HD / 16, NO = HD / 32, KLD = HD + 8;
   __shared__ __align__(16) uint16_t sK[KT * KLD];
   __shared__ __align__(16) uint16_t sV[KT * KLD];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int qb, bh;
   attn_block(a, true, qb, bh);
   const int b = bh / a.H, h = bh % a.H;
@@ -178,7 +194,7 @@ __global__ __launch_bounds__(256, HD <= 64 ? 3 : 2) void attn_fwd_kernel(const A
     const int last_q = min(qb * 128 + 127, a.Tq - 1);
     k_end = min(a.Tk, last_q + shift + 1);
   }
-  Tile<HD> tk, tv;
+  Tile<HD, KT, FAR> tk, tv;
   tk.load(K, a.k_st, 0, a.Tk, a.hd, tid);
   tv.load(V, a.v_st, 0, a.Tk, a.hd, tid);
   for (int k0 = 0; k0 < k_end; k0 += KT) {
@@ -315,12 +331,12 @@ __global__ __launch_bounds__(256) void attn_delta_kernel(const AttnArgs a, float
 // ---------------------------------------------------------------------------------
 // dQ: same tiling as forward (column = query); dQ^T[hd][q] += K^T[hd][kv] dS^T[kv][q]
 // ---------------------------------------------------------------------------------
-template <int DT, int HD>
+template <int DT, int HD, bool FAR = false>
 __global__ __launch_bounds__(256, HD <= 96 ? 2 : 1) void attn_dq_kernel(const AttnArgs a) {
   constexpr int NC = HD / 16, NO = HD / 32, KLD = HD + 8;
   __shared__ __align__(16) uint16_t sK[KT * KLD];
   __shared__ __align__(16) uint16_t sV[KT * KLD];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int qb, bh;
   attn_block(a, true, qb, bh);
   const int b = bh / a.H, h = bh % a.H;
@@ -355,7 +371,7 @@ __global__ __launch_bounds__(256, HD <= 96 ? 2 : 1) void attn_dq_kernel(const At
     const int last_q = min(qb * 128 + 127, a.Tq - 1);
     k_end = min(a.Tk, last_q + shift + 1);
   }
-  Tile<HD> tk, tv;
+  Tile<HD, KT, FAR> tk, tv;
   tk.load(K, a.k_st, 0, a.Tk, a.hd, tid);
   tv.load(V, a.v_st, 0, a.Tk, a.hd, tid);
   for (int k0 = 0; k0 < k_end; k0 += KT) {
@@ -423,7 +439,7 @@ __global__ __launch_bounds__(256, HD <= 96 ? 2 : 1) void attn_dq_kernel(const At
 // tile, its four wavefronts each take a quarter of every staged block of 128 queries, and their
 // accumulators are added at the end through LDS in wavefront order, so that a head's dK/dV come
 // from 4 x ceil(Tk / 32) wavefronts instead of ceil(Tk / 32).
-template <int DT, int HD, bool SPLITQ = false>
+template <int DT, int HD, bool SPLITQ = false, bool FAR = false>
 __global__ __launch_bounds__(256, SPLITQ || HD > 96 ? 1 : 2) void attn_dkv_kernel(const AttnArgs a) {
   constexpr int NC = HD / 16, NO = HD / 32, QLD = HD + 8;
   constexpr int QT = SPLITQ ? 128 : KT;        // queries staged per iteration
@@ -432,7 +448,7 @@ __global__ __launch_bounds__(256, SPLITQ || HD > 96 ? 1 : 2) void attn_dkv_kerne
   uint16_t* sQ = sQD;
   uint16_t* sDO = sQD + QT * QLD;
   __shared__ float sLse[QT], sDelta[QT];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int kb, bh;
   attn_block(a, false, kb, bh);
   const int b = bh / a.H, h = bh % a.H;
@@ -464,7 +480,7 @@ __global__ __launch_bounds__(256, SPLITQ || HD > 96 ? 1 : 2) void attn_dkv_kerne
     q_begin = max(0, (SPLITQ ? kb * 32 : kb * 128) - shift);
     q_begin = q_begin / QT * QT;
   }
-  Tile<HD, QT> tq, tdo;
+  Tile<HD, QT, FAR> tq, tdo;
   float r_lse = 0.f, r_dlt = 0.f;
   auto prefetch = [&](int q0) {
     tq.load(Q, a.q_st, q0, a.Tq, a.hd, tid);
@@ -487,38 +503,41 @@ __global__ __launch_bounds__(256, SPLITQ || HD > 96 ? 1 : 2) void attn_dkv_kerne
     }
     if (q0 + QT < a.Tq) prefetch(q0 + QT);
     __syncthreads();
-    // causal: rows before `first` (of this lane's) do not see its key; a constant against a threshold, 32 sums less per step
-    // than key against query: 2048 tokens x 128 heads backward 354 -> 350 us.  (Lighter still without the `causal` in every
-    // compare, or with vector loads of lse and delta: four registers spill, whose reloads wait for the next tile's loads, 392.)
-    const int first = a.causal ? kj - (q0 + qoff + 4 * (lane >> 5) + shift) : 0;
-    float16_t s[NH], dp[NH];
+    // causal: rows before `first` (of this lane's) do not see its key: a constant against a threshold that the compiler
+    // cannot take apart (it would test `causal` again in every compare).  Each half's P and dS are multiplied before the next half's
+    // scores exist: with both alive four registers spilled as soon as anything else changed, and their reloads wait
+    // for the next tile's loads.  2048 causal tokens x 128 heads backward 350 -> 332 us with the loads through descriptors (see
+    // Tile; without these two 349), 1024 x 80 heads 149 -> 137.
+    int first = a.causal ? kj - (q0 + qoff + 4 * (lane >> 5) + shift) : 0;
+    if constexpr (HD == 64) asm("" : "+v"(first));   // (96 has no register left for it)
 #pragma unroll
     for (int t = 0; t < NH; ++t) {
+      float16_t s, dp;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) s[t][r] = dp[t][r] = 0.f;
+      for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
         const int off = (qoff + t * 32 + (lane & 31)) * QLD + c * 16 + (lane >> 5) * 8;
-        s[t] = M32<DT>::run(*(const uint4*)(sQ + off), kf[c], s[t]);
-        dp[t] = M32<DT>::run(*(const uint4*)(sDO + off), vf[c], dp[t]);
+        s = M32<DT>::run(*(const uint4*)(sQ + off), kf[c], s);
+        dp = M32<DT>::run(*(const uint4*)(sDO + off), vf[c], dp);
       }
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int ql = qoff + t * 32 + acc_row(r, lane);
-        float p = __builtin_amdgcn_exp2f(s[t][r] * sc - sLse[ql]);
+        float p = __builtin_amdgcn_exp2f(s[r] * sc - sLse[ql]);
         if (t * 32 + 8 * (r >> 2) + (r & 3) < first) p = 0.f;
-        s[t][r] = p;                                         // P
-        dp[t][r] = p * (dp[t][r] - sDelta[ql]);              // dS / scale (applied to dK at the end)
+        s[r] = p;                                         // P
+        dp[r] = p * (dp[r] - sDelta[ql]);              // dS / scale (applied to dK at the end)
       }
-    }
 #pragma unroll
-    for (int j = 0; j < 2 * NH; ++j) {
-      const uint4 pf = pack8<DT>(s[j >> 1], 8 * (j & 1));
-      const uint4 dsf = pack8<DT>(dp[j >> 1], 8 * (j & 1));
+      for (int j = 2 * t; j < 2 * t + 2; ++j) {
+        const uint4 pf = pack8<DT>(s, 8 * (j & 1));
+        const uint4 dsf = pack8<DT>(dp, 8 * (j & 1));
 #pragma unroll
-      for (int o = 0; o < NO; ++o) {
-        dv[o] = M32<DT>::run(frag_tr<QLD>(sDO, qoff + 16 * j, o * 32, lane), pf, dv[o]);
-        dk[o] = M32<DT>::run(frag_tr<QLD>(sQ, qoff + 16 * j, o * 32, lane), dsf, dk[o]);
+        for (int o = 0; o < NO; ++o) {
+          dv[o] = M32<DT>::run(frag_tr<QLD>(sDO, qoff + 16 * j, o * 32, lane), pf, dv[o]);
+          dk[o] = M32<DT>::run(frag_tr<QLD>(sQ, qoff + 16 * j, o * 32, lane), dsf, dk[o]);
+        }
       }
     }
   }
@@ -1293,10 +1312,13 @@ int check_common(const pf_attn_desc* d, const char* name) {
 }
 
 // whole operands in LDS: two of them (and their padding) fit for head dims up to 96
+// Do `rows` token rows of each operand that is loaded lie within 2 GiB, so that 32-bit byte offsets reach them?
+bool rows_near(const pf_attn_desc* d, bool bwd, int rows) {
+  auto near = [rows](int64_t st) { return st >= 0 && st < (1 << 30) / rows; };
+  return near(d->q_st) && near(d->k_st) && near(d->v_st) && (!bwd || (near(d->o_st) && near(d->do_st)));
+}
 bool short_ok(const pf_attn_desc* d, bool bwd) {
-  auto near = [](int64_t st) { return st >= 0 && st < (1 << 30) / SHORT_T; };   // (a head's rows within 2 GiB)
-  return d->Tq <= SHORT_T && d->Tk <= SHORT_T && d->hd <= 96 && near(d->q_st) && near(d->k_st) && near(d->v_st) &&
-         (!bwd || (near(d->o_st) && near(d->do_st)));
+  return d->Tq <= SHORT_T && d->Tk <= SHORT_T && d->hd <= 96 && rows_near(d, bwd, SHORT_T);
 }
 
 AttnArgs make_args(const pf_attn_desc* d) {
@@ -1363,17 +1385,18 @@ inline size_t lds_with_shared_tile(size_t operands, int share, int HD) {
     }                                                                                                          \
   } while (0)
 
-#define PF_ATTN_DISPATCH(KERNEL, grid, st, a, dt, hd)                                          \
-  do {                                                                                         \
-    if (dt == PF_F16) {                                                                        \
-      if (hd <= 64) hipLaunchKernelGGL((KERNEL<PF_F16, 64>), grid, dim3(256), 0, st, a);       \
-      else if (hd <= 96) hipLaunchKernelGGL((KERNEL<PF_F16, 96>), grid, dim3(256), 0, st, a);     \
-      else hipLaunchKernelGGL((KERNEL<PF_F16, 128>), grid, dim3(256), 0, st, a);             \
-    } else {                                                                                   \
-      if (hd <= 64) hipLaunchKernelGGL((KERNEL<PF_BF16, 64>), grid, dim3(256), 0, st, a);      \
-      else if (hd <= 96) hipLaunchKernelGGL((KERNEL<PF_BF16, 96>), grid, dim3(256), 0, st, a);    \
-      else hipLaunchKernelGGL((KERNEL<PF_BF16, 128>), grid, dim3(256), 0, st, a);            \
-    }                                                                                          \
+// (...: the kernel's template arguments after type and head dim)
+#define PF_ATTN_DISPATCH(KERNEL, grid, st, a, dt, hd, ...)                                                    \
+  do {                                                                                                       \
+    if (dt == PF_F16) {                                                                                      \
+      if (hd <= 64) hipLaunchKernelGGL((KERNEL<PF_F16, 64, __VA_ARGS__>), grid, dim3(256), 0, st, a);         \
+      else if (hd <= 96) hipLaunchKernelGGL((KERNEL<PF_F16, 96, __VA_ARGS__>), grid, dim3(256), 0, st, a);    \
+      else hipLaunchKernelGGL((KERNEL<PF_F16, 128, __VA_ARGS__>), grid, dim3(256), 0, st, a);                 \
+    } else {                                                                                                 \
+      if (hd <= 64) hipLaunchKernelGGL((KERNEL<PF_BF16, 64, __VA_ARGS__>), grid, dim3(256), 0, st, a);        \
+      else if (hd <= 96) hipLaunchKernelGGL((KERNEL<PF_BF16, 96, __VA_ARGS__>), grid, dim3(256), 0, st, a);   \
+      else hipLaunchKernelGGL((KERNEL<PF_BF16, 128, __VA_ARGS__>), grid, dim3(256), 0, st, a);                \
+    }                                                                                                        \
   } while (0)
 
 extern "C" int pf_attention_fwd(const pf_attn_desc* d, void* stream) {
@@ -1390,7 +1413,8 @@ extern "C" int pf_attention_fwd(const pf_attn_desc* d, void* stream) {
     PF_ATTN_SHORT(attn_fwd_short_kernel, true, rc, d->Tq, d->B * d->H, lds, (hipStream_t)stream, d->dtype, d->hd, a, rows, share);
     if (rc != PF_OK) return rc;
   } else {
-    PF_ATTN_DISPATCH(attn_fwd_kernel, grid, (hipStream_t)stream, a, d->dtype, d->hd);
+    if (rows_near(d, false, 128)) PF_ATTN_DISPATCH(attn_fwd_kernel, grid, (hipStream_t)stream, a, d->dtype, d->hd, false);
+    else PF_ATTN_DISPATCH(attn_fwd_kernel, grid, (hipStream_t)stream, a, d->dtype, d->hd, true);
   }
   PF_CHECK_LAUNCH("pf_attention_fwd");
   return PF_OK;
@@ -1446,7 +1470,8 @@ extern "C" int pf_attention_bwd(const pf_attn_desc* d, void* stream) {
   hipLaunchKernelGGL(attn_delta_kernel, dim3((unsigned)((rows + 31) / 32)), dim3(256), 0, st, ad, d->delta);
   // few keys, many queries (cross attention to a short context): split each key tile's query sweep
   // over the four wavefronts of a workgroup
-  if ((int64_t)gk.x * gk.y < 200 && d->Tq >= 256 && d->hd <= 96) {   // (two 128-row tiles of more do not fit)
+  const bool near = rows_near(d, true, 128);
+  if (near && (int64_t)gk.x * gk.y < 200 && d->Tq >= 256 && d->hd <= 96) {   // (two 128-row tiles of more do not fit)
     const dim3 gs((unsigned)((d->Tk + 31) / 32), (unsigned)(d->B * d->H));
     if (d->dtype == PF_F16) {
       if (d->hd <= 64) hipLaunchKernelGGL((attn_dkv_kernel<PF_F16, 64, true>), gs, dim3(256), 0, st, a);
@@ -1455,10 +1480,13 @@ extern "C" int pf_attention_bwd(const pf_attn_desc* d, void* stream) {
       if (d->hd <= 64) hipLaunchKernelGGL((attn_dkv_kernel<PF_BF16, 64, true>), gs, dim3(256), 0, st, a);
       else hipLaunchKernelGGL((attn_dkv_kernel<PF_BF16, 96, true>), gs, dim3(256), 0, st, a);
     }
+  } else if (near) {
+    PF_ATTN_DISPATCH(attn_dkv_kernel, gk, st, a, d->dtype, d->hd, false, false);
   } else {
-    PF_ATTN_DISPATCH(attn_dkv_kernel, gk, st, a, d->dtype, d->hd);
+    PF_ATTN_DISPATCH(attn_dkv_kernel, gk, st, a, d->dtype, d->hd, false, true);
   }
-  PF_ATTN_DISPATCH(attn_dq_kernel, gq, st, a, d->dtype, d->hd);
+  if (near) PF_ATTN_DISPATCH(attn_dq_kernel, gq, st, a, d->dtype, d->hd, false);
+  else PF_ATTN_DISPATCH(attn_dq_kernel, gq, st, a, d->dtype, d->hd, true);
   PF_CHECK_LAUNCH("pf_attention_bwd");
   return PF_OK;
 }
