@@ -156,7 +156,10 @@ typedef struct pf_gemm_desc {
                       depth, 7 / 8 / 9 / 10 its 256x256 / 128x128 / 256x128 / 192x256 tiles
                       with eight wavefronts side by side, 11..14 register-staged kernel with 128x128 (8 wavefronts),
                       128x128, 128x64, 64x64 tiles, 15 direct-to-LDS kernel with 64x64 tiles, 16 / 17 the tiles of
-                      8 / 9 for row-major operands with K a multiple of 8 (15 takes these as well); PF_ERR_INVALID if it cannot run the problem */
+                      8 / 9 for row-major operands with K a multiple of 8 (15 takes these as well), 18 its 256x256 tile by four
+                      wavefronts, 64 deep, 19 its 192x128 tile (row-major products); PF_ERR_INVALID if it cannot run the
+                      problem.  0 may issue a row-major product as two launches over disjoint rows
+                      (pf_gemm_variant names the first) */
   float* colsum_ws; /* optional, with dact on the direct-to-LDS kernel (pf_gemm_variant ends in ", 5>"): the
                        launch also leaves the column sums of the 16-bit values it stores in C as partial
                        rows, ws[tile_row * N + column] for tile_row < ceil(M / BM) (BM: the variant's first

@@ -20,15 +20,15 @@
   int pf_gemm_x_##DT##_##XT(const pf_gemm_desc& d, hipStream_t st);    \
   int pf_gemm_xgroup_##DT##_##XT(const pf_gemm_desc* d, int n, hipStream_t st);
 #define PF_X_DECL_DT(DT) \
-  PF_X_DECL(DT, 1) PF_X_DECL(DT, 2) PF_X_DECL(DT, 3) PF_X_DECL(DT, 4) PF_X_DECL(DT, 5) PF_X_DECL(DT, 6) PF_X_DECL(DT, 7) PF_X_DECL(DT, 8) PF_X_DECL(DT, 9) PF_X_DECL(DT, 10) PF_X_DECL(DT, 11) PF_X_DECL(DT, 12)
+  PF_X_DECL(DT, 1) PF_X_DECL(DT, 2) PF_X_DECL(DT, 3) PF_X_DECL(DT, 4) PF_X_DECL(DT, 5) PF_X_DECL(DT, 6) PF_X_DECL(DT, 7) PF_X_DECL(DT, 8) PF_X_DECL(DT, 9) PF_X_DECL(DT, 10) PF_X_DECL(DT, 11) PF_X_DECL(DT, 12) PF_X_DECL(DT, 13)
 PF_X_DECL_DT(1)
 PF_X_DECL_DT(2)
 #undef PF_X_DECL_DT
 #undef PF_X_DECL
-static_assert(PF_F16 == 1 && PF_BF16 == 2 && PF_XT_COUNT == 13, "the table below is written out for these ids");
+static_assert(PF_F16 == 1 && PF_BF16 == 2 && PF_XT_COUNT == 14, "the table below is written out for these ids");
 typedef int (*pf_x_fn)(const pf_gemm_desc&, hipStream_t);
 typedef int (*pf_xgroup_fn)(const pf_gemm_desc*, int, hipStream_t);
-#define PF_X_ROW(P, DT) {nullptr, P##DT##_1, P##DT##_2, P##DT##_3, P##DT##_4, P##DT##_5, P##DT##_6, P##DT##_7, P##DT##_8, P##DT##_9, P##DT##_10, P##DT##_11, P##DT##_12}
+#define PF_X_ROW(P, DT) {nullptr, P##DT##_1, P##DT##_2, P##DT##_3, P##DT##_4, P##DT##_5, P##DT##_6, P##DT##_7, P##DT##_8, P##DT##_9, P##DT##_10, P##DT##_11, P##DT##_12, P##DT##_13}
 static const pf_x_fn pf_x_table[3][PF_XT_COUNT] = {{}, PF_X_ROW(pf_gemm_x_, 1), PF_X_ROW(pf_gemm_x_, 2)};
 static const pf_xgroup_fn pf_xgroup_table[3][PF_XT_COUNT] = {{}, PF_X_ROW(pf_gemm_xgroup_, 1), PF_X_ROW(pf_gemm_xgroup_, 2)};
 #undef PF_X_ROW
@@ -589,16 +589,16 @@ int launch16(const pf_gemm_desc& d, hipStream_t st) {
 // Variant ids (pf_gemm_desc.variant; 0 = automatic):
 //   1..10  direct-to-LDS kernel, tiles PF_XT_256x256 / 256x128 / 128x128 / 192x256 / 128x128k2 / 256x128k2 /
 //          256x256w8 / 128x128w8 / 256x128w8 / 192x256w8
-//   18     direct-to-LDS kernel, tile PF_XT_256x256w4
+//   18, 19 direct-to-LDS kernel, tiles PF_XT_256x256w4 / PF_XT_192x128w8
 //   15     direct-to-LDS kernel, tile PF_XT_64x64; 16, 17: 128x128w8 and 256x128w8 for row-major products whose
 //          K is a multiple of 8 only (15 takes these too)
 //   11..14 register-staged kernel: 128x128 by 8 wavefronts, 128x128, 128x64, 64x64 by 4
 enum { V_AUTO = 0, V_X256 = 1, V_X256x128 = 2, V_X128 = 3, V_X192x256 = 4, V_X128K2 = 5, V_X256x128K2 = 6, V_X256W8 = 7, V_X128W8 = 8, V_X256x128W8 = 9, V_X192x256W8 = 10,
-       V_X64 = 15, V_X128W8R = 16, V_X256x128W8R = 17, V_X256W4 = 18, V_R128W8 = 11, V_R128 = 12, V_R128x64 = 13, V_R64 = 14 };
-inline bool is_x_variant(int v) { return (v >= V_X256 && v <= V_X192x256W8) || (v >= V_X64 && v <= V_X256W4); }
+       V_X64 = 15, V_X128W8R = 16, V_X256x128W8R = 17, V_X256W4 = 18, V_X192x128W8 = 19, V_R128W8 = 11, V_R128 = 12, V_R128x64 = 13, V_R64 = 14 };
+inline bool is_x_variant(int v) { return (v >= V_X256 && v <= V_X192x256W8) || (v >= V_X64 && v <= V_X192x128W8); }
 // tile id (PF_XT_*) of a direct-to-LDS variant
 inline int x_tile_of(int v) {
-  return v == V_X64 ? (int)PF_XT_64x64 : v == V_X128W8R ? (int)PF_XT_128x128w8 : v == V_X256x128W8R ? (int)PF_XT_256x128w8 : v == V_X256W4 ? (int)PF_XT_256x256w4 : v;
+  return v == V_X64 ? (int)PF_XT_64x64 : v == V_X128W8R ? (int)PF_XT_128x128w8 : v == V_X256x128W8R ? (int)PF_XT_256x128w8 : v == V_X256W4 ? (int)PF_XT_256x256w4 : v == V_X192x128W8 ? (int)PF_XT_192x128w8 : v;
 }
 
 // Register-staged tiles: 128x128 with two workgroups resident per CU is the largest that keeps
@@ -622,9 +622,9 @@ int choose_staged(const pf_gemm_desc& d) {
 // tile's loads in the first (some tiles, K a multiple of 8).
 bool x_supports(const pf_gemm_desc& d, int v) {
   const int xt = x_tile_of(v), bk = x_tile_bk(xt);
-  if ((xt == PF_XT_192x256 || xt == PF_XT_192x256w8) && d.a_trans) return false;   // no reduction-strided 192-row tile
+  if (x_tile_bm(xt) == 192 && d.a_trans) return false;   // no reduction-strided 192-row tile
   if (d.a_trans != d.b_trans) return false;
-  if (!d.a_trans && d.K % bk != 0 && !(v >= V_X64 && v != V_X256W4 && d.K % 8 == 0)) return false;
+  if (!d.a_trans && d.K % bk != 0 && !(v >= V_X64 && v < V_X256W4 && d.K % 8 == 0)) return false;
   return d.K >= bk;
 }
 
@@ -644,6 +644,7 @@ constexpr TileCost ROW_MAJOR[] = {{V_X256W4, 256, 256, 6.7, 0.95, 0.43, 6.3},
                                   {V_X256W8, 256, 256, 6.5, 0.95, 0.64, 6.2},
                                   {V_X192x256W8, 192, 256, 5.6, 0.78, 0.47, 5.8},
                                   {V_X256x128W8, 256, 128, 4.9, 0.47, 0.33, 4.4},
+                                  {V_X192x128W8, 192, 128, 5.3, 0.33, 0.26, 4.0},
                                   {V_X128W8, 128, 128, 3.6, 0.295, 0.176, 2.2},
                                   {V_X256x128W8R, 256, 128, 5.1, 0.49, 0.34, 4.4},   // (ragged K: only where the two above cannot)
                                   {V_X128W8R, 128, 128, 3.7, 0.305, 0.18, 2.2},
@@ -682,6 +683,11 @@ int choose_tile(const pf_gemm_desc& d, int64_t M, int bm, double& best_t) {
     // longer epilogue costs.  us on eight / four wavefronts, fp16, GELU and GELU': [3072 x 768] . [768 x 4096] 29.9 / 30.4, 34.2 /
     // 33.7; [4096 x 1024] . [1024 x 3152] 35.2 / 35.2, 39.7 / 38.9; over 2048 55.9 / 54.5, 60.6 / 57.8
     if (c.v == V_X256W4 && tiles <= 256 && d.K <= 1024 && (d.act != PF_ACT_NONE || d.dact != PF_ACT_NONE)) return;
+    // One round only: 130 to 200 tiles of 256x128 become 170 to 256 that each move three quarters of the operands.  us on
+    // 256x128 / 192x128, fp16: 4096 x 1280 over 1280 18.1 / 17.2, over 5120 54.9 / 49.7, over 10240 138.9 / 118.3, 3072 x 1408 over
+    // 1408 17.8 / 15.8, 12288 x 384 over 1536 20.0 / 17.8.  Over two rounds it lost to the larger tiles (8192 x 1280 over 1280 33.0
+    // against 28.9, 6168 x 1408 over 6144 118 against 113).
+    if (c.v == V_X192x128W8 && tiles > 256) return;
     const double t = tile_cost(c, tiles, d.K, strided);
     if (best < 0 || t < best_t) { best = c.v; best_t = t; }
   };
@@ -709,7 +715,7 @@ bool plan_split(const pf_gemm_desc& d, Split& s) {
   double best_t = 0.96 * single - 0.5;   // (less is within the model's error and a launch's)
   bool found = false;
   for (const TileCost& c : ROW_MAJOR) {
-    if (c.v == V_X64 || !x_supports(d, c.v)) continue;
+    if (c.v == V_X64 || c.v == V_X192x128W8 || !x_supports(d, c.v)) continue;
     const int64_t tn = (d.N + c.bn - 1) / c.bn;
     for (int64_t round = 1;; ++round) {
       const int64_t blocks = 256 * round / tn, rows = blocks * c.bm;
@@ -794,7 +800,7 @@ int dispatch16(const pf_gemm_desc& d, hipStream_t st) {
     }
   }
   switch (v) {
-    case V_X256: case V_X256x128: case V_X128: case V_X192x256: case V_X128K2: case V_X256x128K2: case V_X256W8: case V_X128W8: case V_X256x128W8: case V_X192x256W8: case V_X64: case V_X128W8R: case V_X256x128W8R: case V_X256W4: {
+    case V_X256: case V_X256x128: case V_X128: case V_X192x256: case V_X128K2: case V_X256x128K2: case V_X256W8: case V_X128W8: case V_X256x128W8: case V_X192x256W8: case V_X64: case V_X128W8R: case V_X256x128W8R: case V_X256W4: case V_X192x128W8: {
       const int xt = x_tile_of(v);
       if (!x_supports(d, v)) {
         pf_set_error("pf_gemm: variant %d needs both operands stored alike and (unless transposed) K a multiple of the stage depth", v);
@@ -956,12 +962,12 @@ extern "C" int pf_gemm_variant(const pf_gemm_desc* desc, char* out, int cap) {
   const char* bt = d.b_trans ? "true" : "false";
   const int v = resolve_variant(d);
   switch (v) {
-    case V_X256: case V_X256x128: case V_X128: case V_X192x256: case V_X128K2: case V_X256x128K2: case V_X256W8: case V_X128W8: case V_X256x128W8: case V_X192x256W8: case V_X64: case V_X128W8R: case V_X256x128W8R: case V_X256W4: {
+    case V_X256: case V_X256x128: case V_X128: case V_X192x256: case V_X128K2: case V_X256x128K2: case V_X256W8: case V_X128W8: case V_X256x128W8: case V_X192x256W8: case V_X64: case V_X128W8R: case V_X256x128W8R: case V_X256W4: case V_X192x128W8: {
       // BM, BN, BK, wavefront rows, columns, reduction split, stages: as rocprofv3 prints the instantiation
       static const char* shapes[PF_XT_COUNT] = {"", "256, 256, 32, 2, 2, 1, 5", "256, 128, 64, 2, 2, 1, 3", "128, 128, 64, 2, 2, 1, 3",
                                                 "192, 256, 32, 2, 2, 1, 5", "128, 128, 64, 2, 2, 2, 3", "256, 128, 64, 2, 2, 2, 3",
                                                 "256, 256, 32, 2, 4, 1, 5", "128, 128, 64, 2, 4, 1, 3", "256, 128, 64, 4, 2, 1, 3",
-                                                "192, 256, 32, 2, 4, 1, 5", "64, 64, 64, 2, 2, 1, 5", "256, 256, 64, 2, 2, 1, 2"};
+                                                "192, 256, 32, 2, 4, 1, 5", "64, 64, 64, 2, 2, 1, 5", "256, 256, 64, 2, 2, 1, 2", "192, 128, 64, 4, 2, 1, 3"};
       if (!x_supports(d, v)) {   // a pinned tile that cannot run this product: say so here, not at launch time
         pf_set_error("pf_gemm_variant: variant %d needs both operands stored alike, K >= %d and (unless both are "
                      "reduction-strided) K a multiple of %d", v, x_tile_bk(x_tile_of(v)), x_tile_bk(x_tile_of(v)));

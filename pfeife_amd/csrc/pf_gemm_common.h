@@ -196,9 +196,11 @@ __device__ __forceinline__ uint4 buf_load16(__amdgpu_buffer_rsrc_t r, uint32_t b
 //   id 11: 64x64 by four wavefronts, two workgroups to a CU, for small outputs
 //   id 12: 256x256 (64 deep, 2 stages, 3 of the right-hand operand) by four wavefronts with their accumulators in
 //   accumulation registers: the fastest per tile wherever K is a multiple of 64
-//   (ids 1-6 run where a descriptor pins them; the automatic choice takes 7-12, which were faster wherever measured)
+//   id 13: 192x128 (64 deep, 3 stages) by eight wavefronts, row-major products only: outputs of 130 to 200 tiles of 256x128, which
+//   leave a third of the compute units without one
+//   (ids 1-6 run where a descriptor pins them; the automatic choice takes 7-13, which were faster wherever measured)
 enum { PF_XT_256x256 = 1, PF_XT_256x128 = 2, PF_XT_128x128 = 3, PF_XT_192x256 = 4, PF_XT_128x128k2 = 5,
-       PF_XT_256x128k2 = 6, PF_XT_256x256w8 = 7, PF_XT_128x128w8 = 8, PF_XT_256x128w8 = 9, PF_XT_192x256w8 = 10, PF_XT_64x64 = 11, PF_XT_256x256w4 = 12, PF_XT_COUNT = 13 };
+       PF_XT_256x128k2 = 6, PF_XT_256x256w8 = 7, PF_XT_128x128w8 = 8, PF_XT_256x128w8 = 9, PF_XT_192x256w8 = 10, PF_XT_64x64 = 11, PF_XT_256x256w4 = 12, PF_XT_192x128w8 = 13, PF_XT_COUNT = 14 };
 // BM, BN, reduction depth per stage, stages, wavefront grid (rows x columns x reduction split) of each tile id
 template <int XT> struct XTile;
 template <> struct XTile<PF_XT_256x256> { static constexpr int BM = 256, BN = 256, BK = 32, ST = 5, WGM = 2, WGN = 2, KS = 1; };
@@ -212,13 +214,14 @@ template <> struct XTile<PF_XT_128x128w8> { static constexpr int BM = 128, BN = 
 template <> struct XTile<PF_XT_256x128w8> { static constexpr int BM = 256, BN = 128, BK = 64, ST = 3, WGM = 4, WGN = 2, KS = 1; };
 template <> struct XTile<PF_XT_192x256w8> { static constexpr int BM = 192, BN = 256, BK = 32, ST = 5, WGM = 2, WGN = 4, KS = 1; };
 template <> struct XTile<PF_XT_256x256w4> { static constexpr int BM = 256, BN = 256, BK = 64, ST = 2, WGM = 2, WGN = 2, KS = 1; };
+template <> struct XTile<PF_XT_192x128w8> { static constexpr int BM = 192, BN = 128, BK = 64, ST = 3, WGM = 4, WGN = 2, KS = 1; };
 template <> struct XTile<PF_XT_64x64> { static constexpr int BM = 64, BN = 64, BK = 64, ST = 5, WGM = 2, WGN = 2, KS = 1; };
 // tiles with a kernel for row-major products whose reduction length is no multiple of the stage depth: the
 // eight-wavefront 128x128 and 256x128 tiles and 64x64
 constexpr bool x_tile_ragged(int bm, int bn, int nw) { return (nw == 8 && bn == 128) || (bm == 64 && bn == 64); }
 constexpr int x_tile_bm(int xt) {
   return xt == PF_XT_64x64 ? 64 : (xt == PF_XT_128x128 || xt == PF_XT_128x128k2 || xt == PF_XT_128x128w8) ? 128
-         : (xt == PF_XT_192x256 || xt == PF_XT_192x256w8) ? 192 : 256;
+         : (xt == PF_XT_192x256 || xt == PF_XT_192x256w8 || xt == PF_XT_192x128w8) ? 192 : 256;
 }
 inline int x_tile_bk(int xt) { return (xt == PF_XT_256x256 || xt == PF_XT_192x256 || xt == PF_XT_256x256w8 || xt == PF_XT_192x256w8) ? 32 : 64; }
 

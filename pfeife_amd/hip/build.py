@@ -30,9 +30,9 @@ SOURCES = [
 ]
 
 # the direct-to-LDS MFMA kernel: one object per (operand dtype id, tile id), all from one source
-# (ids as in csrc/pf_gemm_common.h: dtypes PF_F16 = 1, PF_BF16 = 2; tiles PF_XT_* = 1..12)
+# (ids as in csrc/pf_gemm_common.h: dtypes PF_F16 = 1, PF_BF16 = 2; tiles PF_XT_* = 1..13)
 GEMM_X_SOURCE = "pf_gemm_x_inst.hip"
-GEMM_X_PAIRS = [(dt, xt) for xt in (12, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11) for dt in (1, 2)]
+GEMM_X_PAIRS = [(dt, xt) for xt in (12, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 13) for dt in (1, 2)]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
