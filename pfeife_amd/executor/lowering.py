@@ -472,7 +472,7 @@ class BwdCtx:
             self.flush_dw()          # two products into one accumulator keep their order
             self._dw_big = []
         if tiles >= self.FULL_GRID:
-            self.emit(launch)
+            self._emit_dw(launch)
             self._offer_big(launch, [(launch, grad)])
             return
         held = sum(t for _, _, t in self._dw)
@@ -483,6 +483,10 @@ class BwdCtx:
         self._dw.append((launch, grad, tiles))
         if held + tiles >= self.FULL_GRID - 32:
             self.flush_dw()
+
+    def _emit_dw(self, launch):
+        launch.weight_gradients = True     # (may run anywhere until the end of the job: executor/merge.py)
+        self.emit(launch)
 
     def _offer_big(self, issued, members):
         """`issued` (one launch, already in the job) computes `members`: (product, accumulator) pairs.
@@ -538,7 +542,7 @@ class BwdCtx:
                 bigs = bigs if any(b is None for b in full) else full
             for old, _, _, _ in entries:   # blanked, not deleted: positions in the list stay valid until compact()
                 self.out[next(i for i in range(len(self.out) - 1, -1, -1) if self.out[i] is old)] = None
-            self.emit(self.k.gemm_group(bigs))
+            self._emit_dw(self.k.gemm_group(bigs))
 
     def compact(self, ranges):
         """Drop the blanked launches; `ranges` ((name, first, end) over the list) follow."""
@@ -563,11 +567,11 @@ class BwdCtx:
         self._dw = []
         if len(launches) > 1 and len({l.group_key for l in launches}) > 1:   # (a tile that cannot run one of them)
             for launch, grad in zip(launches, grads):
-                self.emit(launch)
+                self._emit_dw(launch)
                 self._offer_big(launch, [(launch, grad)])
             return
         issued = launches[0] if len(launches) == 1 else self.k.gemm_group(launches)
-        self.emit(issued)
+        self._emit_dw(issued)
         self._offer_big(issued, list(zip(launches, grads)))
 
     def register_lp(self, full, copy, colsum=None):

@@ -199,7 +199,9 @@ def _gemm(m, calls):
         if max(c0["lda"], 2 * c0["ldc"], 2 * c0["ld_res"], c0["ld_aux_in"], c0["ld_aux_out"]) * 2 * rows >= MAX_BYTES:
             raise NoMerge("size")
         return _chains(calls, "M", a="lda", c="ldc", aux_out="ld_aux_out", aux_in="ld_aux_in", residual="ld_res")
-    # a weight gradient that accumulates: a longer reduction
+    # a weight gradient that accumulates: a longer reduction; in 16 bits only where each is short (see Merger.lists)
+    if c0["a"].dtype != torch.float32 and min(c["K"] for c in calls) >= 64:
+        raise NoMerge("weight gradient")
     _same(calls, "M", "c", "aux_out", "aux_in", "residual")
     if not c0["b_trans"] or not c0["beta"] or c0["bias"] is not None or c0["act"] or c0["dact"] or c0["residual"] is not None:
         raise NoMerge("reduction")
@@ -414,9 +416,54 @@ class Merger:
         return self._position(launches[:cut]) + self._position(launches[cut:])
 
     def lists(self, lists):
+        """The merged list, or None.  16-bit weight gradients that accumulate inside the backward jobs (micro-batches of
+        different sizes) are not joined: one product over all rows would add its terms in another order than products per
+        micro-batch do, and after one update some weights round the other way and every activation follows.
+        They need nothing but to run before the job ends: micro-batch by micro-batch there, layers side by side in launches that
+        fill the device, they cost as much (ViT-S, 62 images in four micro-batches: 5.63 ms a step, 5.5 joined; where
+        they stand, a launch per layer and micro-batch, 7.4)."""
         if len({len(l) for l in lists}) != 1:
             return None
-        return [m for pos in zip(*lists) for m in self._position(list(pos))]
+        out, held = [], [[] for _ in lists]
+        for pos in zip(*lists):
+            parts = [self._weight_gradients(l) for l in pos]
+            if len(pos) > 1 and all(parts):
+                for h, p in zip(held, parts):
+                    h += p
+            else:
+                out += self._position(list(pos))
+        return out + [g for h in held for g in self._grouped(h)]
+
+    def _weight_gradients(self, launch):
+        """The products of a launch of 16-bit weight gradients that accumulate, or None."""
+        call = getattr(launch, "call", None)
+        if call is None or not getattr(launch, "weight_gradients", False) or getattr(self.table, "gemm_retiled", None) is None:
+            return None
+        members = call[1]["launches"] if call[0] == "gemm_group" else [launch]
+        return list(members) if all(self.table.gemm_groupable(l) and l.desc.beta == 1 for l in members) else None
+
+    def _grouped(self, launches):
+        """One micro-batch's weight gradients in launches that fill the device on 128x128 tiles (64x64 where all that is
+        left is small: BwdCtx._retile_held has both sides' times)."""
+        def tiles(l):
+            return ((l.desc.M + 127) // 128) * ((l.desc.N + 127) // 128)
+
+        out, i = [], 0
+        while i < len(launches):
+            run, n = [launches[i]], tiles(launches[i])
+            while i + len(run) < len(launches):
+                l = launches[i + len(run)]
+                if len(run) == self.table.GEMM_GROUP_MAX or n + tiles(l) > 256 or l.desc.in_dtype != run[0].desc.in_dtype:
+                    break
+                run.append(l)
+                n += tiles(l)
+            i += len(run)
+            same = [self.table.gemm_retiled(l, 15 if n <= 112 else 8) for l in run]
+            if len(run) > 1 and all(l is not None and self.table.gemm_groupable(l) for l in same):
+                out.append(self.table.gemm_group(same))
+            else:
+                out += run
+        return out
 
     def reduces(self, lists):
         """The deferred column reductions [(ws, offset, partial rows, stride, cols, accumulator)] of every

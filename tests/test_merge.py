@@ -117,6 +117,21 @@ def test_merged_jobs_on_the_device(monkeypatch, family, batch, micro, rows, mixe
             assert d <= tol, (i, k, d)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("family,batch,micro,rows", [("vit", 58, 4, 10 ** 6), ("vit", 59, 4, 140), ("decoder", 26, 3, 10 ** 6)])
+def test_merged_ragged_weight_gradients_keep_their_sums(monkeypatch, family, batch, micro, rows):
+    """Micro-batches of different sizes, of 64 rows and more each (products of fewer are joined): the first step's matrix
+    gradients are those of separate jobs bit for bit."""
+    (want,), _ = _steps(family, "bf16", batch, micro, 0, 1, monkeypatch, "cuda")
+    (got,), w = _steps(family, "bf16", batch, micro, rows, 1, monkeypatch, "cuda")
+    assert any(len(j.mbs) > 1 for j in w.jobs.values())
+    # (not the classifier: one row per sample)
+    linear = [k for k, g in want[1].items() if g.dim() == 2 and "emb" not in k and "tok" not in k and k != "head.weight"]
+    assert want[0] == got[0] and len(linear) >= 4
+    for k in linear:
+        assert torch.equal(want[1][k], got[1][k]), k
+
+
 def test_merged_lists_are_as_short_as_one_micro_batchs(monkeypatch):
     """Nothing but a loss inside the model stays per micro-batch."""
     for family, per_mb in (("vit", 0), ("decoder", 2 * 3)):    # cross entropy forward and backward of the last stage
