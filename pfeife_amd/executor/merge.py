@@ -17,7 +17,7 @@ How many micro-batches (`StageWorker.job_rows`): up to 8192 rows a job.  Step ti
 job, sustained: ViT-L/16 (4 x 3152 rows) 36.7 apart, 34.0 in twos, 33.9 all four (31.8 with today's products, in twos and all);
 1B decoder (8 x 4096) 205.2 apart, 188.8 in twos, 192.5 in fours; ViT-g share (4 x 6168) 53.7 / 51.7 / 51.9 (today - /
 46.0 / 45.0); decoder with wide heads (4 x 1021) 13.1 / - / 10.3; ViT-S fp32 (4 x 788) 9.80 -> 8.64, bf16 with ragged
-micro-batches 6.83 -> 5.96; decoder of four looped stages (8 x 256 rows) 3.98 -> 2.95.  Past some 8192 rows the kernels gain
+micro-batches 6.78 -> 5.69; decoder of four looped stages (8 x 256 rows) 3.98 -> 2.95.  Past some 8192 rows the kernels gain
 little, and jobs of one rank's forward and another's backward, or user code, no longer run beside each other.
 """
 import inspect
