@@ -391,26 +391,35 @@ class StageWorker:
     def form_jobs(self):
         """The jobs of a step from the micro-batches' programs: consecutive micro-batches of one layout and group whose
         launch lists correspond run as one.  A job's forward runs where the schedule has its first micro-batch, its
-        backward where it has its last: every order that the schedule allows stays one."""
+        backward where it has its last: every order that the schedule allows stays one.  All stages or none: a stage in one
+        job between others in several leaves them nothing to run beside (a decoder of two stages, fp32, 12 sequences in
+        eight micro-batches whose single ones have shorter lists: 11.8 ms apart, 12.6 with the first stage in one job)."""
         runs, self.jobs = [], {}
+
+        def shape(mb):
+            return [(len(p.fwd), len(p.bwd), len(p.reduces)) for _, p in sorted(self.mbs[mb].stage_programs.items())]
+
         for mb in sorted(self.mbs):
             lay = self.mbs[mb].layout
             key = None if lay is None else (lay.tag, lay.group(mb))
-            if runs and key is not None and runs[-1][0] == key and runs[-1][1][-1] == mb - 1:
+            if runs and key is not None and runs[-1][0] == key and runs[-1][1][-1] == mb - 1 and shape(mb) == shape(mb - 1):
                 runs[-1][1].append(mb)
             else:
                 runs.append((key, [mb]))
         at = {job: i for i, job in enumerate(self.order)} if runs else {}
         for _, mbs in runs:
+            merged = {}
+            for sid in self.part_graph.nodes if len(mbs) > 1 else ():
+                self.pool.lane = self._lane_key(sid, False) if self.lanes is not None else 0
+                prog = self.lowerer.merge_programs([self.mbs[m].stage_programs[sid] for m in mbs])
+                self.pool.lane = 0
+                if prog is None:
+                    merged = {}
+                    break
+                merged[sid] = prog
             for sid in self.part_graph.nodes:
-                progs = [self.mbs[m].stage_programs[sid] for m in mbs]
-                prog = None
-                if len(mbs) > 1:
-                    self.pool.lane = self._lane_key(sid, False) if self.lanes is not None else 0
-                    prog = self.lowerer.merge_programs(progs)
-                    self.pool.lane = 0
-                for part in ([mbs] if prog is not None else [[m] for m in mbs]):
-                    job = StageJob(prog if prog is not None else self.mbs[part[0]].stage_programs[sid], part,
+                for part in [mbs] if merged else [[m] for m in mbs]:
+                    job = StageJob(merged[sid] if merged else self.mbs[part[0]].stage_programs[sid], part,
                                    min(part, key=lambda m: at[sid, m, True]), max(part, key=lambda m: at[sid, m, False]))
                     for m in part:
                         self.jobs[sid, m] = job
