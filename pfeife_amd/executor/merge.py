@@ -444,7 +444,8 @@ class Merger:
 
     def _grouped(self, launches):
         """One micro-batch's weight gradients in launches that fill the device on 128x128 tiles (64x64 where all that is
-        left is small: BwdCtx._retile_held has both sides' times)."""
+        left is small: BwdCtx._retile_held has both sides' times).  Products into one accumulator (a weight used twice in
+        the stage) keep their order: a launch's products run side by side."""
         def tiles(l):
             return ((l.desc.M + 127) // 128) * ((l.desc.N + 127) // 128)
 
@@ -453,7 +454,8 @@ class Merger:
             run, n = [launches[i]], tiles(launches[i])
             while i + len(run) < len(launches):
                 l = launches[i + len(run)]
-                if len(run) == self.table.GEMM_GROUP_MAX or n + tiles(l) > 256 or l.desc.in_dtype != run[0].desc.in_dtype:
+                if len(run) == self.table.GEMM_GROUP_MAX or n + tiles(l) > 256 or l.desc.in_dtype != run[0].desc.in_dtype \
+                        or any(l.desc.C == r.desc.C for r in run):
                     break
                 run.append(l)
                 n += tiles(l)

@@ -444,11 +444,14 @@ class HipKernels:
         return HipKernels.gemm_groupable(launch)
 
     def gemm_group(self, launches):
-        """One launch for 2..GEMM_GROUP_MAX independent `gemm_groupable` products of the same variant."""
+        """One launch for 2..GEMM_GROUP_MAX independent `gemm_groupable` products of the same variant.  They run side by
+        side and add to C without atomics: two into one C are an error."""
         n = len(launches)
         if not (2 <= n <= self.GEMM_GROUP_MAX) or len({l.group_key for l in launches}) != 1 \
                 or not all(self.gemm_groupable(l) for l in launches):
             raise RuntimeError("gemm_group: needs 2..%d groupable launches of one variant" % self.GEMM_GROUP_MAX)
+        if len({l.desc.C for l in launches}) != n:
+            raise RuntimeError("gemm_group: two products into one C")
         arr = (GemmDesc * n)()
         for i, l in enumerate(launches):
             ctypes.memmove(ctypes.byref(arr[i]), ctypes.byref(l.desc), ctypes.sizeof(GemmDesc))

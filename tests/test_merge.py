@@ -173,3 +173,114 @@ def test_layout_places_do_not_overlap(sizes, rows):
             for (m, (a, _)), (m2, (b, _)) in zip(spans, spans[1:]):
                 if not in_group or lay.group(m) == lay.group(m2):
                     assert b == a + per * sizes[m]
+
+
+class _TwiceThroughABlock(torch.nn.Module):
+    """A stage that uses its weights twice (layers that share parameters)."""
+
+    def __init__(self):
+        super().__init__()
+        self.up, self.down, self.head = torch.nn.Linear(64, 128), torch.nn.Linear(128, 64), torch.nn.Linear(64, 16)
+
+    def forward(self, x):
+        for _ in range(2):
+            x = x + self.down(F.gelu(self.up(x)))
+        return self.head(x)
+
+
+def _grouping_kernels():
+    """The kernel oracle with the device's way to put weight gradients together: the products of one launch run side by
+    side, so each adds to its accumulator as that was before the launch."""
+    from types import SimpleNamespace
+
+    from oracle.kernels_oracle import OracleKernels
+
+    class GroupingKernels(OracleKernels):
+        GEMM_GROUP_MAX = 8
+        groups = []      # every launch of several products, as their accumulators
+
+        def gemm(self, a, b, c, M, N, K, lda, ldb, ldc, a_trans=0, b_trans=0, batch=(1, 1), sa=(0, 0), sb=(0, 0), sc=(0, 0),
+                 alpha=1.0, beta=0, bias=None, round_mid=0, aux_out=None, ld_aux_out=0, act=0, dact=0, aux_in=None, ld_aux_in=0,
+                 residual=None, ld_res=0, variant=0, unscale_by=None, nonfinite_flag=None):
+            launch = super().gemm(a, b, c, M, N, K, lda, ldb, ldc, a_trans, b_trans, batch, sa, sb, sc, alpha, beta, bias, round_mid,
+                                  aux_out, ld_aux_out, act, dact, aux_in, ld_aux_in, residual, ld_res, unscale_by, nonfinite_flag)
+            launch.desc = SimpleNamespace(M=M, N=N, K=K, C=c.data_ptr(), beta=beta, in_dtype=a.dtype)
+            launch.acc = c
+            launch.group_key = "tile %d" % variant if a_trans and b_trans and a.dtype != torch.float32 and K >= 64 else ""
+            return launch
+
+        @staticmethod
+        def gemm_groupable(launch):
+            return getattr(launch, "group_key", "") != ""
+
+        def gemm_retiled(self, launch, variant):
+            new = lambda stream=None: launch(stream)
+            new.desc, new.acc, new.group_key = launch.desc, launch.acc, "tile %d" % variant
+            return new
+
+        def gemm_group(self, launches):
+            assert 2 <= len(launches) <= self.GEMM_GROUP_MAX and len({l.group_key for l in launches}) == 1
+            self.groups.append([l.acc.data_ptr() for l in launches])
+
+            def launch(stream=None):
+                before = [l.acc.clone() for l in launches]
+                for l, acc in zip(launches, before):
+                    l.acc.copy_(acc)
+                    l(stream)
+
+            launch.group_key = "group"
+            return launch
+
+    return GroupingKernels("cpu")
+
+
+def _steps_of_shared_weights(monkeypatch, rows, device="cpu"):
+    from pfeife_amd.mp import PartialRunner, initialize_pfeife, net_states, partial_compiler
+
+    monkeypatch.setenv("PFEIFE_JOB_ROWS", str(rows))
+    torch._dynamo.reset()
+    net_states._reset_state_for_tests()
+    initialize_pfeife(**(dict(device="cpu") if device == "cpu" else {}))
+    torch.manual_seed(0)
+    model = _TwiceThroughABlock().to(device)
+    kernels = _grouping_kernels() if device == "cpu" else None
+    runner = PartialRunner(PipeOption(device_cnt=1, batch_cnt=4, batch_size=1, mixed_precision="bf16", optimizer=dict(type="sgd", lr=0.0)),
+                           kernels=kernels)
+    cmodel = torch.compile(model, backend=partial_compiler, dynamic=False)
+
+    def fn(x):
+        loss = cmodel(x).float().square().mean()
+        loss.backward()
+        return loss.detach()
+
+    runner.set_exec_fn(fn)
+    g = torch.Generator().manual_seed(1)
+    for _ in range(4 if device == "cuda" else 1):     # (launch by launch, captured, from job lists)
+        runner.step(torch.randn(58, 5, 64, generator=g).to(device))
+    return {k: p.grad.cpu().clone() for k, p in model.named_parameters()}, runner.worker, kernels
+
+
+def _same_shared_gradients(want, got):
+    for k in want:
+        if want[k].dim() == 2:
+            assert torch.equal(want[k], got[k]), k
+        assert float((want[k] - got[k]).norm()) <= 1.1e-4 * float(want[k].norm()), k
+
+
+def test_products_into_one_accumulator_are_never_one_launch(monkeypatch):
+    """Weights used twice in a stage, micro-batches of different sizes (15, 15, 14, 14 samples of 5 rows): each accumulator
+    gets the products of separate jobs in their order, so that the weights' gradients are the same bit for bit.  (Biases
+    add at most 75 rows x 2 uses in another order: 150 * 2^-24 = 9e-6 of the sum of magnitudes, some sqrt(150) times the sum's.)"""
+    want, _, _ = _steps_of_shared_weights(monkeypatch, 0)
+    got, w, kernels = _steps_of_shared_weights(monkeypatch, 10 ** 6)
+    assert any(len(j.mbs) > 1 for j in w.jobs.values()) and kernels.groups
+    assert all(len(set(g)) == len(g) for g in kernels.groups), kernels.groups
+    _same_shared_gradients(want, got)
+
+
+@pytest.mark.gpu
+def test_weights_used_twice_on_the_device(monkeypatch):
+    want, _, _ = _steps_of_shared_weights(monkeypatch, 0, "cuda")
+    got, w, _ = _steps_of_shared_weights(monkeypatch, 10 ** 6, "cuda")
+    assert any(len(j.mbs) > 1 for j in w.jobs.values())
+    _same_shared_gradients(want, got)
