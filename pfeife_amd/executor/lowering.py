@@ -291,8 +291,18 @@ class BufferPool:
         # buffer is shared within a lane only.
         self.lane = 0
 
+    def scratch_key(self, slot, shape, dtype):
+        return self.lane, slot, tuple(shape), dtype
+
+    def drop_scratch(self, keys):
+        """Forget scratch that no launch uses any more."""
+        for key in set(keys):
+            t = self._scratch.pop(key, None)
+            if t is not None:
+                self.bytes -= t.numel() * t.element_size()
+
     def scratch(self, slot, shape, dtype):
-        key = (self.lane, slot, tuple(shape), dtype)
+        key = self.scratch_key(slot, shape, dtype)
         t = self._scratch.get(key)
         if t is None:
             t = torch.empty(tuple(shape), dtype=dtype, device=self.device)
@@ -821,6 +831,8 @@ class Lowerer:
         # layout (`MicroBatchLayout`): the micro-batches' forward buffers and the gradients that those products or
         # jobs over several micro-batches read are laid end to end; None: buffers of their own
         self.layout = None
+        # scratch taken by forward jobs that were lowered before the layout's groups were formed (None: others use it too)
+        self.early_scratch = []
         # loss scaling as the once-per-step weight-gradient products see it: (device scale or None,
         # device overflow flag or None, constant factor); set by the worker
         self.dw_unscale = (None, None, 1.0)
@@ -856,11 +868,15 @@ class Lowerer:
                                  self.layout.place(mb, in_group=True), strides, aligned=True)
 
     def scratch(self, slot, mb, shape, dtype):
-        """Scratch that several launches of a job use (forward jobs: their groups are not known yet)."""
-        if self.layout is None or mb is None:
-            return self.pool.scratch(slot, shape, dtype)
-        return self.pool.stacked((self.layout.tag, "s", self.pool.lane, slot, tuple(shape[1:])), shape, dtype,
-                                 self.layout.place(mb))
+        """Scratch that several launches of a job use and that no other job reads: one buffer per lane, where jobs take
+        several micro-batches one for each of them (jobs use these in turn)."""
+        if self.shares_jobs(mb):
+            return self.pool.stacked((self.layout.tag, "s", self.pool.lane, slot, tuple(shape[1:])), shape, dtype,
+                                     self.layout.place(mb, in_group=True))
+        if self.layout is not None and not self.layout.formed:
+            key = self.pool.scratch_key(slot, shape, dtype)
+            self.early_scratch.append(None if key in self.pool._scratch else key)
+        return self.pool.scratch(slot, shape, dtype)
 
     def workspace(self, rows, cols):
         """fp32 scratch for the two-stage column reductions (shared by every launch of that size)."""

@@ -277,35 +277,13 @@ class StageWorker:
             L.dw_unscale = (self.scaler_state[0:1], self.scaler_state[2:3], 1.0)
         else:
             L.dw_unscale = (None, None, 1.0 / float(self.option.loss_scale))
-        stage_out = {}
-        for sid in sorted(pg.nodes):
-            st = pg.nodes[sid]
-            ins = []
-            for k, name in enumerate(st.inputs):
-                gi = st.input_placeholder[k]
-                if gi >= 0:
-                    ins.append(graph_vals[gi])
-                else:
-                    src_stage, oi = st.input_source[k]
-                    pv = stage_out[src_stage][oi]
-                    if isinstance(pv, Val):
-                        bv = Val(pv.buf, req_grad=pv.req_grad, name=name)  # same storage: the handoff is a pointer
-                        bv.boundary = True
-                        ins.append(bv)
-                    elif isinstance(pv, (list, tuple)) and any(isinstance(e, Val) for e in pv):
-                        # its gradient would have to travel back as a tuple as well; the stage
-                        # programs hand over single tensors only
-                        raise Unsupported("the split point in front of stage %d cuts between '%s' (a tuple of "
-                                          "tensors) and its users; move it before the node that makes the tuple "
-                                          "or after the nodes that take it apart" % (sid, name))
-                    else:
-                        ins.append(pv)
-            self.pool.lane = self._lane_key(sid, True) if self.lanes is not None else 0
-            prog = L.lower_forward(st, mb, ins)
-            slot.stage_programs[sid] = prog
-            stage_out[sid] = prog.outputs
+        L.early_scratch = []
+        stage_out = self._lower_forwards(slot, mb, pg, graph_vals)
         if L.layout is not None and not L.layout.formed:
             self._form_groups(L.layout, mb, slot.stage_programs.values())
+            if L.early_scratch and L.shares_jobs(mb):    # (scratch of several micro-batches: only now is it known how many)
+                self.pool.drop_scratch(L.early_scratch)
+                stage_out = self._lower_forwards(slot, mb, pg, graph_vals)
         # graph outputs and the buffers their loss gradients arrive in
         for oi, ref in enumerate(pg.outputs):
             if ref[0] == "const":
@@ -358,6 +336,38 @@ class StageWorker:
         self.graphs_ready = False   # new programs (and possibly new parameters): capture again
         self._drop_begin_graph()
         return slot
+
+    def _lower_forwards(self, slot, mb, pg, graph_vals):
+        """Lowers the forward jobs of every stage into the slot; -> stage -> its outputs."""
+        L = self.lowerer
+        stage_out = {}
+        for sid in sorted(pg.nodes):
+            st = pg.nodes[sid]
+            ins = []
+            for k, name in enumerate(st.inputs):
+                gi = st.input_placeholder[k]
+                if gi >= 0:
+                    ins.append(graph_vals[gi])
+                else:
+                    src_stage, oi = st.input_source[k]
+                    pv = stage_out[src_stage][oi]
+                    if isinstance(pv, Val):
+                        bv = Val(pv.buf, req_grad=pv.req_grad, name=name)  # same storage: the handoff is a pointer
+                        bv.boundary = True
+                        ins.append(bv)
+                    elif isinstance(pv, (list, tuple)) and any(isinstance(e, Val) for e in pv):
+                        # its gradient would have to travel back as a tuple as well; the stage
+                        # programs hand over single tensors only
+                        raise Unsupported("the split point in front of stage %d cuts between '%s' (a tuple of "
+                                          "tensors) and its users; move it before the node that makes the tuple "
+                                          "or after the nodes that take it apart" % (sid, name))
+                    else:
+                        ins.append(pv)
+            self.pool.lane = self._lane_key(sid, True) if self.lanes is not None else 0
+            prog = L.lower_forward(st, mb, ins)
+            slot.stage_programs[sid] = prog
+            stage_out[sid] = prog.outputs
+        return stage_out
 
     def _layout(self, mb, sig):
         """How the buffers of the step's micro-batches lie, for a micro-batch whose inputs have the signature `sig`;

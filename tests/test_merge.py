@@ -140,6 +140,28 @@ def test_merged_lists_are_as_short_as_one_micro_batchs(monkeypatch):
         assert sum(len(p.fwd) + len(p.bwd) for p in w.step_programs()) == one + per_mb
 
 
+@pytest.mark.parametrize("rows,batch,jobs", [(0, 8, 1), (1, 8, 1), (36, 8, 2), (10 ** 6, 8, 4), (36, 11, 2), (0, 7, 1)])
+def test_attention_scratch_is_that_of_one_job(monkeypatch, rows, batch, jobs):
+    """Scores, their gradients and the rounded ones (fp32: attention through memory): one buffer for a lane's jobs, with
+    room for as many micro-batches as a job takes; nothing is left of the ones it was first lowered with."""
+    _, w = _steps("decoder", None, batch, 4, rows, 2, monkeypatch)
+    assert {len(j.mbs) for j in w.jobs.values()} == {jobs}
+    bufs = {}
+    for slot in w.mbs.values():
+        for prog in slot.stage_programs.values():
+            for l in prog.fwd + prog.bwd:
+                for name in {"softmax_fwd": ("s",), "softmax_bwd": ("dp", "ds")}.get(l.call[0] if hasattr(l, "call") else "", ()):
+                    bufs.setdefault(name, set()).add(l.call[1][name])
+    assert set(bufs) == {"s", "dp", "ds"}
+    for name, ts in bufs.items():
+        sizes = sorted(t.numel() for t in ts)
+        assert len({t.data_ptr() for t in ts}) == (jobs if batch == 8 or jobs > 1 else 2), name   # (two shapes: a buffer each)
+        held = {t.untyped_storage().data_ptr(): t.untyped_storage().nbytes() for t in ts}
+        assert sum(held.values()) <= 4 * (jobs * sizes[-1] if jobs > 1 or batch == 8 else sum(set(sizes))), name
+    kept = {id(t) for ts in bufs.values() for t in ts}
+    assert all(id(t) in kept for (_, slot, _, _), t in w.pool._scratch.items() if str(slot).startswith("attn"))
+
+
 def test_a_micro_batch_that_differs_keeps_its_own_launches(monkeypatch):
     """Operands that do not follow each other: the launches stay as they are, in order."""
     from oracle.kernels_oracle import OracleKernels
