@@ -44,23 +44,19 @@ from ..worker import StageWorker
 STEP_TOKEN = "###<<STEP_TOKEN>>###"
 
 
-def _same_shapes(args, kwargs):
-    """Do the micro-batches of a step agree in the shapes and dtypes of all their tensors?  (A batch
-    that does not divide evenly gives the first micro-batches one row more, pfeife/batch.py:45.)"""
+def _shapes(args, kwargs):
+    """-> (do the micro-batches of a step agree in the shapes and dtypes of all their tensors, how many samples each has:
+    the rows of its first tensor).  (A batch that does not divide evenly gives the first micro-batches one row more,
+    pfeife/batch.py:45.)"""
     from torch.utils._pytree import tree_flatten
 
-    sigs = set()
+    sigs, samples = set(), []
     for a, k in zip(args, kwargs):
         leaves, _ = tree_flatten((a, k))
-        sigs.add(tuple((tuple(t.shape), t.dtype) for t in leaves if torch.is_tensor(t)))
-    return len(sigs) <= 1
-
-
-def _samples(args, kwargs):
-    """How many samples a micro-batch has: the rows of its first tensor."""
-    from torch.utils._pytree import tree_flatten
-
-    return next((int(t.shape[0]) for t in tree_flatten((args, kwargs))[0] if torch.is_tensor(t) and t.dim() > 0), 1)
+        sig = tuple((tuple(t.shape), t.dtype) for t in leaves if torch.is_tensor(t))
+        sigs.add(sig)
+        samples.append(next((int(s[0]) for s, _ in sig if s), 1))
+    return len(sigs) <= 1, samples
 
 
 class _ExecError:
@@ -122,8 +118,7 @@ class PartialRunner:
             raise RuntimeError("call set_exec_fn() before step()")
         option = self.option
         args, kwargs = split_args_kwargs(args, kwargs, option.batch_cnt)
-        self.worker.uniform_mbs = _same_shapes(args, kwargs)
-        self.worker.mb_sizes = [_samples(a, k) for a, k in zip(args, kwargs)]
+        self.worker.uniform_mbs, self.worker.mb_sizes = _shapes(args, kwargs)
 
         if not self._compiled:
             self._probe_forward(args[0], kwargs[0])

@@ -181,6 +181,30 @@ def test_a_micro_batch_that_differs_keeps_its_own_launches(monkeypatch):
     assert m.lists([[calls[0]], []]) is None                                       # another structure
 
 
+def test_shapes_of_a_step_take_one_walk_per_micro_batch(monkeypatch):
+    import torch.utils._pytree as pytree
+    from pfeife_amd.mp.partial.module import PartialRunner
+
+    walks, steps = [], []
+    flatten = pytree.tree_flatten
+    runner = make_runner(PipeOption(device_cnt=1, batch_cnt=3, batch_size=1))
+    runner.set_exec_fn(lambda *a, **k: None)
+    monkeypatch.setattr(PartialRunner, "_probe_forward", lambda self, *a: None)
+    monkeypatch.setattr(PartialRunner, "_run_step", lambda self, *a: steps.append((self.worker.uniform_mbs, self.worker.mb_sizes)))
+    for args, kwargs, want in [((torch.zeros(8, 2),), dict(y=torch.zeros(8)), (False, [3, 3, 2])),
+                               ((torch.zeros(6, 2), torch.zeros(6)), {}, (True, [2, 2, 2]))]:
+        runner.step(*args, **kwargs)
+        with monkeypatch.context() as m:      # (the split walks too: how often beside that)
+            m.setattr(pytree, "tree_flatten", lambda *a, **k: walks.append(1) or flatten(*a, **k))
+            from pfeife_amd.batch import split_args_kwargs
+            split_args_kwargs(args, kwargs, 3)
+            split, walks[:] = len(walks), []
+            runner.step(*args, **kwargs)
+            assert len(walks) - split == 3
+            walks.clear()
+        assert steps[-1] == want
+
+
 @pytest.mark.parametrize("sizes", [[2] * 5, [3, 3, 2, 2], [1, 1, 0, 0], [4]])
 @pytest.mark.parametrize("rows", [1, 7, 10 ** 6])
 def test_layout_places_do_not_overlap(sizes, rows):
