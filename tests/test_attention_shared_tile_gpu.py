@@ -1,7 +1,7 @@
 """Attention over 257 to 288 tokens: the ninth tile of 32, which a workgroup's eight wavefronts share (the queries of
-the forward and of dQ, the keys of dK / dV), one row of it to all, beside long, short and one-token other axes (their
-operands in LDS are then smaller than the partial results), with and without a causal mask (rows that see no key of a
-wavefront's share), against the kernel oracle and torch's attention."""
+the forward and of dQ, the keys of dK / dV) where there is no mask and the other axis has more than 192 tokens, and
+the calls beside that rule, which the eight or four wavefronts take tile by tile (a causal mask, a short other axis, 256 tokens and
+less), against the kernel oracle and torch's attention."""
 import pytest
 import torch
 
@@ -18,6 +18,16 @@ pytestmark = pytest.mark.gpu
     (270, 40, 64, 0), (33, 270, 40, 1), (271, 271, 80, 1), (129, 160, 96, 0), (256, 256, 72, 1)])
 def test_ninth_tile(hip, oracle, dtype, Tq, Tk, hd, causal):  # noqa: F811
     base.test_fused_attention(hip, oracle, dtype, dict(B=2, H=3, Tq=Tq, Tk=Tk, hd=hd, causal=causal, packed=False))
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("B,H,Tq,Tk,hd", [
+    (2, 3, 257, 200, 64), (2, 3, 200, 257, 64), (2, 3, 288, 193, 96), (2, 3, 193, 288, 96), (2, 3, 257, 224, 88), (1, 3, 224, 288, 40),
+    (3, 43, 257, 257, 88), (3, 43, 288, 288, 96), (3, 43, 257, 193, 80), (1, 129, 200, 260, 72)])
+def test_shared_tile_sweeps(hip, oracle, dtype, B, H, Tq, Tk, hd):  # noqa: F811
+    """Sweeps of 193 to 224 tokens leave the eighth wavefront without a tile (no maximum, no sum) and their operands take less
+    LDS than the partial results; above head dim 64 dK / dV run on eight wavefronts, which share, for more than 128 heads only."""
+    base.test_fused_attention(hip, oracle, dtype, dict(B=B, H=H, Tq=Tq, Tk=Tk, hd=hd, causal=0, packed=False))
 
 
 @pytest.mark.parametrize("T,hd,causal", [(70, 64, 0), (130, 96, 1), (65, 128, 0)])
