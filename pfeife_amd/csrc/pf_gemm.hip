@@ -715,6 +715,10 @@ bool plan_split(const pf_gemm_desc& d, Split& s) {
   double best_t = 0.96 * single - 0.5;   // (less is within the model's error and a launch's)
   bool found = false;
   for (const TileCost& c : ROW_MAJOR) {
+    // (A GELU product's first round may be the four-wavefront tile's at any depth, which choose_tile refuses for one round on its
+    // own.  48 products of 4700 to 15800 rows over 384 to 1024, with that rule here too: GELU 5.9 % slower on average, GELU' 1.0 %
+    // faster; us as here / with it: 11426 x 1536 over 1024 47.7 / 54.2, 13593 x 1536 over 1024 56.6 / 61.6, GELU' 10441 x 2048 over
+    // 768 58.3 / 56.3, 14381 x 1536 over 1024 64.9 / 70.0)
     if (c.v == V_X64 || c.v == V_X192x128W8 || !x_supports(d, c.v)) continue;
     const int64_t tn = (d.N + c.bn - 1) / c.bn;
     for (int64_t round = 1;; ++round) {
