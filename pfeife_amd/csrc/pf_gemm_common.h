@@ -218,7 +218,7 @@ template <> struct XTile<PF_XT_192x128w8> { static constexpr int BM = 192, BN = 
 template <> struct XTile<PF_XT_64x64> { static constexpr int BM = 64, BN = 64, BK = 64, ST = 5, WGM = 2, WGN = 2, KS = 1; };
 // tiles with a kernel for row-major products whose reduction length is no multiple of the stage depth: the
 // eight-wavefront 128x128 and 256x128 tiles and 64x64
-constexpr bool x_tile_ragged(int bm, int bn, int nw) { return (nw == 8 && bn == 128) || (bm == 64 && bn == 64); }
+constexpr bool x_tile_ragged(int bm, int bn, int nw) { return (nw == 8 && bn == 128 && bm != 192) || (bm == 64 && bn == 64); }
 constexpr int x_tile_bm(int xt) {
   return xt == PF_XT_64x64 ? 64 : (xt == PF_XT_128x128 || xt == PF_XT_128x128k2 || xt == PF_XT_128x128w8) ? 128
          : (xt == PF_XT_192x256 || xt == PF_XT_192x256w8 || xt == PF_XT_192x128w8) ? 192 : 256;
