@@ -825,6 +825,8 @@ int norm_bwd(const void* dy, int dy_dt, const void* x, int x_dt, const float* ga
   // ... or everything is one 16-bit dtype and there is no side copy
   const bool io16 = (x_dt == PF_F16 || x_dt == PF_BF16) && dx_dt == x_dt && dy_dt == x_dt && (!dx_add || add_dt == x_dt) &&
                     !dx_lp;
+  // a team stores its partial rows 16 bytes at a time
+  const bool team = pf_aligned(ws, 16);
 #define PF_NBC(NV, LP, DY) PF_NBI(NV, PF_F32, LP, DY)
 #define PF_NBI(NV, IO, LP, DY)                                                                                       \
   hipLaunchKernelGGL((norm_bwd_kernel<8, NV, IO, LP, DY>), dim3(blocks), dim3(256), 0, st, dy, dy_dt, x, x_dt, gamma, \
@@ -833,7 +835,8 @@ int norm_bwd(const void* dy, int dy_dt, const void* x, int x_dt, const float* ga
   hipLaunchKernelGGL((norm_bwd_team_kernel<NWV, TEAMS, IO, LP, DY>), dim3(blocks), dim3(64 * NWV * TEAMS), 0, st, dy, x, gamma, mean, \
                      rstd, dx_add, dx, ws, rows, d, rms, want, dx_lp, want_colsum)
 #define PF_NBTD(NWV, TEAMS, ELSE)                                                           \
-  if (io32 && dy_dt == PF_F16 && (!dx_lp || lp_dt == PF_F16)) PF_NBT(NWV, TEAMS, PF_F32, PF_F16, PF_F16);    \
+  if (!team) ELSE;                                                                          \
+  else if (io32 && dy_dt == PF_F16 && (!dx_lp || lp_dt == PF_F16)) PF_NBT(NWV, TEAMS, PF_F32, PF_F16, PF_F16);    \
   else if (io32 && dy_dt == PF_BF16 && (!dx_lp || lp_dt == PF_BF16)) PF_NBT(NWV, TEAMS, PF_F32, PF_BF16, PF_BF16); \
   else if (io32 && dy_dt == PF_F32 && (!dx_lp || lp_dt == PF_F16)) PF_NBT(NWV, TEAMS, PF_F32, PF_F16, PF_F32);    \
   else if (io32 && dy_dt == PF_F32 && lp_dt == PF_BF16) PF_NBT(NWV, TEAMS, PF_F32, PF_BF16, PF_F32);         \

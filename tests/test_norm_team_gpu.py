@@ -67,3 +67,26 @@ def test_non_finite_rows_stay_in_their_rows(rows, d):
     torch.cuda.synchronize()
     bad = ~torch.isfinite(dx).all(dim=1)
     assert bad.nonzero().flatten().tolist() == [7]
+
+
+@pytest.mark.parametrize("rows,d", [(5, 520), (700, 1408), (300, 2048)])
+def test_partial_rows_at_any_fp32_address(rows, d):
+    """The workspace needs no more than its type's alignment: the partial rows are the same sums at every offset (of at
+    most `rows` fp32 terms, in another order: rows * 2^-24 of the sum of their magnitudes)."""
+    from pfeife_amd.hip import HipKernels
+
+    hip = HipKernels(0)
+    dy, x = rnd((rows, d), BF16, 1).cuda(), rnd((rows, d), F32, 2).cuda()
+    gamma, mean, rstd = rnd((d,), F32, 4).cuda(), torch.zeros(rows, device="cuda"), torch.ones(rows, device="cuda")
+    nb, res = hip.norm_bwd_partials(rows), []
+    for off in (0, 1, 2, 3):
+        dx, lp = torch.zeros(rows, d, device="cuda"), torch.zeros(rows, d, dtype=BF16, device="cuda")
+        ws = torch.zeros(nb * 3 * d + 4, device="cuda")[off:off + nb * 3 * d]
+        hip.norm_bwd_fused(dy, x, gamma, mean, rstd, None, dx, lp, ws, rows, d, True, True)(torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        res.append((dx.cpu(), ws.view(nb, 3, d).double().sum(0).cpu()))
+    bound = rows * 2.0 ** -24 * torch.stack([(dy.double() * x.double()).abs().sum(0), dy.double().abs().sum(0)]).cpu()
+    for dx, sums in res[1:]:
+        torch.testing.assert_close(dx, res[0][0], rtol=2e-5, atol=8e-5)
+        assert bool(((sums - res[0][1])[:2].abs() <= bound + 1e-6).all())
+        assert float((sums - res[0][1])[2].abs().max()) <= 2.0 ** -7 * float(res[0][0].abs().sum(0).max())   # (a rounding the other way)
