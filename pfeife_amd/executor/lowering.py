@@ -27,7 +27,7 @@ import os
 import torch
 import torch.nn.functional as F
 
-from .merge import CallRecorder, Merger
+from .merge import MAX_BYTES, CallRecorder, Merger
 from .values import Val, as_matrix, collapse_for_copy, dense_like, is_dense
 
 ACT_NONE, ACT_GELU, ACT_GELU_TANH, ACT_SILU, ACT_RELU = 0, 1, 2, 3, 4
@@ -991,7 +991,7 @@ class Lowerer:
         """The once-per-step weight-gradient job of one stage.  `progs`: the stage's programs, one
         per micro-batch, in micro-batch order.  Product i of every program reads that micro-batch's
         layer-output gradient and layer input; where those lie end to end in memory (equal
-        micro-batches, stacked buffers) the micro-batches are ONE product over all their rows:
+        micro-batches, stacked buffers, no operand of 2 GiB) the micro-batches are ONE product over all their rows:
         one launch and one read-modify-write of the fp32 accumulator instead of one per micro-batch
         (ViT-L: a quarter of a weight-gradient launch was that pass).  Otherwise (ragged batch, an
         operand in a buffer of its own) one product per micro-batch, in micro-batch order.
@@ -1013,7 +1013,10 @@ class Lowerer:
                        (r["rows"], r["n_out"], r["n_in"], r["ld_dy"], r["ld_x"]) ==
                        (r0["rows"], r0["n_out"], r0["n_in"], r0["ld_dy"], r0["ld_x"]) and
                        r["dy"].dtype == r0["dy"].dtype and r["x"].dtype == r0["x"].dtype for r in recs)
-            stacked = same and len(recs) > 1 and r0["rows"] > 0 and all(
+            # (a matrix operand of a 16-bit product stays below 2 GiB: the logits' gradient of 131072 rows over 8192
+            # classes does not)
+            fits = es == 4 or (sum(r["rows"] for r in recs) + 256) * max(r0["ld_dy"], r0["ld_x"]) * es < MAX_BYTES
+            stacked = same and fits and len(recs) > 1 and r0["rows"] > 0 and all(
                 r["dy"].untyped_storage().data_ptr() == r0["dy"].untyped_storage().data_ptr() and
                 r["x"].untyped_storage().data_ptr() == r0["x"].untyped_storage().data_ptr() and
                 r["dy"].data_ptr() == r0["dy"].data_ptr() + j * r0["rows"] * r0["ld_dy"] * es and

@@ -162,6 +162,24 @@ def test_attention_scratch_is_that_of_one_job(monkeypatch, rows, batch, jobs):
     assert all(id(t) in kept for (_, slot, _, _), t in w.pool._scratch.items() if str(slot).startswith("attn"))
 
 
+@pytest.mark.parametrize("mixed,products", [("bf16", 4), (None, 1)])
+def test_weight_gradients_over_the_step_keep_to_the_operand_limit(monkeypatch, mixed, products):
+    """Rows of all micro-batches that make an operand of a 16-bit product larger than pf_gemm takes: a product per
+    micro-batch, the same gradients (sums of at most 40 rows in another order, 40 * 2^-24 = 2.4e-6).  fp32 has no such limit."""
+    import pfeife_amd.executor.lowering as lowering
+
+    (want,), w0 = _steps("vit", mixed, 8, 4, 0, 1, monkeypatch)
+    monkeypatch.setattr(lowering, "MAX_BYTES", (300 * 128) * 2)        # (40 rows in all; qkv has 192 columns)
+    (got,), w = _steps("vit", mixed, 8, 4, 0, 1, monkeypatch)
+    for worker, n in ((w0, 1), (w, products)):
+        job = [l.call[1]["c"].data_ptr() for l in worker.dw_jobs[0][0] if getattr(l, "call", ("",))[0] == "gemm"]
+        qkv = [p.grad.data_ptr() for p in worker.params.params if tuple(p.shape) == (192, 64)]
+        assert {job.count(c) for c in qkv if c in job} == {n}
+    assert want[0] == got[0]
+    for k in want[1]:
+        assert float((want[1][k] - got[1][k]).norm()) <= 2.4e-5 * float(want[1][k].norm()), k
+
+
 def test_a_micro_batch_that_differs_keeps_its_own_launches(monkeypatch):
     """Operands that do not follow each other: the launches stay as they are, in order."""
     from oracle.kernels_oracle import OracleKernels
