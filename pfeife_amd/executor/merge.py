@@ -13,7 +13,7 @@ hold (a loss inside the model averages over its micro-batch) the launches stay a
 other.  Every row is computed from the same operands as before, products on the tile that suits the longer
 operand; gradients that sum over rows (biases, norm weights) add their fp32 terms in another order.
 
-How many micro-batches (`StageWorker.job_rows`): up to 8192 rows a job.  Step times on one card in ms, by rows to a
+How many micro-batches (`StageWorker.job_rows`): as few as give a job 8192 rows, so that it has up to about twice that many.  Step times on one card in ms, by rows to a
 job, sustained: ViT-L/16 (4 x 3152 rows) 36.7 apart, 34.0 in twos, 33.9 all four (31.8 with today's products, in twos and all);
 1B decoder (8 x 4096) 205.2 apart, 188.8 in twos, 192.5 in fours; ViT-g share (4 x 6168) 53.7 / 51.7 / 51.9 (today - /
 46.0 / 45.0); decoder with wide heads (4 x 1021) 13.1 / - / 10.3; ViT-S fp32 (4 x 788) 9.80 -> 8.64, bf16 with ragged

@@ -115,8 +115,8 @@ class StageWorker:
         # shapes stack their buffers (`uniform_mbs`, set by the runner before the step's first job)
         self.stack_dw = os.environ.get("PFEIFE_DW_STACK", "1") != "0"
         self.uniform_mbs = getattr(self, "uniform_mbs", True)
-        # Consecutive micro-batches share a stage's jobs until these have this many rows (PFEIFE_JOB_ROWS; 0: every
-        # micro-batch has jobs of its own)
+        # Consecutive micro-batches share a stage's jobs until these have this many rows (PFEIFE_JOB_ROWS; a job of several
+        # has up to about twice as many; 0: every micro-batch has jobs of its own)
         self.job_rows = int(os.environ.get("PFEIFE_JOB_ROWS", str(JOB_ROWS)))
         self.mb_sizes = getattr(self, "mb_sizes", [1] * self.option.batch_cnt)    # samples, set by the runner
         self._layouts = {}         # tag -> MicroBatchLayout
