@@ -957,8 +957,7 @@ extern "C" int pf_gemm_variant(const pf_gemm_desc* desc, char* out, int cap) {
   if (d.batch2 <= 0) d.batch2 = 1;
   if (d.in_dtype == PF_F32 || d.K == 0) {
     if (d.in_dtype != PF_F32 || d.K == 0) snprintf(out, (size_t)cap, "gemm32_kernel");
-    else if (pf_gemm_f32_direct_ok(d))
-      snprintf(out, (size_t)cap, "gemm32d_kernel<%s, %s, %s>", pf_gemm_f32_direct_shape(d), d.a_trans ? "true" : "false", d.b_trans ? "true" : "false");
+    else if (pf_gemm_f32_direct_ok(d)) pf_gemm_f32_direct_name(d, out, (size_t)cap);
     else snprintf(out, (size_t)cap, "gemm32x_kernel<64, 64, 64>");
     return PF_OK;
   }

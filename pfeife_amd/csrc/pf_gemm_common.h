@@ -276,5 +276,5 @@ inline int x_epi_class(const pf_gemm_desc& d, int vec_ok, int bm) {
 
 // pf_gemm_f32.hip: fp32 products straight from 16-byte-aligned operands
 bool pf_gemm_f32_direct_ok(const pf_gemm_desc& d);
-const char* pf_gemm_f32_direct_shape(const pf_gemm_desc& d);
+void pf_gemm_f32_direct_name(const pf_gemm_desc& d, char* out, size_t cap);   // the kernel, as the profiler prints it
 int pf_gemm_f32_direct(const pf_gemm_desc& d, hipStream_t st);

@@ -1,5 +1,5 @@
-// fp32 matrix products on v_mfma_f32_16x16x4_f32, operands straight from global memory into LDS.
-#include "pf_gemm_common.h"
+// fp32 matrix products on v_mfma_f32_16x16x4_f32, operands straight from global memory into LDS: shallow ones, and the choice.
+#include "pf_gemm_f32.h"
 
 namespace {
 
@@ -25,32 +25,7 @@ namespace {
 // 788 x 384 x 1536 55.2 -> 20.3, 788 x 1536 x 384 27.2 -> 17.3, 3152 x 1536 x 384 64.1 -> 37.9, 4096 x 4096 x 1024
 // 307 -> 261 (131 TFLOP/s); weight gradients over 3152 rows: 384 x 384 83 -> 24, 1536 x 384 84 -> 57.
 // ---------------------------------------------------------------------------
-#define PF_LDS(T) __attribute__((address_space(3))) T*
-typedef float float2_t __attribute__((ext_vector_type(2)));
 constexpr int FK = 32;   // depth of a tile
-
-// Fragments are read by inline assembly (the compiler would make an LDS read wait for every outstanding
-// direct-to-LDS load); it takes their registers for complete where the read is issued.  arrived(), after the wait,
-// keeps what uses them below it, and the registers theirs until then.
-template <bool TRANS> struct FragF;
-template <> struct FragF<false> {
-  float4_t v;
-  template <int E> __device__ __forceinline__ float get() const { return v[E]; }
-  __device__ __forceinline__ void arrived() { asm volatile("" : "+v"(v)); }
-  // zero the reduction indices from `left` on (k: the lane's first one)
-  __device__ __forceinline__ void mask(int k, int left) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = k + e < left ? v[e] : 0.f;
-  }
-};
-template <> struct FragF<true> {
-  float2_t lo, hi;
-  template <int E> __device__ __forceinline__ float get() const { return E == 0 ? lo.x : E == 1 ? lo.y : E == 2 ? hi.x : hi.y; }
-  __device__ __forceinline__ void arrived() { asm volatile("" : "+v"(lo), "+v"(hi)); }
-  __device__ __forceinline__ void mask(int, int) {}   // (k-rows past K arrive as zeros)
-};
-template <int N> __device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory"); }
-template <int N> __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
 template <int R, int NW, bool TRANS> struct FTile {
   static constexpr int BYTES = R * FK * 4;
@@ -188,7 +163,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm32d_kernel(const pf_gemm_d
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[S][H][i].template get<E>(), fb[S][H][j].template get<E>(), acc[i][j], 0, 0, 0);
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[S][H][i].get(E), fb[S][H][j].get(E), acc[i][j], 0, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
   };
   constexpr std::integral_constant<int, 0> c0{};
@@ -249,82 +224,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm32d_kernel(const pf_gemm_d
   arrived(c1);
   __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the dropped requests past K
 
-  // Epilogue.  D layout of v_mfma_f32_16x16x*: lane l holds column l % 16 and rows 4*(l/16) + r: 16 lanes cover 64
-  // consecutive bytes.  With fp32 operands throughout (vec_epi), everything one step reads is requested before any of it is used;
-  // the buffers' range checks drop rows past M, columns past N are sent out of range.
-  const Epi epi = make_epi(p);
-  const int64_t row0 = m0 + wm0 + 4 * (lane >> 4), col0 = n0 + wn0 + (lane & 15);
-  if (!g.vec_epi) {
-#pragma nounroll
-    for (int h = 0; h < TM * TN; ++h) {
-      float4_t x;
-      static_for<TM * TN>([&](auto hc) {
-        constexpr int c = decltype(hc)::value;
-        if (h == c) x = acc[c / TN][c % TN];
-      });
-      const int64_t col = col0 + 16 * (h % TN);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t row = row0 + 16 * (h / TN) + r;
-        if (row < M && col < N) epilogue_scalar(epi, c_base, row, col, x[r]);
-      }
-    }
-    return;
-  }
-  const int rows_left = (int)(M - m0 < BM ? M - m0 : BM);
-  auto buffer = [&](const void* x, int64_t ld) {   // rows m0 .. of an operand of C's shape
-    return make_rsrc((const float*)x + m0 * ld, (uint32_t)(((rows_left - 1) * ld + N) * 4));
-  };
-  auto offset = [&](int i, int j, int r, int64_t ld) {
-    const int64_t col = col0 + 16 * j;
-    return col < N ? (int)(((wm0 + 16 * i + 4 * (lane >> 4) + r) * ld + col) * 4) : (int)0x80000000;
-  };
-  auto each = [&](auto&& f) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) f(i, j, r);
-  };
-  float4_t x[TM][TN];
-  auto load = [&](const void* src, int64_t ld) {
-    const __amdgpu_buffer_rsrc_t rs = buffer(src, ld);
-    each([&](int i, int j, int r) { x[i][j][r] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, offset(i, j, r, ld), 0, 0)); });
-  };
-  each([&](int i, int j, int r) { acc[i][j][r] *= epi.alpha; });
-  if (epi.bias) {
-    const __amdgpu_buffer_rsrc_t rs = make_rsrc(epi.bias, (uint32_t)(N * 4));
-    float b[TN];
-#pragma unroll
-    for (int j = 0; j < TN; ++j) b[j] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, (int)((col0 + 16 * j) * 4), 0, 0));
-    each([&](int i, int j, int r) { acc[i][j][r] += b[j]; });
-  }
-  if (epi.aux_out) {
-    const __amdgpu_buffer_rsrc_t rs = buffer(epi.aux_out, epi.ld_aux_out);
-    each([&](int i, int j, int r) { __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(acc[i][j][r]), rs, offset(i, j, r, epi.ld_aux_out), 0, 0); });
-  }
-  if (epi.act == PF_ACT_GELU) {
-    each([&](int i, int j, int r) { acc[i][j][r] = pf_gelu_erf(acc[i][j][r]); });
-  } else if (epi.act != PF_ACT_NONE) {
-    each([&](int i, int j, int r) { acc[i][j][r] = pf_act(epi.act, acc[i][j][r]); });
-  }
-  if (epi.dact != PF_ACT_NONE) {
-    load(epi.aux_in, epi.ld_aux_in);
-    if (epi.dact == PF_ACT_GELU) each([&](int i, int j, int r) { acc[i][j][r] *= pf_gelu_erf_grad(x[i][j][r]); });
-    else each([&](int i, int j, int r) { acc[i][j][r] *= pf_act_grad(epi.dact, x[i][j][r]); });
-  }
-  if (epi.residual) {
-    load(epi.residual, epi.ld_res);
-    each([&](int i, int j, int r) { acc[i][j][r] += x[i][j][r]; });
-  }
-  const float* C = (const float*)epi.C + c_base;
-  if (epi.beta) {
-    load(C, epi.ldc);
-    each([&](int i, int j, int r) { acc[i][j][r] += x[i][j][r]; });
-  }
-  const __amdgpu_buffer_rsrc_t rs = buffer(C, epi.ldc);
-  each([&](int i, int j, int r) { __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(acc[i][j][r]), rs, offset(i, j, r, epi.ldc), 0, 0); });
+  // D layout of v_mfma_f32_16x16x*: lane l holds column l % 16 and rows 4*(l/16) + r
+  epilogue_f32<BM>(p, g, acc, m0, wm0 + 4 * (lane >> 4), n0 + wn0 + (lane & 15), c_base);
 }
 
 template <int BM, int BN, int WGM, int WGN, int ST, bool AT, bool BT>
@@ -344,9 +245,7 @@ int launch(const pf_gemm_desc& d, hipStream_t st) {
   g.tiles_m = (int)((d.M + BM - 1) / BM);
   g.tiles_n = (int)((d.N + BN - 1) / BN);
   g.per_xcd = (int)(((int64_t)g.tiles_m * g.tiles_n + 7) / 8);
-  const int64_t lim = (1ll << 31) / (4 * BM) - 1;
-  g.vec_epi = d.c_dtype == PF_F32 && (!d.bias || d.bias_dtype == PF_F32) && (!d.residual || d.res_dtype == PF_F32) && d.ldc < lim &&
-              (!d.residual || d.ld_res < lim) && (!d.aux_in || d.ld_aux_in < lim) && (!d.aux_out || d.ld_aux_out < lim);
+  g.vec_epi = epi_f32_vec_ok(d, BM);
   const dim3 grid((unsigned)(g.per_xcd * 8), (unsigned)(d.batch1 * d.batch2), 1);
   if (d.a_trans && d.b_trans) return launch_one<BM, BN, WGM, WGN, ST, true, true>(d, g, grid, st);
   if (d.a_trans) return launch_one<BM, BN, WGM, WGN, ST, true, false>(d, g, grid, st);
@@ -390,9 +289,20 @@ bool pf_gemm_f32_direct_ok(const pf_gemm_desc& d) {
          d.a_stride2 % 4 == 0 && d.b_stride1 % 4 == 0 && d.b_stride2 % 4 == 0 && d.lda < lim && d.ldb < lim && d.K < (1ll << 31) &&
          d.N < (1ll << 29);
 }
-const char* pf_gemm_f32_direct_shape(const pf_gemm_desc& d) { return TILES[choose(d)].shape; }
+
+// Depths from 129 on go to the wavefronts that split the depth, unless its stages of 64 would be a fifth empty.  us here / there: 3152 x 384 over 384
+// 17.6 / 12.8, 788 x 384 over 1536 20.8 / 14.9, 442 x 1476 over 176 8.6 / 7.2, 4877 x 80 over 281 7.1 / 7.3; 96 products of 197 x 64 over 197 16.9 / 18.2,
+// 8675 x 364 over 69 12.6 / 16.7, 7967 x 4996 over 126 122 / 128, 96 products of 197 x 197 over 64 19.3 / 20.0
+static bool by_depth(const pf_gemm_desc& d) { return d.K > 128 && (d.K + 63) / 64 * 64 * 4 <= d.K * 5; }
+
+void pf_gemm_f32_direct_name(const pf_gemm_desc& d, char* out, size_t cap) {
+  const char* layouts = d.a_trans ? (d.b_trans ? "true, true" : "true, false") : (d.b_trans ? "false, true" : "false, false");
+  if (by_depth(d)) snprintf(out, cap, "gemm32k_kernel<%s, %s>", pf_gemm_f32_depth_shape(d), layouts);
+  else snprintf(out, cap, "gemm32d_kernel<%s, %s>", TILES[choose(d)].shape, layouts);
+}
 
 int pf_gemm_f32_direct(const pf_gemm_desc& d, hipStream_t st) {
+  if (by_depth(d)) return pf_gemm_f32_depth(d, st);
   switch (choose(d)) {
     case 0: return launch<128, 128, 2, 4, 4>(d, st);
     case 1: return launch<64, 64, 4, 2, 4>(d, st);

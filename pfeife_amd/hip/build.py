@@ -21,6 +21,7 @@ SOURCES = [
     "pf_issuer.cpp",
     "pf_gemm.hip",
     "pf_gemm_f32.hip",
+    "pf_gemm_f32_depth.hip",
     "pf_attention.hip",
     "pf_norm.hip",
     "pf_elementwise.hip",
