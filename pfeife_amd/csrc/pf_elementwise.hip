@@ -1,7 +1,9 @@
 // HBM-bound streaming kernels: activations, gated MLP, axpby, bias add, casts,
 // fills, strided copies, rotary embedding and the fp32 gradient accumulation.
-// All of them move 16 bytes (8 x 16-bit) or 32 bytes (8 x fp32) per lane per
-// step in a grid-stride loop sized to keep every CU busy.
+// All of them move 16 bytes (8 x 16-bit) or 32 bytes (8 x fp32) per lane, once: a workgroup to every 256 of these, in
+// the order of memory.  The dispatcher then keeps what is in flight to a narrow window that moves over the operands;
+// workgroups that stay and loop drift apart, and memory's open pages with them (1 GiB copied at 5.5 against 6.6 TB/s, Adam's seven streams
+// at 5.2 against 6.2).
 #include <math.h>
 
 #include "pf_common.h"
@@ -9,7 +11,7 @@
 namespace {
 
 constexpr int EW_BLOCK = 256;
-constexpr int EW_MAX_BLOCKS = 256 * 16;  // 16 workgroups per CU is plenty of bytes in flight
+constexpr int64_t EW_MAX_BLOCKS = 1 << 23;  // (a launch has less than 2^32 threads: beyond, they loop)
 
 inline dim3 ew_grid(int64_t work_items) {
   int64_t b = (work_items + EW_BLOCK - 1) / EW_BLOCK;
@@ -34,6 +36,19 @@ int ew_launch(const F& f, int64_t n, bool vec, hipStream_t st, const char* name)
   hipLaunchKernelGGL(ew_kernel<F>, ew_grid(vec ? (n + 7) / 8 : n), dim3(EW_BLOCK), 0, st, f, n, vec ? 1 : 0);
   PF_CHECK_LAUNCH(name);
   return PF_OK;
+}
+
+// Quotient and remainder of an index: in 32 bits where it fits (a 64-bit division is some 150 instructions, several times what the
+// loads and stores of eight elements cost)
+__device__ __forceinline__ void div_mod(int64_t i, int64_t d, int64_t& q, int64_t& r) {
+  if ((uint64_t)(i | d) >> 32) {
+    q = i / d;
+    r = i - q * d;
+  } else {
+    const uint32_t q32 = (uint32_t)i / (uint32_t)d;
+    q = q32;
+    r = (uint32_t)i - q32 * (uint32_t)d;
+  }
 }
 
 inline bool al16(const void* p) { return pf_aligned(p, 16); }
@@ -128,7 +143,8 @@ template <int DT = -1>
 struct GluFwd {
   const void* gate; const void* up; void* y; int64_t ldg, ldu, ldy, cols; int dt, act;
   template <int W> __device__ void run(int64_t i) const {
-    const int64_t r = i / cols, c = i % cols;
+    int64_t r, c;
+    div_mod(i, cols, r, c);
     const int edt = DT >= 0 ? DT : dt;
     float g[W], u[W];
     ld_vec_c<W, DT>(gate, r * ldg + c, dt, g);
@@ -143,7 +159,8 @@ struct GluBwd {
   const void* dy; const void* gate; const void* up; void* dgate; void* dup;
   int64_t lddy, ldg, ldu, lddg, lddu, cols; int dt, act;
   template <int W> __device__ void run(int64_t i) const {
-    const int64_t r = i / cols, c = i % cols;
+    int64_t r, c;
+    div_mod(i, cols, r, c);
     const int edt = DT >= 0 ? DT : dt;
     float d[W], g[W], u[W], dg[W], du[W];
     ld_vec_c<W, DT>(dy, r * lddy + c, dt, d);
@@ -173,8 +190,8 @@ __global__ __launch_bounds__(EW_BLOCK) void copy_strided_kernel(const void* src,
 #pragma unroll
     for (int k = 5; k >= 0; --k) {
       if (k < cd.ndim) {
-        const int64_t idx = rem % cd.size[k];
-        rem /= cd.size[k];
+        int64_t idx;
+        div_mod(rem, cd.size[k], rem, idx);
         const int64_t mul = (k == cd.ndim - 1) ? W : 1;
         so += idx * cd.ss[k] * mul;
         dof += idx * cd.ds[k] * mul;
@@ -201,8 +218,8 @@ __global__ __launch_bounds__(EW_BLOCK) void copy_strided_raw_kernel(const U* src
 #pragma unroll
     for (int k = 5; k >= 0; --k) {
       if (k < cd.ndim) {
-        const int64_t idx = rem % cd.size[k];
-        rem /= cd.size[k];
+        int64_t idx;
+        div_mod(rem, cd.size[k], rem, idx);
         so += idx * cd.ss[k];
         dof += idx * cd.ds[k];
       }
@@ -429,13 +446,6 @@ __global__ void adam_coefficients_kernel(float* state, double lr, double beta1, 
   state[5] = (float)sqrt(1.0 - pow(beta2, t));
 }
 
-// Bound by memory: 16 bytes read and 12 written per parameter.  The tensors of a model differ in size by four
-// orders of magnitude, so they are cut into chunks and every workgroup of a grid that just fills the chip gets the
-// same number of consecutive ones (with a fixed number of workgroups per tensor the largest, an embedding, was left
-// to 64 of them).  Gradients and moments are next used a step later and bypass the caches.  337 M parameters, 131 M of
-// them in two embeddings: 2278 -> 1858 us alone (5.07 TB/s; a copy of 1 GiB reaches 5.15), 3.0 -> 1.9 ms in a step;
-// 303 M in 288 tensors 1773 -> 1681 us.
-constexpr int ADAM_CHUNK = 2048;
 __device__ __forceinline__ float4 ld_once(const float* p) {
   const float4_t x = __builtin_nontemporal_load((const float4_t*)p);
   return make_float4(x.x, x.y, x.z, x.w);
@@ -444,24 +454,75 @@ __device__ __forceinline__ void st_once(float* p, const float4& v) {
   const float4_t x = {v.x, v.y, v.z, v.w};
   __builtin_nontemporal_store(x, (float4_t*)p);
 }
-__global__ __launch_bounds__(256) void adam_kernel(const pf_adam_item* items, int n_items, float lr, float omb1, float beta2, float omb2,
-                                                   float eps, float weight_decay, float step_size,
-                                                   float bias_c2_sqrt, int adamw, const float* scaler_state) {
-  // omb1 = 1 - beta1, omb2 = 1 - beta2, step_size = lr / (1 - beta1^t): formed in double
-  // like torch does, then rounded once
-  if (scaler_state != nullptr) {
-    if (scaler_state[2] != 0.f) return;   // uniform over the grid
-    step_size = scaler_state[4];
-    bias_c2_sqrt = scaler_state[5];
+// omb1 = 1 - beta1, omb2 = 1 - beta2, step_size = lr / (1 - beta1^t): formed in double like torch does, then rounded once
+struct AdamCoef {
+  float lr, omb1, beta2, omb2, eps, weight_decay, step_size, bias_c2_sqrt;
+  int adamw;
+  // with a loss scaler: its state says whether there is an update (uniform over the grid) and has the last two
+  __device__ __forceinline__ bool scaled(const float* state) {
+    if (state == nullptr) return true;
+    step_size = state[4];
+    bias_c2_sqrt = state[5];
+    return state[2] == 0.f;
   }
-  const auto update = [&](float& p, float g, float& m, float& v) {
+  __device__ __forceinline__ void update(float& p, float g, float& m, float& v) const {
     if (adamw) p *= 1.f - lr * weight_decay;
     else if (weight_decay != 0.f) g += weight_decay * p;
     m = m + omb1 * (g - m);
     v = v * beta2 + omb2 * g * g;
     const float denom = sqrtf(v) / bias_c2_sqrt + eps;
     p = p - step_size * (m / denom);
-  };
+  }
+  // the four elements from i on of an item
+  __device__ __forceinline__ void update4(const pf_adam_item& it, int64_t i) const {
+    if (i + 4 <= it.n) {
+      float4 p = ld_once(it.param + i), m = ld_once(it.exp_avg + i), v = ld_once(it.exp_avg_sq + i);
+      const float4 g = ld_once(it.grad + i);
+      update(p.x, g.x, m.x, v.x);
+      update(p.y, g.y, m.y, v.y);
+      update(p.z, g.z, m.z, v.z);
+      update(p.w, g.w, m.w, v.w);
+      st_once(it.param + i, p);
+      st_once(it.exp_avg + i, m);
+      st_once(it.exp_avg_sq + i, v);
+    } else {
+      for (int64_t j = i; j < it.n; ++j) {
+        float p = it.param[j], m = it.exp_avg[j], v = it.exp_avg_sq[j];
+        update(p, it.grad[j], m, v);
+        it.param[j] = p; it.exp_avg[j] = m; it.exp_avg_sq[j] = v;
+      }
+    }
+  }
+};
+
+// Bound by memory: 16 bytes read and 12 written per parameter.  The tensors of a model differ in size by four orders of
+// magnitude, so they are cut into chunks of 1024, and a workgroup updates one: all that is in flight then lies in a narrow window that moves over the
+// seven streams (see the top of this file).  2048 workgroups that stay, with consecutive chunks each, reach 5.2 TB/s over 268 M parameters, chunks dealt
+// out in turn 4.9, two chunks to a workgroup 5.7, one 6.2.  Everything is next used a step later and bypasses the caches.
+// Which item: `ends`, the chunks up to and including each item's last, is searched by each wavefront, 64 ways at a time.
+constexpr int ADAM_CHUNK = PF_ADAM_CHUNK;
+__global__ __launch_bounds__(256) void adam_chunk_kernel(const pf_adam_item* items, const int64_t* ends, int n_items, AdamCoef c,
+                                                         const float* scaler_state) {
+  if (!c.scaled(scaler_state)) return;
+  const int64_t chunk = blockIdx.x;
+  const int lane = threadIdx.x & 63;
+  int lo = 0, hi = n_items - 1;      // the item is one of these: the first whose end is past the chunk
+  while (lo < hi) {
+    const int step = (hi - lo + 64) / 64;
+    int at = lo + (lane + 1) * step - 1;
+    if (at > hi) at = hi;
+    const int k = __ffsll((unsigned long long)__ballot(ends[at] > chunk)) - 1;   // (the last item's end is)
+    hi = lo + (k + 1) * step - 1 < hi ? lo + (k + 1) * step - 1 : hi;
+    lo = lo + k * step;
+  }
+  lo = __builtin_amdgcn_readfirstlane(lo);
+  c.update4(items[lo], (chunk - (lo > 0 ? ends[lo - 1] : 0)) * ADAM_CHUNK + threadIdx.x * 4);
+}
+
+// The same for callers who have the items only: workgroups that stay, each with the same number of consecutive chunks, which it finds by adding up the
+// items' sizes itself.
+__global__ __launch_bounds__(256) void adam_kernel(const pf_adam_item* items, int n_items, AdamCoef c, const float* scaler_state) {
+  if (!c.scaled(scaler_state)) return;
   // this workgroup's chunks of the items laid end to end, first .. last - 1
   __shared__ int64_t wave_sum[4];
   __shared__ int64_t found[2];   // item that holds the first chunk, the chunk's index in it
@@ -508,38 +569,8 @@ __global__ __launch_bounds__(256) void adam_kernel(const pf_adam_item* items, in
       it = items[++item];
       chunk = 0;
     }
-    const int64_t i0 = chunk * ADAM_CHUNK + tid * 4;
+    c.update4(it, chunk * ADAM_CHUNK + tid * 4);
     ++chunk;
-    constexpr int U = ADAM_CHUNK / 1024;
-    if ((chunk * ADAM_CHUNK) <= it.n) {
-      float4 p[U], g[U], m[U], v[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t i = i0 + u * 1024;
-        p[u] = *(const float4*)(it.param + i), g[u] = ld_once(it.grad + i);
-        m[u] = ld_once(it.exp_avg + i), v[u] = ld_once(it.exp_avg_sq + i);
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t i = i0 + u * 1024;
-        float* pp = (float*)&p[u];
-        float* mm = (float*)&m[u];
-        float* vv = (float*)&v[u];
-        const float* gg = (const float*)&g[u];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) update(pp[k], gg[k], mm[k], vv[k]);
-        *(float4*)(it.param + i) = p[u];
-        st_once(it.exp_avg + i, m[u]);
-        st_once(it.exp_avg_sq + i, v[u]);
-      }
-    } else {
-      for (int u = 0; u < U; ++u)
-        for (int64_t j = i0 + u * 1024; j < i0 + u * 1024 + 4 && j < it.n; ++j) {
-          float p = it.param[j], m = it.exp_avg[j], v = it.exp_avg_sq[j];
-          update(p, it.grad[j], m, v);
-          it.param[j] = p; it.exp_avg[j] = m; it.exp_avg_sq[j] = v;
-        }
-    }
   }
 }
 
@@ -553,11 +584,10 @@ __global__ __launch_bounds__(EW_BLOCK) void rope_kernel(const void* x, void* y, 
   const int64_t total = B * T * H * half;
   const int64_t gsz = (int64_t)gridDim.x * blockDim.x;
   for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += gsz) {
-    const int64_t i = idx % half;
-    int64_t r = idx / half;
-    const int64_t h = r % H;
-    r /= H;
-    const int64_t t = r % T, b = r / T;
+    int64_t i, r, h, t, b;
+    div_mod(idx, half, r, i);
+    div_mod(r, H, r, h);
+    div_mod(r, T, b, t);
     const int64_t xo = b * xsb + t * xst + h * xsh, yo = b * ysb + t * yst + h * ysh;
     const float x1 = pf_load_as_f32(x, xo + i, dt), x2 = pf_load_as_f32(x, xo + i + half, dt);
     const float c = cos_t[t * tab_ld + i];
@@ -799,11 +829,11 @@ __global__ __launch_bounds__(EW_BLOCK) void rope_vec_kernel(const uint16_t* x, u
   const int64_t total = B * T * H * hv;
   const int64_t gsz = (int64_t)gridDim.x * blockDim.x;
   for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += gsz) {
-    const int64_t i = (idx % hv) * 8;
-    int64_t r = idx / hv;
-    const int64_t h = r % H;
-    r /= H;
-    const int64_t t = r % T, b = r / T;
+    int64_t i, r, h, t, b;
+    div_mod(idx, hv, r, i);
+    i *= 8;
+    div_mod(r, H, r, h);
+    div_mod(r, T, b, t);
     const int64_t xo = b * xsb + t * xst + h * xsh + i, yo = b * ysb + t * yst + h * ysh + i;
     float x1[8], x2[8], c[8], sn[8], o1[8], o2[8];
     Vec8<DT>::load(x, xo, x1);
@@ -947,10 +977,7 @@ extern "C" int pf_scaler_unscale(float* grads, int64_t n, float* state, void* st
   PF_REQUIRE(n >= 0, "pf_scaler_unscale: negative size");
   if (n == 0) return PF_OK;
   PF_REQUIRE(grads && state && pf_aligned(grads, 16), "pf_scaler_unscale: null or unaligned pointer");
-  int64_t blocks = (n / 4 + 255) / 256;
-  if (blocks > 2048) blocks = 2048;
-  if (blocks < 1) blocks = 1;
-  hipLaunchKernelGGL(scaler_unscale_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, grads, n, state);
+  hipLaunchKernelGGL(scaler_unscale_kernel, ew_grid((n + 3) / 4), dim3(256), 0, (hipStream_t)stream, grads, n, state);
   PF_CHECK_LAUNCH("pf_scaler_unscale");
   return PF_OK;
 }
@@ -973,35 +1000,48 @@ extern "C" int pf_scale_by_state(const void* src, int src_dtype, const float* st
   PF_REQUIRE(pf_is_float_dtype(src_dtype) && pf_is_float_dtype(dst_dtype), "pf_scale_by_state: bad dtype");
   ScaleByState f{src, src_dtype, state, dst, dst_dtype};
   const int vec = pf_aligned(src, 16) && pf_aligned(dst, 16);
-  int64_t blocks = ((vec ? n / 8 : n) + 255) / 256;
-  if (blocks > 2048) blocks = 2048;
-  if (blocks < 1) blocks = 1;
-  hipLaunchKernelGGL(scale_by_state_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, f, n, vec);
+  hipLaunchKernelGGL(scale_by_state_kernel, ew_grid(vec ? (n + 7) / 8 : n), dim3(256), 0, (hipStream_t)stream, f, n, vec);
   PF_CHECK_LAUNCH("pf_scale_by_state");
   return PF_OK;
 }
 
 namespace {
+AdamCoef adam_coef(double lr, double beta1, double beta2, double eps, double weight_decay, int64_t step, int adamw) {
+  const double bc1 = 1.0 - pow(beta1, (double)step), bc2 = 1.0 - pow(beta2, (double)step);
+  return {(float)lr, (float)(1.0 - beta1), (float)beta2, (float)(1.0 - beta2), (float)eps, (float)weight_decay, (float)(lr / bc1), (float)sqrt(bc2), adamw};
+}
+
 int adam_launch(const pf_adam_item* items_dev, int n_items, int64_t max_n, double lr, double beta1, double beta2,
                 double eps, double weight_decay, int64_t step, int adamw, float* scaler_state, void* stream,
                 const char* name) {
   PF_REQUIRE(n_items >= 0 && max_n >= 0, "%s: bad arguments", name);
   if (n_items == 0 || max_n == 0) return PF_OK;
   PF_REQUIRE(items_dev != nullptr && n_items <= 65535, "%s: bad item list", name);
-  const double bc1 = 1.0 - pow(beta1, (double)step);
-  const double bc2 = 1.0 - pow(beta2, (double)step);
   int64_t blocks = (max_n + ADAM_CHUNK - 1) / ADAM_CHUNK * n_items;
   if (blocks > 2048) blocks = 2048;   // eight to a CU, all resident
   if (scaler_state != nullptr)
     hipLaunchKernelGGL(adam_coefficients_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, scaler_state, lr, beta1,
                        beta2);
-  hipLaunchKernelGGL(adam_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, items_dev, n_items, (float)lr,
-                     (float)(1.0 - beta1), (float)beta2, (float)(1.0 - beta2), (float)eps, (float)weight_decay,
-                     (float)(lr / bc1), (float)sqrt(bc2), adamw, scaler_state);
+  hipLaunchKernelGGL(adam_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, items_dev, n_items,
+                     adam_coef(lr, beta1, beta2, eps, weight_decay, step, adamw), scaler_state);
   PF_CHECK_LAUNCH(name);
   return PF_OK;
 }
 }  // namespace
+
+extern "C" int pf_adam_step_chunks(const pf_adam_item* items_dev, const int64_t* chunk_ends_dev, int n_items, int64_t n_chunks, double lr,
+                                   double beta1, double beta2, double eps, double weight_decay, int64_t step, int adamw,
+                                   float* scaler_state, void* stream) {
+  PF_REQUIRE(n_items >= 0 && n_chunks >= 0 && (scaler_state != nullptr || step >= 1), "pf_adam_step_chunks: bad arguments");
+  if (n_items == 0 || n_chunks == 0) return PF_OK;
+  PF_REQUIRE(items_dev != nullptr && chunk_ends_dev != nullptr && n_chunks < (1ll << 24), "pf_adam_step_chunks: bad item list");
+  if (scaler_state != nullptr)
+    hipLaunchKernelGGL(adam_coefficients_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, scaler_state, lr, beta1, beta2);
+  hipLaunchKernelGGL(adam_chunk_kernel, dim3((unsigned)n_chunks), dim3(256), 0, (hipStream_t)stream, items_dev, chunk_ends_dev, n_items,
+                     adam_coef(lr, beta1, beta2, eps, weight_decay, scaler_state != nullptr ? 1 : step, adamw), scaler_state);
+  PF_CHECK_LAUNCH("pf_adam_step_chunks");
+  return PF_OK;
+}
 
 extern "C" int pf_shadow_batch(const pf_shadow_item* items_dev, int n_items, int64_t max_tiles, void* stream) {
   PF_REQUIRE(n_items >= 0 && max_tiles >= 0, "pf_shadow_batch: bad arguments");

@@ -20,6 +20,7 @@ ABI_VERSION = 5
 
 PF_F32, PF_F16, PF_BF16, PF_I64, PF_I32, PF_U8 = 0, 1, 2, 3, 4, 5
 ACT_NONE, ACT_GELU, ACT_GELU_TANH, ACT_SILU, ACT_RELU = 0, 1, 2, 3, 4
+ADAM_CHUNK = 1024   # PF_ADAM_CHUNK
 
 _DTYPE_CODE = {
     torch.float32: PF_F32,
@@ -142,6 +143,8 @@ _SIGNATURES = {
                      _I, _P],
     "pf_adam_step_scaled": [_P, _I, _L, ctypes.c_double, ctypes.c_double, ctypes.c_double, ctypes.c_double,
                             ctypes.c_double, _I, _P, _P],
+    "pf_adam_step_chunks": [_P, _P, _I, _L, ctypes.c_double, ctypes.c_double, ctypes.c_double, ctypes.c_double,
+                            ctypes.c_double, _L, _I, _P, _P],
     "pf_scale_by_state": [_P, _I, _P, _P, _I, _L, _P],
     "pf_scaler_unscale": [_P, _L, _P, _P],
     "pf_scaler_update": [_P, ctypes.c_double, ctypes.c_double, _I, _P],
@@ -666,26 +669,31 @@ class HipKernels:
         return self._prep("pf_transpose_cast", args, (src, dst), rows * cols * (_es(src) + _es(dst)))
 
     def adam_table(self, params, grads, exp_avgs, exp_avg_sqs):
-        """Device table of pf_adam_item for one param group (built once, pointers are static)."""
-        rows = [[p.data_ptr(), g.data_ptr(), m.data_ptr(), v.data_ptr(), p.numel()]
-                for p, g, m, v in zip(params, grads, exp_avgs, exp_avg_sqs)]
-        for r in rows:
-            if any(x % 16 for x in r[:4]):
+        """Device table of one param group: its pf_adam_items, then the running count of their chunks (built once, pointers
+        are static).  -> (table, items, chunks)"""
+        rows, ends, chunks = [], [], 0
+        for p, g, m, v in zip(params, grads, exp_avgs, exp_avg_sqs):
+            row = [p.data_ptr(), g.data_ptr(), m.data_ptr(), v.data_ptr(), p.numel()]
+            if any(x % 16 for x in row[:4]):
                 raise RuntimeError("adam: tensors must be 16-byte aligned")
-        table = torch.tensor(rows, dtype=torch.int64).to(params[0].device)
-        return table, len(rows), max(r[4] for r in rows)
+            chunks += -(-row[4] // ADAM_CHUNK)
+            rows += row
+            ends.append(chunks)
+        table = torch.tensor(rows + ends, dtype=torch.int64).to(params[0].device)
+        return table, len(ends), chunks
 
-    def adam_step(self, table, n_items, max_n, lr, beta1, beta2, eps, weight_decay, step, adamw, stream):
-        rc = self.lib.pf_adam_step(table.data_ptr(), n_items, max_n, lr, beta1, beta2, eps, weight_decay, step,
-                                   int(adamw), stream)
+    def _adam(self, table, n_items, n_chunks, lr, beta1, beta2, eps, weight_decay, step, adamw, state, stream):
+        items = table.data_ptr()
+        rc = self.lib.pf_adam_step_chunks(items, items + 40 * n_items, n_items, n_chunks, lr, beta1, beta2, eps, weight_decay, step,
+                                          int(adamw), state, stream)
         if rc != 0:
-            raise RuntimeError("pf_adam_step failed: %s" % self.lib.pf_last_error().decode())
+            raise RuntimeError("pf_adam_step_chunks failed: %s" % self.lib.pf_last_error().decode())
 
-    def adam_step_scaled(self, table, n_items, max_n, lr, beta1, beta2, eps, weight_decay, adamw, state, stream):
-        rc = self.lib.pf_adam_step_scaled(table.data_ptr(), n_items, max_n, lr, beta1, beta2, eps, weight_decay,
-                                          int(adamw), state.data_ptr(), stream)
-        if rc != 0:
-            raise RuntimeError("pf_adam_step_scaled failed: %s" % self.lib.pf_last_error().decode())
+    def adam_step(self, table, n_items, n_chunks, lr, beta1, beta2, eps, weight_decay, step, adamw, stream):
+        self._adam(table, n_items, n_chunks, lr, beta1, beta2, eps, weight_decay, step, adamw, None, stream)
+
+    def adam_step_scaled(self, table, n_items, n_chunks, lr, beta1, beta2, eps, weight_decay, adamw, state, stream):
+        self._adam(table, n_items, n_chunks, lr, beta1, beta2, eps, weight_decay, 1, adamw, state.data_ptr(), stream)
 
     # -- dynamic loss scaling (state: float32[8] on the device) ----------------------------
     def scale_by_state(self, src, state, dst, n):

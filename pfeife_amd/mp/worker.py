@@ -856,19 +856,19 @@ class StageWorker:
             groups.append((g, params, ent[1]))
         if scaled and rebuilt:
             self._seed_device_step_count(opt, groups)
-        for g, params, (table, n_items, max_n) in groups:
+        for g, params, (table, n_items, n_chunks) in groups:
             b1, b2 = g["betas"]
             if scaled:
                 # skipped on overflow; the bias corrections use the device's count of completed steps.
                 # The host-side `step` entries are brought up to date from that count when somebody
                 # reads them (sync_optimizer_steps: optimizer.state_dict() calls it)
-                self.kernels.adam_step_scaled(table, n_items, max_n, float(g["lr"]), float(b1), float(b2),
+                self.kernels.adam_step_scaled(table, n_items, n_chunks, float(g["lr"]), float(b1), float(b2),
                                               float(g["eps"]), float(g["weight_decay"]),
                                               type(opt) is torch.optim.AdamW, self.scaler_state, s)
                 self._host_steps_stale = True
             else:
                 step = int(opt.state[params[0]]["step"].item()) + 1
-                self.kernels.adam_step(table, n_items, max_n, float(g["lr"]), float(b1), float(b2), float(g["eps"]),
+                self.kernels.adam_step(table, n_items, n_chunks, float(g["lr"]), float(b1), float(b2), float(g["eps"]),
                                        float(g["weight_decay"]), step, type(opt) is torch.optim.AdamW, s)
                 for p in params:
                     opt.state[p]["step"] += 1
