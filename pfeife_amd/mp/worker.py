@@ -537,12 +537,16 @@ class StageWorker:
         for job in self.dw_jobs.values():
             if job[1] is None and job[0]:
                 job[1] = self.kernels.capture(job[0], s)
-        pre = self.params.zero_launches() + self.params.refresh_launches()
+        pre = self.begin_launches()
         self._drop_begin_graph()
         self.begin_graph = self.kernels.capture(pre, s) if pre else None
         self._begin_len = (len(self.params.zero), len(self.params.refresh))
         self.graphs_ready = True
         self._drop_step_plan()
+
+    def begin_launches(self):
+        """What a step begins with: optimizer.zero_grad(set_to_none=False), and one master -> 16-bit cast."""
+        return self.params.zero_launches() + self.params.refresh_launches()
 
     def distribute_input(self, mb, placeholder_idx, value):
         """Copy one micro-batch slab into the stage input buffer it was built for."""
