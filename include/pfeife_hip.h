@@ -76,6 +76,16 @@ int pf_issuer_create(int device, void** issuer_out);
 int pf_issuer_push(void* issuer, const pf_job* jobs, int n, int64_t* ticket);
 int pf_issuer_wait(void* issuer, int64_t ticket);
 int pf_issuer_destroy(void* issuer);
+
+/* ---- control from thread to thread -----------------------------------------------------------------
+ * Of the thread that calls step() and the threads of its micro-batches exactly one runs at a time (the reference hands over through
+ * queues, pfeife/mp/partial/module.py:87-89, 145-159).  A baton has `slots` counts of tokens, all zero: pf_baton_switch gives one to slot `to`
+ * (to < 0: none) and then takes one from slot `own` (own < 0: none), for at most timeout_us (< 0: as long as it takes): *came = 1 if it got
+ * it, 0 if not (the caller goes on waiting with to = -1).  One thread at a time may wait at a slot.  pf_baton_alert wakes the thread that sleeps at
+ * a slot shortly before its token comes.  A baton is not freed: threads may be waiting at it for as long as the process lives. */
+int pf_baton_create(int slots, void** baton_out);
+int pf_baton_alert(void* baton, int slot);
+int pf_baton_switch(void* baton, int to, int own, int64_t timeout_us, int* came);
 /* events that order streams (no timing) */
 int pf_event_create(void** event_out);
 int pf_event_destroy(void* event);

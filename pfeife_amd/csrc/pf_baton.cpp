@@ -1,0 +1,102 @@
+// Hands control from thread to thread: of the caller of a step and its micro-batches' threads one runs at a time.
+//
+// A queue does that too, but the thread it wakes has been asleep (some 40 us until it runs), and wakes while the other still
+// holds the Python interpreter (and then sleeps again until that one waits).  A step of eight micro-batches hands over 32 times.  Here
+// giving away and waiting are one call, made without the interpreter, and a waiting thread looks for its token for a while before it
+// sleeps; pf_baton_alert wakes a sleeping one ahead of its turn, so that it is looking when the token comes.
+// A step of a decoder with eight micro-batches of 256 tokens 2.3 -> 2.1 ms, of a two-layer ViT with two 0.78 -> 0.72 (queues / this, the rest alike).
+#include <atomic>
+#include <chrono>
+#include <condition_variable>
+#include <exception>
+#include <memory>
+#include <mutex>
+
+#include "pf_common.h"
+
+namespace {
+
+struct Slot {
+  std::atomic<int> tokens{0};
+  std::mutex mutex;
+  std::condition_variable wake;
+  bool alerted = false;
+};
+
+struct Baton {
+  explicit Baton(int n) : n(n), slots(new Slot[n]) {}
+  const int n;
+  const std::unique_ptr<Slot[]> slots;
+};
+
+using Clock = std::chrono::steady_clock;
+// How long a thread looks for its token before it sleeps.  One whose turn is announced, and the caller of a step, whom a micro-batch's
+// loss and backward hooks keep for some 100 us: LOOK; the other micro-batches' threads, who may have long to wait, shortly.
+constexpr auto LOOK = std::chrono::microseconds(300), GLANCE = std::chrono::microseconds(20);
+
+bool take(Slot& s) {
+  int t = s.tokens.load(std::memory_order_acquire);
+  while (t > 0)
+    if (s.tokens.compare_exchange_weak(t, t - 1, std::memory_order_acquire)) return true;
+  return false;
+}
+
+void give(Slot& s) {
+  s.tokens.fetch_add(1, std::memory_order_release);
+  { std::lock_guard<std::mutex> lock(s.mutex); }   // (a waiter is either before its check or asleep)
+  s.wake.notify_one();
+}
+
+// timeout_us < 0: none.  -> has the token come?
+bool wait(Slot& s, int64_t timeout_us) {
+  const Clock::time_point start = Clock::now();
+  auto look = timeout_us < 0 ? GLANCE : LOOK;
+  for (;;) {
+    const Clock::time_point until = Clock::now() + look;
+    do {
+      for (int i = 0; i < 64; ++i) {
+        if (take(s)) return true;
+        __builtin_ia32_pause();
+      }
+    } while (Clock::now() < until);
+    std::unique_lock<std::mutex> lock(s.mutex);
+    const auto ready = [&] { return s.alerted || s.tokens.load(std::memory_order_acquire) > 0; };
+    if (timeout_us < 0) s.wake.wait(lock, ready);
+    else if (!s.wake.wait_until(lock, start + std::chrono::microseconds(timeout_us), ready)) return false;
+    s.alerted = false;
+    look = LOOK;
+  }
+}
+
+}  // namespace
+
+extern "C" int pf_baton_create(int slots, void** out) {
+  PF_REQUIRE(out != nullptr && slots > 0, "pf_baton_create: bad arguments");
+  *out = nullptr;
+  try {
+    *out = new Baton(slots);
+  } catch (const std::exception& e) {
+    pf_set_error("pf_baton_create: %s", e.what());
+    return PF_ERR_HIP;
+  }
+  return PF_OK;
+}
+
+extern "C" int pf_baton_alert(void* baton, int slot) {
+  PF_REQUIRE(baton != nullptr && slot >= 0 && slot < ((Baton*)baton)->n, "pf_baton_alert: bad arguments");
+  Slot& s = ((Baton*)baton)->slots[slot];
+  {
+    std::lock_guard<std::mutex> lock(s.mutex);
+    s.alerted = true;
+  }
+  s.wake.notify_one();
+  return PF_OK;
+}
+
+extern "C" int pf_baton_switch(void* baton, int to, int own, int64_t timeout_us, int* came) {
+  PF_REQUIRE(baton != nullptr && came != nullptr && to < ((Baton*)baton)->n && own < ((Baton*)baton)->n, "pf_baton_switch: bad arguments");
+  Baton& b = *(Baton*)baton;
+  if (to >= 0) give(b.slots[to]);
+  *came = own < 0 || wait(b.slots[own], timeout_us) ? 1 : 0;
+  return PF_OK;
+}

@@ -102,6 +102,9 @@ _SIGNATURES = {
     "pf_issuer_push": [_P, _P, _I, POINTER(c_int64)],
     "pf_issuer_wait": [_P, _L],
     "pf_issuer_destroy": [_P],
+    "pf_baton_create": [_I, POINTER(c_void_p)],
+    "pf_baton_alert": [_P, _I],
+    "pf_baton_switch": [_P, _I, _I, _L, POINTER(c_int)],
     "pf_event_create": [POINTER(c_void_p)],
     "pf_event_destroy": [_P],
     "pf_gemm": [POINTER(GemmDesc), _P],
@@ -268,6 +271,36 @@ class Issuer:
         if self._h:
             self.lib.pf_issuer_destroy(self._h)
             self._h = None
+
+
+class Baton:
+    """Control of a step, handed from thread to thread (`pf_baton_*`; the calls release the interpreter)."""
+
+    def __init__(self, slots):
+        self._lib = load()
+        h = c_void_p()
+        self._check(self._lib.pf_baton_create(slots, byref(h)))
+        self._h = h.value
+
+    @staticmethod
+    def _check(rc):
+        if rc != 0:
+            raise RuntimeError("pfeife_amd: %s" % last_error())
+
+    def alert(self, slot):
+        """The thread that waits at `slot` is next."""
+        self._check(self._lib.pf_baton_alert(self._h, slot))
+
+    def switch(self, to, own, patience=-1):
+        """Wakes the thread at slot `to` (None: nobody) and waits at slot `own` until woken.  patience: microseconds after which
+        the interpreter may look at signals in between."""
+        came = c_int(0)
+        to = -1 if to is None else to
+        while True:
+            self._check(self._lib.pf_baton_switch(self._h, to, own, patience, byref(came)))
+            if came.value:
+                return
+            to = -1
 
 
 class HipKernels:

@@ -19,6 +19,7 @@ OBJ_DIR = os.path.join(HERE, "build")
 SOURCES = [
     "pf_runtime.cpp",
     "pf_issuer.cpp",
+    "pf_baton.cpp",
     "pf_gemm.hip",
     "pf_gemm_f32.hip",
     "pf_gemm_f32_depth.hip",

@@ -36,6 +36,7 @@ from ...batch import split_args_kwargs
 from ...executor.values import Val
 from ...graph.canonicalize import canonicalize
 from ...graph.partition_graph import compute_nodes, is_static_placeholder, partition_by_split_points
+from ...hip import Baton
 from ...option import PipeOption
 from ...utils import get_logger, to_device
 from ..net_states import get_state
@@ -83,6 +84,9 @@ class PartialRunner:
         self._probing = False
         self._train_queues = [SimpleQueue() for _ in range(self.option.batch_cnt)]
         self._return_queues = [SimpleQueue() for _ in range(self.option.batch_cnt)]
+        # control goes from thread to thread by the baton, with what is handed over in the queues: slots i and n + i are what micro-batch
+        # i's thread and, for it, the caller of step() wait at
+        self._baton = Baton(2 * self.option.batch_cnt)
         self._batch_threads = []
         self.results = []
         self.worker = StageWorker(self, self.option, self.net_state.device, kernels)
@@ -117,6 +121,7 @@ class PartialRunner:
         if self.exec_fn is None:
             raise RuntimeError("call set_exec_fn() before step()")
         option = self.option
+        self._baton.alert(0)
         args, kwargs = split_args_kwargs(args, kwargs, option.batch_cnt)
         self.worker.uniform_mbs, self.worker.mb_sizes = _shapes(args, kwargs)
 
@@ -135,13 +140,24 @@ class PartialRunner:
             self.worker.settle_failed_step()
             raise
 
+    def _hand_over(self, bid):
+        """Micro-batch `bid`'s thread runs, until it hands back; -> what it hands over."""
+        self._baton.switch(bid, self.option.batch_cnt + bid, patience=50000)
+        return self._return_queues[bid].get()
+
+    def _hand_back(self, bid, what, queue):
+        """Micro-batch `bid`'s thread hands `what` over and waits for its next turn; -> what `queue` then holds."""
+        self._return_queues[bid].put(what)
+        self._baton.switch(self.option.batch_cnt + bid, bid)
+        return queue.get()
+
     def _abort_parked(self):
         """A failed step leaves the micro-batch threads that already handed their inputs over
         parked inside the compiled model; wake them with an abort so that each one unwinds out of
         exec_fn and is ready for the next step()."""
         for bid in sorted(self._parked):
             PartialModule._module_queues[bid].put(_ABORT)
-            self._return_queues[bid].get()
+            self._hand_over(bid)
         self._parked = set()
 
     def _run_step(self, args, kwargs):
@@ -153,7 +169,9 @@ class PartialRunner:
         # inputs to the worker and parks there
         for bid in range(option.batch_cnt):
             self._train_queues[bid].put((args[bid], kwargs[bid]))
-            tok = self._return_queues[bid].get()
+            if bid + 1 < option.batch_cnt:
+                self._baton.alert(bid + 1)
+            tok = self._hand_over(bid)
             if isinstance(tok, _ExecError):
                 raise tok.exc
             if tok is STEP_TOKEN:
@@ -171,10 +189,10 @@ class PartialRunner:
         plan = worker.begin_planned_step()
         if plan is not None:
             for turn, mb in plan.turns:
+                self._baton.alert(mb)
                 plan.advance(turn)
                 self.finalize_output(mb)
-            plan.end()
-            worker.optimizer_step()
+            worker.optimizer_step(plan.end())
             worker.steps_done += 1
             return self._take_results()
 
@@ -198,7 +216,7 @@ class PartialRunner:
         """Wake micro-batch `batch_idx`: its outputs exist; wait until its exec_fn has
         returned (loss computed, backward hooks fired)."""
         PartialModule._module_queues[batch_idx].put(None)
-        ret = self._return_queues[batch_idx].get()
+        ret = self._hand_over(batch_idx)
         self._parked.discard(batch_idx)
         if isinstance(ret, _ExecError):
             raise ret.exc
@@ -239,19 +257,20 @@ class PartialRunner:
 
     # -- helpers --------------------------------------------------------------------
     def _exec_loop(self, batch_idx):
-        q = self._train_queues[batch_idx]
+        q, stream = self._train_queues[batch_idx], self.worker.stream_obj
+        self._baton.switch(None, batch_idx)
+        args, kwargs = q.get()
         while True:
-            args, kwargs = q.get()
             try:
-                if self.worker.stream_obj is not None:
+                if stream is not None:
                     torch.cuda.set_device(self.net_state.device)
-                    with torch.cuda.stream(self.worker.stream_obj):   # user code shares the step's stream
-                        ret = self.exec_fn(*args, **kwargs)
-                else:
-                    ret = self.exec_fn(*args, **kwargs)
+                    if torch.cuda.current_stream() != stream:    # user code shares the step's stream
+                        torch.cuda.set_stream(stream)
+                ret = self.exec_fn(*args, **kwargs)
             except BaseException as e:  # surfaced on the thread that called step()
                 ret = _ExecError(e)
-            self._return_queues[batch_idx].put(ret)
+            args = kwargs = None     # (not kept alive until the next step)
+            args, kwargs = self._hand_back(batch_idx, ret, q)
 
     def _probe_forward(self, args, kwargs):
         self._probing = True
@@ -289,6 +308,7 @@ class PartialModule(nn.Module):
                   % (len(self._all_modules) + 1, len(gm.graph.nodes), self.should_pp))
             gm.graph.print_tabular()
         self.partition_graph = None
+        self._dynamic = None        # (the graph's static placeholders, the indices of the others)
         self._canonical, self._folded = False, []
         # TorchDynamo recompiles when a micro-batch arrives with a new shape (ragged last chunk);
         # a structurally identical graph is the same pipeline, run by the module that owns the programs
@@ -356,9 +376,11 @@ class PartialModule(nn.Module):
         del ex
 
     def _dynamic_inputs(self, args):
-        pg = self.partition_graph
-        return {i: (to_device(a, self.device) if not torch.is_tensor(a) else a)
-                for i, a in enumerate(args) if not pg.static_placeholder[i]}
+        static = self.partition_graph.static_placeholder
+        if self._dynamic is None or self._dynamic[0] is not static:
+            self._dynamic = static, [i for i in range(len(static)) if not static[i]]
+        return {i: (args[i] if torch.is_tensor(args[i]) else to_device(args[i], self.device))
+                for i in self._dynamic[1] if i < len(args)}
 
     def _ensure_programs(self, mb, args):
         worker = self._runner.worker
@@ -416,8 +438,8 @@ class PartialModule(nn.Module):
         for i, v in dyn.items():
             if torch.is_tensor(v):
                 worker.distribute_input(mb, i, v)
-        runner._return_queues[mb].put(STEP_TOKEN)   # inputs are in place; main thread may schedule
-        if self._module_queues[mb].get() is _ABORT:  # parked until this micro-batch's outputs exist
+        # inputs are in place, the main thread may schedule; parked until this micro-batch's outputs exist
+        if runner._hand_back(mb, STEP_TOKEN, self._module_queues[mb]) is _ABORT:
             raise _StepAborted()
         return self._outputs_for_user(mb, probe=False)
 

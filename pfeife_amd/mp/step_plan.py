@@ -179,8 +179,11 @@ class StepPlan:
         self.issuer.wait(ticket)
 
     def end(self):
-        """The rest, and the main stream after every lane."""
+        """Hands over the rest, and the main stream after every lane; -> what returns once all of it has been issued."""
         self.issuer.push(self._end)
+        return self._settle
+
+    def _settle(self):
         self.issuer.wait()
         self.started = False
 

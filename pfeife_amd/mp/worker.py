@@ -777,7 +777,7 @@ class StageWorker:
         """Current loss scale (synchronises; for logging and tests)."""
         return float(self.scaler_state[0].item()) if self.dyn_scale else float(self.option.loss_scale)
 
-    def _dynamic_optimizer_step(self, opt):
+    def _dynamic_optimizer_step(self, opt, adam):
         """GradScaler.unscale_ + step + update on the device (pfeife/mp/worker.py:1432-1436): the
         gradients are unscaled in place and checked; an Adam/AdamW step reads the overflow flag
         itself, any other optimizer is skipped after one host read of the flag."""
@@ -789,18 +789,24 @@ class StageWorker:
             self._unscale_key = key
         for launch in self._unscale:
             launch(s)
-        if opt is not None:
-            if self._fused_adam_applicable(opt):
-                self._fused_adam_step(opt, scaled=True)
-            elif float(self.scaler_state[2].item()) == 0.0:
-                opt.step()
+        if adam is not None:
+            adam()
+        elif opt is not None and float(self.scaler_state[2].item()) == 0.0:
+            opt.step()
         o = self.option
         self.kernels.scaler_update(self.scaler_state, o.growth_factor, o.backoff_factor, o.growth_interval)(s)
 
-    def optimizer_step(self):
+    def optimizer_step(self, settle=None):
+        """settle: returns when all jobs of the step have been issued; what the fused Adam step looks over on the host it looks
+        over before."""
         opt = self.optimizer
+        adam = None
+        if opt is not None and self._fused_adam_applicable(opt):
+            adam = self._fused_adam_prepare(opt, self.dyn_scale)
+        if settle is not None:
+            settle()
         if self.dyn_scale:
-            return self._dynamic_optimizer_step(opt)
+            return self._dynamic_optimizer_step(opt, adam)
         if self.option.loss_scale != 1.0:   # gradients leave the step unscaled, with or without an optimizer
             key = (len(self.params.params), len(self.params.zero))
             if getattr(self, "_unscale_key", None) != key:
@@ -808,11 +814,9 @@ class StageWorker:
                 self._unscale_key = key
             for launch in self._unscale:
                 launch(self.stream())
-        if opt is None:
-            return
-        if self._fused_adam_applicable(opt):
-            self._fused_adam_step(opt)
-        else:
+        if adam is not None:
+            adam()
+        elif opt is not None:
             opt.step()
 
     def _fused_adam_applicable(self, opt):
@@ -834,48 +838,61 @@ class StageWorker:
         return True
 
     def _fused_adam_step(self, opt, scaled=False):
+        self._fused_adam_prepare(opt, scaled)()
+
+    def _fused_adam_prepare(self, opt, scaled):
+        """The tables of the param groups, as their tensors are now; -> the call that makes the step."""
         cache = self.__dict__.setdefault("_adam_tables", {})
-        s = self.stream()
         rebuilt = False
         groups = []
         for gi, g in enumerate(opt.param_groups):
-            params = [p for p in g["params"] if p.grad is not None]
-            if not params:
-                continue
-            for p in params:   # state exactly as torch.optim.Adam initialises it
+            params, sig, state = [], [], []
+            for p in g["params"]:
+                if p.grad is None:
+                    continue
                 st = opt.state[p]
-                if len(st) == 0:
+                if len(st) == 0:       # state exactly as torch.optim.Adam initialises it
                     st["step"] = torch.tensor(0.0, dtype=torch.float32)
                     st["exp_avg"] = torch.zeros_like(p, memory_format=torch.preserve_format)
                     st["exp_avg_sq"] = torch.zeros_like(p, memory_format=torch.preserve_format)
-            sig = tuple((p.numel(), p.data_ptr(), p.grad.data_ptr(), opt.state[p]["exp_avg"].data_ptr(),
-                         opt.state[p]["exp_avg_sq"].data_ptr()) for p in params)   # (all that the table holds)
+                params.append(p)
+                state.append(st)
+                sig.append((p.numel(), p.data_ptr(), p.grad.data_ptr(), st["exp_avg"].data_ptr(), st["exp_avg_sq"].data_ptr()))
+            if not params:
+                continue
             ent = cache.get(gi)
-            if ent is None or ent[0] != sig:
+            if ent is None or ent[0] != sig:    # (all that the table holds)
                 table = self.kernels.adam_table([p.data for p in params], [p.grad for p in params],
-                                                [opt.state[p]["exp_avg"] for p in params],
-                                                [opt.state[p]["exp_avg_sq"] for p in params])
+                                                [st["exp_avg"] for st in state], [st["exp_avg_sq"] for st in state])
                 ent = cache[gi] = (sig, table)
                 rebuilt = True
-            groups.append((g, params, ent[1]))
-        if scaled and rebuilt:
-            self._seed_device_step_count(opt, groups)
-        for g, params, (table, n_items, n_chunks) in groups:
-            b1, b2 = g["betas"]
-            if scaled:
-                # skipped on overflow; the bias corrections use the device's count of completed steps.
-                # The host-side `step` entries are brought up to date from that count when somebody
-                # reads them (sync_optimizer_steps: optimizer.state_dict() calls it)
-                self.kernels.adam_step_scaled(table, n_items, n_chunks, float(g["lr"]), float(b1), float(b2),
-                                              float(g["eps"]), float(g["weight_decay"]),
-                                              type(opt) is torch.optim.AdamW, self.scaler_state, s)
-                self._host_steps_stale = True
-            else:
-                step = int(opt.state[params[0]]["step"].item()) + 1
-                self.kernels.adam_step(table, n_items, n_chunks, float(g["lr"]), float(b1), float(b2), float(g["eps"]),
-                                       float(g["weight_decay"]), step, type(opt) is torch.optim.AdamW, s)
-                for p in params:
-                    opt.state[p]["step"] += 1
+            groups.append((g, params, state, ent[1]))
+
+        def step():
+            s = self.stream()
+            if scaled and rebuilt:
+                self._seed_device_step_count(opt, groups)
+            for g, params, state, (table, n_items, n_chunks) in groups:
+                b1, b2 = g["betas"]
+                if scaled:
+                    # skipped on overflow; the bias corrections use the device's count of completed steps.
+                    # The host-side `step` entries are brought up to date from that count when somebody
+                    # reads them (sync_optimizer_steps: optimizer.state_dict() calls it)
+                    self.kernels.adam_step_scaled(table, n_items, n_chunks, float(g["lr"]), float(b1), float(b2),
+                                                  float(g["eps"]), float(g["weight_decay"]),
+                                                  type(opt) is torch.optim.AdamW, self.scaler_state, s)
+                    self._host_steps_stale = True
+                else:
+                    t = int(state[0]["step"].item()) + 1
+                    self.kernels.adam_step(table, n_items, n_chunks, float(g["lr"]), float(b1), float(b2), float(g["eps"]),
+                                           float(g["weight_decay"]), t, type(opt) is torch.optim.AdamW, s)
+                    if all(torch.is_tensor(st["step"]) for st in state):
+                        torch._foreach_add_([st["step"] for st in state], 1)
+                    else:
+                        for st in state:
+                            st["step"] += 1
+
+        return step
 
     def _seed_device_step_count(self, opt, groups):
         """The fused step under dynamic loss scaling takes Adam's bias corrections from the device's
@@ -885,7 +902,7 @@ class StageWorker:
         One counter serves every parameter: an optimizer whose parameters disagree is refused."""
         if getattr(self, "_host_steps_stale", False) and getattr(self, "_steps_owner", None) is opt:
             self.sync_optimizer_steps()
-        steps = {int(float(opt.state[p]["step"])) for _, params, _ in groups for p in params}
+        steps = {int(float(st["step"])) for _, _, state, _ in groups for st in state}
         if len(steps) > 1:
             raise RuntimeError("fused Adam step with dynamic loss scaling: the optimizer's parameters are at "
                                "different step counts %s; one device-side counter serves them all" % sorted(steps))
