@@ -1435,6 +1435,14 @@ def lower_sdpa(L, node):
     kern = L.kernels
     if L.mixed and hv == hd and hd % 8 == 0 and hd <= getattr(kern, "MAX_FUSED_HEAD_DIM", 0):
         return _lower_sdpa_fused(L, (q, k, v), (qt, kt, vt), (Bn, H, Tq, Tk, hd), scale, causal, req)
+    # fp32: a workgroup of the fused kernels sweeps the other side's tokens for 16 of one side, in a quarter of them one after the
+    # other.  Few of them over long sequences leave the device idle where products through memory fill it (us forward + backward, memory /
+    # fused: 1 head, 64 queries of 4096 keys, 4 workgroups: 130 / 137; 4096 of 64 at head dim 128: 58 / 281; 2 heads of 1500, 188
+    # workgroups: 125 / 110)
+    few = max(Tq, Tk) > 1024 and Bn * H * ((min(Tq, Tk) + 15) // 16) < 128
+    if (not L.mixed and hv == hd and hd % 4 == 0 and hd <= getattr(kern, "FUSED_F32_HEAD_DIM", 0) and scale > 0 and not few
+            and all(_f32_heads(t) for t in (qt, kt, vt))):
+        return _lower_sdpa_fused(L, (q, k, v), (qt, kt, vt), (Bn, H, Tq, Tk, hd), scale, causal, req)
     S = L.scratch("attn_s", L.cur.mb, (Bn, H, Tq, Tkp), torch.float32)
     P = L.alloc((Bn, H, Tq, Tkp), cd)
     O = L.alloc((Bn, Tq, H, hv), cd)           # token-major, so that transpose(1,2).reshape is a view
@@ -1492,17 +1500,38 @@ def lower_sdpa(L, node):
     return outv
 
 
+def _f32_heads(t):
+    """Whether the fp32 attention kernels can read and write this [B, H, T, hd] tensor (16-byte accesses, tokens apart)."""
+    return (t.dtype == torch.float32 and t.numel() > 0 and t.stride(3) == 1 and t.stride(2) >= t.shape[3] and t.data_ptr() % 16 == 0
+            and all(s % 4 == 0 for s in t.stride()[:3]))
+
+
+def _apart(vals):
+    """Whether the gradients of these values are different memory (targets may then be taken for all of them before any is written)."""
+    def chain(val):
+        nodes = []
+        while val.kind != "base":
+            if val.kind == "part":
+                nodes.append(id(val))
+            val = val.base
+        return nodes + [id(val)]
+
+    chains = [chain(val) for val in vals]
+    return not any(i != j and a[0] in b for i, a in enumerate(chains) for j, b in enumerate(chains))
+
+
 def _lower_sdpa_fused(L, vals, tensors, dims, scale, causal, req):
-    """softmax(QK^T)V as one kernel (no score matrix in memory) and a three-kernel backward."""
+    """softmax(QK^T)V as one kernel (no score matrix in memory) and its backward in two or three."""
     q, k, v = vals
     qt, kt, vt = tensors
     Bn, H, Tq, Tk, hd = dims
     cd = L.cd
     O = L.alloc((Bn, Tq, H, hd), cd)            # token-major, so that transpose(1,2).reshape is a view
     Ov = O.permute(0, 2, 1, 3)
-    lse = L.alloc((Bn, H, Tq), torch.float32)
+    # (fp32 keeps a row's maximum and its sum apart)
+    lse = L.alloc((Bn, H, Tq if L.mixed else 2 * Tq), torch.float32)
     # (wide heads keep O to twice its digits for the backward pass, see attn_delta_kernel)
-    o_lo = L.alloc((Bn, Tq, H, hd), cd).permute(0, 2, 1, 3) if req and hd > L.kernels.O_LO_HEAD_DIM else None
+    o_lo = L.alloc((Bn, Tq, H, hd), cd).permute(0, 2, 1, 3) if L.mixed and req and hd > L.kernels.O_LO_HEAD_DIM else None
     L.emit(L.kernels.attention_fwd(qt, kt, vt, Ov, lse, scale, causal, o_lo))
     outv = Val(Ov, req_grad=req)
 
@@ -1510,18 +1539,19 @@ def _lower_sdpa_fused(L, vals, tensors, dims, scale, causal, req):
         g = B.grad_of(outv)
         if g is None:
             return
-        if g.dtype != cd or g.stride(3) != 1 or any(s % 8 for s in g.stride()[:3]):
+        if not _f32_heads(g) if not L.mixed else g.dtype != cd or g.stride(3) != 1 or any(s % 8 for s in g.stride()[:3]):
             t = B.new_like(Ov)
             B.copy(g, t)
             g = t
         delta = L.scratch("attn_delta", B.program.mb, (Bn, H, Tq), torch.float32)
         plan = []
         outs = []
-        for val, like in ((q, qt), (k, kt), (v, vt)):
-            if val.req_grad:
+        apart = _apart([val for val in vals if val.req_grad])
+        for val in vals:
+            if val.req_grad and apart:
                 dst, prev = B.grad_target(val)
                 direct = (prev is None and dst.dtype == cd and dst.stride(3) == 1
-                          and all(s % 4 == 0 for s in dst.stride()[:3]))
+                          and all(s % 4 == 0 for s in dst.stride()[:3]) and (L.mixed or _f32_heads(dst)))
                 buf = dst if direct else B.temp(val.shape, cd)
                 plan.append((val, dst, prev, buf, direct))
             else:
@@ -1532,6 +1562,12 @@ def _lower_sdpa_fused(L, vals, tensors, dims, scale, causal, req):
             if not direct:
                 B.merge(buf, dst, prev)
             B.commit(val, dst)
+        if not apart:
+            for val, buf in zip(vals, outs):      # (each sees what the one before it left)
+                if val.req_grad:
+                    dst, prev = B.grad_target(val)
+                    B.merge(buf, dst, prev)
+                    B.commit(val, dst)
 
     if req:
         L.add_backward(bwd)

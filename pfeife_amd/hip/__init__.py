@@ -112,6 +112,8 @@ _SIGNATURES = {
     "pf_gemm_variant": [POINTER(GemmDesc), ctypes.c_char_p, _I],
     "pf_attention_fwd": [POINTER(AttnDesc), _P],
     "pf_attention_bwd": [POINTER(AttnDesc), _P],
+    "pf_attention_f32_fwd": [POINTER(AttnDesc), _P],
+    "pf_attention_f32_bwd": [POINTER(AttnDesc), _P],
     "pf_norm_bwd_fused": [POINTER(NormBwdDesc), _P],
     "pf_layernorm_fwd": [_P, _I, _P, _P, _P, _I, _P, _P, _L, _L, _F, _P],
     "pf_layernorm_bwd": [_P, _I, _P, _I, _P, _P, _P, _P, _I, _P, _I, _P, _P, _P, _L, _L, _I, _P],
@@ -500,6 +502,7 @@ class HipKernels:
 
     # -- fused attention -----------------------------------------------------------
     MAX_FUSED_HEAD_DIM = 128
+    FUSED_F32_HEAD_DIM = 128
     O_LO_HEAD_DIM = 96     # above it the forward pass may keep what rounding O lost, for the backward pass
 
     @staticmethod
@@ -526,11 +529,11 @@ class HipKernels:
 
     def attention_fwd(self, q, k, v, o, lse, scale, causal, o_lo=None):
         d = self._attn_desc(q, k, v, o, lse, scale, causal, o_lo=o_lo)
-        return self._prep("pf_attention_fwd", (byref(d),), (d, q, k, v, o, lse, o_lo))
+        return self._prep("pf_attention_f32_fwd" if q.dtype == torch.float32 else "pf_attention_fwd", (byref(d),), (d, q, k, v, o, lse, o_lo))
 
     def attention_bwd(self, q, k, v, o, d_o, lse, delta, dq, dk, dv, scale, causal, o_lo=None):
         d = self._attn_desc(q, k, v, o, lse, scale, causal, d_o, dq, dk, dv, delta, o_lo)
-        return self._prep("pf_attention_bwd", (byref(d),), (d, q, k, v, o, d_o, lse, delta, dq, dk, dv, o_lo))
+        return self._prep("pf_attention_f32_bwd" if q.dtype == torch.float32 else "pf_attention_bwd", (byref(d),), (d, q, k, v, o, d_o, lse, delta, dq, dk, dv, o_lo))
 
     # -- normalisation -----------------------------------------------------------
     def layernorm_fwd(self, x, gamma, beta, y, mean, rstd, rows, d, eps):

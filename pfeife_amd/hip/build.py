@@ -24,6 +24,7 @@ SOURCES = [
     "pf_gemm_f32.hip",
     "pf_gemm_f32_depth.hip",
     "pf_attention.hip",
+    "pf_attention_f32.hip",
     "pf_norm.hip",
     "pf_elementwise.hip",
     "pf_softmax_loss.hip",
