@@ -13,21 +13,33 @@ namespace {
 
 constexpr int COLRED_MAX_BLOCKS = 1024;
 
+// over L neighbouring lanes
+template <int L>
+__device__ __forceinline__ float lanes_sum(float v) {
+  if constexpr (L == 64) return pf_wave_sum(v);
+#pragma unroll
+  for (int off = 1; off < L; off <<= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
 // ---- forward ---------------------------------------------------------------
 // NV > 0: the row (d <= 64*W*NV) is loaded ONCE into registers, all loads in flight together;
 // mean, then the sum of squared deviations, then the output come from the registers: one memory
 // round trip per row instead of three dependent ones (the kernel is latency-bound, a row is
 // 2-8 KB).  NV == 0: any d, three sweeps over the row (the second and third hit L2).
 // XDT / YDT: dtypes of x and y when known at compile time (-1: read x_dt / y_dt at run time).
-template <int W, int NV, int XDT = -1, int YDT = -1>
+// L: lanes to a row (NV = 1, d <= L * W): rows of up to half a wavefront's columns share it.  us, one row to a wavefront / L = 8 and 32, fp32 to
+// bf16: 50000 x 64 14.5 / 4.4, 50000 x 256 16.6 / 12.7.
+template <int W, int NV, int XDT = -1, int YDT = -1, int L = 64>
 __global__ __launch_bounds__(256) void norm_fwd_kernel(const void* x, int x_dt, const float* gamma, const float* beta,
                                                        void* y, int y_dt, float* mean, float* rstd, int64_t rows,
                                                        int64_t d, float eps, int rms) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t row = (int64_t)blockIdx.x * 4 + wave;
-  if (row >= rows) return;
+  const int lane = threadIdx.x % L;
+  const int64_t row = (int64_t)blockIdx.x * (256 / L) + threadIdx.x / L;
+  if (row >= rows) return;      // (a row's lanes leave together)
   const int64_t base = row * d;
   if constexpr (NV > 0) {
+    static_assert(L == 64 || NV == 1, "one column group to a lane where rows share a wavefront");
     // nothing around the loads branches: out-of-range lanes read column 0 and are masked out of
     // the sums and the stores; a missing beta reads gamma instead and is not added
     float v[NV][W], g[NV][W], b[NV][W];
@@ -51,7 +63,7 @@ __global__ __launch_bounds__(256) void norm_fwd_kernel(const void* x, int x_dt, 
       for (int i = 0; i < NV; ++i)
 #pragma unroll
         for (int k = 0; k < W; ++k) s += ok[i] ? v[i][k] : 0.f;
-      mu = pf_wave_sum(s) / (float)d;
+      mu = lanes_sum<L>(s) / (float)d;
     }
     float q = 0.f;
 #pragma unroll
@@ -62,7 +74,7 @@ __global__ __launch_bounds__(256) void norm_fwd_kernel(const void* x, int x_dt, 
         q += ok[i] ? t * t : 0.f;
       }
     }
-    const float var = pf_wave_sum(q) / (float)d;
+    const float var = lanes_sum<L>(q) / (float)d;
     const float rs = 1.0f / sqrtf(var + eps);
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -127,9 +139,7 @@ __global__ __launch_bounds__(256) void norm_fwd_kernel(const void* x, int x_dt, 
 // ---- backward ----------------------------------------------------------------
 // NV = column groups a lane owns (d <= 64 * W * NV).  Column partials for
 // dgamma/dbeta stay in registers across the rows a wavefront processes.
-// IODT: dtype of x, dx_add and dx when they all share one known at compile time (-1: run time);
-// LPDT: dtype of dx_lp likewise; DYDT: dtype of dy likewise.
-template <int W, int NV, int IODT = -1, int LPDT = -1, int DYDT = -1>
+template <int W, int NV>
 __global__ __launch_bounds__(256) void norm_bwd_kernel(const void* dy, int dy_dt, const void* x, int x_dt,
                                                        const float* gamma, const float* mean, const float* rstd,
                                                        const void* dx_add, int add_dt, void* dx, int dx_dt,
@@ -153,87 +163,6 @@ __global__ __launch_bounds__(256) void norm_bwd_kernel(const void* dy, int dy_dt
     for (int k = 0; k < W; ++k) ps[i][k] = 0.f;
 
   constexpr bool CACHE = (NV * W <= 32);   // keep the row's dy and x in registers between the two passes
-  // Straight-line variants with at most two column groups per lane: the operands of the wavefront's
-  // NEXT row are requested before the current row is reduced and stored, so a wavefront that
-  // owns two rows pays one memory round trip, not two.  Nothing around the loads branches (row and
-  // column indices are clamped, out-of-range lanes contribute zeros and store nothing).
-  constexpr bool PIPE = CACHE && NV <= 4 && IODT >= 0 && DYDT >= 0 && W == 8;
-  if constexpr (PIPE) {
-    const int64_t stride = (int64_t)gridDim.x * 4;
-    int64_t row = (int64_t)blockIdx.x * 4 + wave;
-    const bool has_add = dx_add != nullptr;
-    bool ok[NV];
-    int64_t col[NV];
-    float g[NV][W];
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int64_t c = ((int64_t)lane + i * 64) * W;
-      ok[i] = c < d;
-      col[i] = ok[i] ? c : 0;
-      ld_vec_c<W, PF_F32>(gamma, col[i], PF_F32, g[i]);
-    }
-    float ndy[NV][W], nx[NV][W], nadd[NV][W], nmu, nrs;
-    auto fetch = [&](int64_t r) {
-      const int64_t rr = r < rows ? r : rows - 1;
-#pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        ld_vec_c<W, DYDT>(dy, rr * d + col[i], dy_dt, ndy[i]);
-        ld_vec_c<W, IODT>(x, rr * d + col[i], x_dt, nx[i]);
-        if (has_add) ld_vec_c<W, IODT>(dx_add, rr * d + col[i], add_dt, nadd[i]);
-      }
-      nmu = rms ? 0.f : mean[rr];
-      nrs = rstd[rr];
-    };
-    if (row < rows) fetch(row);
-    while (row < rows) {
-      float cdy[NV][W], cx[NV][W], cadd[NV][W];
-      const float mu = nmu, rs = nrs;
-#pragma unroll
-      for (int i = 0; i < NV; ++i)
-#pragma unroll
-        for (int k = 0; k < W; ++k) {
-          cdy[i][k] = ok[i] ? ndy[i][k] : 0.f;
-          cx[i][k] = nx[i][k];
-          cadd[i][k] = has_add ? nadd[i][k] : 0.f;
-        }
-      fetch(row + stride);
-      float c1 = 0.f, c2 = 0.f;
-      float xh[NV][W], gg[NV][W];
-#pragma unroll
-      for (int i = 0; i < NV; ++i)
-#pragma unroll
-        for (int k = 0; k < W; ++k) {
-          gg[i][k] = cdy[i][k] * g[i][k];
-          xh[i][k] = ok[i] ? (cx[i][k] - mu) * rs : 0.f;
-          c1 += gg[i][k];
-          c2 += gg[i][k] * xh[i][k];
-        }
-      c1 = rms ? 0.f : pf_wave_sum(c1) / (float)d;
-      c2 = pf_wave_sum(c2) / (float)d;
-      const int64_t base = row * d;
-#pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        float o[W];
-#pragma unroll
-        for (int k = 0; k < W; ++k) {
-          o[k] = rs * (gg[i][k] - c1 - xh[i][k] * c2) + cadd[i][k];
-          pg[i][k] += cdy[i][k] * xh[i][k];
-          pb[i][k] += cdy[i][k];
-        }
-        if (ok[i]) {
-          st_vec_c<W, IODT>(dx, base + col[i], dx_dt, o);
-          if (dx_lp) {
-            st_vec_c<W, LPDT>(dx_lp, base + col[i], lp_dt, o);
-            if (want_colsum) {
-#pragma unroll
-              for (int k = 0; k < W; ++k) ps[i][k] += pf_round_to(LPDT >= 0 ? LPDT : lp_dt, o[k]);
-            }
-          }
-        }
-      }
-      row += stride;
-    }
-  } else
   for (int64_t row = (int64_t)blockIdx.x * 4 + wave; row < rows; row += (int64_t)gridDim.x * 4) {
     const int64_t base = row * d;
     const float mu = rms ? 0.f : mean[row];
@@ -245,13 +174,13 @@ __global__ __launch_bounds__(256) void norm_bwd_kernel(const void* dy, int dy_dt
       const int64_t c = ((int64_t)lane + i * 64) * W;
       if (c < d) {
         float vdy[W], vx[W], g[W];
-        ld_vec_c<W, DYDT>(dy, base + c, dy_dt, vdy);
-        ld_vec_c<W, IODT>(x, base + c, x_dt, vx);
-        ld_vec_c<W, PF_F32>(gamma, c, PF_F32, g);
+        ld_vec<W>(dy, base + c, dy_dt, vdy);
+        ld_vec<W>(x, base + c, x_dt, vx);
+        ld_vec<W>(gamma, c, PF_F32, g);
         // the gradient already accumulated on x: requested with the other operands, so that the
         // row costs one memory round trip, not a second one after the reductions
         if constexpr (CACHE) {
-          if (dx_add) ld_vec_c<W, IODT>(dx_add, base + c, add_dt, cadd[i]);
+          if (dx_add) ld_vec<W>(dx_add, base + c, add_dt, cadd[i]);
         }
 #pragma unroll
         for (int k = 0; k < W; ++k) {
@@ -283,9 +212,9 @@ __global__ __launch_bounds__(256) void norm_bwd_kernel(const void* dy, int dy_dt
           }
         } else {
           float vx[W], g[W];
-          ld_vec_c<W, DYDT>(dy, base + c, dy_dt, vdy);
-          ld_vec_c<W, IODT>(x, base + c, x_dt, vx);
-          ld_vec_c<W, PF_F32>(gamma, c, PF_F32, g);
+          ld_vec<W>(dy, base + c, dy_dt, vdy);
+          ld_vec<W>(x, base + c, x_dt, vx);
+          ld_vec<W>(gamma, c, PF_F32, g);
 #pragma unroll
           for (int k = 0; k < W; ++k) {
             ggv[k] = vdy[k] * g[k];
@@ -304,18 +233,18 @@ __global__ __launch_bounds__(256) void norm_bwd_kernel(const void* dy, int dy_dt
             for (int k = 0; k < W; ++k) o[k] += cadd[i][k];
           } else {
             float a[W];
-            ld_vec_c<W, IODT>(dx_add, base + c, add_dt, a);
+            ld_vec<W>(dx_add, base + c, add_dt, a);
 #pragma unroll
             for (int k = 0; k < W; ++k) o[k] += a[k];
           }
         }
-        st_vec_c<W, IODT>(dx, base + c, dx_dt, o);
+        st_vec<W>(dx, base + c, dx_dt, o);
         if (dx_lp) {
-          st_vec_c<W, LPDT>(dx_lp, base + c, lp_dt, o);
+          st_vec<W>(dx_lp, base + c, lp_dt, o);
           if constexpr (NS == NV) {
             if (want_colsum) {
 #pragma unroll
-              for (int k = 0; k < W; ++k) ps[i][k] += pf_round_to(LPDT >= 0 ? LPDT : lp_dt, o[k]);
+              for (int k = 0; k < W; ++k) ps[i][k] += pf_round_to(lp_dt, o[k]);
             }
           }
         }
@@ -626,6 +555,94 @@ __global__ __launch_bounds__(256) void groupnorm_bwd_apply_kernel(const void* dy
   }
 }
 
+// Rows of up to 512 columns, dtypes known: L lanes to a row, eight columns to a lane, 64 / L rows to a wavefront and G of them to a workgroup at
+// a time.  Eight wavefronts to a workgroup, two workgroups to a CU: with 48 to 80 bytes a lane in flight for the row at hand and as many for
+// the next one that hides the memory's latency; fewer than 512 workgroups would not, more would leave more partial rows behind.  Sums of a row
+// stay inside its lanes, so nothing waits for another wavefront before the column sums at the end, which all threads add up.
+// us, a row to a wavefront with two column groups to a lane and four wavefronts to a workgroup / this, with the 16-bit copy and its column
+// sums: 12214 x 384 16.5 / 14.0 (5.6 TB/s), 3152 x 384 8.1 / 6.2, 12214 x 192 14.0 / 7.6, 50000 x 64 40.8 / 10.5, 20 x 64 4.6 / 3.7.
+template <int L, int IODT, int LPDT, int DYDT>
+__global__ __launch_bounds__(512, 4) void norm_bwd_narrow_kernel(
+    const void* dy, const void* x, const float* gamma, const float* mean, const float* rstd, const void* dx_add, void* dx,
+    float* ws, int64_t rows, int64_t d, int rms, int want_wgrad, void* dx_lp, int want_colsum) {
+  constexpr int W = 8, G = 512 / L;
+  __shared__ __align__(16) float red[3][G][L * W];
+  const int group = threadIdx.x / L;
+  const int64_t c = (int64_t)(threadIdx.x % L) * W;
+  const bool ok = c < d, has_add = dx_add != nullptr;
+  const int64_t col = ok ? c : 0;
+  float g[W], pg[W], pb[W], ps[W];
+  ld_vec_c<W, PF_F32>(gamma, col, PF_F32, g);
+#pragma unroll
+  for (int k = 0; k < W; ++k) pg[k] = pb[k] = ps[k] = 0.f;
+  const int64_t stride = (int64_t)gridDim.x * G;
+  float ndy[W], nx[W], nadd[W], nmu, nrs;
+  auto fetch = [&](int64_t r) {
+    const int64_t rr = r < rows ? r : rows - 1;
+    ld_vec_c<W, DYDT>(dy, rr * d + col, DYDT, ndy);
+    ld_vec_c<W, IODT>(x, rr * d + col, IODT, nx);
+    if (has_add) ld_vec_c<W, IODT>(dx_add, rr * d + col, IODT, nadd);
+    nmu = rms ? 0.f : mean[rr];
+    nrs = rstd[rr];
+  };
+  int64_t row = (int64_t)blockIdx.x * G + group;
+  fetch(row);
+  // (the wavefront's rows end together: its last ones may be past the end, which sum zeros and store nothing)
+  for (int64_t first = row - group % (64 / L); first < rows; first += stride, row += stride) {
+    const bool mine = row < rows && ok;
+    const float mu = nmu, rs = nrs;
+    float gg[W], xh[W], cdy[W], cadd[W];
+    float c1 = 0.f, c2 = 0.f;
+#pragma unroll
+    for (int k = 0; k < W; ++k) {
+      cdy[k] = mine ? ndy[k] : 0.f;
+      cadd[k] = has_add ? nadd[k] : 0.f;
+      gg[k] = cdy[k] * g[k];
+      xh[k] = mine ? (nx[k] - mu) * rs : 0.f;
+      c1 += gg[k];
+      c2 += gg[k] * xh[k];
+    }
+    fetch(row + stride);
+    c1 = rms ? 0.f : lanes_sum<L>(c1) / (float)d;
+    c2 = lanes_sum<L>(c2) / (float)d;
+    if (mine) {
+      float o[W];
+#pragma unroll
+      for (int k = 0; k < W; ++k) {
+        o[k] = rs * (gg[k] - c1 - xh[k] * c2) + cadd[k];
+        pg[k] += cdy[k] * xh[k];
+        pb[k] += cdy[k];
+      }
+      st_vec_c<W, IODT>(dx, row * d + c, IODT, o);
+      if (dx_lp) {
+        st_vec_c<W, LPDT>(dx_lp, row * d + c, LPDT, o);
+        if (want_colsum) {
+#pragma unroll
+          for (int k = 0; k < W; ++k) ps[k] += pf_round_to(LPDT, o[k]);
+        }
+      }
+    }
+  }
+  if (!want_wgrad && !want_colsum) return;
+  // one partial row of each kind per workgroup: ws [gridDim.x][2 or 3][d]
+  st_vec_c<W, PF_F32>(red[0][group], c, PF_F32, pg);
+  st_vec_c<W, PF_F32>(red[1][group], c, PF_F32, pb);
+  st_vec_c<W, PF_F32>(red[2][group], c, PF_F32, ps);
+  __syncthreads();
+  const int kinds = want_colsum ? 3 : 2;
+  float* wrow = ws + (int64_t)blockIdx.x * kinds * d;
+  for (int at = threadIdx.x; at < kinds * L * W; at += 512) {
+    const int which = at / (L * W), cc = at % (L * W);
+    if (cc >= d || (which < 2 && !want_wgrad)) continue;
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+    for (int q = 0; q < G; q += 4)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[e] += red[which][q + e][cc];
+    wrow[which * d + cc] = (s[0] + s[1]) + (s[2] + s[3]);
+  }
+}
+
 // Rows of 513 to 2048 columns, dtypes known: NWV wavefronts (a team) share a row, eight columns to a lane, TEAMS rows
 // to a workgroup at a time.  A wavefront that owns a whole row of 2048 holds 32 columns in each of ten operands and sums, more
 // registers than leave a second wavefront on its SIMD, and then waits out every memory round trip (measured: 143 MB
@@ -773,22 +790,25 @@ int norm_fwd(const void* x, int x_dt, const float* gamma, const float* beta, voi
   const bool v = vec_ok(x, x_dt, d) && vec_ok(y, y_dt, d) && vec_ok(gamma, PF_F32, d) && vec_ok(beta, PF_F32, d);
 #define PF_NF(W, NV) \
   hipLaunchKernelGGL((norm_fwd_kernel<W, NV>), grid, dim3(256), 0, st, x, x_dt, gamma, beta, y, y_dt, mean, rstd, rows, d, eps, rms)
-#define PF_NFC(NV, XD, YD) \
-  hipLaunchKernelGGL((norm_fwd_kernel<8, NV, XD, YD>), grid, dim3(256), 0, st, x, x_dt, gamma, beta, y, y_dt, mean, rstd, rows, d, eps, rms)
+#define PF_NFC(NV, L, XD, YD) \
+  hipLaunchKernelGGL((norm_fwd_kernel<8, NV, XD, YD, L>), dim3((unsigned)((rows * L + 255) / 256)), dim3(256), 0, st, x, x_dt, gamma, beta, y, y_dt, mean, rstd, rows, d, eps, rms)
   // the residual stream is fp32 and the consumers are matrix products (16-bit) or fp32, or the
   // whole stream is 16-bit (a UNet's transformer blocks under autocast): those pairs get
   // straight-line code
-#define PF_NFD(NV)                                                     \
-  if (x_dt == PF_F32 && y_dt == PF_F16) PF_NFC(NV, PF_F32, PF_F16);     \
-  else if (x_dt == PF_F32 && y_dt == PF_BF16) PF_NFC(NV, PF_F32, PF_BF16); \
-  else if (x_dt == PF_F32 && y_dt == PF_F32) PF_NFC(NV, PF_F32, PF_F32); \
-  else if (x_dt == PF_F16 && y_dt == PF_F16) PF_NFC(NV, PF_F16, PF_F16); \
-  else if (x_dt == PF_BF16 && y_dt == PF_BF16) PF_NFC(NV, PF_BF16, PF_BF16); \
+#define PF_NFD(NV, L)                                                     \
+  if (x_dt == PF_F32 && y_dt == PF_F16) PF_NFC(NV, L, PF_F32, PF_F16);     \
+  else if (x_dt == PF_F32 && y_dt == PF_BF16) PF_NFC(NV, L, PF_F32, PF_BF16); \
+  else if (x_dt == PF_F32 && y_dt == PF_F32) PF_NFC(NV, L, PF_F32, PF_F32); \
+  else if (x_dt == PF_F16 && y_dt == PF_F16) PF_NFC(NV, L, PF_F16, PF_F16); \
+  else if (x_dt == PF_BF16 && y_dt == PF_BF16) PF_NFC(NV, L, PF_BF16, PF_BF16); \
   else PF_NF(8, NV)
-  if (v && d <= 64 * 8 * 1) { PF_NFD(1); }
-  else if (v && d <= 64 * 8 * 2) { PF_NFD(2); }
-  else if (v && d <= 64 * 8 * 3) { PF_NFD(3); }
-  else if (v && d <= 64 * 8 * 4) { PF_NFD(4); }
+  if (v && d <= 8 * 8) { PF_NFD(1, 8); }
+  else if (v && d <= 16 * 8) { PF_NFD(1, 16); }
+  else if (v && d <= 32 * 8) { PF_NFD(1, 32); }
+  else if (v && d <= 64 * 8 * 1) { PF_NFD(1, 64); }
+  else if (v && d <= 64 * 8 * 2) { PF_NFD(2, 64); }
+  else if (v && d <= 64 * 8 * 3) { PF_NFD(3, 64); }
+  else if (v && d <= 64 * 8 * 4) { PF_NFD(4, 64); }
   else if (v) PF_NF(8, 0);
   else PF_NF(1, 0);
 #undef PF_NFD
@@ -827,35 +847,29 @@ int norm_bwd(const void* dy, int dy_dt, const void* x, int x_dt, const float* ga
                     !dx_lp;
   // a team stores its partial rows 16 bytes at a time
   const bool team = pf_aligned(ws, 16);
-#define PF_NBC(NV, LP, DY) PF_NBI(NV, PF_F32, LP, DY)
-#define PF_NBI(NV, IO, LP, DY)                                                                                       \
-  hipLaunchKernelGGL((norm_bwd_kernel<8, NV, IO, LP, DY>), dim3(blocks), dim3(256), 0, st, dy, dy_dt, x, x_dt, gamma, \
-                     mean, rstd, dx_add, add_dt, dx, dx_dt, ws, rows, d, rms, want, dx_lp, lp_dt, want_colsum)
+#define PF_NBN(L, IO, LP, DY)                                                                                          \
+  hipLaunchKernelGGL((norm_bwd_narrow_kernel<L, IO, LP, DY>), dim3(blocks), dim3(512), 0, st, dy, x, gamma, mean, rstd, dx_add, \
+                     dx, ws, rows, d, rms, want, dx_lp, want_colsum)
 #define PF_NBT(NWV, TEAMS, IO, LP, DY)                                                                                       \
   hipLaunchKernelGGL((norm_bwd_team_kernel<NWV, TEAMS, IO, LP, DY>), dim3(blocks), dim3(64 * NWV * TEAMS), 0, st, dy, x, gamma, mean, \
                      rstd, dx_add, dx, ws, rows, d, rms, want, dx_lp, want_colsum)
-#define PF_NBTD(NWV, TEAMS, ELSE)                                                           \
+#define PF_NBTD(ELSE, KERNEL, ...)                                                          \
   if (!team) ELSE;                                                                          \
-  else if (io32 && dy_dt == PF_F16 && (!dx_lp || lp_dt == PF_F16)) PF_NBT(NWV, TEAMS, PF_F32, PF_F16, PF_F16);    \
-  else if (io32 && dy_dt == PF_BF16 && (!dx_lp || lp_dt == PF_BF16)) PF_NBT(NWV, TEAMS, PF_F32, PF_BF16, PF_BF16); \
-  else if (io32 && dy_dt == PF_F32 && (!dx_lp || lp_dt == PF_F16)) PF_NBT(NWV, TEAMS, PF_F32, PF_F16, PF_F32);    \
-  else if (io32 && dy_dt == PF_F32 && lp_dt == PF_BF16) PF_NBT(NWV, TEAMS, PF_F32, PF_BF16, PF_F32);         \
-  else if (io16 && x_dt == PF_F16) PF_NBT(NWV, TEAMS, PF_F16, PF_F16, PF_F16);               \
-  else if (io16 && x_dt == PF_BF16) PF_NBT(NWV, TEAMS, PF_BF16, PF_BF16, PF_BF16);           \
+  else if (io32 && dy_dt == PF_F16 && (!dx_lp || lp_dt == PF_F16)) KERNEL(__VA_ARGS__, PF_F32, PF_F16, PF_F16);    \
+  else if (io32 && dy_dt == PF_BF16 && (!dx_lp || lp_dt == PF_BF16)) KERNEL(__VA_ARGS__, PF_F32, PF_BF16, PF_BF16); \
+  else if (io32 && dy_dt == PF_F32 && (!dx_lp || lp_dt == PF_F16)) KERNEL(__VA_ARGS__, PF_F32, PF_F16, PF_F32);    \
+  else if (io32 && dy_dt == PF_F32 && lp_dt == PF_BF16) KERNEL(__VA_ARGS__, PF_F32, PF_BF16, PF_F32);         \
+  else if (io16 && x_dt == PF_F16) KERNEL(__VA_ARGS__, PF_F16, PF_F16, PF_F16);               \
+  else if (io16 && x_dt == PF_BF16) KERNEL(__VA_ARGS__, PF_BF16, PF_BF16, PF_BF16);           \
   else ELSE
-#define PF_NBD(NV)                                                                          \
-  if (io32 && dy_dt == PF_F16 && (!dx_lp || lp_dt == PF_F16)) PF_NBC(NV, PF_F16, PF_F16);    \
-  else if (io32 && dy_dt == PF_BF16 && (!dx_lp || lp_dt == PF_BF16)) PF_NBC(NV, PF_BF16, PF_BF16); \
-  else if (io32 && dy_dt == PF_F32 && (!dx_lp || lp_dt == PF_F16)) PF_NBC(NV, PF_F16, PF_F32);    \
-  else if (io32 && dy_dt == PF_F32 && lp_dt == PF_BF16) PF_NBC(NV, PF_BF16, PF_F32);         \
-  else if (io16 && x_dt == PF_F16) PF_NBI(NV, PF_F16, PF_F16, PF_F16);                       \
-  else if (io16 && x_dt == PF_BF16) PF_NBI(NV, PF_BF16, PF_BF16, PF_BF16);                   \
-  else PF_NB(8, NV)
   if (v) {
-    if (d <= 64 * 8) { PF_NBD(2); }
-    else if (d <= 64 * 8 * 2) { PF_NBTD(2, 4, PF_NB(8, 2)); }
-    else if (d <= 64 * 8 * 3) { PF_NBTD(3, 2, PF_NB(8, 3)); }
-    else if (d <= 64 * 8 * 4) { PF_NBTD(4, 2, PF_NB(8, 4)); }
+    if (d <= 8 * 8) { PF_NBTD(PF_NB(8, 1), PF_NBN, 8); }
+    else if (d <= 16 * 8) { PF_NBTD(PF_NB(8, 1), PF_NBN, 16); }
+    else if (d <= 32 * 8) { PF_NBTD(PF_NB(8, 1), PF_NBN, 32); }
+    else if (d <= 64 * 8) { PF_NBTD(PF_NB(8, 1), PF_NBN, 64); }
+    else if (d <= 64 * 8 * 2) { PF_NBTD(PF_NB(8, 2), PF_NBT, 2, 4); }
+    else if (d <= 64 * 8 * 3) { PF_NBTD(PF_NB(8, 3), PF_NBT, 3, 2); }
+    else if (d <= 64 * 8 * 4) { PF_NBTD(PF_NB(8, 4), PF_NBT, 4, 2); }
     else if (d <= 64 * 8 * 8) PF_NB(8, 8);
     else if (d <= 64 * 8 * 16) PF_NB(8, 16);
     else { pf_set_error("%s: d=%lld exceeds 8192", name, (long long)d); return PF_ERR_UNSUPPORTED; }
@@ -864,11 +878,9 @@ int norm_bwd(const void* dy, int dy_dt, const void* x, int x_dt, const float* ga
     else if (d <= 64 * 64) PF_NB(1, 64);
     else { pf_set_error("%s: unaligned d=%lld exceeds 4096", name, (long long)d); return PF_ERR_UNSUPPORTED; }
   }
-#undef PF_NBD
 #undef PF_NBTD
 #undef PF_NBT
-#undef PF_NBC
-#undef PF_NBI
+#undef PF_NBN
 #undef PF_NB
   PF_CHECK_LAUNCH(name);
   if (want && !defer) {
