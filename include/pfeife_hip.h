@@ -175,7 +175,8 @@ typedef struct pf_gemm_desc {
                        rows, ws[tile_row * N + column] for tile_row < ceil(M / BM) (BM: the variant's first
                        tile dimension): the bias gradient of the layer whose pre-activation gradient C is
                        (aten.sum of the reference's autograd, pfeife/mp/worker.py:1585-1587), finished by
-                       pf_colreduce_finalize(_batch).  PF_ERR_UNSUPPORTED on any other kernel path. */
+                       pf_colreduce_finalize(_batch).  A product in two launches leaves more of them if its second
+                       tile is less high, which it is only where colsum_rows has room (pf_gemm_colsum_rows: how many).  PF_ERR_UNSUPPORTED on any other kernel path. */
   const float* unscale_by; /* optional: device pointer to a loss scale s > 0, read when the kernel runs: the
                        product is multiplied by alpha / s[0] instead of alpha, so a gradient computed from a scaled
                        loss leaves the product unscaled (GradScaler.unscale_ of pfeife/mp/worker.py:1432-1436 without
@@ -184,6 +185,7 @@ typedef struct pf_gemm_desc {
                        the same unscale_); only where the direct-to-LDS kernel stores or accumulates an fp32 C without
                        activation or residual (pf_gemm_variant ends in ", 1>" or ", 4>", or in ", -1>" for such a
                        product with both operands transposed and a bias or round_mid), PF_ERR_UNSUPPORTED elsewhere */
+  int64_t colsum_rows; /* partial rows that colsum_ws has room for (0: ceil(M / BM)) */
 } pf_gemm_desc;
 
 int pf_gemm(const pf_gemm_desc* desc, void* stream);
@@ -212,6 +214,8 @@ int pf_mfma16_rate(int dtype, const void* operands, int64_t iters, int workgroup
  * b_trans, epilogue class) or "gemm16_kernel<1, 128, 64, 64, 2, 2, false, true>".  Lets a harness attribute
  * measured kernel time to problem shapes.  No counterpart in the reference. */
 int pf_gemm_variant(const pf_gemm_desc* desc, char* out, int cap);
+/* Partial rows of column sums that the product leaves given room for them (before colsum_ws is set), -1: none. */
+int64_t pf_gemm_colsum_rows(const pf_gemm_desc* desc);
 
 /* ---- normalisation (HBM-bound, one wavefront per row) ---------------------
  * LayerNorm over the last dimension d of a [rows, d] matrix; gamma/beta are

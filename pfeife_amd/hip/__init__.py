@@ -59,7 +59,7 @@ class GemmDesc(Structure):
         ("aux_in", c_void_p), ("ld_aux_in", c_int64),
         ("residual", c_void_p), ("ld_res", c_int64),
         ("res_dtype", c_int32), ("variant", c_int32),
-        ("colsum_ws", c_void_p), ("unscale_by", c_void_p), ("nonfinite_flag", c_void_p),
+        ("colsum_ws", c_void_p), ("unscale_by", c_void_p), ("nonfinite_flag", c_void_p), ("colsum_rows", c_int64),
     ]
 
 
@@ -163,7 +163,8 @@ _SIGNATURES = {
     "pf_mfma_rate": [_I, _P, _L, _I, _P, _P],
     "pf_mfma16_rate": [_I, _P, _L, _I, _P, _P],
 }
-_RET_I64 = {"pf_colreduce_workspace": [_L, _L], "pf_reduce_workspace": [_L], "pf_groupnorm_workspace": [_L, _L, _I],
+_RET_I64 = {"pf_gemm_colsum_rows": [POINTER(GemmDesc)], "pf_colreduce_workspace": [_L, _L], "pf_reduce_workspace": [_L],
+            "pf_groupnorm_workspace": [_L, _L, _I],
             "pf_colsum_static_capacity": []}
 EXPORTED_SYMBOLS = sorted(list(_SIGNATURES) + list(_RET_I64) + ["pf_version", "pf_last_error"])
 
@@ -435,10 +436,9 @@ class HipKernels:
             return None
         if d.batch1 * d.batch2 != 1 or d.colsum_ws:
             return None
-        bm = int(v.split("<")[1].split(",")[1])
-        nb = (d.M + bm - 1) // bm
+        nb = int(self.lib.pf_gemm_colsum_rows(byref(d)))
         ws = alloc((nb, d.N), torch.float32)
-        d.colsum_ws = ws.data_ptr()
+        d.colsum_ws, d.colsum_rows = ws.data_ptr(), nb
         launch.colsum_ws = ws
         return ws, 0, nb, d.N
 

@@ -158,3 +158,35 @@ def test_products_in_two_launches(hip, dtype, M, N, K):
         if w0 is not None:
             want = c0[:, :N].double().sum(0)
             assert float((w0.double().sum(0) - want).abs().max()) <= 256 * 2.0 ** -24 * float(c0[:, :N].double().abs().sum(0).max())
+
+
+@pytest.mark.parametrize("M,N,K", [(12214, 1536, 384), (12922, 1536, 1024), (4728, 4096, 512)])
+def test_column_sums_of_two_launches(hip, M, N, K):
+    """Two launches of tiles of different heights: as many partial rows as announced, stored values as without them; a workspace for the
+    first tile's height alone gets rows of that height.  (Bound: fp32 sums of at most 256 values each.)"""
+    dy, w, h = rnd((M, K), BF16, 1).cuda(), rnd((N, K), BF16, 2, 0.1).cuda(), rnd((M, N), BF16, 3).cuda()
+    c = [torch.zeros(M, N, dtype=BF16, device="cuda") for _ in range(3)]
+    kw = dict(M=M, N=N, K=K, lda=K, ldb=K, ldc=N, dact=1, aux_in=h, ld_aux_in=N)
+    s = torch.cuda.current_stream().cuda_stream
+    hip.gemm(dy, w, c[0], **kw)(s)
+    any_height, one_height = hip.gemm(dy, w, c[1], **kw), hip.gemm(dy, w, c[2], **kw)
+    got = []
+
+    def alloc(shape, dtype):
+        got.append(torch.full((shape[0] * shape[1] + 64,), float("nan"), dtype=dtype, device="cuda"))
+        return got[-1][:shape[0] * shape[1]].view(shape)
+
+    _, _, nb, _ = hip.gemm_attach_colsum(any_height, alloc)
+    low = (M + 255) // 256
+    assert nb > low and "256, 256, 64, 2, 2" in any_height.variant
+    whole = torch.full((low * N + 64,), float("nan"), device="cuda")
+    one_height.desc.colsum_ws = whole.data_ptr()
+    any_height(s)
+    one_height(s)
+    torch.cuda.synchronize()
+    assert torch.equal(c[0], c[1]) and torch.equal(c[0], c[2])
+    want = c[0].double().sum(0)
+    for ws, rows in ((got[0], nb), (whole, low)):
+        assert ws[rows * N:].isnan().all()
+        err = (ws[:rows * N].view(rows, N).double().sum(0) - want).abs().max()
+        assert float(err) <= 256 * 2.0 ** -24 * float(c[0].double().abs().sum(0).max())
