@@ -1116,9 +1116,10 @@ __global__ __launch_bounds__(NT) void attn_dkv_short_kernel(const AttnArgs a, in
 // wavefront first forms delta and dQ for its 32 queries (sweeping the keys), then, after one barrier,
 // dK and dV for its 32 keys (sweeping the queries); against the two-kernel form this saves a launch and
 // one load of the head.  Same arithmetic, in the same order, as attn_dq_short_kernel and
-// attn_dkv_short_kernel.
+// attn_dkv_short_kernel.  Heads from `whole` on have two workgroups each: there four wavefronts form dQ of half of the queries
+// beside four that form dK and dV of half of the keys.
 template <int DT, int HD>
-__global__ __launch_bounds__(512) void attn_bwd_short_fused_kernel(const AttnArgs a, float* delta_out, int rows_q, int rows_k) {
+__global__ __launch_bounds__(512) void attn_bwd_short_fused_kernel(const AttnArgs a, float* delta_out, int rows_q, int rows_k, int whole) {
   constexpr int NC = HD / 16, NO = HD / 32, LD = HD + 8, NT = 512;
   extern __shared__ __align__(16) uint16_t smem[];
   uint16_t* sK = smem;
@@ -1128,19 +1129,20 @@ __global__ __launch_bounds__(512) void attn_bwd_short_fused_kernel(const AttnArg
   float* sLse = (float*)(sDO + rows_q * LD);
   float* sDelta = sLse + rows_q;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int bh = blockIdx.y, b = bh / a.H, h = bh % a.H;
+  // heads from `whole` on: two workgroups each
+  const int part = (int)blockIdx.y - whole, bh = part < 0 ? (int)blockIdx.y : whole + part / 2, b = bh / a.H, h = bh % a.H;
   const uint16_t* OO = a.o + b * a.o_sb + h * a.o_sh;
   const float sc = a.scale * LOG2E;
   const int shift = a.Tk - a.Tq;
 
   // delta = rowsum(dO * O) and lse of this lane's query row
-  const int q0 = wave * 32, qi = q0 + (lane & 31);
-  const bool qok = qi < a.Tq;
+  int q0 = wave * 32, qi = q0 + (lane & 31);
+  bool qok = qi < a.Tq;
   const HeadRows rdo(a.d_o + b * a.do_sb + h * a.do_sh, a.do_st, a.Tq, a.hd), ro(OO, a.o_st, a.Tq, a.hd);
   const HeadRows rq(a.q + b * a.q_sb + h * a.q_sh, a.q_st, a.Tq, a.hd);
   const HeadRows rk(a.k + b * a.k_sb + h * a.k_sh, a.k_st, a.Tk, a.hd), rv(a.v + b * a.v_sb + h * a.v_sh, a.v_st, a.Tk, a.hd);
   float dlt = 0.f;
-  const float lse2 = qok ? a.lse[(int64_t)bh * a.Tq + qi] * LOG2E : INFINITY;
+  float lse2 = qok ? a.lse[(int64_t)bh * a.Tq + qi] * LOG2E : INFINITY;
   {
     HeadPair<HD, NT> kv, qd;
     uint4 dof[NC], of[NC];
@@ -1172,6 +1174,19 @@ __global__ __launch_bounds__(512) void attn_bwd_short_fused_kernel(const AttnArg
   __syncthreads();
 
   // ---- dQ for queries q0 .. q0+31
+  int kw0 = q0;
+  if (part >= 0) {
+    // half of the head: dQ by the first four wavefronts and dK, dV by the others, at the same time
+    const int hq = (rows_q / 32 + 1) / 2, hk = (rows_k / 32 + 1) / 2;
+    q0 = wave < hq && wave < 4 ? ((part & 1) * hq + wave) * 32 : a.Tq;
+    kw0 = wave >= 4 && wave - 4 < hk ? ((part & 1) * hk + wave - 4) * 32 : a.Tk;
+    qi = q0 + (lane & 31);
+    qok = qi < a.Tq;
+    if (q0 < a.Tq) {
+      lse2 = sLse[qi];
+      dlt = sDelta[qi];
+    }
+  }
   if (q0 < a.Tq) {
     uint4 qf[NC], dof[NC];
 #pragma unroll
@@ -1231,7 +1246,7 @@ __global__ __launch_bounds__(512) void attn_bwd_short_fused_kernel(const AttnArg
   }
 
   // ---- dK, dV for keys kw0 .. kw0+31 (sLse / sDelta were complete at the barrier above)
-  const int kw0 = wave * 32, kj = kw0 + (lane & 31);
+  const int kj = kw0 + (lane & 31);
   if (kw0 >= a.Tk) return;
   const bool kok = kj < a.Tk;
   uint4 kf[NC], vf[NC];
@@ -1441,9 +1456,13 @@ extern "C" int pf_attention_bwd(const pf_attn_desc* d, void* stream) {
     if (d->hd <= 64 && d->Tq <= 256 && d->Tk <= 256 && (d->Tq > 128 || d->Tk > 128)) {
       // one workgroup per head forms dQ, dK and dV from a single load of the head
       const size_t lds = (size_t)2 * (rows_k + rows_q) * (64 + 8) * 2 + (size_t)rows_q * 8;
-      const dim3 gf(1, (unsigned)(d->B * d->H));
-      if (d->dtype == PF_F16) rc = launch_short(attn_bwd_short_fused_kernel<PF_F16, 64>, gf, 512, lds, st, a, d->delta, rows_q, rows_k);
-      else rc = launch_short(attn_bwd_short_fused_kernel<PF_BF16, 64>, gf, 512, lds, st, a, d->delta, rows_q, rows_k);
+      // A CU has LDS for one of them.  Up to 128 heads that are left after rounds of 256 go to two workgroups each, half of the queries and
+      // half of the keys to one (us, a workgroup / two, 197 tokens, head dim 64: 24 heads 17.6 / 13.3, 60 18.5 / 14.2, 120 20.0 / 16.7,
+      // 258 40.0 / 35.0, 372 42.0 / 40.1).
+      const int heads = d->B * d->H, rest = heads % 256, whole = rest <= 128 ? heads - rest : heads;
+      const dim3 gf(1, (unsigned)(2 * heads - whole));
+      if (d->dtype == PF_F16) rc = launch_short(attn_bwd_short_fused_kernel<PF_F16, 64>, gf, 512, lds, st, a, d->delta, rows_q, rows_k, whole);
+      else rc = launch_short(attn_bwd_short_fused_kernel<PF_BF16, 64>, gf, 512, lds, st, a, d->delta, rows_q, rows_k, whole);
       if (rc != PF_OK) return rc;
       PF_CHECK_LAUNCH("pf_attention_bwd");
       return PF_OK;
