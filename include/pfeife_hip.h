@@ -428,7 +428,8 @@ typedef struct pf_shadow_item {
   void* plain;
   void* transposed;
   int64_t rows, cols;
-  int32_t dtype, reserved;
+  int32_t dtype;
+  int32_t ld_t; /* elements between rows of `transposed`, a multiple of 4 (0: rows) */
 } pf_shadow_item;
 int pf_shadow_batch(const pf_shadow_item* items_dev, int n_items, int64_t max_tiles, void* stream);
 /* dst[c*ld_dst + r] = src[r*ld_src + c] with dtype conversion: the transposed 16-bit

@@ -418,6 +418,7 @@ __global__ __launch_bounds__(256) void shadow_batch_kernel(const pf_shadow_item*
   }
   __syncthreads();
   if (!it.transposed) return;
+  const int64_t ld_t = it.ld_t ? it.ld_t : it.rows;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int lc = ty + 16 * i;             // source column = row of the transposed shadow
@@ -425,7 +426,7 @@ __global__ __launch_bounds__(256) void shadow_batch_kernel(const pf_shadow_item*
     if (c < it.cols && r < it.rows) {
       const uint32_t lo = (uint32_t)tile[tx * 4][lc] | ((uint32_t)tile[tx * 4 + 1][lc] << 16);
       const uint32_t hi = (uint32_t)tile[tx * 4 + 2][lc] | ((uint32_t)tile[tx * 4 + 3][lc] << 16);
-      *(uint2*)((uint16_t*)it.transposed + c * it.rows + r) = make_uint2(lo, hi);
+      *(uint2*)((uint16_t*)it.transposed + c * ld_t + r) = make_uint2(lo, hi);
     }
   }
 }

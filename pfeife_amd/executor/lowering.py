@@ -87,13 +87,47 @@ class ParamStore:
             self._keep.append(tensor)
         return sh
 
+    def shadow_joint(self, tensors, dtype):
+        """One [sum of rows, columns] matrix of the shadows of several weight matrices, one below the other, or None if one of
+        them has a shadow of its own already."""
+        keys = [(t.data_ptr(), tuple(t.shape), t.dtype, dtype) for t in tensors]
+        sh = self._shadow.get(("joint", *keys))
+        if sh is None:
+            if len(set(keys)) < len(keys) or any(k in self._shadow or t.dtype == dtype or not t.is_contiguous() for k, t in zip(keys, tensors)):
+                return None
+            sh = torch.empty((sum(t.shape[0] for t in tensors), tensors[0].shape[1]), dtype=dtype, device=tensors[0].device)
+            for t, key, piece in zip(tensors, keys, sh.split([t.shape[0] for t in tensors])):
+                if hasattr(self.kernels, "cast_batch"):
+                    self.cast_pairs.append((t.detach(), piece))
+                else:
+                    self.refresh.append(self.kernels.cast(t.detach(), piece, piece.numel()))
+                self._shadow[key] = piece
+                self._keep.append(t)
+            self._shadow[("joint", *keys)] = sh
+        return sh
+
+    def shadow_joint_t(self, tensors, dtype):
+        """The transposed shadows of the same matrices side by side: [columns, sum of rows]."""
+        key = ("joint T", *((t.data_ptr(), tuple(t.shape), t.dtype, dtype) for t in tensors))
+        sh = self._shadow.get(key)
+        if sh is None:
+            sh = torch.empty((tensors[0].shape[1], sum(t.shape[0] for t in tensors)), dtype=dtype, device=tensors[0].device)
+            self.shadow_t_pairs += [(t.detach(), piece) for t, piece in zip(tensors, sh.split([t.shape[0] for t in tensors], 1))]
+            self._shadow[key] = sh
+        return sh
+
     def refresh_launches(self):
         """Launches that bring every shadow up to date with its master (once per step): weight
         matrices get their plain and transposed shadows from one read of the master, in one
         launch for all of them; the remaining casts share a second launch."""
         out = list(self.refresh)
         pairs = list(self.cast_pairs)
-        t_of = {src.data_ptr(): (src, sh) for src, sh in self.shadow_t_pairs}
+        t_of, more = {}, []
+        for src, sh in self.shadow_t_pairs:
+            if src.data_ptr() in t_of:          # (a matrix that has one beside others and one of its own)
+                more.append((src, sh))
+            else:
+                t_of[src.data_ptr()] = (src, sh)
         batch = getattr(self.kernels, "shadow_batch", None)
         duals, rest = [], []
         for src, sh in pairs:
@@ -104,12 +138,12 @@ class ParamStore:
                 del t_of[src.data_ptr()]
             else:
                 rest.append((src, sh))
-        for src, sh in t_of.values():           # transposed shadow only (or not batchable)
+        for src, sh in list(t_of.values()) + more:      # transposed shadow only (or not batchable)
             if batch is not None and self.kernels.shadow_batch_ok(src, None, sh):
                 duals.append((src, None, sh))
             else:
                 rows, cols = src.shape
-                out.append(self.kernels.transpose_cast(src, cols, sh, rows, rows, cols))
+                out.append(self.kernels.transpose_cast(src, cols, sh, sh.stride(0), rows, cols))
         if duals:
             out.insert(0, batch(duals))
         if rest:
@@ -1160,7 +1194,155 @@ def _is_add_node(n):
     return n.op == "call_function" and n.target in (operator.add, operator.iadd, torch.add)
 
 
+def _input_gradient(B, x, dy, wb, K, kw2, alone):
+    """x's gradient of a linear layer, dy times the weight (wb, as kw2 says).  alone: no other layer reads x."""
+    dst, prev = B.grad_target(x)
+    dm = as_matrix(dst)
+    if x.preact is not None and alone and prev is None:
+        kw2.update(dact=x.preact[0], aux_in=x.preact[1], ld_aux_in=K)
+        x.grad_is_preact = True
+    if dm is not None:
+        if prev is dst:
+            kw2["beta"] = 1
+        elif prev is not None:
+            pm = as_matrix(prev)
+            if pm is None:
+                raise Unsupported("accumulating into a non-matrix gradient")
+            kw2.update(residual=prev, ld_res=pm[2])
+        launch = B.k.gemm(dy, wb, dst, ldc=dm[2], **kw2)
+        B.emit(launch)
+        B.commit(x, dst)
+        if ("dact" in kw2 and hasattr(B.k, "gemm_attach_colsum") and dm[2] == K
+                and os.environ.get("PFEIFE_EPILOGUE_COLSUM", "1") != "0"):
+            # dst now holds the gradient of the producing layer's pre-activation: its column sums
+            # are that layer's bias gradient, and the product's epilogue can leave them behind
+            cs = B.k.gemm_attach_colsum(launch, B.temp)
+            if cs is not None:
+                B.register_lp(dst, dst, colsum=cs)
+    else:
+        # target is not a plain matrix (e.g. a permuted view): go through a temp
+        tmp = B.temp(tuple(x.shape), x.dtype)
+        B.emit(B.k.gemm(dy, wb, tmp, ldc=K, **kw2))
+        if prev is None:
+            B.copy(tmp, dst)
+        elif prev is dst:
+            B.copy(tmp, dst, accumulate=True)
+        else:
+            B.copy(prev, dst)
+            B.copy(tmp, dst, accumulate=True)
+        B.commit(x, dst)
+
+
+def _joins_at(L, node):
+    """The attention or gated product that a linear layer's result goes to through nothing but views and rotary embedding, or None."""
+    while True:
+        users = list(node.users)
+        root = next((r for r, p in L.patterns.items() if p[0] is node), None)
+        if root is not None and all(u in L.pattern_skip for u in users):
+            node = root
+            continue
+        if len(users) != 1:
+            return None
+        u = users[0]
+        if _is(u, F.scaled_dot_product_attention, torch._C._nn.scaled_dot_product_attention):
+            return u if node in u.args[:3] else None
+        gate = L.sole_user(u) if _act_of_node(u) is not None else u
+        if gate is not None and _is(gate, operator.mul, torch.mul) and all(isinstance(a, torch.fx.Node) for a in gate.args[:2]):
+            return gate
+        if not ((u.op == "call_method" and u.target in ("view", "reshape", "transpose", "permute", "unflatten"))
+                or _is(u, torch.transpose, torch.permute, torch.reshape)):
+            return None
+        node = u
+
+
+def _joint_layers(L, node):
+    """The linear layers without bias that read what `node` reads and whose results meet its result in one attention or gated
+    product (`node` the first), or None.  As one layer they are one product forward and one for the input's
+    gradient, summed in fp32 over all of them, where there were as many of each, with a 16-bit sum after every one.  us a step, one
+    by one / joint: four decoder layers of 2048 with 4084 tokens 9977 / 9650, the 30 attention blocks of 4 x 1024 tokens of 1280
+    53400 / 51900, sixteen decoder layers of 2048 with 4 x 8192 tokens 190000 / 187500."""
+    def eligible(n):
+        if not _is(n, F.linear, torch._C._nn.linear) or n.args[0] is not node.args[0] or n in L.env or _kw(n, 2, "bias") is not None:
+            return False
+        w = L.env.get(_kw(n, 1, "weight"))
+        return (isinstance(w, Val) and w.kind == "base" and w.param is not None and w.buf.dim() == 2 and w.buf.dtype == torch.float32
+                and w.shape[0] % 8 == 0 and w.shape[1] % 8 == 0)
+
+    if not L.mixed or not isinstance(node.args[0], torch.fx.Node) or not eligible(node):
+        return None
+    at = _joins_at(L, node)
+    nodes = [node] + [n for n in node.args[0].users if at is not None and n is not node and eligible(n) and _joins_at(L, n) is at]
+    if len(nodes) < 2:
+        return None
+    x = L.arg(node.args[0])
+    K, N = x.shape[-1], sum(L.env[_kw(n, 1, "weight")].shape[0] for n in nodes)
+    rows = x.buf.numel() // K
+    if L.layout is not None and L.layout.sizes and L.cur.mb is not None and L.layout.sizes[L.cur.mb] > 0:
+        rows = rows * sum(L.layout.sizes) // L.layout.sizes[L.cur.mb]
+    # (what the products read and write stays below 2 GiB, the weight gradients' operands over all micro-batches too)
+    if any(L.env[_kw(n, 1, "weight")].shape[1] != K for n in nodes) or rows == 0 or (rows + 256) * N * 4 >= MAX_BYTES:
+        return None
+    return nodes
+
+
+def _lower_joint(L, nodes):
+    x = L.arg(nodes[0].args[0])
+    ws = [L.env[_kw(n, 1, "weight")] for n in nodes]
+    w_cd = L.params.shadow_joint([w.buf for w in ws], L.cd)
+    if w_cd is None:
+        return None
+    cd, K, sizes = L.cd, x.shape[-1], [w.shape[0] for w in ws]
+    N = sum(sizes)
+    xm = L.matrix_in(x.buf, cd)
+    M, _, lda = as_matrix(xm)
+    w_t = L.params.shadow_joint_t([w.buf for w in ws], cd) if x.req_grad and M >= 256 else None
+    out = L.alloc(tuple(x.shape[:-1]) + (N,), cd)
+    L.emit(L.kernels.gemm(xm, w_cd, out, M=M, N=N, K=K, lda=lda, ldb=K, ldc=N, round_mid=1))
+    outv = Val(out, req_grad=x.req_grad or any(w.req_grad for w in ws), name=nodes[0].name)
+    parts = []
+    for i, n in enumerate(nodes):
+        fn = (lambda t, i=i: t.split(sizes, -1)[i])
+        part = Val(fn(out), req_grad=outv.req_grad, kind="part", base=outv, view_fn=fn, name=n.name)
+        part.tiled = True
+        parts.append(part)
+        L.fused[n] = part
+    L.cur.tile_groups.append(parts)
+    if L.defer_dw and any(w.req_grad for w in ws):
+        L.cur.dw_sigs.add((M * N, cd))
+
+    def bwd(B):
+        g = B.grad_of(outv)
+        if g is None:
+            return
+        dy = B.matrix_in(g, cd)
+        _, _, ld_dy = as_matrix(dy)
+        at = 0
+        for n, w, size in zip(nodes, ws, sizes):
+            piece = torch.as_strided(dy, (M, size), (ld_dy, 1), dy.storage_offset() + at)
+            at += size
+            if not w.req_grad:
+                continue
+            wg = L.params.grad(w.param, (B.program.stage, n.name) if L.defer_dw else None)
+            if L.defer_dw:
+                B.program.dw_deferred.append(dict(name=n.name, dy=piece, x=xm, wg=wg, param=w.param, rows=M, n_out=size, n_in=K,
+                                                  ld_dy=ld_dy, ld_x=lda))
+            else:
+                B.emit_dw(B.k.gemm(piece, xm, wg, M=size, N=K, K=M, lda=ld_dy, ldb=lda, ldc=K, a_trans=1, b_trans=1, beta=1), wg)
+        if x.req_grad:
+            wb, kw = (w_t, dict(ldb=N, b_trans=0)) if w_t is not None else (w_cd, dict(ldb=K, b_trans=1))
+            _input_gradient(B, x, dy, wb, K, dict(M=M, N=K, K=N, lda=ld_dy, **kw), False)
+
+    if outv.req_grad:
+        L.add_backward(bwd)
+    return parts[0]
+
+
 def lower_linear(L, node):
+    joint = _joint_layers(L, node)
+    if joint is not None:
+        out = _lower_joint(L, joint)
+        if out is not None:
+            return out
     x = L.arg(node.args[0])
     w = L.arg(node.args[1])
     b = L.arg(_kw(node, 2, "bias"))
@@ -1260,49 +1442,15 @@ def lower_linear(L, node):
             else:
                 B.colsum_into(dy, M, N, ld_dy, bg)
         if x.req_grad:
-            dst, prev = B.grad_target(x)
-            dm = as_matrix(dst)
             if w_t is not None:
                 wb, kw2 = w_t, dict(M=M, N=K, K=N, lda=ld_dy, ldb=N, b_trans=0)
             else:
                 wb, kw2 = w_cd, dict(M=M, N=K, K=N, lda=ld_dy, ldb=K, b_trans=1)
-            if x.preact is not None and x_users == 1 and prev is None:
-                kw2.update(dact=x.preact[0], aux_in=x.preact[1], ld_aux_in=K)
-                x.grad_is_preact = True
-            if dm is not None:
-                if prev is dst:
-                    kw2["beta"] = 1
-                elif prev is not None:
-                    pm = as_matrix(prev)
-                    if pm is None:
-                        raise Unsupported("accumulating into a non-matrix gradient")
-                    kw2.update(residual=prev, ld_res=pm[2])
-                launch = B.k.gemm(dy, wb, dst, ldc=dm[2], **kw2)
-                B.emit(launch)
-                B.commit(x, dst)
-                if ("dact" in kw2 and hasattr(B.k, "gemm_attach_colsum") and dm[2] == K
-                        and os.environ.get("PFEIFE_EPILOGUE_COLSUM", "1") != "0"):
-                    # dst now holds the gradient of the producing layer's pre-activation: its column sums
-                    # are that layer's bias gradient, and the product's epilogue can leave them behind
-                    cs = B.k.gemm_attach_colsum(launch, B.temp)
-                    if cs is not None:
-                        B.register_lp(dst, dst, colsum=cs)
-            else:
-                # target is not a plain matrix (e.g. a permuted view): go through a temp
-                tmp = B.temp(tuple(x.shape), x.dtype)
-                B.emit(B.k.gemm(dy, wb, tmp, ldc=K, **kw2))
-                if prev is None:
-                    B.copy(tmp, dst)
-                elif prev is dst:
-                    B.copy(tmp, dst, accumulate=True)
-                else:
-                    B.copy(prev, dst)
-                    B.copy(tmp, dst, accumulate=True)
-                B.commit(x, dst)
+            _input_gradient(B, x, dy, wb, K, kw2, x_users == 1)
 
     if req:
         L.add_backward(bwd)
-    return outv if out_node is node else outv
+    return outv
 
 
 def lower_layer_norm(L, node, rms=False):

@@ -684,8 +684,11 @@ class HipKernels:
             return False
         if src.shape[0] % 4 or src.shape[1] % 4 or src.data_ptr() % 16:
             return False
-        return all(t is None or (t.is_contiguous() and t.data_ptr() % 8 == 0 and t.dtype in (torch.float16, torch.bfloat16))
-                   for t in (plain, transposed))
+        if plain is not None and not plain.is_contiguous():
+            return False
+        if transposed is not None and (transposed.stride(1) != 1 or transposed.stride(0) % 4 or transposed.stride(0) >= 1 << 31):
+            return False
+        return all(t is None or (t.data_ptr() % 8 == 0 and t.dtype in (torch.float16, torch.bfloat16)) for t in (plain, transposed))
 
     def shadow_batch(self, items):
         """One launch writing the plain and/or transposed 16-bit shadow of every (src, plain, transposed)."""
@@ -694,7 +697,7 @@ class HipKernels:
             r, c = src.shape
             dt = dtype_code((plain if plain is not None else tr).dtype)
             rows.append([src.data_ptr(), 0 if plain is None else plain.data_ptr(), 0 if tr is None else tr.data_ptr(),
-                         r, c, dt])
+                         r, c, dt | (0 if tr is None else tr.stride(0)) << 32])
         table = torch.tensor(rows, dtype=torch.int64).to(items[0][0].device)
         tiles = max(((r[3] + 63) // 64) * ((r[4] + 63) // 64) for r in rows)
         nbytes = sum(r[3] * r[4] * (4 + 2 * (r[1] != 0) + 2 * (r[2] != 0)) for r in rows)
