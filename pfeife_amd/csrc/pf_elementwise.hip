@@ -470,7 +470,7 @@ struct AdamCoef {
     if (adamw) p *= 1.f - lr * weight_decay;
     else if (weight_decay != 0.f) g += weight_decay * p;
     m = m + omb1 * (g - m);
-    v = v * beta2 + omb2 * g * g;
+    v = fmaf(omb2, g * g, v * beta2);      // (rounded as mul_ and addcmul_ round)
     const float denom = sqrtf(v) / bias_c2_sqrt + eps;
     p = p - step_size * (m / denom);
   }
