@@ -422,7 +422,8 @@ int pf_cast_batch(const pf_cast_item* items_dev, int n_items, int64_t max_n, voi
  * be NULL.  Every matrix is contiguous with rows % 4 == 0 and cols % 4 == 0, src 16-byte and
  * the destinations 8-byte aligned (the caller checks; other matrices go through pf_cast_batch /
  * pf_transpose_cast).  max_tiles = max over items of ceil(rows/64) * ceil(cols/64).  The master
- * is read once instead of once per shadow (autocast re-casts the weight at every use). */
+ * is read once instead of once per shadow (autocast re-casts the weight at every use).  dtype PF_F32: a
+ * transposed copy alone, 16-byte aligned. */
 typedef struct pf_shadow_item {
   const float* src;
   void* plain;

@@ -392,12 +392,35 @@ __global__ __launch_bounds__(256) void cast_batch_kernel(const pf_cast_item* ite
 // lane, 256-byte runs), the plain shadow is written from registers (8 bytes per lane), the
 // transposed shadow through a 16-bit LDS tile (8 bytes per lane, 128-byte runs).
 __global__ __launch_bounds__(256) void shadow_batch_kernel(const pf_shadow_item* items) {
-  __shared__ uint16_t tile[64][64 + 2];
+  __shared__ float tile32[64][64 + 1];
+  uint16_t (*tile)[64 + 2] = (uint16_t (*)[64 + 2])tile32;
   const pf_shadow_item it = items[blockIdx.y];
   const int64_t tiles_c = (it.cols + 63) / 64, tiles_r = (it.rows + 63) / 64;
   if ((int64_t)blockIdx.x >= tiles_c * tiles_r) return;   // uniform over the block
   const int64_t r0 = ((int64_t)blockIdx.x / tiles_c) * 64, c0 = ((int64_t)blockIdx.x % tiles_c) * 64;
   const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+  const int64_t ld_t = it.ld_t ? it.ld_t : it.rows;
+  if (it.dtype == PF_F32) {
+    // a transposed copy of fp32 products' weights.  us, a launch to each / together: the 48 of twelve ViT-S layers (85 MB) 518 / 31
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int64_t r = r0 + ty + 16 * i, c = c0 + tx * 4;
+      float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (r < it.rows && c < it.cols) v = *(const float4*)(it.src + r * it.cols + c);
+      float* to = &tile32[ty + 16 * i][tx * 4];
+      to[0] = v.x; to[1] = v.y; to[2] = v.z; to[3] = v.w;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int lc = ty + 16 * i;
+      const int64_t c = c0 + lc, r = r0 + tx * 4;
+      if (c < it.cols && r < it.rows)
+        *(float4*)((float*)it.transposed + c * ld_t + r) =
+            make_float4(tile32[tx * 4][lc], tile32[tx * 4 + 1][lc], tile32[tx * 4 + 2][lc], tile32[tx * 4 + 3][lc]);
+    }
+    return;
+  }
   const bool bf = it.dtype == PF_BF16;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -418,7 +441,6 @@ __global__ __launch_bounds__(256) void shadow_batch_kernel(const pf_shadow_item*
   }
   __syncthreads();
   if (!it.transposed) return;
-  const int64_t ld_t = it.ld_t ? it.ld_t : it.rows;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int lc = ty + 16 * i;             // source column = row of the transposed shadow

@@ -477,9 +477,10 @@ class HipKernels:
 
     @staticmethod
     def gemm_stores_checked(launch):
-        """Does this product run on a kernel whose epilogue honours `nonfinite_flag` (the fp32 classes
-        of the direct-to-LDS kernel)?"""
-        return HipKernels.gemm_groupable(launch)
+        """Does this product store what was asked for: on any kernel without `nonfinite_flag` and `unscale_by`, else on one whose
+        epilogue honours the flag (the fp32 classes of the direct-to-LDS kernel)?"""
+        d = launch.desc
+        return HipKernels.gemm_groupable(launch) or (not d.nonfinite_flag and not d.unscale_by)
 
     def gemm_group(self, launches):
         """One launch for 2..GEMM_GROUP_MAX independent `gemm_groupable` products of the same variant.  They run side by
@@ -688,6 +689,8 @@ class HipKernels:
             return False
         if transposed is not None and (transposed.stride(1) != 1 or transposed.stride(0) % 4 or transposed.stride(0) >= 1 << 31):
             return False
+        if plain is None and transposed is not None and transposed.dtype == torch.float32:
+            return transposed.data_ptr() % 16 == 0
         return all(t is None or (t.data_ptr() % 8 == 0 and t.dtype in (torch.float16, torch.bfloat16)) for t in (plain, transposed))
 
     def shadow_batch(self, items):
@@ -700,7 +703,7 @@ class HipKernels:
                          r, c, dt | (0 if tr is None else tr.stride(0)) << 32])
         table = torch.tensor(rows, dtype=torch.int64).to(items[0][0].device)
         tiles = max(((r[3] + 63) // 64) * ((r[4] + 63) // 64) for r in rows)
-        nbytes = sum(r[3] * r[4] * (4 + 2 * (r[1] != 0) + 2 * (r[2] != 0)) for r in rows)
+        nbytes = sum(src.numel() * 4 + sum(t.numel() * t.element_size() for t in (plain, tr) if t is not None) for src, plain, tr in items)
         return self._prep("pf_shadow_batch", (table.data_ptr(), len(rows), tiles), (table, items), nbytes)
 
     def transpose_cast(self, src, ld_src, dst, ld_dst, rows, cols):
