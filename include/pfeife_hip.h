@@ -438,6 +438,9 @@ int pf_shadow_batch(const pf_shadow_item* items_dev, int n_items, int64_t max_ti
  * product dx = dy W read W with its reduction dimension contiguous. */
 int pf_transpose_cast(const void* src, int src_dtype, int64_t ld_src, void* dst, int dst_dtype, int64_t ld_dst,
                       int64_t rows, int64_t cols, void* stream);
+/* dst[b, y, x, 3 i + j, c] = src[b, y + i - 1, x + j - 1, c] (flip: y + 1 - i, x + 1 - j), zero outside: a channels-last image's
+ * windows as the left operand of a 3x3 "same" convolution (flip: of its input gradient).  C * element size % 16 == 0, 16-byte aligned. */
+int pf_im2col3x3(const void* src, void* dst, int dtype, int64_t B, int64_t H, int64_t W, int64_t C, int flip, void* stream);
 /* dst[i] = value for n elements of a 4-byte or 2-byte float dtype
  * (optimizer.zero_grad(set_to_none=False), pfeife/mp/worker.py:583-597). */
 int pf_fill(void* dst, int dtype, float value, int64_t n, void* stream);

@@ -541,6 +541,16 @@ class OracleKernels:
 
         return launch
 
+    def im2col3x3(self, src, dst, B, H, W, C, flip=0):
+        def launch(stream=None):
+            pad = torch.nn.functional.pad(_flat(src, B * H * W * C).view(B, H, W, C), (0, 0, 1, 1, 1, 1))
+            out = _flat(dst, 9 * B * H * W * C).view(B, H, W, 9, C)
+            for t in range(9):
+                i, j = (2 - t // 3, 2 - t % 3) if flip else (t // 3, t % 3)
+                out[:, :, :, t] = pad[:, i:i + H, j:j + W]
+
+        return launch
+
     def rope(self, x, y, cos_t, sin_t, B, T, H, D, xs, ys, inverse, tab_ld=None):
         def launch(stream=None):
             half = D // 2

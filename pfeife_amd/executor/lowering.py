@@ -1820,19 +1820,27 @@ def _lower_conv_same(L, x, w, b, k):
     O = w.shape[0]
     M = Bn * H * W
     xn = as_nhwc(L, x.buf, cd)
+    whole = lambda n: M > 0 and n * xn.element_size() % 16 == 0      # pixels of n channels are whole 16-byte pieces
     if k == 1:
         cols, Kc = xn.reshape(M, C), C
         w_cd = L.params.shadow(w.buf, cd).reshape(O, C)
     else:
         Kc = 9 * C
-        padded = L.alloc((Bn, H + 2, W + 2, C), cd).zero_()  # border stays zero for good
-        L.copy(xn, padded[:, 1:H + 1, 1:W + 1, :])
         cols = L.alloc((M, Kc), cd)
-        ps = padded.stride()
-        win = torch.as_strided(padded, (Bn, H, W, 3, 3, C), (ps[0], ps[1], ps[2], ps[1], ps[2], 1))
-        L.copy(win, cols.view(Bn, H, W, 3, 3, C))
+        if whole(C) and xn.is_contiguous() and xn.data_ptr() % 16 == 0:
+            L.emit(L.kernels.im2col3x3(xn, cols, Bn, H, W, C))
+        else:
+            padded = L.alloc((Bn, H + 2, W + 2, C), cd).zero_()  # border stays zero for good
+            L.copy(xn, padded[:, 1:H + 1, 1:W + 1, :])
+            ps = padded.stride()
+            win = torch.as_strided(padded, (Bn, H, W, 3, 3, C), (ps[0], ps[1], ps[2], ps[1], ps[2], 1))
+            L.copy(win, cols.view(Bn, H, W, 3, 3, C))
         w_cd = L.params.shadow_perm(w.buf, cd, (0, 2, 3, 1)).reshape(O, Kc)
     b_cd = None if b is None else L.params.shadow(b.buf, cd)
+    # the weight with the output channels last, [C, taps * O]: what the input gradient multiplies by
+    w_t = None
+    if x.req_grad and w.buf.is_contiguous() and M >= 256 and whole(O) and whole(C):
+        w_t = L.params.shadow_t(w.buf.view(O, Kc), cd).view(C, k * k * O)
     out = L.alloc((Bn, H, W, O), cd)
     L.emit(L.kernels.gemm(cols, w_cd, out, M=M, N=O, K=Kc, lda=Kc, ldb=Kc, ldc=O, bias=b_cd,
                           round_mid=1 if L.mixed else 0))
@@ -1860,7 +1868,21 @@ def _lower_conv_same(L, x, w, b, k):
             if k == 1:
                 direct = prev is None and dstn.is_contiguous()
                 t = dstn if direct else B.temp((Bn, H, W, C), x.dtype)
-                B.emit(B.k.gemm(dy, w_cd, t, M=M, N=C, K=O, lda=O, ldb=C, ldc=C, b_trans=1))
+                if w_t is not None:
+                    B.emit(B.k.gemm(dy, w_t, t, M=M, N=C, K=O, lda=O, ldb=O, ldc=C))
+                else:
+                    B.emit(B.k.gemm(dy, w_cd, t, M=M, N=C, K=O, lda=O, ldb=C, ldc=C, b_trans=1))
+                if not direct:
+                    B.merge(t, dstn, None if prev is None else prev.permute(0, 2, 3, 1))
+            elif w_t is not None and dy.data_ptr() % 16 == 0:
+                # the input gradient is a convolution of dy with the taps in reverse: nine windows side by side, one product that adds
+                # up all taps in fp32.  4096 x 1280 over 9 x 1280, fp16: 129 us; as a product of all windows (16-bit results) and nine
+                # shifted sums 280
+                dcols = B.temp((M, 9 * O), cd)
+                B.emit(B.k.im2col3x3(dy, dcols, Bn, H, W, O, flip=1))
+                direct = prev is None and dstn.is_contiguous()
+                t = dstn if direct else B.temp((Bn, H, W, C), x.dtype)
+                B.emit(B.k.gemm(dcols, w_t, t, M=M, N=C, K=9 * O, lda=9 * O, ldb=9 * O, ldc=C))
                 if not direct:
                     B.merge(t, dstn, None if prev is None else prev.permute(0, 2, 3, 1))
             else:

@@ -262,6 +262,12 @@ def _groupnorm(m, calls):
     return kw
 
 
+def _im2col(m, calls):
+    _same(calls, "H", "W", "C", "flip")
+    per = calls[0]["H"] * calls[0]["W"] * calls[0]["C"]
+    return _chains(calls, "B", src=per, dst=9 * per)
+
+
 def _softmax(*operands):
     def rule(m, calls):
         _same(calls, "cols", *("ld_" + o for o in operands), *(("scale",) if "scale" in calls[0] else ("q_len", "causal")))
@@ -349,7 +355,7 @@ RULES = {
     "axpby": _flat_rule("a", "b", "out", same=("alpha", "beta")),
     "cast": _flat_rule("src", "dst"), "fill": _flat_rule("dst", same=("value",)),
     "glu_fwd": _glu("gate", "up", "y"), "glu_bwd": _glu("dy", "gate", "up", "dgate", "dup"),
-    "bias_add": _bias_add, "copy_strided": _copy_strided, "rope": _rope,
+    "bias_add": _bias_add, "copy_strided": _copy_strided, "im2col3x3": _im2col, "rope": _rope,
     "embedding_fwd": _embedding_fwd, "embedding_bwd": _embedding_bwd,
 }
 

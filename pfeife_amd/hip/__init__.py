@@ -154,6 +154,7 @@ _SIGNATURES = {
     "pf_scaler_unscale": [_P, _L, _P, _P],
     "pf_scaler_update": [_P, ctypes.c_double, ctypes.c_double, _I, _P],
     "pf_copy_strided": [_P, _I, POINTER(c_int64), _P, _I, POINTER(c_int64), POINTER(c_int64), _I, _I, _P],
+    "pf_im2col3x3": [_P, _P, _I, _L, _L, _L, _L, _I, _P],
     "pf_rope": [_P, _P, _I, _P, _P, _L, _L, _L, _L, _L, _L, _L, _L, _L, _L, _L, _I, _P],
     "pf_grad_accumulate_f32": [_P, _P, _I, _L, _P],
     "pf_split_gather": [_P, _P, _L, _L, _L, _P, _P],
@@ -768,6 +769,9 @@ class HipKernels:
         ss, ds, sz = arr(*src_strides), arr(*dst_strides), arr(*sizes)
         args = (_ptr(src), _dt(src), ss, _ptr(dst), _dt(dst), ds, sz, nd, int(accumulate))
         return self._prep("pf_copy_strided", args, (src, dst, ss, ds, sz))
+
+    def im2col3x3(self, src, dst, B, H, W, C, flip=0):
+        return self._prep("pf_im2col3x3", (_ptr(src), _ptr(dst), _dt(src), B, H, W, C, int(flip)), (src, dst), 10 * B * H * W * C * _es(src))
 
     def rope(self, x, y, cos_t, sin_t, B, T, H, D, xs, ys, inverse, tab_ld=None):
         tab_ld = D // 2 if tab_ld is None else tab_ld

@@ -1,0 +1,73 @@
+"""3x3 and 1x1 "same" convolutions: the input gradient as one product with the taps in reverse (kernel table double on the CPU)."""
+import copy
+
+import pytest
+import torch
+import torch.nn as nn
+
+from oracle.kernels_oracle import OracleKernels
+from pfeife_amd.mp import net_states
+from pfeife_amd.option import PipeOption
+
+
+class Convs(nn.Module):
+    def __init__(self, a, b, c, k):
+        super().__init__()
+        self.c0 = nn.Conv2d(a, b, 1)
+        self.c1 = nn.Conv2d(b, c, k, padding=k // 2)
+        self.c2 = nn.Conv2d(c, b, 3, padding=1, bias=False)
+
+    def forward(self, x):
+        x = self.c0(x)
+        return x + self.c2(self.c1(x))          # the first gradient is added to, the others stored
+
+
+@pytest.mark.parametrize("mixed", [None, "bf16"])
+@pytest.mark.parametrize("channels,k,H,W,wide", [((8, 16, 24), 3, 13, 11, True), ((8, 8, 16), 1, 20, 9, True), ((8, 16, 24), 3, 5, 3, False),
+                                                 ((4, 12, 20), 3, 13, 11, None)])
+def test_input_gradients(channels, k, H, W, wide, mixed):
+    """Against autograd in fp32.  wide: 256 pixels and more in a micro-batch and channels of whole 16 bytes, the condition of the one product
+    (None: in fp32 alone)."""
+    from pfeife_amd.mp import PartialRunner, initialize_pfeife, partial_compiler
+
+    if mixed and wide is None:
+        pytest.skip("16-bit products need channels in eights")
+    calls = []
+
+    class Table(OracleKernels):
+        def im2col3x3(self, src, dst, B, H, W, C, flip=0):
+            calls.append(flip)
+            return super().im2col3x3(src, dst, B, H, W, C, flip)
+
+    torch._dynamo.reset()
+    net_states._reset_state_for_tests()
+    initialize_pfeife(device="cpu")
+    torch.manual_seed(0)
+    model = Convs(*channels, k)
+    ref = copy.deepcopy(model)
+    runner = PartialRunner(PipeOption(device_cnt=2, batch_cnt=2, batch_size=2, split_points=["c2"], mixed_precision=mixed,
+                                      optimizer=dict(type="sgd", lr=0.0)), kernels=Table("cpu"))
+    cmodel = torch.compile(model, backend=partial_compiler)
+
+    def fn(x):
+        loss = cmodel(x).float().square().mean()
+        loss.backward()
+        return loss.detach()
+
+    runner.set_exec_fn(fn)
+    x = torch.randn(4, channels[0], H, W, generator=torch.Generator().manual_seed(1))
+    for _ in range(2):
+        losses = runner.step(x)
+        want = []
+        ref.zero_grad()
+        for i in (0, 2):
+            loss = ref(x[i:i + 2]).square().mean()
+            loss.backward()
+            want.append(float(loss.detach()))
+        tol = 1e-5 if mixed is None else 2e-2
+        for a, b in zip(losses, want):
+            assert abs(float(a) - b) <= tol * b
+        for (n, p), (_, q) in zip(model.named_parameters(), ref.named_parameters()):
+            assert (p.grad - q.grad).norm() <= tol * q.grad.norm(), n
+    one = wide or wide is None
+    assert (1 in calls) == one and (0 in calls) == (wide is not None or mixed is None)
