@@ -371,6 +371,15 @@ int pf_cross_entropy_fwd(const void* logits, int l_dtype, const int64_t* targets
 int pf_cross_entropy_bwd(const void* logits, int l_dtype, const int64_t* targets, const float* row_lse,
                          const float* dloss, const float* n_valid, void* dlogits, int dl_dtype, int64_t rows,
                          int64_t classes, int64_t ignore_index, void* stream);
+/* The same for rows in whole groups of `group` that are followed by `gap` rows which take no part: logits is
+ * [rows / group, group + gap, classes], targets / row_loss / row_lse have the `rows` rows alone; dlogits is laid out
+ * like logits and the rows in its gaps are written as zeros. */
+int pf_cross_entropy_gap_fwd(const void* logits, int l_dtype, const int64_t* targets, float* row_loss,
+                             float* row_lse, float* loss, int64_t rows, int64_t classes, int64_t ignore_index,
+                             int64_t group, int64_t gap, void* stream);
+int pf_cross_entropy_gap_bwd(const void* logits, int l_dtype, const int64_t* targets, const float* row_lse,
+                             const float* dloss, const float* n_valid, void* dlogits, int dl_dtype, int64_t rows,
+                             int64_t classes, int64_t ignore_index, int64_t group, int64_t gap, void* stream);
 /* Mean squared error (F.mse_loss, bench_models/models/train_sdxl.py:1422-1424):
  * loss[0] = mean((a-b)^2) computed in fp32; partial: fp32 [pf_reduce_workspace(n)]. */
 int64_t pf_reduce_workspace(int64_t n);

@@ -63,6 +63,13 @@ def _flat(t, n):
     return _strided(t, (n,), (1,))
 
 
+def _gap_rows(t, rows, classes, group, gap):
+    """[groups, group + gap, classes] over t (group 0: one group of all rows)."""
+    group = group or rows
+    n = rows // group if group else 1
+    return torch.as_strided(t, (n, group + gap, classes), ((group + gap) * classes, classes, 1))
+
+
 def _rows(t, rows, cols, ld):
     return _strided(t, (rows, cols), (ld, 1))
 
@@ -351,9 +358,9 @@ class OracleKernels:
 
         return launch
 
-    def cross_entropy_fwd(self, logits, targets, row_loss, row_lse, loss, rows, classes, ignore_index):
+    def cross_entropy_fwd(self, logits, targets, row_loss, row_lse, loss, rows, classes, ignore_index, group=0, gap=0):
         def launch(stream=None):
-            L = _rows(logits, rows, classes, classes).float()
+            L = _gap_rows(logits, rows, classes, group, gap)[:, :group or rows].reshape(rows, classes).float()
             t = _flat(targets, rows)
             lse = torch.logsumexp(L, dim=1)
             valid = t != ignore_index
@@ -368,9 +375,9 @@ class OracleKernels:
 
         return launch
 
-    def cross_entropy_bwd(self, logits, targets, row_lse, dloss, loss, dlogits, rows, classes, ignore_index):
+    def cross_entropy_bwd(self, logits, targets, row_lse, dloss, loss, dlogits, rows, classes, ignore_index, group=0, gap=0):
         def launch(stream=None):
-            L = _rows(logits, rows, classes, classes).float()
+            L = _gap_rows(logits, rows, classes, group, gap)[:, :group or rows].reshape(rows, classes).float()
             t = _flat(targets, rows)
             lse = _flat(row_lse, rows).float()
             g = (1.0 if dloss is None else _flat(dloss, 1).float()[0]) / _flat(loss, 2)[1]
@@ -379,7 +386,9 @@ class OracleKernels:
             tt = torch.where(valid, t, torch.zeros_like(t))
             sm.scatter_add_(1, tt[:, None], -torch.ones(rows, 1, dtype=sm.dtype, device=sm.device))
             sm = sm * g * valid[:, None].float()
-            _rows(dlogits, rows, classes, classes).copy_(sm.to(dlogits.dtype))
+            out = _gap_rows(dlogits, rows, classes, group, gap)
+            out[:, :group or rows].copy_(sm.to(dlogits.dtype).view(-1, group or rows, classes))
+            out[:, group or rows:].zero_()
 
         return launch
 

@@ -1955,6 +1955,29 @@ def lower_group_norm(L, node):
     return outv
 
 
+def _rows_in_place(L, node, x, out):
+    """(group, gap) when the reshape `node` of x = whole[:, :-gap] into rows feeds cross entropy alone: a language model's
+    logits without each sequence's last positions.  The loss kernels read such rows where they lie, and backward write
+    the gradient of the whole; any other slice, and any other reader, takes a copy of the rows."""
+    if x.kind != "part" or x.buf.dim() != 3 or x.buf.numel() == 0 or tuple(out.shape) != (x.shape[0] * x.shape[1], x.shape[2]):
+        return None
+    whole = x.base.buf
+    if whole.dim() != 3 or not whole.is_contiguous() or whole.data_ptr() != x.buf.data_ptr() \
+            or whole.stride() != x.buf.stride() or (whole.shape[0], whole.shape[2]) != (x.shape[0], x.shape[2]):
+        return None
+
+    def loss(n):
+        return n.op == "call_function" and n.target is F.cross_entropy
+
+    def same(n):     # x.float() that makes no copy, see lower_float
+        return n.op == "call_method" and n.target == "float" and (L.mixed or x.dtype == torch.float32) and n.users and \
+            all(loss(u) and u.args and u.args[0] is n for u in n.users)
+
+    if not node.users or not all(loss(u) and u.args and u.args[0] is node or same(u) for u in node.users):
+        return None
+    return x.shape[1], whole.shape[1] - x.shape[1]
+
+
 def _view_handler(fn_of_node):
     """Builds a handler for an op that is a pure view of its first argument."""
 
@@ -1965,6 +1988,11 @@ def _view_handler(fn_of_node):
         fn = fn_of_node(L, node)
         out = fn(x.buf)
         if out.untyped_storage().data_ptr() != x.buf.untyped_storage().data_ptr():
+            gap_rows = _rows_in_place(L, node, x, out)
+            if gap_rows is not None:
+                outv = Val(x.buf, req_grad=x.req_grad, kind="view", base=x, view_fn=lambda t: t)
+                outv.gap_rows = gap_rows
+                return outv
             # the op had to copy (reshape of a non-viewable layout): materialise with the copy kernel
             shape = tuple(out.shape)
             dense = L.alloc(x.shape, x.dtype)
@@ -2333,6 +2361,12 @@ def lower_pad(L, node):
     return Val(out, req_grad=False)
 
 
+def _region_of(val):
+    while val.kind == "view":
+        val = val.base
+    return val
+
+
 def lower_cross_entropy(L, node):
     logits = L.arg(node.args[0])
     target = L.arg(node.args[1])
@@ -2341,16 +2375,18 @@ def lower_cross_entropy(L, node):
     ignore_index = int(node.kwargs.get("ignore_index", -100))
     if node.kwargs.get("reduction", "mean") != "mean":
         raise Unsupported("cross entropy with reduction other than mean")
-    if logits.buf.dim() != 2 or not logits.buf.is_contiguous() or target.dtype != torch.int64:
+    group, gap = logits.gap_rows or (0, 0)
+    if not gap and (logits.buf.dim() != 2 or not logits.buf.is_contiguous()) or target.dtype != torch.int64:
         raise Unsupported("cross entropy expects contiguous [rows, classes] logits and int64 targets")
-    rows, classes = logits.shape
+    classes = logits.shape[-1]
+    rows = logits.buf.numel() // classes if gap else logits.shape[0]
     tgt = target.buf if target.buf.is_contiguous() else None
     if tgt is None:
         raise Unsupported("non-contiguous cross entropy targets")
     row_loss = L.alloc((rows,), torch.float32)
     row_lse = L.alloc((rows,), torch.float32)
     loss2 = L.alloc((2,), torch.float32)
-    L.emit(L.kernels.cross_entropy_fwd(logits.buf, tgt, row_loss, row_lse, loss2, rows, classes, ignore_index))
+    L.emit(L.kernels.cross_entropy_fwd(logits.buf, tgt, row_loss, row_lse, loss2, rows, classes, ignore_index, group, gap))
     outv = Val(loss2[0], req_grad=logits.req_grad)
 
     def bwd(B):
@@ -2359,6 +2395,19 @@ def lower_cross_entropy(L, node):
             return
         if g.dtype != torch.float32:
             raise Unsupported("loss gradient must be fp32")
+        if gap:
+            part = _region_of(logits)
+            whole, root = part.base, _region_of(part.base)
+            alone = root.kind == "base" and root.param is None and root.grad is None
+            dst, prev = B.grad_target(whole if alone else logits)
+            if alone and prev is None and dst.is_contiguous() and dst.dtype == logits.dtype:
+                B.emit(B.k.cross_entropy_bwd(logits.buf, tgt, row_lse, g, loss2, dst, rows, classes, ignore_index, group, gap))
+            else:
+                tmp = B.temp(whole.shape, logits.dtype)
+                B.emit(B.k.cross_entropy_bwd(logits.buf, tgt, row_lse, g, loss2, tmp, rows, classes, ignore_index, group, gap))
+                B.merge(tmp if alone else part.view_fn(tmp), dst, prev)
+            B.commit(whole if alone else logits, dst)
+            return
         dst, prev = B.grad_target(logits)
         if prev is None and dst.is_contiguous() and dst.dtype == logits.dtype:
             B.emit(B.k.cross_entropy_bwd(logits.buf, tgt, row_lse, g, loss2, dst, rows, classes, ignore_index))
@@ -2379,6 +2428,10 @@ def lower_float(L, node):
     """x.float() / x.to(float32): under the mixed-precision policy a no-op for fp32 values,
     a cast kernel otherwise."""
     x = L.arg(node.args[0])
+    if x.gap_rows is not None:
+        outv = Val(x.buf, req_grad=x.req_grad, kind="view", base=x, view_fn=lambda t: t)
+        outv.gap_rows = x.gap_rows
+        return outv
     if L.mixed and node.users and all(u.op == "call_function" and u.target is F.cross_entropy for u in node.users):
         # the loss kernels read 16-bit logits and do their arithmetic in fp32: no fp32 copy of the logits
         return Val(x.buf, req_grad=x.req_grad, kind="view", base=x, view_fn=lambda t: t)

@@ -71,7 +71,7 @@ class Val:
     """A tensor value of a stage program."""
 
     __slots__ = ("buf", "req_grad", "kind", "base", "view_fn", "param", "grad", "grad_shared", "written",
-                 "partial_only", "tiled", "name", "preact", "grad_is_preact", "pending_act", "boundary", "lp_grad")
+                 "partial_only", "tiled", "name", "preact", "grad_is_preact", "pending_act", "boundary", "lp_grad", "gap_rows")
 
     def __init__(self, buf, req_grad=False, kind="base", base=None, view_fn=None, param=None, name=""):
         self.buf = buf
@@ -90,6 +90,7 @@ class Val:
         self.grad_is_preact = False
         self.lp_grad = None       # dict(colsum, cols) when backward reads this value's gradient as a 16-bit matrix
         self.boundary = False     # stage input produced by another stage: its gradient outlives the backward job
+        self.gap_rows = None      # (group, gap) when this is a matrix of rows read in place, see lowering._rows_in_place
         self.pending_act = None   # (act, source value) when this is the not-yet-applied gate of a gated MLP
 
     @property

@@ -128,6 +128,8 @@ _SIGNATURES = {
     "pf_softmax_bwd": [_P, _L, _P, _I, _L, _P, _I, _L, _L, _L, _F, _P],
     "pf_cross_entropy_fwd": [_P, _I, _P, _P, _P, _P, _L, _L, _L, _P],
     "pf_cross_entropy_bwd": [_P, _I, _P, _P, _P, _P, _P, _I, _L, _L, _L, _P],
+    "pf_cross_entropy_gap_fwd": [_P, _I, _P, _P, _P, _P, _L, _L, _L, _L, _L, _P],
+    "pf_cross_entropy_gap_bwd": [_P, _I, _P, _P, _P, _P, _P, _I, _L, _L, _L, _L, _L, _P],
     "pf_mse_fwd": [_P, _I, _P, _I, _P, _P, _L, _P],
     "pf_mse_bwd": [_P, _I, _P, _I, _P, _P, _I, _L, _P],
     "pf_sum_fwd": [_P, _I, _P, _P, _L, _P],
@@ -617,17 +619,20 @@ class HipKernels:
         args = (_ptr(dp), ld_dp, _ptr(p), _dt(p), ld_p, _ptr(ds), _dt(ds), ld_ds, rows, cols, scale)
         return self._prep("pf_softmax_bwd", args, (dp, p, ds), rows * cols * (_es(dp) + _es(p) + _es(ds)))
 
-    def cross_entropy_fwd(self, logits, targets, row_loss, row_lse, loss, rows, classes, ignore_index):
+    def cross_entropy_fwd(self, logits, targets, row_loss, row_lse, loss, rows, classes, ignore_index, group=0, gap=0):
+        """gap: rows that follow every `group` rows of the logits and take no part."""
         args = (_ptr(logits), _dt(logits), _ptr(targets), _ptr(row_loss), _ptr(row_lse), _ptr(loss), rows, classes,
                 ignore_index)
-        return self._prep("pf_cross_entropy_fwd", args, (logits, targets, row_loss, row_lse, loss), rows * classes * _es(logits))
+        return self._prep("pf_cross_entropy_gap_fwd" if gap else "pf_cross_entropy_fwd", args + ((group, gap) if gap else ()),
+                          (logits, targets, row_loss, row_lse, loss), rows * classes * _es(logits))
 
-    def cross_entropy_bwd(self, logits, targets, row_lse, dloss, loss, dlogits, rows, classes, ignore_index):
+    def cross_entropy_bwd(self, logits, targets, row_lse, dloss, loss, dlogits, rows, classes, ignore_index, group=0, gap=0):
+        """gap: dlogits has the gaps of the logits as well, and zeros are written there."""
         n_valid = loss.data_ptr() + 4
         args = (_ptr(logits), _dt(logits), _ptr(targets), _ptr(row_lse), _ptr(dloss), n_valid, _ptr(dlogits),
                 _dt(dlogits), rows, classes, ignore_index)
-        return self._prep("pf_cross_entropy_bwd", args, (logits, targets, row_lse, dloss, loss, dlogits),
-                          rows * classes * (_es(logits) + _es(dlogits)))
+        return self._prep("pf_cross_entropy_gap_bwd" if gap else "pf_cross_entropy_bwd", args + ((group, gap) if gap else ()),
+                          (logits, targets, row_lse, dloss, loss, dlogits), rows * classes * (_es(logits) + _es(dlogits)))
 
     def mse_fwd(self, a, b, partial, loss, n):
         args = (_ptr(a), _dt(a), _ptr(b), _dt(b), _ptr(partial), _ptr(loss), n)
