@@ -30,7 +30,7 @@ constexpr float O_LO = 2048.f;   // scale of what rounding O lost: at most as la
 struct AttnArgs {
   const uint16_t* q; const uint16_t* k; const uint16_t* v; const uint16_t* o; const uint16_t* d_o;
   uint16_t* out; uint16_t* o_lo; uint16_t* dq; uint16_t* dk; uint16_t* dv;
-  float* lse; const float* delta;
+  float* lse; float* delta;
   int64_t q_sb, q_sh, q_st, k_sb, k_sh, k_st, v_sb, v_sh, v_st, o_sb, o_sh, o_st;
   int64_t do_sb, do_sh, do_st, dq_sb, dq_sh, dq_st, dk_sb, dk_sh, dk_st, dv_sb, dv_sh, dv_st;
   int B, H, Tq, Tk, hd, causal;
@@ -72,6 +72,21 @@ __device__ __forceinline__ int acc_row(int r, int lane) { return 8 * (r >> 2) + 
 __device__ __forceinline__ uint4 load_row8(const uint16_t* base, int64_t st, int t, int T, int h0, int hd) {
   if (t < T && h0 < hd) return *(const uint4*)(base + (int64_t)t * st + h0);
   return make_uint4(0, 0, 0, 0);
+}
+
+template <int DT>
+__device__ __forceinline__ void unpack8(const uint4& r, float (&v)[8]) {
+  const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if constexpr (DT == PF_F16) {
+      v[2 * k] = pf_f16_bits_to_f32((uint16_t)(w[k] & 0xffffu));
+      v[2 * k + 1] = pf_f16_bits_to_f32((uint16_t)(w[k] >> 16));
+    } else {
+      v[2 * k] = __uint_as_float(w[k] << 16);
+      v[2 * k + 1] = __uint_as_float(w[k] & 0xffff0000u);
+    }
+  }
 }
 
 // One [ROWS tokens][HD] tile in flight: NV 16-byte vectors per thread, loaded from global into
@@ -293,43 +308,14 @@ __global__ __launch_bounds__(256, HD <= 64 ? 3 : 2) void attn_fwd_kernel(const A
   }
 }
 
-// delta[b,h,q] = sum_hd dO * O : 8 lanes per row (16-byte loads), 8 rows per wavefront.  With o_lo, from O to twice its
-// digits: where one key has most of a query's weight, dP - delta is a small difference, and the rounding of O is the
-// largest error in it.
-__global__ __launch_bounds__(256) void attn_delta_kernel(const AttnArgs a, float* delta) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t rows = (int64_t)a.B * a.H * a.Tq;
-  const int64_t row = ((int64_t)blockIdx.x * 4 + wave) * 8 + (lane >> 3);
-  const bool bf = (a.causal & 0x100) != 0;
-  float s = 0.f;
-  if (row < rows) {
-    const int q = (int)(row % a.Tq);
-    const int bh = (int)(row / a.Tq), b = bh / a.H, h = bh % a.H;
-    const uint16_t* O = a.o + b * a.o_sb + h * a.o_sh + (int64_t)q * a.o_st;
-    const uint16_t* D = a.d_o + b * a.do_sb + h * a.do_sh + (int64_t)q * a.do_st;
-    for (int c = (lane & 7) * 8; c < a.hd; c += 64) {
-      float x[8], y[8];
-      if (bf) { Vec8<PF_BF16>::load(O, c, x); Vec8<PF_BF16>::load(D, c, y); }
-      else { Vec8<PF_F16>::load(O, c, x); Vec8<PF_F16>::load(D, c, y); }
-      if (a.o_lo != nullptr) {
-        float z[8];
-        if (bf) Vec8<PF_BF16>::load(a.o_lo + (O - a.o), c, z);
-        else Vec8<PF_F16>::load(a.o_lo + (O - a.o), c, z);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) x[k] += z[k] * (1.f / O_LO);
-      }
-#pragma unroll
-      for (int k = 0; k < 8; ++k) s += x[k] * y[k];
-    }
-  }
-  s += __shfl_xor(s, 1, 64);
-  s += __shfl_xor(s, 2, 64);
-  s += __shfl_xor(s, 4, 64);
-  if (row < rows && (lane & 7) == 0) delta[row] = s;
-}
-
 // ---------------------------------------------------------------------------------
 // dQ: same tiling as forward (column = query); dQ^T[hd][q] += K^T[hd][kv] dS^T[kv][q]
+//
+// It holds its queries' rows of dO and so also forms delta[b,h,q] = sum_hd dO * O, for itself and for the dK/dV kernel that is launched
+// after it; a kernel of its own read dO once more (7.2 us of 43 + 7 at 4096 x 20 heads of 64, 41 us beside another stage's work at
+// 8192 x 32 heads; a step of 30 transformer blocks 50.1 -> 49.3 ms, a 1B decoder's 189.2 -> 188.5).  With o_lo, from O to
+// twice its digits: where one key has most of a query's weight, dP - delta is a small difference, and the rounding of O is the
+// largest error in it.
 // ---------------------------------------------------------------------------------
 template <int DT, int HD, bool FAR = false>
 __global__ __launch_bounds__(256, HD <= 96 ? 2 : 1) void attn_dq_kernel(const AttnArgs a) {
@@ -358,7 +344,29 @@ __global__ __launch_bounds__(256, HD <= 96 ? 2 : 1) void attn_dq_kernel(const At
   const bool qok = qi < a.Tq;
   // a query row past the end keeps lse = +inf so that its probabilities are exactly zero
   const float lse2 = qok ? a.lse[(int64_t)bh * a.Tq + qi] * LOG2E : INFINITY;
-  const float dlt = qok ? a.delta[(int64_t)bh * a.Tq + qi] : 0.f;
+  float dlt = 0.f;
+  {
+    const uint16_t* O = a.o + b * a.o_sb + h * a.o_sh;
+    uint4 of[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) of[c] = load_row8(O, a.o_st, qi, a.Tq, c * 16 + (lane >> 5) * 8, a.hd);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      float x[8], y[8];
+      unpack8<DT>(of[c], x);
+      unpack8<DT>(dof[c], y);
+      if (a.o_lo != nullptr) {
+        float z[8];
+        unpack8<DT>(load_row8(a.o_lo + (O - a.o), a.o_st, qi, a.Tq, c * 16 + (lane >> 5) * 8, a.hd), z);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) x[k] += z[k] * (1.f / O_LO);
+      }
+#pragma unroll
+      for (int k = 0; k < 8; ++k) dlt += x[k] * y[k];
+    }
+    dlt += __shfl_xor(dlt, 32, 64);   // (the other half of the row's chunks)
+    if (qok && (lane >> 5) == 0) a.delta[(int64_t)bh * a.Tq + qi] = dlt;
+  }
 
   float16_t acc[NO];
 #pragma unroll
@@ -598,20 +606,6 @@ __global__ __launch_bounds__(256, SPLITQ || HD > 96 ? 1 : 2) void attn_dkv_kerne
 // so no transposed copy is made.
 // =================================================================================
 constexpr int SHORT_T = 288;   // 2 operands x 288 rows x (96 + 8) x 2 bytes = 117 KB of the 160 KB
-template <int DT>
-__device__ __forceinline__ void unpack8(const uint4& r, float (&v)[8]) {
-  const uint32_t w[4] = {r.x, r.y, r.z, r.w};
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    if constexpr (DT == PF_F16) {
-      v[2 * k] = pf_f16_bits_to_f32((uint16_t)(w[k] & 0xffffu));
-      v[2 * k + 1] = pf_f16_bits_to_f32((uint16_t)(w[k] >> 16));
-    } else {
-      v[2 * k] = __uint_as_float(w[k] << 16);
-      v[2 * k + 1] = __uint_as_float(w[k] & 0xffff0000u);
-    }
-  }
-}
 
 // One head's [T][hd] operand for 16-byte loads without a branch: rows past T and chunks past hd get an offset out of the
 // buffer's range, which reads zeros.  (T * st * 2 bytes are below 2 GiB, see short_ok.)
@@ -1447,8 +1441,6 @@ extern "C" int pf_attention_bwd(const pf_attn_desc* d, void* stream) {
              "pf_attention_bwd: gradient operands must be 8-byte aligned with strides that are multiples of 4");
   AttnArgs a = make_args(d);
   hipStream_t st = (hipStream_t)stream;
-  AttnArgs ad = a;
-  if (d->dtype == PF_BF16) ad.causal |= 0x100;  // dtype flag for the delta kernel
   const dim3 gq((unsigned)((d->Tq + 127) / 128), (unsigned)(d->B * d->H));
   const dim3 gk((unsigned)((d->Tk + 127) / 128), (unsigned)(d->B * d->H));
   if (short_ok(d, true)) {
@@ -1485,11 +1477,12 @@ extern "C" int pf_attention_bwd(const pf_attn_desc* d, void* stream) {
     PF_CHECK_LAUNCH("pf_attention_bwd");
     return PF_OK;
   }
-  const int64_t rows = (int64_t)d->B * d->H * d->Tq;
-  hipLaunchKernelGGL(attn_delta_kernel, dim3((unsigned)((rows + 31) / 32)), dim3(256), 0, st, ad, d->delta);
+  const bool near = rows_near(d, true, 128);
+  // dQ first: it also leaves delta for the dK/dV kernel
+  if (near) PF_ATTN_DISPATCH(attn_dq_kernel, gq, st, a, d->dtype, d->hd, false);
+  else PF_ATTN_DISPATCH(attn_dq_kernel, gq, st, a, d->dtype, d->hd, true);
   // few keys, many queries (cross attention to a short context): split each key tile's query sweep
   // over the four wavefronts of a workgroup
-  const bool near = rows_near(d, true, 128);
   if (near && (int64_t)gk.x * gk.y < 200 && d->Tq >= 256 && d->hd <= 96) {   // (two 128-row tiles of more do not fit)
     const dim3 gs((unsigned)((d->Tk + 31) / 32), (unsigned)(d->B * d->H));
     if (d->dtype == PF_F16) {
@@ -1504,8 +1497,6 @@ extern "C" int pf_attention_bwd(const pf_attn_desc* d, void* stream) {
   } else {
     PF_ATTN_DISPATCH(attn_dkv_kernel, gk, st, a, d->dtype, d->hd, false, true);
   }
-  if (near) PF_ATTN_DISPATCH(attn_dq_kernel, gq, st, a, d->dtype, d->hd, false);
-  else PF_ATTN_DISPATCH(attn_dq_kernel, gq, st, a, d->dtype, d->hd, true);
   PF_CHECK_LAUNCH("pf_attention_bwd");
   return PF_OK;
 }

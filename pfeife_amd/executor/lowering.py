@@ -1678,7 +1678,7 @@ def _lower_sdpa_fused(L, vals, tensors, dims, scale, causal, req):
     Ov = O.permute(0, 2, 1, 3)
     # (fp32 keeps a row's maximum and its sum apart)
     lse = L.alloc((Bn, H, Tq if L.mixed else 2 * Tq), torch.float32)
-    # (wide heads keep O to twice its digits for the backward pass, see attn_delta_kernel)
+    # (wide heads keep O to twice its digits for the backward pass, see attn_dq_kernel)
     o_lo = L.alloc((Bn, Tq, H, hd), cd).permute(0, 2, 1, 3) if L.mixed and req and hd > L.kernels.O_LO_HEAD_DIM else None
     L.emit(L.kernels.attention_fwd(qt, kt, vt, Ov, lse, scale, causal, o_lo))
     outv = Val(Ov, req_grad=req)
