@@ -1190,6 +1190,13 @@ def _act_of_node(n):
     return None
 
 
+def _factor_beside(product, node):
+    """The other operand of a tensor*tensor product that `node` is an operand of, or None."""
+    if product is None or not _is(product, operator.mul, torch.mul) or not all(isinstance(a, torch.fx.Node) for a in product.args[:2]):
+        return None
+    return next((a for a in product.args[:2] if a is not node), None)
+
+
 def _is_add_node(n):
     return n.op == "call_function" and n.target in (operator.add, operator.iadd, torch.add)
 
@@ -1246,9 +1253,12 @@ def _joins_at(L, node):
         u = users[0]
         if _is(u, F.scaled_dot_product_attention, torch._C._nn.scaled_dot_product_attention):
             return u if node in u.args[:3] else None
-        gate = L.sole_user(u) if _act_of_node(u) is not None else u
-        if gate is not None and _is(gate, operator.mul, torch.mul) and all(isinstance(a, torch.fx.Node) for a in gate.args[:2]):
-            return gate
+        act = _act_of_node(u)
+        gate = L.sole_user(u) if act is not None else u
+        other = _factor_beside(gate, u if act is not None else node)
+        if other is not None:
+            # (a ReLU, and one of two activations, is not the product's gate and has a kernel of its own, for dense operands)
+            return gate if act is None or act != ACT_RELU and _act_of_node(other) is None else None
         if not ((u.op == "call_method" and u.target in ("view", "reshape", "transpose", "permute", "unflatten"))
                 or _is(u, torch.transpose, torch.permute, torch.reshape)):
             return None
@@ -2563,11 +2573,12 @@ def _lower_glu(L, gate, up, act):
 
 def lower_act_maybe_gate(L, node):
     """silu/gelu whose single user is a tensor*tensor product is the gate of a gated MLP:
-    defer it to the product so that one kernel computes act(gate) * up."""
+    defer it to the product so that one kernel computes act(gate) * up.  The kernel has one gate: of two activations
+    the second is computed here, and one that is multiplied by itself is no gate."""
     user = L.sole_user(node)
     x = L.arg(node.args[0])
-    if (user is not None and user.op == "call_function" and user.target in (operator.mul, torch.mul)
-            and all(isinstance(a, torch.fx.Node) for a in user.args[:2])):
+    other = _factor_beside(user, node)
+    if other is not None and not (other in L.env and isinstance(L.env[other], Val) and L.env[other].pending_act is not None):
         v = Val(x.buf, req_grad=x.req_grad, kind="view", base=x, view_fn=lambda t: t)
         v.pending_act = (_act_of_node(node), x)
         return v
