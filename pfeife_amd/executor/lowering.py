@@ -1241,12 +1241,20 @@ def _input_gradient(B, x, dy, wb, K, kw2, alone):
 
 
 def _joins_at(L, node):
-    """The attention or gated product that a linear layer's result goes to through nothing but views and rotary embedding, or None."""
+    """The attention or gated product that a linear layer's result goes to through nothing but views and rotary embedding, or None.  On
+    the way the result has to do as a range of a wider matrix's columns as well: what is a view of it apart is one of such a
+    range, and the gated product gets a matrix."""
+    lead, size = tuple(L.arg(node.args[0]).shape[:-1]), L.env[_kw(node, 1, "weight")].shape[0]
+    apart = torch.empty(lead + (size,), device="meta")
+    part = torch.empty(lead + (2 * size,), device="meta")[..., :size]      # (any wider matrix)
     while True:
         users = list(node.users)
         root = next((r for r, p in L.patterns.items() if p[0] is node), None)
         if root is not None and all(u in L.pattern_skip for u in users):
-            node = root
+            if part.dim() != 4:
+                return None
+            node, apart = root, torch.empty([part.shape[i] for i in (0, 2, 1, 3)], device="meta").permute(0, 2, 1, 3)
+            part = apart      # (written anew, see lower_rope)
             continue
         if len(users) != 1:
             return None
@@ -1258,9 +1266,20 @@ def _joins_at(L, node):
         other = _factor_beside(gate, u if act is not None else node)
         if other is not None:
             # (a ReLU, and one of two activations, is not the product's gate and has a kernel of its own, for dense operands)
-            return gate if act is None or act != ACT_RELU and _act_of_node(other) is None else None
-        if not ((u.op == "call_method" and u.target in ("view", "reshape", "transpose", "permute", "unflatten"))
+            gated = act is None or act != ACT_RELU and _act_of_node(other) is None
+            return gate if gated and (as_matrix(part) is not None or as_matrix(apart) is None) else None
+        if not ((u.op == "call_method" and u.target in ("view", "reshape", "transpose", "permute"))
                 or _is(u, torch.transpose, torch.permute, torch.reshape)):
+            return None
+        if any(isinstance(a, torch.fx.Node) for a in u.args[1:]):
+            return None
+        view = L._handler(u).view_of(L, u)
+        try:
+            nodes = [(t, view(t)) for t in (apart, part)]
+        except RuntimeError:
+            return None
+        (apart, copied), (part, copies) = [(new, new.untyped_storage()._cdata != t.untyped_storage()._cdata) for t, new in nodes]
+        if copies and not copied:
             return None
         node = u
 
@@ -2020,6 +2039,7 @@ def _view_handler(fn_of_node):
             return outv
         return Val(out, req_grad=x.req_grad, kind="view", base=x, view_fn=fn)
 
+    handler.view_of = fn_of_node
     return handler
 
 
