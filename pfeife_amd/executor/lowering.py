@@ -1866,9 +1866,11 @@ def _lower_conv_same(L, x, w, b, k):
             L.copy(win, cols.view(Bn, H, W, 3, 3, C))
         w_cd = L.params.shadow_perm(w.buf, cd, (0, 2, 3, 1)).reshape(O, Kc)
     b_cd = None if b is None else L.params.shadow(b.buf, cd)
-    # the weight with the output channels last, [C, taps * O]: what the input gradient multiplies by
+    # the weight with the output channels last, [C, taps * O]: what the input gradient multiplies by (where it and the gradient's windows
+    # are operands that a 16-bit product takes: with more channels out than in they may not be where the forward pass' are)
     w_t = None
-    if x.req_grad and w.buf.is_contiguous() and M >= 256 and whole(O) and whole(C):
+    fits = xn.element_size() == 4 or (max(M, C) + 256) * k * k * O * xn.element_size() < MAX_BYTES
+    if x.req_grad and w.buf.is_contiguous() and M >= 256 and whole(O) and whole(C) and fits:
         w_t = L.params.shadow_t(w.buf.view(O, Kc), cd).view(C, k * k * O)
     out = L.alloc((Bn, H, W, O), cd)
     L.emit(L.kernels.gemm(cols, w_cd, out, M=M, N=O, K=Kc, lda=Kc, ldb=Kc, ldc=O, bias=b_cd,

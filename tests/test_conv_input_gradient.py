@@ -1,5 +1,6 @@
 """3x3 and 1x1 "same" convolutions: the input gradient as one product with the taps in reverse (kernel table double on the CPU)."""
 import copy
+import functools
 
 import pytest
 import torch
@@ -71,3 +72,58 @@ def test_input_gradients(channels, k, H, W, wide, mixed):
             assert (p.grad - q.grad).norm() <= tol * q.grad.norm(), n
     one = wide or wide is None
     assert (1 in calls) == one and (0 in calls) == (wide is not None or mixed is None)
+
+
+class Wider(nn.Module):
+    def __init__(self):
+        super().__init__()
+        self.c0, self.c1, self.c2 = nn.Conv2d(8, 16, 1), nn.Conv2d(16, 48, 3, padding=1), nn.Conv2d(48, 8, 1)
+
+    def forward(self, x):
+        return self.c2(self.c1(self.c0(x)))
+
+
+@pytest.mark.parametrize("limit,one", [(300_000, False), (600_000, True)])
+def test_windows_of_the_gradient_fit_an_operand(limit, one, monkeypatch):
+    """More channels out than in: the forward windows may fit the size a 16-bit operand can have and the gradient's may not, which then takes the
+    product with the windows as its result.  The limit is lowered, and held to as pf_gemm holds to it."""
+    from pfeife_amd.executor import lowering, merge
+    from pfeife_amd.mp import PartialRunner, initialize_pfeife, partial_compiler
+
+    monkeypatch.setattr(lowering, "MAX_BYTES", limit)
+    monkeypatch.setattr(merge, "MAX_BYTES", limit)
+    gemm, calls = OracleKernels.gemm, []
+
+    @functools.wraps(gemm)
+    def checked(self, a, b, c, **kw):
+        for rows, ld in ((kw["K"] if kw.get("a_trans") else kw["M"], kw["lda"]), (kw["K"] if kw.get("b_trans") else kw["N"], kw["ldb"])):
+            assert (rows + 256) * ld * 2 < limit
+        calls.append((kw["N"], kw["K"]))
+        return gemm(self, a, b, c, **kw)
+
+    monkeypatch.setattr(OracleKernels, "gemm", checked)
+    torch._dynamo.reset()
+    net_states._reset_state_for_tests()
+    initialize_pfeife(device="cpu")
+    torch.manual_seed(0)
+    model = Wider()
+    ref = copy.deepcopy(model)
+    runner = PartialRunner(PipeOption(device_cnt=2, batch_cnt=2, batch_size=2, split_points=["c2"], mixed_precision="bf16",
+                                      optimizer=dict(type="sgd", lr=0.0)), kernels=OracleKernels("cpu"))
+    cmodel = torch.compile(model, backend=partial_compiler)
+
+    def fn(x):
+        loss = cmodel(x).float().square().mean()
+        loss.backward()
+        return loss.detach()
+
+    runner.set_exec_fn(fn)
+    x = torch.randn(4, 8, 13, 11, generator=torch.Generator().manual_seed(1))
+    for _ in range(2):
+        runner.step(x)
+        ref.zero_grad()
+        for i in (0, 2):
+            ref(x[i:i + 2]).square().mean().backward()
+        for (n, p), (_, q) in zip(model.named_parameters(), ref.named_parameters()):
+            assert (p.grad - q.grad).norm() <= 2e-2 * q.grad.norm(), n      # (as above)
+    assert ((16, 9 * 48) in calls) == one and ((9 * 16, 48) in calls) != one
