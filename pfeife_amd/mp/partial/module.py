@@ -24,6 +24,7 @@ of the right shape so that user code can run through its loss once; like the
 reference's probe it contributes nothing to the gradients.
 """
 import threading
+import weakref
 from functools import partial
 from queue import SimpleQueue
 from typing import List
@@ -70,6 +71,26 @@ class _StepAborted(BaseException):
 
 
 _ABORT = object()
+_END = object()
+
+
+def _exec_loop(runner, bid, n, baton, train_queue, return_queue):
+    """Micro-batch `bid`'s thread.  Between its turns it holds the runner by a weak reference alone, and nothing of the last step: a
+    runner that is dropped goes away with its buffers, and the threads end."""
+    baton.switch(None, bid)
+    while True:
+        work = train_queue.get()
+        if work is _END:
+            return
+        return_queue.put(runner()._exec(*work))
+        del work
+        baton.switch(n + bid, bid)
+
+
+def _end_loops(baton, train_queues):
+    for bid, q in enumerate(train_queues):
+        q.put(_END)
+        baton.switch(bid, -1)
 
 
 class PartialRunner:
@@ -95,9 +116,11 @@ class PartialRunner:
         torch._dynamo.config.automatic_dynamic_shapes = False
         PartialModule.set_runner(self)
         for i in range(self.option.batch_cnt):
-            t = threading.Thread(target=self._exec_loop, args=(i,), daemon=True, name="pfeife-mb%d" % i)
+            t = threading.Thread(target=_exec_loop, daemon=True, name="pfeife-mb%d" % i,
+                                 args=(weakref.ref(self), i, self.option.batch_cnt, self._baton, self._train_queues[i], self._return_queues[i]))
             self._batch_threads.append(t)
             t.start()
+        weakref.finalize(self, _end_loops, self._baton, self._train_queues).atexit = False
 
     def set_exec_fn(self, exec_fn):
         self.exec_fn = exec_fn
@@ -256,21 +279,17 @@ class PartialRunner:
         """No-op, as in the reference (pfeife/mp/partial/module.py:179-181)."""
 
     # -- helpers --------------------------------------------------------------------
-    def _exec_loop(self, batch_idx):
-        q, stream = self._train_queues[batch_idx], self.worker.stream_obj
-        self._baton.switch(None, batch_idx)
-        args, kwargs = q.get()
-        while True:
-            try:
-                if stream is not None:
-                    torch.cuda.set_device(self.net_state.device)
-                    if torch.cuda.current_stream() != stream:    # user code shares the step's stream
-                        torch.cuda.set_stream(stream)
-                ret = self.exec_fn(*args, **kwargs)
-            except BaseException as e:  # surfaced on the thread that called step()
-                ret = _ExecError(e)
-            args = kwargs = None     # (not kept alive until the next step)
-            args, kwargs = self._hand_back(batch_idx, ret, q)
+    def _exec(self, args, kwargs):
+        """exec_fn on the thread of a micro-batch."""
+        stream = self.worker.stream_obj
+        try:
+            if stream is not None:
+                torch.cuda.set_device(self.net_state.device)
+                if torch.cuda.current_stream() != stream:    # user code shares the step's stream
+                    torch.cuda.set_stream(stream)
+            return self.exec_fn(*args, **kwargs)
+        except BaseException as e:  # surfaced on the thread that called step()
+            return _ExecError(e)
 
     def _probe_forward(self, args, kwargs):
         self._probing = True

@@ -59,7 +59,6 @@ class StageWorker:
     jobs = None                # (stage, micro-batch) -> StageJob; None: to be formed from the slots
 
     def __init__(self, runner, option, device, kernels=None):
-        self.runner = runner
         self.option = option
         self.device = torch.device(device)
         if kernels is None:
