@@ -37,7 +37,7 @@ enum pf_act { PF_ACT_NONE = 0, PF_ACT_GELU = 1, PF_ACT_GELU_TANH = 2, PF_ACT_SIL
 
 /* ---- library state ------------------------------------------------------- */
 
-/* ABI version of this header (bumped when a signature changes). */
+/* ABI version of this header (bumped when a signature or a structure changes). */
 int pf_version(void);
 /* Text of the last error raised on the calling host thread ("" if none). */
 const char* pf_last_error(void);

@@ -11,7 +11,7 @@
 
 int pf_norm_init_device();   // pf_norm.hip
 
-#define PF_ABI_VERSION 5
+#define PF_ABI_VERSION 6
 
 static thread_local char g_err[512] = "";
 
