@@ -1841,9 +1841,25 @@ def _grad_nhwc(B, g, dtype):
     return t
 
 
+def _windows_of_gradient(M, C, O, size):
+    """Whether a 3x3 convolution's input gradient multiplies the windows of the output gradient, [M, 9 O], or makes windows of
+    the input's, [M, 9 C], and adds them up.  A 16-bit operand has to stay below 2 GiB, which the forward windows say nothing about; and the more
+    channels go out than in, the more the first form reads and the deeper its sums are.  us, windows of the input's / of the output's, M x C -> O:
+    fp16 4096 x 1280 -> 1280 280 / 130, 16384 x 640 -> 1280 552 / 409, x 320 -> 1280 271 / 290, x 160 -> 640 129 / 90, x 64 -> 512 79 / 65,
+    x 64 -> 1024 93 / 160, 4096 x 8 -> 320 37 / 24, x 8 -> 1280 45 / 56; fp32 4096 x 320 -> 1280 286 / 259, x 64 -> 512 65 / 50, x 64 -> 1024 82 / 90,
+    16384 x 64 -> 512 137 / 196.  Of 210 such
+    products of 256 to 32768 pixels the first form is nowhere taken where it is the slower one; the second is where the first would be up to 1.3
+    times as fast (256 x 64 -> 1024)."""
+    windows = 9 * M * O * size
+    if size == 2 and (max(M, C) + 256) * 9 * O * size >= MAX_BYTES:
+        return False
+    return O <= 3 * C or windows <= (200e6 if O <= 4 * C or O <= min(768, 8 * C) else 80e6 if O <= 768 else 0)
+
+
 def _lower_conv_same(L, x, w, b, k):
     """1x1 or 3x3 stride-1 'same' convolution as one GEMM over channels-last rows
-    (3x3: the nine shifted windows of a zero-bordered copy are laid side by side first)."""
+    (3x3: the image's nine shifted windows are laid side by side first, straight from it where its pixels are whole 16-byte pieces,
+    else from a zero-bordered copy)."""
     cd = L.cd
     Bn, C, H, W = x.shape
     O = w.shape[0]
@@ -1866,11 +1882,9 @@ def _lower_conv_same(L, x, w, b, k):
             L.copy(win, cols.view(Bn, H, W, 3, 3, C))
         w_cd = L.params.shadow_perm(w.buf, cd, (0, 2, 3, 1)).reshape(O, Kc)
     b_cd = None if b is None else L.params.shadow(b.buf, cd)
-    # the weight with the output channels last, [C, taps * O]: what the input gradient multiplies by (where it and the gradient's windows
-    # are operands that a 16-bit product takes: with more channels out than in they may not be where the forward pass' are)
+    # the weight with the output channels last, [C, taps * O]: what the input gradient multiplies by
     w_t = None
-    fits = xn.element_size() == 4 or (max(M, C) + 256) * k * k * O * xn.element_size() < MAX_BYTES
-    if x.req_grad and w.buf.is_contiguous() and M >= 256 and whole(O) and whole(C) and fits:
+    if x.req_grad and w.buf.is_contiguous() and M >= 256 and whole(O) and whole(C) and (k == 1 or _windows_of_gradient(M, C, O, xn.element_size())):
         w_t = L.params.shadow_t(w.buf.view(O, Kc), cd).view(C, k * k * O)
     out = L.alloc((Bn, H, W, O), cd)
     L.emit(L.kernels.gemm(cols, w_cd, out, M=M, N=O, K=Kc, lda=Kc, ldb=Kc, ldc=O, bias=b_cd,

@@ -75,40 +75,34 @@ def test_input_gradients(channels, k, H, W, wide, mixed):
 
 
 class Wider(nn.Module):
-    def __init__(self):
+    def __init__(self, c=16, o=48):
         super().__init__()
-        self.c0, self.c1, self.c2 = nn.Conv2d(8, 16, 1), nn.Conv2d(16, 48, 3, padding=1), nn.Conv2d(48, 8, 1)
+        self.c0, self.c1, self.c2 = nn.Conv2d(8, c, 1), nn.Conv2d(c, o, 3, padding=1), nn.Conv2d(o, 8, 1)
 
     def forward(self, x):
         return self.c2(self.c1(self.c0(x)))
 
 
-@pytest.mark.parametrize("limit,one", [(300_000, False), (600_000, True)])
-def test_windows_of_the_gradient_fit_an_operand(limit, one, monkeypatch):
-    """More channels out than in: the forward windows may fit the size a 16-bit operand can have and the gradient's may not, which then takes the
-    product with the windows as its result.  The limit is lowered, and held to as pf_gemm holds to it."""
-    from pfeife_amd.executor import lowering, merge
+def wider_steps(mixed, channels, monkeypatch, check):
+    """Two steps' gradients against autograd in fp32; -> (N, K) of the products."""
     from pfeife_amd.mp import PartialRunner, initialize_pfeife, partial_compiler
 
-    monkeypatch.setattr(lowering, "MAX_BYTES", limit)
-    monkeypatch.setattr(merge, "MAX_BYTES", limit)
     gemm, calls = OracleKernels.gemm, []
 
     @functools.wraps(gemm)
-    def checked(self, a, b, c, **kw):
-        for rows, ld in ((kw["K"] if kw.get("a_trans") else kw["M"], kw["lda"]), (kw["K"] if kw.get("b_trans") else kw["N"], kw["ldb"])):
-            assert (rows + 256) * ld * 2 < limit
+    def seen(self, a, b, c, **kw):
+        check(kw)
         calls.append((kw["N"], kw["K"]))
         return gemm(self, a, b, c, **kw)
 
-    monkeypatch.setattr(OracleKernels, "gemm", checked)
+    monkeypatch.setattr(OracleKernels, "gemm", seen)
     torch._dynamo.reset()
     net_states._reset_state_for_tests()
     initialize_pfeife(device="cpu")
     torch.manual_seed(0)
-    model = Wider()
+    model = Wider(*channels)
     ref = copy.deepcopy(model)
-    runner = PartialRunner(PipeOption(device_cnt=2, batch_cnt=2, batch_size=2, split_points=["c2"], mixed_precision="bf16",
+    runner = PartialRunner(PipeOption(device_cnt=2, batch_cnt=2, batch_size=2, split_points=["c2"], mixed_precision=mixed,
                                       optimizer=dict(type="sgd", lr=0.0)), kernels=OracleKernels("cpu"))
     cmodel = torch.compile(model, backend=partial_compiler)
 
@@ -125,5 +119,40 @@ def test_windows_of_the_gradient_fit_an_operand(limit, one, monkeypatch):
         for i in (0, 2):
             ref(x[i:i + 2]).square().mean().backward()
         for (n, p), (_, q) in zip(model.named_parameters(), ref.named_parameters()):
-            assert (p.grad - q.grad).norm() <= 2e-2 * q.grad.norm(), n      # (as above)
+            assert (p.grad - q.grad).norm() <= (2e-2 if mixed else 1e-5) * q.grad.norm(), n      # (as above)
+    return calls
+
+
+@pytest.mark.parametrize("limit,one", [(300_000, False), (600_000, True)])
+def test_windows_of_the_gradient_fit_an_operand(limit, one, monkeypatch):
+    """More channels out than in: the forward windows may fit the size a 16-bit operand can have and the gradient's may not, which then takes the
+    product with the windows as its result.  The limit is lowered, and held to as pf_gemm holds to it."""
+    from pfeife_amd.executor import lowering, merge
+
+    monkeypatch.setattr(lowering, "MAX_BYTES", limit)
+    monkeypatch.setattr(merge, "MAX_BYTES", limit)
+
+    def check(kw):
+        for rows, ld in ((kw["K"] if kw.get("a_trans") else kw["M"], kw["lda"]), (kw["K"] if kw.get("b_trans") else kw["N"], kw["ldb"])):
+            assert (rows + 256) * ld * 2 < limit
+
+    calls = wider_steps("bf16", (16, 48), monkeypatch, check)
     assert ((16, 9 * 48) in calls) == one and ((9 * 16, 48) in calls) != one
+
+
+@pytest.mark.parametrize("mixed", [None, "bf16"])
+@pytest.mark.parametrize("channels,one", [((8, 768), True), ((8, 776), False), ((200, 776), True)])
+def test_many_channels_out_of_few_keep_the_product_of_windows(channels, one, mixed, monkeypatch):
+    c, o = channels
+    calls = wider_steps(mixed, channels, monkeypatch, lambda kw: None)
+    assert ((c, 9 * o) in calls) == one and ((9 * c, o) in calls) != one
+
+
+def test_the_form_of_the_input_gradient():
+    from pfeife_amd.executor.lowering import _windows_of_gradient as one
+
+    assert one(1 << 15, 320, 960, 4) and not one(1 << 15, 320, 968, 4)                       # three times as many at any size
+    assert one(20_000, 128, 512, 2) and not one(22_000, 128, 512, 2) and not one(22_000, 64, 512, 2)    # eight times: up to 200 MB
+    assert one(9_000, 300, 1200, 2) and not one(9_000, 299, 1200, 2) and not one(10_000, 300, 1200, 2)                        # ... above 768 of them four times
+    assert one(5_000, 8, 768, 2) and not one(6_000, 8, 768, 2)                               # others: up to 80 MB
+    assert one(100_000, 640, 640, 2) and not one(196_608, 320, 640, 2) and one(196_608, 320, 640, 4)   # 2 GiB of 16 bits
