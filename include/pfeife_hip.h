@@ -490,7 +490,8 @@ int pf_adam_step(const pf_adam_item* items_dev, int n_items, int64_t max_n, doub
                  double eps, double weight_decay, int64_t step, int adamw, void* stream);
 /* The same in one pass over memory, for a caller that also keeps, in DEVICE memory, the running count of the items'
  * chunks of PF_ADAM_CHUNK elements: chunk_ends_dev[i] = sum over k <= i of ceil(items[k].n / PF_ADAM_CHUNK), n_chunks =
- * the last of them.  scaler_state NULL: as pf_adam_step; else as pf_adam_step_scaled (`step` is not read). */
+ * the last of them.  scaler_state NULL: as pf_adam_step; else as pf_adam_step_scaled (`step` is not read).  The framework's own steps
+ * are this call; the results are the same bit for bit. */
 #define PF_ADAM_CHUNK 1024
 int pf_adam_step_chunks(const pf_adam_item* items_dev, const int64_t* chunk_ends_dev, int n_items, int64_t n_chunks,
                         double lr, double beta1, double beta2, double eps, double weight_decay, int64_t step, int adamw,
