@@ -524,10 +524,10 @@ struct AdamCoef {
 // out in turn 4.9, two chunks to a workgroup 5.7, one 6.2.  Everything is next used a step later and bypasses the caches.
 // Which item: `ends`, the chunks up to and including each item's last, is searched by each wavefront, 64 ways at a time.
 constexpr int ADAM_CHUNK = PF_ADAM_CHUNK;
-__global__ __launch_bounds__(256) void adam_chunk_kernel(const pf_adam_item* items, const int64_t* ends, int n_items, AdamCoef c,
+__global__ __launch_bounds__(256) void adam_chunk_kernel(const pf_adam_item* items, const int64_t* ends, int64_t first, int n_items, AdamCoef c,
                                                          const float* scaler_state) {
   if (!c.scaled(scaler_state)) return;
-  const int64_t chunk = blockIdx.x;
+  const int64_t chunk = first + blockIdx.x;
   const int lane = threadIdx.x & 63;
   int lo = 0, hi = n_items - 1;      // the item is one of these: the first whose end is past the chunk
   while (lo < hi) {
@@ -1116,11 +1116,15 @@ extern "C" int pf_adam_step_chunks(const pf_adam_item* items_dev, const int64_t*
                                    float* scaler_state, void* stream) {
   PF_REQUIRE(n_items >= 0 && n_chunks >= 0 && (scaler_state != nullptr || step >= 1), "pf_adam_step_chunks: bad arguments");
   if (n_items == 0 || n_chunks == 0) return PF_OK;
-  PF_REQUIRE(items_dev != nullptr && chunk_ends_dev != nullptr && n_chunks < (1ll << 24), "pf_adam_step_chunks: bad item list");
+  PF_REQUIRE(items_dev != nullptr && chunk_ends_dev != nullptr, "pf_adam_step_chunks: bad item list");
   if (scaler_state != nullptr)
     hipLaunchKernelGGL(adam_coefficients_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, scaler_state, lr, beta1, beta2);
-  hipLaunchKernelGGL(adam_chunk_kernel, dim3((unsigned)n_chunks), dim3(256), 0, (hipStream_t)stream, items_dev, chunk_ends_dev, n_items,
-                     adam_coef(lr, beta1, beta2, eps, weight_decay, scaler_state != nullptr ? 1 : step, adamw), scaler_state);
+  const AdamCoef c = adam_coef(lr, beta1, beta2, eps, weight_decay, scaler_state != nullptr ? 1 : step, adamw);
+  for (int64_t first = 0; first < n_chunks; first += EW_MAX_BLOCKS) {      // (a launch has less than 2^32 threads)
+    const int64_t blocks = n_chunks - first < EW_MAX_BLOCKS ? n_chunks - first : EW_MAX_BLOCKS;
+    hipLaunchKernelGGL(adam_chunk_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, items_dev, chunk_ends_dev, first, n_items, c,
+                       scaler_state);
+  }
   PF_CHECK_LAUNCH("pf_adam_step_chunks");
   return PF_OK;
 }
