@@ -1612,13 +1612,7 @@ def lower_sdpa(L, node):
     kern = L.kernels
     if L.mixed and hv == hd and hd % 8 == 0 and hd <= getattr(kern, "MAX_FUSED_HEAD_DIM", 0):
         return _lower_sdpa_fused(L, (q, k, v), (qt, kt, vt), (Bn, H, Tq, Tk, hd), scale, causal, req)
-    # fp32: a workgroup of the fused kernels sweeps the other side's tokens for 16 of one side, in a quarter of them one after the
-    # other.  Few of them over long sequences leave the device idle where products through memory fill it (us forward + backward, memory /
-    # fused: 1 head, 64 queries of 4096 keys, 4 workgroups: 130 / 137; 4096 of 64 at head dim 128: 58 / 281; 2 heads of 1500, 188
-    # workgroups: 125 / 110)
-    few = max(Tq, Tk) > 1024 and Bn * H * ((min(Tq, Tk) + 15) // 16) < 128
-    if (not L.mixed and hv == hd and hd % 4 == 0 and hd <= getattr(kern, "FUSED_F32_HEAD_DIM", 0) and scale > 0 and not few
-            and all(_f32_heads(t) for t in (qt, kt, vt))):
+    if not L.mixed and hd <= getattr(kern, "FUSED_F32_HEAD_DIM", 0) and _fused_f32(qt, kt, vt, scale):
         return _lower_sdpa_fused(L, (q, k, v), (qt, kt, vt), (Bn, H, Tq, Tk, hd), scale, causal, req)
     S = L.scratch("attn_s", L.cur.mb, (Bn, H, Tq, Tkp), torch.float32)
     P = L.alloc((Bn, H, Tq, Tkp), cd)
@@ -1678,9 +1672,22 @@ def lower_sdpa(L, node):
 
 
 def _f32_heads(t):
-    """Whether the fp32 attention kernels can read and write this [B, H, T, hd] tensor (16-byte accesses, tokens apart)."""
-    return (t.dtype == torch.float32 and t.numel() > 0 and t.stride(3) == 1 and t.stride(2) >= t.shape[3] and t.data_ptr() % 16 == 0
+    """Whether the fp32 attention kernels can read and write this [B, H, T, hd] tensor (16-byte accesses, tokens apart, a tile of 16 of them within
+    32-bit offsets)."""
+    return (t.dtype == torch.float32 and t.numel() > 0 and t.stride(3) == 1 and t.shape[3] <= t.stride(2) < 1 << 23 and t.data_ptr() % 16 == 0
             and all(s % 4 == 0 for s in t.stride()[:3]))
+
+
+def _fused_f32(q, k, v, scale):
+    """Whether fp32 attention of up to 128 head dims runs on the fused kernels.  A workgroup of them sweeps the other side's tokens for 16 of
+    one side, in a quarter of them one after the other.  Few of them over long sequences leave the device idle where products through memory
+    fill it (us forward + backward, memory / fused: 1 head, 64 queries of 4096 keys, 4 workgroups: 130 / 137; 4096 of 64 at head dim
+    128: 58 / 281; 2 heads of 1500, 188 workgroups: 125 / 110); a launch has 65535 of them to a head at most.  (The result's tokens
+    are H * hd apart.)"""
+    (Bn, H, Tq, hd), Tk = q.shape, k.shape[2]
+    few = max(Tq, Tk) > 1024 and Bn * H * ((min(Tq, Tk) + 15) // 16) < 128
+    return (v.shape[3] == hd and hd % 4 == 0 and scale > 0 and not few and max(Tq, Tk) <= 65535 * 16 and Bn * H < 1 << 23 and H * hd < 1 << 23
+            and all(_f32_heads(t) for t in (q, k, v)))
 
 
 def _apart(vals):
