@@ -82,10 +82,11 @@ int pf_issuer_destroy(void* issuer);
  * queues, pfeife/mp/partial/module.py:87-89, 145-159).  A baton has `slots` counts of tokens, all zero: pf_baton_switch gives one to slot `to`
  * (to < 0: none) and then takes one from slot `own` (own < 0: none), for at most timeout_us (< 0: as long as it takes): *came = 1 if it got
  * it, 0 if not (the caller goes on waiting with to = -1).  One thread at a time may wait at a slot.  pf_baton_alert wakes the thread that sleeps at
- * a slot shortly before its token comes.  A baton is not freed: threads may be waiting at it for as long as the process lives. */
+ * a slot shortly before its token comes.  pf_baton_destroy: no thread may be at it, or come to it. */
 int pf_baton_create(int slots, void** baton_out);
 int pf_baton_alert(void* baton, int slot);
 int pf_baton_switch(void* baton, int to, int own, int64_t timeout_us, int* came);
+int pf_baton_destroy(void* baton);
 /* events that order streams (no timing) */
 int pf_event_create(void** event_out);
 int pf_event_destroy(void* event);

@@ -100,3 +100,8 @@ extern "C" int pf_baton_switch(void* baton, int to, int own, int64_t timeout_us,
   *came = own < 0 || wait(b.slots[own], timeout_us) ? 1 : 0;
   return PF_OK;
 }
+
+extern "C" int pf_baton_destroy(void* baton) {
+  delete (Baton*)baton;
+  return PF_OK;
+}

@@ -105,6 +105,7 @@ _SIGNATURES = {
     "pf_baton_create": [_I, POINTER(c_void_p)],
     "pf_baton_alert": [_P, _I],
     "pf_baton_switch": [_P, _I, _I, _L, POINTER(c_int)],
+    "pf_baton_destroy": [_P],
     "pf_event_create": [POINTER(c_void_p)],
     "pf_event_destroy": [_P],
     "pf_gemm": [POINTER(GemmDesc), _P],
@@ -307,6 +308,11 @@ class Baton:
             if came.value:
                 return
             to = -1
+
+    def __del__(self):      # (a thread that is at it holds it)
+        if getattr(self, "_h", None):
+            self._lib.pf_baton_destroy(self._h)
+            self._h = None
 
 
 class HipKernels:

@@ -70,3 +70,16 @@ def test_a_dropped_runner_leaves_nothing(fail, release):
         t.join(10)
         assert not t.is_alive()
     assert threading.active_count() <= before + len(other[2])
+
+
+def test_a_dropped_runner_gives_its_baton_back(monkeypatch):
+    from pfeife_amd import hip
+
+    lib, gone = hip.load(), []
+    destroy = lib.pf_baton_destroy
+    monkeypatch.setattr(lib, "pf_baton_destroy", lambda h: (gone.append(h), destroy(h))[1])
+    threads = [runner_after_steps(False, False)[2] for _ in range(3)]
+    gc.collect()
+    for t in threads[0] + threads[1]:
+        t.join(10)
+    assert len(set(gone)) >= 2        # (the last runner still is the compiled models')
