@@ -352,8 +352,9 @@ typedef struct pf_attn_desc {
 int pf_attention_fwd(const pf_attn_desc* desc, void* stream);
 int pf_attention_bwd(const pf_attn_desc* desc, void* stream);
 /* The same in fp32 (dtype PF_F32): head dim a multiple of 4 and at most 128, strides multiples of 4 elements with tokens hd or
- * more apart, operands 16-byte aligned, scale > 0.  `lse` has 2 Tq values per head: the rows' maxima of the raw scores, then the
- * reciprocals of the sums of exp((s - max) * scale).  `o_lo` is not used. */
+ * more apart, operands 16-byte aligned, scale > 0.  `lse` has 2 Tq values per head, with x = s * scale * log2(e) of a raw score s: for each row
+ * a reference exponent R near its largest x, but not at it (a whole number unless the scores are huge; it follows the maximum in steps), then
+ * 1 / sum(exp2(x - R)).  The row's log-sum-exp is R * ln 2 - ln of the second.  `o_lo` is not used. */
 int pf_attention_f32_fwd(const pf_attn_desc* desc, void* stream);
 int pf_attention_f32_bwd(const pf_attn_desc* desc, void* stream);
 
