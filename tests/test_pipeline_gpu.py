@@ -2,7 +2,7 @@
 against the CPU oracle of the reference's stage execution (oracle/stage_oracle.py)
 on identical seeded inputs and weights.
 
-Tolerances (from the task's north star): micro-batch split bit-exact; loss within
+Tolerances: micro-batch split bit-exact; loss within
 1e-5 relative in fp32 and 2e-2 relative in bf16/fp16; gradients: fp32
 max|d| <= 1e-4 * max|g| per tensor, 16-bit relative L2 <= 2e-2 per tensor
 (fp32 accumulation of 16-bit products on both sides)."""
