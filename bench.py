@@ -266,7 +266,7 @@ def hbm_kernel_rates(runner, reps=3):
         ms = timed(lambda: w._fused_adam_step(opt, scaled=w.dyn_scale))
         nb = 28.0 * n_par   # read p, g, m, v; write p, m, v (fp32)
         gbs = nb / (ms * 1e-3) / 1e9
-        out.append(dict(kernel="pf_adam_step", on_path=True, launches_per_step=len(opt.param_groups),
+        out.append(dict(kernel="pf_adam_step_chunks", on_path=True, launches_per_step=len(opt.param_groups),
                         ms_per_step=round(ms, 3), avg_launch_us=round(1e3 * ms / len(opt.param_groups), 2),
                         bytes_per_launch=round(nb / len(opt.param_groups)), achieved=round(gbs, 1), peak=PEAK_HBM_GBS,
                         unit="GB/s", frac=round(gbs / PEAK_HBM_GBS, 4)))
